@@ -8,8 +8,6 @@ CalibComputeInt8ToFp32; registered as `calib` with aliases `fp32_to_int8` and
 as (pointer, element count); the work is done by the HIP kernels behind
 pl_calib_fp32_to_int8 / pl_calib_int8_to_fp32.
 """
-import ctypes as C
-
 from . import capi
 
 
@@ -36,11 +34,12 @@ class _CalibCompute(object):
 
     def Run(self, stream=0):
         p = self.param
-        n = int(p.input.numel())
-        if int(p.output.numel()) != n:
+        n = p.input.numel()
+        if p.output.numel() != n:
             raise ValueError("calib: Out must have the shape of Input")
-        fn = getattr(capi.lib(), self._entry)
-        capi.check(fn(C.c_void_p(p.input.data_ptr()), C.c_void_p(p.output.data_ptr()), n, C.c_float(p.scale), C.c_void_p(stream)))
+        rc = getattr(capi.lib(), self._entry)(p.input.data_ptr(), p.output.data_ptr(), n, p.scale, stream)
+        if rc < 0:
+            capi.check(rc)
 
     Launch = Run
 

@@ -207,6 +207,22 @@ def lib():
     return L
 
 
+_raw_stream = None
+
+
+def current_stream(device):
+    """Raw handle of torch's current stream on `device` (a torch device of type cuda).
+
+    torch.cuda.current_stream() builds a Stream object on every call (1.9 us of the 8.6 us that a small layer's
+    Run took on the host); the call behind it that returns the handle alone takes 0.14 us."""
+    global _raw_stream
+    if _raw_stream is None:
+        import torch
+
+        _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda index: torch.cuda.current_stream(index).cuda_stream)
+    return _raw_stream(device.index)
+
+
 def last_error():
     return lib().pl_last_error().decode("utf-8", "replace")
 

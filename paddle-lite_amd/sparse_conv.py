@@ -161,6 +161,7 @@ class SparseConvKernel(object):
         self.tuning = tuning  # capi.Tuning or None (every rule of the library applies)
         self.reference_quirks = reference_quirks
         self._handle = None
+        self._bound = None  # what Run looks up once (_bind)
         self._first_epoch = True
         self.w_scale_ = []
         self.bias_ = None
@@ -234,6 +235,7 @@ class SparseConvKernel(object):
         capi.check(capi.lib().pl_sparse_conv_prepare(C.byref(d), C.byref(h)))
         self._release()
         self._handle = h
+        self._bound = None
         self._first_epoch = False
 
     # -- KernelBase::Launch
@@ -243,29 +245,40 @@ class SparseConvKernel(object):
         return self.Run(x, out, stream)
 
     # -- SparseConvCompute::Run; x and out are CUDA-device torch tensors
+    # A small layer runs for 4 us on the device and the C entry point takes 3.1 - 4.1 us of host time, so what
+    # surrounds it counts: tensor types, channel counts and the entry point are looked up once per handle (_bind),
+    # the stream comes as a raw handle (capi.current_stream).  Host time of a call: 8.6 -> 6.3 us, with `out`
+    # 7.2 -> 5.1 (of which the entry point 3.1 before and, on a slower machine, 4.1 after).
     def Run(self, x, out=None, stream=None):
-        import torch
-
         if self._handle is None:
             raise RuntimeError("PrepareForRun has not been called")
+        in_dtype, out_dtype, ic, oc, empty, run = self._bound or self._bind()
         if not x.is_cuda or not x.is_contiguous():
             raise ValueError("x must be a contiguous device tensor")
-        want_in = {capi.KIND_FP32: torch.float32, capi.KIND_FP16: torch.float16}.get(self.kind, torch.int8)
-        if x.dtype != want_in or x.dim() != 4 or x.shape[1] != self.param.weights.ic:
-            raise ValueError("x must be %s NCHW with %d channels" % (want_in, self.param.weights.ic))
-        n, _, hh, ww = x.shape
-        odt = {capi.KIND_FP32: torch.float32, capi.KIND_INT8_FP32: torch.float32, capi.KIND_INT8_INT8: torch.int8, capi.KIND_INT8_ACC32: torch.int32, capi.KIND_FP16: torch.float16}[self.kind]
+        shape = x.shape
+        if x.dtype != in_dtype or len(shape) != 4 or shape[1] != ic:
+            raise ValueError("x must be %s NCHW with %d channels" % (in_dtype, ic))
+        n, _, hh, ww = shape
         # output shape as SparseConvOp::InferShapeImpl for 1x1 / stride 1 / pad 0
         # (reference: lite/operators/sparse_conv_op.cc:46-65)
-        shape = (n, self.param.weights.oc, hh, ww)
+        shape = (n, oc, hh, ww)
+        device = x.device
         if out is None:
-            out = torch.empty(shape, dtype=odt, device=x.device)
-        elif tuple(out.shape) != shape or out.dtype != odt or not out.is_contiguous() or out.device != x.device:
-            raise ValueError("out must be a contiguous %s tensor of shape %s on %s" % (odt, shape, x.device))
-        if stream is None:
-            stream = torch.cuda.current_stream(x.device).cuda_stream
-        capi.check(capi.lib().pl_sparse_conv_run(self._handle, x.data_ptr(), out.data_ptr(), n, hh * ww, C.c_void_p(stream)))
+            out = empty(shape, dtype=out_dtype, device=device)
+        elif out.shape != shape or out.dtype != out_dtype or not out.is_contiguous() or out.device != device:
+            raise ValueError("out must be a contiguous %s tensor of shape %s on %s" % (out_dtype, shape, device))
+        rc = run(self._handle, x.data_ptr(), out.data_ptr(), n, hh * ww, capi.current_stream(device) if stream is None else stream)
+        if rc < 0:
+            capi.check(rc)
         return out
+
+    def _bind(self):
+        import torch
+
+        in_dtype = {capi.KIND_FP32: torch.float32, capi.KIND_FP16: torch.float16}.get(self.kind, torch.int8)
+        out_dtype = {capi.KIND_FP32: torch.float32, capi.KIND_INT8_FP32: torch.float32, capi.KIND_INT8_INT8: torch.int8, capi.KIND_INT8_ACC32: torch.int32, capi.KIND_FP16: torch.float16}[self.kind]
+        self._bound = (in_dtype, out_dtype, self.param.weights.ic, self.param.weights.oc, torch.empty, capi.lib().pl_sparse_conv_run)
+        return self._bound
 
     def info(self):
         i = capi.Info()
