@@ -84,7 +84,10 @@ enum {
  * chooses per call by batch and H*W (the image kernels where the whole map
  * fits, or in slabs while batch * slabs * oc / 128 is at most half the CU
  * count; else the row walk for at most 256 positions in all;
- * else the block kernel): see pl_sparse_conv_algo_for(). */
+ * else the block kernel): see pl_sparse_conv_algo_for().  Calls with many
+ * channels or few positions among them run as dense 16x64 weight tiles with
+ * the channels taken chunk by chunk, whichever of the three that names; so
+ * do such calls of a handle prepared for PL_ALGO_BLOCK_MFMA. */
 enum { PL_ALGO_AUTO = 0, PL_ALGO_ROW_WALK = 1, PL_ALGO_BLOCK_MFMA = 2, PL_ALGO_IMAGE_MFMA = 3 };
 
 /* Activation constants, used as given (replaces the fields of

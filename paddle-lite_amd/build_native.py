@@ -38,6 +38,7 @@ SOURCES = [
     ("tile_walk_kernels.hip", "tile_walk_kernels.o", []),
     ("fp16_walk_kernels.hip", "fp16_walk_kernels.o", []),
     ("dwconv_kernels.hip", "dwconv_kernels.o", []),
+    ("chunk_mfma_kernels.hip", "chunk_mfma_kernels.o", []),
     ("image_mfma_kernels.hip", "image_mfma_kernels.o", []),
     ("image_tr_kernels.hip", "image_tr_kernels.o", []),
     ("image_rows_kernels.hip", "image_rows_kernels.o", []),

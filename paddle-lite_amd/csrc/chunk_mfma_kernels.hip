@@ -1,0 +1,336 @@
+// Chunk MFMA: int8 sparse 1x1 convolution as a dense product on the matrix cores that takes the input channels chunk
+// by chunk, for layers with many channels and for calls of few positions.
+//
+// One workgroup of eight wavefronts makes a tile of 128 output rows x up to 64 NW positions; wavefront w multiplies
+// one tile of 16 rows with all of them.  Per chunk of 512 / NW channels a thread loads, for 16 consecutive channels,
+// the dword (four positions) of one position quad, turns the 16 x 4 bytes into four 16-byte operand cells (16
+// channels of one position) with two stages of byte permutes and writes them to one of two 32 KB LDS buffers.  The
+// accumulators stay in registers over all chunks.  While a chunk is multiplied (v_mfma_i32_16x16x64_i8) the next one
+// is written to the other buffer, a quarter behind each of the first multiplies, and the loads of the one three
+// ahead are issued; the weights (dense tiles in operand order, straight into registers: every wavefront needs its own
+// rows only) are requested one chunk ahead.  One barrier per chunk.
+//
+// What bounds it: the operand reads from LDS.  Every wavefront reads the whole chunk (32 KB at 128 bytes per clock and
+// CU: 2048 clocks for the eight of them, and about 500 for the writes), while the chunk's 256 matrix instructions take
+// 1024 clocks of each SIMD.  A chunk takes 2500 - 3300 clocks with everything in L2; a workgroup whose wavefronts own
+// two or four row tiles and split the channels halves the reads but was no faster on a full chip (25.4 us on
+// 2048 -> 2048 @14x14 x 16 against 24.6: there L2, which serves 170 - 220 MB per launch, limits both).
+// 31.4 -> 24.6 us on that layer (128-position tiles of the block kernel, one 8-step chunk at a time, before), 512 -> 512
+// @14x14 on one image 6.4 -> 4.2, 2048 -> 512 @7x7 on 16 images 28.7 -> 10.9.
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+#include <type_traits>
+
+#include "epilogue.h"
+#include "launch_lds.h"
+#include "sparse_conv_kernels.h"
+
+namespace pl {
+namespace {
+
+using epilogue::ActivateT;
+using epilogue::ActQuantF;
+using epilogue::DispatchAct;
+using epilogue::TruncPackI8x4;
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+
+constexpr int kBufCells = 2048;  // 16-byte cells of one chunk: (channel group of 16, position of the tile)
+
+template <int NW, int OUT>
+__device__ __forceinline__ void ChunkBody(const ChunkMfmaParams& p, uint4* xt) {
+  constexpr int QT = 16 * NW;    // position quads a tile has room for
+  constexpr int NG = 512 / QT;   // channel groups of a chunk
+  constexpr int KS = NG / 4;     // 64-channel steps of a chunk
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // each XCD owns a contiguous range of tiles, the row groups of one tile follow each other there
+  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+  const int first_tile = (xcd * p.tiles) >> 3, last_tile = ((xcd + 1) * p.tiles) >> 3;
+  const int tile = first_tile + slot / p.row_groups, rg = slot % p.row_groups;
+  if (tile >= last_tile) return;
+
+  // the thread's part of a chunk: quad j, channel group kgl; a partial quad (the end of an image whose size is not
+  // a multiple of 4) is read from the last four positions of its channel row and shifted, threads behind the tile's or
+  // the tensor's last quad repeat that one
+  const int j = tid & (QT - 1), kgl = tid / QT;
+  const uint32_t tile_quad0 = (uint32_t)tile * (uint32_t)p.tile_quads;
+  const uint32_t quad = min(tile_quad0 + (uint32_t)min(j, p.tile_quads - 1), p.total_quads - 1u);
+  const uint32_t img = quad / (uint32_t)p.qpi;
+  const int pp = 4 * (int)(quad - img * (uint32_t)p.qpi);
+  const int first = min(pp, p.hw - 4), shift = 8 * (pp - first);
+  const uint32_t vbase = img * (uint32_t)p.K * (uint32_t)p.hw + (uint32_t)first;
+  uint32_t r[2][16];
+  // loads [4 piece, 4 piece + 4) of the thread's 16 of a chunk
+  auto issue = [&](uint32_t (&rd)[16], int chunk, int piece) {
+    // the last group of a channel count that is no multiple of 16 holds the last 16 channels; groups behind it repeat
+    // it against weights of zero
+    const uint32_t voff = vbase + (uint32_t)(min(chunk * 16 * NG + 16 * kgl, p.K - 16) * p.hw);
+    const int8_t* base = p.x + (size_t)(4 * piece) * p.hw;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      rd[4 * piece + i] = *reinterpret_cast<const uint32_t*>(base + voff);
+      base += p.hw;
+    }
+  };
+  auto issue_all = [&](uint32_t (&rd)[16], int chunk) {
+#pragma unroll
+    for (int piece = 0; piece < 4; ++piece) issue(rd, chunk, piece);
+  };
+  // Two stages of byte permutes, in four pieces: bytes of neighbouring channels paired up for positions 0 and 1, their
+  // cells made and written, then the same for positions 2 and 3.
+  uint4* const cells = xt + kgl * (4 * QT) + j;
+  uint32_t pair[4][2];
+  auto commit = [&](uint32_t (&rd)[16], int buf, int piece) {
+    if (piece == 0 && !p.quad_aligned) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) rd[i] >>= shift;
+    }
+    if ((piece & 1) == 0) {
+      const uint32_t sel = piece == 0 ? 0x05010400u : 0x07030602u;
+#pragma unroll
+      for (int b4 = 0; b4 < 4; ++b4) {
+        pair[b4][0] = __builtin_amdgcn_perm(rd[4 * b4 + 1], rd[4 * b4], sel);
+        pair[b4][1] = __builtin_amdgcn_perm(rd[4 * b4 + 3], rd[4 * b4 + 2], sel);
+      }
+    } else {
+      uint4* dst = cells + buf * kBufCells;
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const uint32_t sel = c ? 0x07060302u : 0x05040100u;
+        dst[(piece - 1 + c) * QT] = make_uint4(__builtin_amdgcn_perm(pair[0][1], pair[0][0], sel), __builtin_amdgcn_perm(pair[1][1], pair[1][0], sel),
+                                               __builtin_amdgcn_perm(pair[2][1], pair[2][0], sel), __builtin_amdgcn_perm(pair[3][1], pair[3][0], sel));
+      }
+    }
+  };
+  auto commit_all = [&](uint32_t (&rd)[16], int buf) {
+#pragma unroll
+    for (int piece = 0; piece < 4; ++piece) commit(rd, buf, piece);
+  };
+
+  // the wavefront's row tile (past the last one: the last one again, not stored)
+  const int rt = rg * 8 + wave;
+  const v4i* const wt = static_cast<const v4i*>(p.wtiles) + (size_t)min(rt, p.row_tiles - 1) * p.padded_ksteps * 64 + lane;
+  v4i a[KS];
+  auto load_weights = [&](int chunk, int ks) { a[ks] = wt[(chunk * KS + ks) * 64]; };
+  const int n = lane & 15, kq = lane >> 4;
+  const uint4* const operand = xt + kq * (4 * QT) + n;
+  v4i acc[NW][4];
+#pragma unroll
+  for (int w = 0; w < NW; ++w)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[w][c] = v4i{0, 0, 0, 0};
+
+  // One chunk: eight (step, window of 16 quads) pairs of four multiplies.  The operand cells are read from LDS PF cells
+  // ahead.  Behind the first four pairs the next chunk's activations go to the other buffer, so that the vector ALU
+  // and the LDS writes work while the matrix cores do; behind the last four the loads of the chunk three ahead are
+  // issued into the registers this frees.  The weights of a step are requested for the next chunk as soon as the
+  // step has used their registers.  AHEAD: 1 there are such chunks, 0 there are none, 2 maybe; a condition around
+  // loads makes the wait for older ones wait for these too, hence only near the end.
+  constexpr int PF = 8;
+  auto run_chunk = [&](auto ahead_c, int chunk, uint32_t (&rn)[16]) {
+    constexpr int AHEAD = decltype(ahead_c)::value;
+    const uint4* const cells_in = operand + (chunk & 1) * kBufCells;
+    uint4 b[PF + 1];
+    auto read = [&](int v) {
+      const int u = v >> 2, c = v & 3;
+      b[v % (PF + 1)] = cells_in[(u / NW) * 4 * (4 * QT) + c * QT + 16 * (u % NW)];
+    };
+#pragma unroll
+    for (int d = 0; d < PF; ++d) read(d);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int ks = u / NW, w = u % NW;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int v = 4 * u + c;
+        if (v + PF < 32) read(v + PF);
+        __builtin_amdgcn_sched_barrier(0);  // the reads stay ahead of the multiply
+        const uint4 q = b[v % (PF + 1)];
+        acc[w][c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[ks], v4i{(int)q.x, (int)q.y, (int)q.z, (int)q.w}, acc[w][c], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (w == NW - 1 && (AHEAD == 1 || chunk + 1 < p.chunks)) load_weights(chunk + 1, ks);
+      if (u < 4) {
+        if (AHEAD == 1 || chunk + 1 < p.chunks) commit(rn, (chunk + 1) & 1, u);
+      } else if (AHEAD == 1 || (AHEAD == 2 && chunk + 3 < p.chunks)) {
+        issue(rn, chunk + 3, u - 4);
+      }
+    }
+    __syncthreads();
+  };
+  issue_all(r[0], 0);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) load_weights(0, ks);
+  __builtin_amdgcn_sched_barrier(0);
+  if (p.chunks >= 3) {
+    issue_all(r[1], 1);
+    __builtin_amdgcn_sched_barrier(0);
+    commit_all(r[0], 0);
+    issue_all(r[0], 2);
+  } else {
+    if (p.chunks == 2) issue_all(r[1], 1);
+    commit_all(r[0], 0);
+  }
+  __syncthreads();
+  using Always = std::integral_constant<int, 1>;
+  using Maybe = std::integral_constant<int, 2>;
+  using Never = std::integral_constant<int, 0>;
+  int chunk = 0;
+  for (; chunk + 5 <= p.chunks; chunk += 2) {
+    run_chunk(Always(), chunk, r[1]);
+    run_chunk(Always(), chunk + 1, r[0]);
+  }
+  // one to four chunks are left
+  run_chunk(Maybe(), chunk, r[1]);
+  if (chunk + 1 < p.chunks) {
+    run_chunk(Maybe(), chunk + 1, r[0]);
+    if (chunk + 2 < p.chunks) {
+      run_chunk(Never(), chunk + 2, r[1]);
+      if (chunk + 3 < p.chunks) run_chunk(Never(), chunk + 3, r[0]);
+    }
+  }
+
+  // epilogue: lane (n, kq) holds rows 4 kq .. 4 kq + 3 of the row tile at the four positions of quad 16 w + n
+  const int row0 = rt * 16 + 4 * kq;
+  if (row0 >= p.M) return;
+  float sc[4], bi[4];
+  if (OUT != kOutAcc32) {
+    // arrays are padded to a multiple of 32 rows
+    const float4 s4 = *reinterpret_cast<const float4*>(p.scale + row0), b4 = *reinterpret_cast<const float4*>(p.bias + row0);
+    sc[0] = s4.x, sc[1] = s4.y, sc[2] = s4.z, sc[3] = s4.w;
+    bi[0] = b4.x, bi[1] = b4.y, bi[2] = b4.z, bi[3] = b4.w;
+  }
+  constexpr uint32_t kElem = OUT == kOutI8 ? 1u : 4u;
+  // output rows that start on 64-byte boundaries are stored as streaming data; others share sectors with their
+  // neighbours, which merge in L2 only if stored plainly (384 -> 384 @28x28 x 16, fp32: 9.2 against 12.2 us;
+  // 192 -> 384 @17x17 x 64: 16.2 against 13.4)
+  const bool stream = OUT != kOutI8 && (p.hw & 15) == 0;
+  DispatchAct(OUT == kOutAcc32 ? 0 : epilogue::LeakyAsMax(p.act), [&](auto act_c) {
+    constexpr int ACT = decltype(act_c)::value;
+    char* dst[NW];
+    int valid[NW];
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const uint32_t q = tile_quad0 + 16u * w + (uint32_t)n;
+      const uint32_t on = q / (uint32_t)p.qpi;
+      const int opp = 4 * (int)(q - on * (uint32_t)p.qpi);
+      valid[w] = 16 * w + n >= p.tile_quads || q >= p.total_quads ? 0 : min(4, p.hw - opp);
+      dst[w] = static_cast<char*>(p.out) + (((size_t)on * p.M + row0) * p.hw + opp) * kElem;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        if (row0 + i < p.M) {
+          u4 v;
+          if (OUT == kOutAcc32) {
+            v = u4{(uint32_t)acc[w][0][i], (uint32_t)acc[w][1][i], (uint32_t)acc[w][2][i], (uint32_t)acc[w][3][i]};
+          } else {
+            float f[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) f[c] = __builtin_fmaf((float)acc[w][c][i], sc[i], bi[i]);
+            if (OUT == kOutI8) {
+              v = u4{TruncPackI8x4(ActQuantF<ACT>(f[0], p.act), ActQuantF<ACT>(f[1], p.act), ActQuantF<ACT>(f[2], p.act), ActQuantF<ACT>(f[3], p.act)), 0u, 0u, 0u};
+            } else {
+#pragma unroll
+              for (int c = 0; c < 4; ++c) f[c] = ActivateT<ACT>(f[c], p.act);
+              v = u4{__float_as_uint(f[0]), __float_as_uint(f[1]), __float_as_uint(f[2]), __float_as_uint(f[3])};
+            }
+          }
+          if (valid[w] == 4) {
+            if (OUT == kOutI8) {
+              *reinterpret_cast<uint32_t*>(dst[w]) = v.x;
+            } else if (stream) {
+              __builtin_nontemporal_store(v, reinterpret_cast<u4*>(dst[w]));
+            } else {
+              *reinterpret_cast<u4*>(dst[w]) = v;
+            }
+          } else {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+              if (c < valid[w]) {
+                if (OUT == kOutI8) {
+                  reinterpret_cast<int8_t*>(dst[w])[c] = static_cast<int8_t>(v.x >> (8 * c));
+                } else {
+                  reinterpret_cast<uint32_t*>(dst[w])[c] = v[c];
+                }
+              }
+            }
+          }
+        }
+        dst[w] += (size_t)p.hw * kElem;
+      }
+    }
+  });
+}
+
+template <int NW, int OUT>
+__global__ void __launch_bounds__(512, 2) ChunkMfmaKernel(const ChunkMfmaParams p) {
+  extern __shared__ uint4 xt[];
+  ChunkBody<NW, OUT>(p, xt);
+}
+
+template <int OUT>
+hipError_t Launch(int nw, const ChunkMfmaParams& p, dim3 grid, hipStream_t s) {
+  const dim3 block(512);
+  const size_t lds = 2 * kBufCells * 16;
+  if (nw == 4) return LaunchWithLds(ChunkMfmaKernel<4, OUT>, grid, block, lds, s, p);
+  if (nw == 2) return LaunchWithLds(ChunkMfmaKernel<2, OUT>, grid, block, lds, s, p);
+  return LaunchWithLds(ChunkMfmaKernel<1, OUT>, grid, block, lds, s, p);
+}
+
+}  // namespace
+
+int ChunkMfmaPaddedSteps(int K) { return (K + 511) / 512 * 8; }
+bool ChunkMfmaFits(int K, int hw) { return K >= 16 && hw >= 4; }
+
+hipError_t LaunchChunkMfma(int out_kind, int cus, const ChunkMfmaParams& p, hipStream_t stream) {
+  if (p.batch <= 0 || p.M <= 0) return hipSuccess;
+  if (!ChunkMfmaFits(p.K, p.hw)) return hipErrorInvalidValue;
+  const int64_t positions = (int64_t)p.batch * p.hw;
+  // tensor offsets are kept in 32 bits
+  if (positions * p.K >= (1ll << 31) || positions >= (1ll << 31) - 512) return hipErrorInvalidValue;
+  ChunkMfmaParams q = p;
+  q.qpi = (p.hw + 3) / 4;
+  q.quad_aligned = p.hw % 4 == 0;
+  q.total_quads = (uint32_t)p.batch * (uint32_t)q.qpi;
+  q.row_tiles = (p.M + 15) / 16;
+  q.ksteps = (p.K + 63) / 64;
+  q.padded_ksteps = ChunkMfmaPaddedSteps(p.K);
+  q.row_groups = (q.row_tiles + 7) / 8;
+  // whole images per tile where they fit: their channel rows lie back to back, so no line is fetched in parts
+  auto tile_quads = [&](int nw) { return q.qpi <= 16 * nw ? 16 * nw / q.qpi * q.qpi : 16 * nw; };
+  auto tiles = [&](int nw) { return (int)((q.total_quads + tile_quads(nw) - 1) / tile_quads(nw)); };
+  // The tile width: a CU holds one workgroup, a workgroup takes about 3 us and 1.35 us per chunk, so the fewest rounds
+  // times that, rounds being what the XCD with the most workgroups needs.  2048 -> 2048 @14x14 x 16: 256 positions 24.6 us
+  // (one round of 16 chunks), 128 36.6 (two of 8), 64 44.7 (four of 4); 1024 -> 256 @14x14 x 32: 14.6, 12.7 and 9.9 (one
+  // round each); 608 -> 736 @9x8 x 42: 11.4 (one round), 13.2 and 12.9 (two).
+  int nw = 1;
+  int64_t best = 0;
+  for (int w : {1, 2, 4}) {
+    const int64_t rounds = ((int64_t)((tiles(w) + 7) / 8) * q.row_groups * 8 + cus - 1) / cus;
+    const int64_t cost = rounds * (300 + 135 * ((q.ksteps + 8 / w - 1) / (8 / w)));
+    if (w == 1 || cost < best) best = cost, nw = w;
+  }
+  q.tile_quads = tile_quads(nw);
+  q.tiles = tiles(nw);
+  q.chunks = (q.ksteps + 8 / nw - 1) / (8 / nw);
+  const int64_t wgs = 8ll * q.row_groups * ((q.tiles + 7) / 8);
+  if (wgs > (1ll << 30)) return hipErrorInvalidValue;
+  const dim3 grid((uint32_t)wgs);
+  switch (out_kind) {
+    case kOutF32:
+      return Launch<kOutF32>(nw, q, grid, stream);
+    case kOutI8:
+      return Launch<kOutI8>(nw, q, grid, stream);
+    case kOutAcc32:
+      return Launch<kOutAcc32>(nw, q, grid, stream);
+    default:
+      return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace pl

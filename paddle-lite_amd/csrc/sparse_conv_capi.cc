@@ -180,6 +180,7 @@ struct pl_sparse_conv_handle {
   DevBuf wblocks, kmask;
   int wg_slots = 512;       // workgroups resident at once (2 per CU)
   int wg_slots_default = 512;  // the same before any override: twice the device's CU count
+  DevBuf wchunk;            // dense 16x64 tiles of the kernel that takes the channels chunk by chunk
   int mfma_stream = 1;      // streaming block MFMA: 0 never, 1 when the shape suits it, 2 whenever the shape allows
   int mfma_i8_wide = 1;
   int mfma_tile_quads = 0;  // 0 = chosen per problem
@@ -202,7 +203,7 @@ struct pl_sparse_conv_handle {
   int padded_rows = 0;
 
   int64_t DeviceBytes() const {
-    return static_cast<int64_t>(groups.bytes + kidx.bytes + wts.bytes + cw_desc.bytes + cw_idx.bytes + cw_wts.bytes + hw_kidx.bytes + hw_wts.bytes + hw_bias.bytes + wblocks.bytes + kmask.bytes + wtiles.bytes + wtiles_rg.bytes + wtiles_tr.bytes + wtiles_rows.bytes + tw.DeviceBytes() + tw_narrow.DeviceBytes() + scale.bytes + bias.bytes);
+    return static_cast<int64_t>(groups.bytes + kidx.bytes + wts.bytes + cw_desc.bytes + cw_idx.bytes + cw_wts.bytes + hw_kidx.bytes + hw_wts.bytes + hw_bias.bytes + wblocks.bytes + kmask.bytes + wchunk.bytes + wtiles.bytes + wtiles_rg.bytes + wtiles_tr.bytes + wtiles_rows.bytes + tw.DeviceBytes() + tw_narrow.DeviceBytes() + scale.bytes + bias.bytes);
   }
 };
 
@@ -577,6 +578,28 @@ int BuildBlockMfma(const pl::DecodedLayout& L, pl_sparse_conv_handle* h) {
   return PL_OK;
 }
 
+// Dense 16x64 tiles of consecutive rows for the kernel that takes the channels chunk by chunk
+// (ChunkMfmaParams::wtiles).
+int BuildChunkMfma(const pl::DecodedLayout& L, pl_sparse_conv_handle* h) {
+  const int row_tiles = CeilDiv(L.oc, 16), kss = pl::ChunkMfmaPaddedSteps(L.ic);
+  std::vector<int8_t> tiles(static_cast<size_t>(row_tiles) * kss * 1024, 0);
+  const uint32_t whole = static_cast<uint32_t>(L.ic) / 16u * 16u;  // channels in whole groups of 16
+  auto put = [&](int row, uint32_t c, uint32_t wbits) {
+    const uint32_t t = c < whole ? c & 15u : 16u - (static_cast<uint32_t>(L.ic) - c);
+    const uint32_t lane = (static_cast<uint32_t>(row) & 15u) + 16u * ((c >> 4) & 3u);
+    tiles[((static_cast<size_t>(row >> 4) * kss + (c >> 6)) * 64 + lane) * 16 + t] = static_cast<int8_t>(wbits & 0xffu);
+  };
+  for (const pl::RowGroup& g : L.groups) {
+    for (uint32_t j = 0; j < g.count; ++j) {
+      put(g.row0, L.ic_index[g.first + j], L.w0[g.first + j]);
+      if (g.nrows == 2) put(g.row0 + 1, L.ic_index[g.first + j], L.w1[g.first + j]);
+    }
+  }
+  const hipError_t e = h->wchunk.Upload(tiles.data(), tiles.size());
+  if (e != hipSuccess) return FailHip(e, "uploading the weight tiles");
+  return PL_OK;
+}
+
 // Device-side form for the image MFMA path: the weight matrix as dense 16x64
 // int8 tiles in matrix-core operand order.  The 16 rows of a tile are four
 // apart (rho, rho + 4, ...): they all start at the same offset inside a
@@ -771,6 +794,45 @@ int AlgoForCall(const pl_sparse_conv_handle* h, int batch, int im_size, bool ali
   return h->algo;
 }
 
+// Whether the kernel that takes the channels chunk by chunk (chunk_mfma_kernels.hip) runs a call that AlgoForCall gives
+// to `call_algo`.  It spreads a call over the chip in workgroups of 128 rows x 64 - 256 positions, pays one short load -
+// multiply chain per 512 channels and does not care about the map's alignment.  Measured at 85 % zeros with fp32
+// output (us, it against what ran before):
+//  * more than 512 channels: 512 rows of 2048 channels on 7 x 7 maps 10.0 / 10.9 / 13.5 against 21.3 / 28.7 / 27.6 at
+//    1 / 16 / 64 images, 768 -> 768 @12x12 7.8 against 19.8 at 16, 2048 -> 2048 @14x14 24.7 against 31.5 at 16; level with
+//    the block kernel on 1024 -> 256 @14x14 at 64 (14.5 / 13.6, int8 output 12.8 / 13.4);
+//  * maps that are no multiple of four positions, which the block kernel loads with clamped addresses, up to two of its
+//    tiles per CU: 192 -> 384 @17x17 5.7 against 8.4 at 8 images, 13.4 against 14.7 at 64; 146 -> 231 @35x35 20.9 against 17.5
+//    at 36 (690 tiles); with at most 128 channels up to half a tile per CU: 96 -> 128 @13x11 5.6 against 8.3 at 23; 99 -> 143
+//    @27x24 10.4 against 6.4 at 32 (324 tiles);
+//  * channel counts that are no multiple of 16, likewise clamped there, up to a tile for every fourth CU: 117 -> 91 @8x8 4.1
+//    against 7.2 at 9; 125 -> 227 @18x18 6.2 against 5.2 at 17 (88 tiles);
+//  * up to 512 channels otherwise only where the block kernel has a tile for less than half the CUs: 512 -> 128
+//    @28x28 5.6 against 7.3 at 8 images but 10.8 against 8.2 at 32, 384 -> 96 @14x14 5.3 against 7.6 at 16, 256 -> 64
+//    @56x56 4.4 against 4.6 at 1 but 10.0 against 6.3 at 16;
+//  * calls of at most 256 positions, in place of the row walk, from 8192 weights on: 96 -> 576 @14x14 4.2 against 5.2, 160 ->
+//    960 @7x7 4.8 against 11.3, 288 -> 32 @8x8 3.7 against 3.8; the walk is ahead on 160 -> 32 @8x8 x 2, 3.2 against 3.7;
+//  * in place of the image kernels while those have work items for less than three CUs of eight: 512 -> 512 @14x14 4.2 /
+//    5.4 / 6.2 / 10.5 against 6.4 / 6.5 / 6.9 / 7.3 at 1 / 4 / 16 / 32 images, 1024 -> 1024 @7x7 6.9 / 7.6 against 7.9 / 8.9 at
+//    1 / 16; with 256 channels only up to eight items: 256 -> 512 @14x14 4.2 / 5.2 against 4.6 / 4.7 at 1 / 4.
+bool ChunkMfmaPays(const pl_sparse_conv_handle* h, int call_algo, int batch, int im_size) {
+  const int64_t positions = static_cast<int64_t>(batch) * im_size;
+  if (!h->wchunk.ptr || !pl::ChunkMfmaFits(h->ic, im_size) || positions * h->ic >= (1ll << 31)) return false;
+  const int cus = std::max(1, h->wg_slots_default / 2);
+  if (call_algo == PL_ALGO_ROW_WALK) return h->auto_int8 && h->oc * h->ic > 8192;
+  if (call_algo == PL_ALGO_IMAGE_MFMA) {
+    if (!h->auto_int8 || h->image_kernel != 0 || h->ic < 256) return false;
+    const int64_t images = im_size == 49 ? (batch + 1) / 2 : static_cast<int64_t>(batch) * (im_size > 256 ? im_size / 196 : 1);
+    const int64_t items = images * (h->oc / 128);
+    return h->ic < 512 ? items <= 8 : items * 8 < 3 * cus;
+  }
+  if (h->mfma_tile_quads != 0 || h->mfma_sub_tiles != 1 || h->mfma_stream != 1) return false;  // the block kernel in a form asked for
+  if (h->ic > 512 || positions <= 256) return true;
+  const int64_t block_tiles = (positions + 127) / 128 * CeilDiv(h->oc, 128);
+  if (h->ic <= 128) return im_size % 4 != 0 ? block_tiles * 2 <= cus : h->ic % 16 != 0 && block_tiles * 4 <= cus;
+  return block_tiles <= (im_size % 4 != 0 ? 2 * cus : cus / 2);
+}
+
 }  // namespace
 
 extern "C" {
@@ -922,6 +984,7 @@ int pl_sparse_conv_prepare(const pl_sparse_conv_desc* desc, pl_sparse_conv_handl
     h->auto_walk = rc == PL_OK;
   }
   if (rc == PL_OK && algo == PL_ALGO_BLOCK_MFMA) rc = BuildBlockMfma(L, h);
+  if (rc == PL_OK && algo == PL_ALGO_BLOCK_MFMA && desc->ic > 64) rc = BuildChunkMfma(L, h);
   if (rc == PL_OK && (algo == PL_ALGO_IMAGE_MFMA || (h->auto_int8 && (pl::ImageMfmaFits(desc->oc, desc->ic, 16) || pl::ImageMfmaFits(desc->oc, desc->ic, 49))))) rc = BuildImageMfma(L, h);
   if (rc == PL_OK && h->wtiles.ptr && pl::ImageTrMfmaFits(desc->oc, desc->ic, 20)) rc = BuildImageTrMfma(L, h);
   if (rc == PL_OK && h->wtiles.ptr && pl::ImageMfmaRegroupsByTransposingReads(desc->ic, 196)) rc = BuildImageMfmaTrRegroup(L, h);
@@ -1128,6 +1191,19 @@ int pl_sparse_conv_run(pl_sparse_conv_handle* h, const void* x_dev, void* out_de
     p.groups_per_slice = CeilDiv(h->n_groups, slices);
     p.slices = CeilDiv(h->n_groups, p.groups_per_slice);
     e = pl::LaunchHalfWalk(h->semi ? 2 : 1, tp, threads, p, s);
+  } else if (h->int8 && ChunkMfmaPays(h, call_algo, batch, im_size)) {
+    pl::ChunkMfmaParams p{};
+    p.x = static_cast<const int8_t*>(x_dev);
+    p.out = out_dev;
+    p.wtiles = h->wchunk.ptr;
+    p.scale = static_cast<const float*>(h->scale.ptr);
+    p.bias = static_cast<const float*>(h->bias.ptr);
+    p.K = h->ic;
+    p.M = h->oc;
+    p.hw = im_size;
+    p.batch = batch;
+    p.act = h->act;
+    e = pl::LaunchChunkMfma(OutKind(h->kind), std::max(1, h->wg_slots_default / 2), p, s);
   } else if (call_algo == PL_ALGO_IMAGE_MFMA) {
     // larger maps of a multiple of 196 positions are taken slab by slab by the kernel with one row tile per wavefront
     const bool slabs = h->wtiles_rows.ptr != nullptr && (h->image_kernel == 0 || h->image_kernel == 3) && pl::ImageRowsSlabFits(h->oc, h->ic, im_size);

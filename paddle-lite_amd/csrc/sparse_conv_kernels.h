@@ -288,6 +288,36 @@ struct MfmaConfig {
 
 hipError_t LaunchBlockMfma(const MfmaConfig& cfg, const MfmaParams& p, hipStream_t stream);
 
+// Chunk MFMA SpMM (int8, chunk_mfma_kernels.hip): dense 16x64 weight tiles, the channels taken chunk by chunk.
+struct ChunkMfmaParams {
+  const int8_t* x;
+  void* out;
+  // [row tile of 16][64-channel step][64 lanes][16 bytes]; lane l of a tile holds row l % 16, byte t channel
+  // 64 step + 16 (l / 16) + t; in the last, partial group of 16 channels byte t is channel K - 16 + t (zero where
+  // that channel belongs to the group before)
+  const void* wtiles;
+  const float* scale;  // padded to a multiple of 32 rows
+  const float* bias;   // likewise (zeros when the op has no bias)
+  int K, M;
+  int hw;
+  int batch;
+  DevAct act;
+  // filled in by the launcher
+  int qpi;               // position quads per image = ceil(hw / 4)
+  int quad_aligned;      // hw % 4 == 0
+  uint32_t total_quads;  // batch * qpi
+  int row_tiles;         // ceil(M / 16)
+  int ksteps;            // ceil(K / 64)
+  int padded_ksteps;     // steps wtiles holds, the last ones zero
+  int chunks;
+  int tile_quads;        // position quads of a tile
+  int tiles, row_groups;
+};
+
+int ChunkMfmaPaddedSteps(int K);  // 64-channel steps of the weight tiles: whole chunks of the widest kind
+bool ChunkMfmaFits(int K, int hw);
+hipError_t LaunchChunkMfma(int out_kind, int cus, const ChunkMfmaParams& p, hipStream_t stream);
+
 // Image MFMA SpMM (int8, image_mfma_kernels.hip): one workgroup per (image,
 // 128 output rows) with the whole image's activations in LDS.
 struct ImageMfmaParams {

@@ -1,0 +1,46 @@
+"""The int8 kernel that takes the input channels chunk by chunk, against the CPU oracle through the C ABI, bit for
+bit: channel counts around a group of 16, a step of 64 and a chunk, one to seven chunks (each way the loop over the
+chunks can end), rows around a tile of 16 and a group of 128, maps of four positions and more with every remainder
+modulo four, tiles of whole images and tiles that cross images, and each of the three tile widths."""
+import sys
+
+import numpy as np
+import pytest
+
+from helpers import capi, workloads, pla, oracle_pack, run_hip, run_oracle, assert_same
+
+pytestmark = pytest.mark.gpu
+
+AP = pla.ActivationParam
+KINDS = {"acc32": capi.KIND_INT8_ACC32, "fp32out": capi.KIND_INT8_FP32, "int8out": capi.KIND_INT8_INT8}
+# (batch, ic, oc, h, w).  64-position tiles hold chunks of 512 channels, 128: 256, 256: 128.
+NARROW = [(1, 513, 17, 2, 2), (3, 520, 1, 1, 5), (5, 527, 127, 2, 3), (2, 600, 129, 7, 7), (1, 1024, 16, 14, 14), (1, 1025, 40, 9, 11), (9, 1536, 33, 3, 3),
+          (1, 2049, 130, 5, 13), (2, 2561, 20, 8, 8), (1, 3100, 24, 1, 7), (4, 79, 140, 5, 9), (2, 65, 200, 3, 5), (1, 512, 512, 14, 14), (1, 200, 72, 12, 12)]
+MIDDLE = [(16, 520, 4096, 8, 8), (3, 1030, 2200, 17, 17)]
+WIDE = [(2, 130, 4096, 31, 33), (2, 330, 4096, 31, 33), (2, 900, 4096, 32, 32)]
+
+
+def check(shape, kind, act, paired, seed):
+    print("CASE chunk", shape, kind, file=sys.stderr, flush=True)
+    batch, ic, oc, h, w = shape
+    k = KINDS[kind]
+    case = workloads.make_int8("chunk", batch, ic, oc, h, w, 0.8, paired, AP() if kind == "acc32" else act, out_int8=(kind == "int8out"), seed=seed,
+                               output_scale=0.2 * float(np.sqrt(ic / 64.0)) if kind == "int8out" else 1.0)
+    case.kind = k
+    got = run_hip(case, capi.ALGO_BLOCK_MFMA)
+    few = case.x[:1] if batch * h * w > 1000 else case.x
+    assert_same(case, got[:len(few)], run_oracle(case, oracle_pack(case), x=few), "chunk %s %s" % (shape, kind))
+    if len(few) != batch:  # the last image too: it ends the last tile
+        assert_same(case, got[-1:], run_oracle(case, oracle_pack(case), x=case.x[-1:]), "chunk %s %s, last image" % (shape, kind))
+
+
+@pytest.mark.parametrize("kind", sorted(KINDS))
+@pytest.mark.parametrize("shape", NARROW, ids=lambda s: "x".join(map(str, s)))
+def test_narrow_tiles(shape, kind):
+    check(shape, kind, [AP("relu"), AP("hard_swish"), AP("leaky_relu", Leaky_relu_alpha=0.1), AP("relu6")][shape[1] % 4], shape[2] % 2 == 0, shape[1])
+
+
+@pytest.mark.parametrize("kind", sorted(KINDS))
+@pytest.mark.parametrize("shape", MIDDLE + WIDE, ids=lambda s: "x".join(map(str, s)))
+def test_wide_tiles(shape, kind):
+    check(shape, kind, AP("relu"), False, shape[1])
