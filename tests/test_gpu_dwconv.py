@@ -105,6 +105,20 @@ def test_mobilenet_shapes(layer):
 ITEM_SHAPES = {1: [(2, 1), (4, 1), (1, 2), (2, 2), (4, 2), (1, 4), (2, 4)], 2: [(2, 1), (1, 2), (2, 2), (1, 4)]}
 
 
+# the first and the last plane, whose rows are read in one piece moved inside the tensor: tensors around the 12 - 36 bytes
+# that a piece has, and every remainder of the row length, so that a piece starts before, ends behind and straddles both
+ENDS = [(1, 1, 3, 3), (1, 1, 4, 3), (1, 1, 3, 5), (1, 1, 4, 4), (1, 1, 4, 5), (1, 1, 5, 4), (1, 1, 4, 6), (1, 1, 5, 7), (1, 1, 4, 9), (1, 1, 2, 18), (1, 2, 1, 37), (1, 1, 6, 6), (2, 1, 17, 30),
+        (1, 3, 25, 31), (1, 1, 26, 32), (1, 2, 24, 33)]
+
+
+@pytest.mark.parametrize("stride,rows,cols", [(s, r, c) for s in (1, 2) for (r, c) in ITEM_SHAPES[s]])
+@pytest.mark.parametrize("pad", [0, 1])
+def test_ends_of_the_tensor(stride, rows, cols, pad):
+    for i, (n, c, h, w) in enumerate(ENDS):
+        if min(h, w) + 2 * pad >= 3:
+            run_case(n, c, h, w, stride, pad, "int8", ACTS["none"](), True, seed=i + 31 * stride + pad, guard=64 + i % 4, item_rows=rows, item_cols=cols)
+
+
 @pytest.mark.parametrize("stride,rows,cols", [(s, r, c) for s in (1, 2) for (r, c) in ITEM_SHAPES[s]])
 @pytest.mark.parametrize("out", ["int8", "fp32"])
 def test_item_shapes(stride, rows, cols, out):
