@@ -74,6 +74,12 @@ using epilogue::DispatchAct;
 constexpr int kWaves = kTileWalkWaves;  // wavefronts per workgroup = list streams
 constexpr int kChunkBytes = kTileWalkChunkBytes;
 
+// The value that lane E of the four lanes around it holds.
+template <int E>
+__device__ __forceinline__ uint32_t QuadLane(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x55 * E, 0xf, 0xf, true);
+}
+
 // One tile: stage it, then walk the streams of one part (0 main, 1 spare).
 template <int NR, int ACT, int G, bool RAGGED>
 __device__ __forceinline__ void WalkOneTile(const TileWalkParams& p, float* tile, int tile_id, int part) {
@@ -219,6 +225,16 @@ __device__ __forceinline__ void WalkOneTile(const TileWalkParams& p, float* tile
         if (NR == 2) acc[NR - 1][q] = __builtin_fmaf(x[q], w1, acc[NR - 1][q]);
       }
     };
+    // The byte offsets of a record.  From four row groups per step on, every lane reads one of them and the address add
+    // takes it from the lane among four that has it: a 4-byte LDS read costs 2.5 clocks, a 16-byte one 4.4.  64 x 512 ->
+    // 512 @14x14 35.0 -> 33.6 us, 64 x 1024 -> 1024 @7x7 with row pairs 60.9 -> 59.2.  Pairs of row groups keep the
+    // 16-byte read (32 x 256 -> 512 @28x28 with row pairs 21.0, 21.3 the other way), and so do the weights, which
+    // would each cost a move (33.6 -> 37.3 together with reading the next record one step ahead).
+    auto offsets = [&](const char* r) {
+      if (G < 4) return *reinterpret_cast<const u4*>(r);
+      const uint32_t own = *reinterpret_cast<const uint32_t*>(r + 4 * (lane & 3));
+      return u4{QuadLane<0>(own), QuadLane<1>(own), QuadLane<2>(own), QuadLane<3>(own)};
+    };
     auto weights = [&](const char* r, float (&w)[4 * NR]) {
       const u4 wa = *reinterpret_cast<const u4*>(r + 16);
       w[0] = __uint_as_float(wa.x), w[1] = __uint_as_float(wa.y), w[2] = __uint_as_float(wa.z), w[3] = __uint_as_float(wa.w);
@@ -230,7 +246,7 @@ __device__ __forceinline__ void WalkOneTile(const TileWalkParams& p, float* tile
     const uint32_t batches = entries >> 2, rem = entries & 3u;
     for (uint32_t b = 0; b < batches; ++b) {
       const char* r = next();
-      const u4 off = *reinterpret_cast<const u4*>(r);
+      const u4 off = offsets(r);
       float w[4 * NR];
       weights(r, w);
       vx x[4];
@@ -247,7 +263,7 @@ __device__ __forceinline__ void WalkOneTile(const TileWalkParams& p, float* tile
     }
     if (rem != 0) {  // the last, partly filled batch: only its real entries
       const char* r = next();
-      const u4 off = *reinterpret_cast<const u4*>(r);
+      const u4 off = offsets(r);
       float w[4 * NR];
       weights(r, w);
       entry(off[0], w[0], w[NR - 1]);
