@@ -68,7 +68,7 @@ def parse():
     ap.add_argument("--steps", type=int, default=2000)
     ap.add_argument("--warmup", type=int, default=200)
     ap.add_argument("--config", default="c3", choices=["c1", "c2", "c3", "c4", "c5", "calib", "mobilenet", "density-sweep", "floors", "store-shapes", "device-rates", "custom", "small-batch", "float-layers"])
-    ap.add_argument("--algo", default="auto", choices=["auto", "walk", "mfma", "image"])
+    ap.add_argument("--algo", default="auto", choices=["auto", "walk", "mfma", "image", "chunk"])
     ap.add_argument("--image-kernel", default="rule", choices=["rule", "regroup", "transpose", "rows"], help="which image MFMA kernel a handle uses where both apply (pl_sparse_conv_tuning.image_kernel)")
     ap.add_argument("--image-regroup", default="rule", choices=["rule", "valu"], help="regrouping image kernel: by transposing LDS reads where that exists (rule) or by the vector ALU everywhere (pl_sparse_conv_tuning.image_tr_regroup)")
     # --config custom: any shape through the same measurement (parity-checked against the oracle on two images)
@@ -271,7 +271,7 @@ def run_density_sweep(args):
     capi, wl = helpers.capi, helpers.workloads
     L = capi.lib()
     stream = torch.cuda.current_stream().cuda_stream
-    names = {capi.ALGO_ROW_WALK: "row_walk", capi.ALGO_BLOCK_MFMA: "block_mfma", capi.ALGO_IMAGE_MFMA: "image_mfma"}
+    names = helpers.ALGO_NAMES
     steps = max(50, min(args.steps, 300))
     rows = []
     for shape in ("metric", "wide"):
@@ -290,9 +290,9 @@ def run_density_sweep(args):
                     op = (C.c_void_p * n_sets)(*[t.data_ptr() for t in outs])
                 want = helpers.run_oracle(case, x=case.x[:1])
                 row = {"shape": "N=%d %d->%d @%dx%d" % (batch, ic, oc, hw, hw), "sparsity": sparsity, "zeros": "blocks" if blocked else "random", "nnz": case.nnz, "kernel_us": {}}
-                for a in (capi.ALGO_ROW_WALK, capi.ALGO_BLOCK_MFMA, capi.ALGO_IMAGE_MFMA, capi.ALGO_AUTO):
+                for a in sorted(names) + [capi.ALGO_AUTO]:
                     try:
-                        kernel, _ = helpers.make_kernel(case, algo=a)
+                        kernel, _ = helpers.make_kernel(case, **helpers.forced_algo(a))
                     except capi.SparseConvError:
                         continue  # the shape is outside this algorithm's range
                     if a == capi.ALGO_AUTO:
@@ -592,7 +592,7 @@ def run_c5(args):
         case = wl.config5_layer(i)
         if args.algo == "image":
             raise SystemExit("--algo image applies to single layers; the stack holds shapes outside the image kernel's range (use auto)")
-        kernel, weights = helpers.make_kernel(case, algo={"auto": capi.ALGO_AUTO, "walk": capi.ALGO_ROW_WALK, "mfma": capi.ALGO_BLOCK_MFMA}[args.algo])
+        kernel, weights = helpers.make_kernel(case, **helpers.forced_algo({"auto": capi.ALGO_AUTO, "walk": capi.ALGO_ROW_WALK, "mfma": capi.ALGO_BLOCK_MFMA, "chunk": capi.ALGO_CHUNK_MFMA}[args.algo]))
         ic, oc, hw = wl.MOBILENET_V1_POINTWISE[i]
         chained = prev_out is not None and tuple(prev_out.shape[1:]) == (ic, hw, hw)
         x = prev_out if chained else torch.from_numpy(case.x).cuda()
@@ -911,9 +911,10 @@ def main():
         case.x = case.x.astype(np.float16)
         case.name += "_fp16"
         args.no_cpu_baseline = True  # the CPU baselines are fp32 / int8 paths
-    algo = {"auto": capi.ALGO_AUTO, "walk": capi.ALGO_ROW_WALK, "mfma": capi.ALGO_BLOCK_MFMA, "image": capi.ALGO_IMAGE_MFMA}[args.algo]
+    algo = {"auto": capi.ALGO_AUTO, "walk": capi.ALGO_ROW_WALK, "mfma": capi.ALGO_BLOCK_MFMA, "image": capi.ALGO_IMAGE_MFMA, "chunk": capi.ALGO_AUTO}[args.algo]
     tune = capi.tuning(image_kernel={"rule": 0, "regroup": capi.IMAGE_KERNEL_REGROUP, "transpose": capi.IMAGE_KERNEL_TRANSPOSE, "rows": capi.IMAGE_KERNEL_ROWS}[args.image_kernel],
-                       image_tr_regroup=capi.TUNE_NEVER if args.image_regroup == "valu" else capi.TUNE_RULE)
+                       image_tr_regroup=capi.TUNE_NEVER if args.image_regroup == "valu" else capi.TUNE_RULE,
+                       chunk_mfma={"auto": capi.TUNE_RULE, "chunk": capi.TUNE_ALWAYS}.get(args.algo, capi.TUNE_NEVER))
     kernel, weights = helpers.make_kernel(case, algo=algo, tuning=tune)
     info = kernel.info()
     ops = case.algorithmic_ops()
@@ -985,7 +986,7 @@ def main():
         copy_gbs = 2.0 * (1 << 30) * 10 / (c0.elapsed_time(c1) * 1e-3) / 1e9
         del src, dst
     achieved = nbytes / (kernel_ms * 1e-3) / 1e9
-    algo_names = {capi.ALGO_ROW_WALK: "row_walk", capi.ALGO_BLOCK_MFMA: "block_mfma", capi.ALGO_IMAGE_MFMA: "image_mfma"}
+    algo_names = helpers.ALGO_NAMES
     algo_name = algo_names[capi.check(L.pl_sparse_conv_algo_for(kernel._handle, case.batch, case.im_size))]
     traffic, traffic_detail = measured_traffic(case.name, algo_name)
     # int8: the same launch through every algorithm the shape allows (same rotating buffers, 200 untimed then 1000 timed launches each)
@@ -1001,10 +1002,11 @@ def main():
             if name in per_algo:
                 continue
             try:
+                forced = helpers.forced_algo(a)
                 other_tune = {"image_mfma_regroup_in_lds": capi.tuning(image_kernel=capi.IMAGE_KERNEL_REGROUP),
                               "image_mfma_valu_regroup": capi.tuning(image_kernel=capi.IMAGE_KERNEL_REGROUP, image_tr_regroup=capi.TUNE_NEVER),
-                              "image_mfma_transposing_reads": capi.tuning(image_kernel=capi.IMAGE_KERNEL_TRANSPOSE)}.get(name)
-                other, _ = helpers.make_kernel(case, algo=a, tuning=other_tune)
+                              "image_mfma_transposing_reads": capi.tuning(image_kernel=capi.IMAGE_KERNEL_TRANSPOSE)}.get(name, forced["tuning"])
+                other, _ = helpers.make_kernel(case, algo=forced["algo"], tuning=other_tune)
             except capi.SparseConvError:
                 continue  # this shape is outside the algorithm's range
             if L.pl_sparse_conv_run_sequence(other._handle, xp, op, n_sets, case.batch, case.im_size, 200, C.c_void_p(stream), None) < 0:

@@ -84,11 +84,14 @@ enum {
  * chooses per call by batch and H*W (the image kernels where the whole map
  * fits, or in slabs while batch * slabs * oc / 128 is at most half the CU
  * count; else the row walk for at most 256 positions in all;
- * else the block kernel): see pl_sparse_conv_algo_for().  Calls with many
- * channels or few positions among them run as dense 16x64 weight tiles with
- * the channels taken chunk by chunk, whichever of the three that names; so
- * do such calls of a handle prepared for PL_ALGO_BLOCK_MFMA. */
-enum { PL_ALGO_AUTO = 0, PL_ALGO_ROW_WALK = 1, PL_ALGO_BLOCK_MFMA = 2, PL_ALGO_IMAGE_MFMA = 3 };
+ * else the block kernel).  Calls with many channels, ragged maps or few
+ * positions among these run as dense 16x64 weight tiles with the channels
+ * taken chunk by chunk instead, and so do such calls of a handle prepared
+ * for PL_ALGO_BLOCK_MFMA; tuning.chunk_mfma forces or forbids it.
+ * pl_sparse_conv_algo_for() reports the choice, that kernel as
+ *   PL_ALGO_CHUNK_MFMA (a report only: pl_sparse_conv_desc.algo takes the
+ *                     others). */
+enum { PL_ALGO_AUTO = 0, PL_ALGO_ROW_WALK = 1, PL_ALGO_BLOCK_MFMA = 2, PL_ALGO_IMAGE_MFMA = 3, PL_ALGO_CHUNK_MFMA = 4 };
 
 /* Activation constants, used as given (replaces the fields of
  * ActivationParam the math functions read,
@@ -145,6 +148,11 @@ typedef struct pl_sparse_conv_tuning {
                                 tiles).  NEVER = one row group per instruction:
                                 that form exists up to 271 channels and for maps
                                 of a multiple of 4 positions only             */
+  int32_t chunk_mfma;        /* (switch) int8 calls with the channels taken chunk
+                                by chunk (PL_ALGO_CHUNK_MFMA), PL_ALGO_AUTO and
+                                PL_ALGO_BLOCK_MFMA; it takes 16 channels and maps
+                                of 4 positions and more                       */
+  int32_t chunk_positions;   /* that kernel: positions per tile, 64, 128 or 256 */
 } pl_sparse_conv_tuning;
 
 /* Everything PrepareForRun() knows.  All pointers are HOST pointers and are
@@ -169,7 +177,8 @@ typedef struct pl_sparse_conv_desc {
   const float* bias;             /* oc merged biases or NULL                */
   pl_activation act;
   pl_sparse_conv_tuning tuning;  /* struct_size may also be the offset of this
-                                    field: then every rule applies            */
+                                    field or of tuning.chunk_mfma: the rules
+                                    apply to what lies behind it              */
 } pl_sparse_conv_desc;
 
 typedef struct pl_sparse_conv_info {
@@ -229,8 +238,8 @@ int pl_sparse_conv_run_sequence(pl_sparse_conv_handle* handle,
 int pl_sparse_conv_get_info(const pl_sparse_conv_handle* handle,
                             pl_sparse_conv_info* info);
 
-/* The algorithm (PL_ALGO_*, never PL_ALGO_AUTO) a pl_sparse_conv_run() call
- * with this batch and H*W would use on 16-byte aligned tensors, or a negative
+/* The algorithm (ROW_WALK, BLOCK_MFMA, IMAGE_MFMA or CHUNK_MFMA) a
+ * pl_sparse_conv_run() call with this batch and H*W would use on 16-byte aligned tensors, or a negative
  * status.  No counterpart in the reference, whose kernel choice is fixed by
  * the registration (lite/kernels/arm/sparse_conv_compute.cc:369-430). */
 int pl_sparse_conv_algo_for(const pl_sparse_conv_handle* handle, int32_t batch,

@@ -11,6 +11,7 @@ PL_OK, PL_ERR_BAD_ARG, PL_ERR_BAD_LAYOUT, PL_ERR_UNSUPPORTED, PL_ERR_HIP, PL_ERR
 KIND_FP32, KIND_INT8_FP32, KIND_INT8_INT8, KIND_INT8_ACC32, KIND_FP16 = 0, 1, 2, 3, 4
 ACT_NONE, ACT_RELU, ACT_RELU6, ACT_LEAKY_RELU, ACT_HARD_SWISH = 0, 1, 2, 4, 10
 ALGO_AUTO, ALGO_ROW_WALK, ALGO_BLOCK_MFMA, ALGO_IMAGE_MFMA = 0, 1, 2, 3
+ALGO_CHUNK_MFMA = 4  # reported by pl_sparse_conv_algo_for, not accepted by prepare
 TUNE_RULE, TUNE_NEVER, TUNE_ALWAYS = 0, 1, 2
 IMAGE_KERNEL_REGROUP, IMAGE_KERNEL_TRANSPOSE, IMAGE_KERNEL_ROWS = 1, 2, 3
 
@@ -70,6 +71,8 @@ class Tuning(C.Structure):
         ("walk_slices", C.c_int32),
         ("image_tr_regroup", C.c_int32),
         ("walk_pairs", C.c_int32),
+        ("chunk_mfma", C.c_int32),
+        ("chunk_positions", C.c_int32),
     ]
 
 

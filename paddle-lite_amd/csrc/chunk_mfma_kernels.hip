@@ -287,7 +287,7 @@ hipError_t Launch(int nw, const ChunkMfmaParams& p, dim3 grid, hipStream_t s) {
 int ChunkMfmaPaddedSteps(int K) { return (K + 511) / 512 * 8; }
 bool ChunkMfmaFits(int K, int hw) { return K >= 16 && hw >= 4; }
 
-hipError_t LaunchChunkMfma(int out_kind, int cus, const ChunkMfmaParams& p, hipStream_t stream) {
+hipError_t LaunchChunkMfma(int out_kind, int cus, int tile_positions, const ChunkMfmaParams& p, hipStream_t stream) {
   if (p.batch <= 0 || p.M <= 0) return hipSuccess;
   if (!ChunkMfmaFits(p.K, p.hw)) return hipErrorInvalidValue;
   const int64_t positions = (int64_t)p.batch * p.hw;
@@ -315,6 +315,7 @@ hipError_t LaunchChunkMfma(int out_kind, int cus, const ChunkMfmaParams& p, hipS
     const int64_t cost = rounds * (300 + 135 * ((q.ksteps + 8 / w - 1) / (8 / w)));
     if (w == 1 || cost < best) best = cost, nw = w;
   }
+  if (tile_positions != 0) nw = tile_positions / 64;
   q.tile_quads = tile_quads(nw);
   q.tiles = tiles(nw);
   q.chunks = (q.ksteps + 8 / nw - 1) / (8 / nw);

@@ -181,6 +181,8 @@ struct pl_sparse_conv_handle {
   int wg_slots = 512;       // workgroups resident at once (2 per CU)
   int wg_slots_default = 512;  // the same before any override: twice the device's CU count
   DevBuf wchunk;            // dense 16x64 tiles of the kernel that takes the channels chunk by chunk
+  int chunk_mfma = 1;       // that kernel: 0 never, 1 by the rule, 2 whenever the shape allows
+  int chunk_positions = 0;  // positions per tile of that kernel; 0 = chosen per problem
   int mfma_stream = 1;      // streaming block MFMA: 0 never, 1 when the shape suits it, 2 whenever the shape allows
   int mfma_i8_wide = 1;
   int mfma_tile_quads = 0;  // 0 = chosen per problem
@@ -766,7 +768,7 @@ pl::WalkConfig ChooseWalk(const pl_sparse_conv_handle* h, uint32_t P) {
   return c;
 }
 
-// The algorithm one call uses.  Handles prepared for one algorithm use it.  An int8 handle prepared with
+// The algorithm of one call that is not taken chunk by chunk.  Handles prepared for one algorithm use it.  An int8 handle prepared with
 // PL_ALGO_AUTO holds the forms of every algorithm its shape allows and picks per call, by what was measured on
 // the pointwise shapes of MobileNetV1 at 1 to 64 images per launch:
 //  * the image kernels wherever their shape conditions hold: they tie with or beat the block kernel at every
@@ -777,7 +779,7 @@ pl::WalkConfig ChooseWalk(const pl_sparse_conv_handle* h, uint32_t P) {
 //    block kernel would have one or two tiles);
 //  * else the block kernel.
 // tuning.image_min_items raises the number of (image, 128-row group) work items the image kernels ask for.
-int AlgoForCall(const pl_sparse_conv_handle* h, int batch, int im_size, bool aligned16) {
+int AlgoBesideChunkMfma(const pl_sparse_conv_handle* h, int batch, int im_size, bool aligned16) {
   if (!h->auto_int8) return h->algo;
   // work items: (image, row group), for 7 x 7 maps (pair of images, row group)
   const int64_t image_items = static_cast<int64_t>(im_size == 49 ? (batch + 1) / 2 : batch) * (h->oc / 128);
@@ -794,8 +796,8 @@ int AlgoForCall(const pl_sparse_conv_handle* h, int batch, int im_size, bool ali
   return h->algo;
 }
 
-// Whether the kernel that takes the channels chunk by chunk (chunk_mfma_kernels.hip) runs a call that AlgoForCall gives
-// to `call_algo`.  It spreads a call over the chip in workgroups of 128 rows x 64 - 256 positions, pays one short load -
+// Whether the kernel that takes the channels chunk by chunk (chunk_mfma_kernels.hip) runs a call that
+// AlgoBesideChunkMfma gives to `call_algo`.  It spreads a call over the chip in workgroups of 128 rows x 64 - 256 positions, pays one short load -
 // multiply chain per 512 channels and does not care about the map's alignment.  Measured at 85 % zeros with fp32
 // output (us, it against what ran before):
 //  * more than 512 channels: 512 rows of 2048 channels on 7 x 7 maps 10.0 / 10.9 / 13.5 against 21.3 / 28.7 / 27.6 at
@@ -818,6 +820,7 @@ int AlgoForCall(const pl_sparse_conv_handle* h, int batch, int im_size, bool ali
 bool ChunkMfmaPays(const pl_sparse_conv_handle* h, int call_algo, int batch, int im_size) {
   const int64_t positions = static_cast<int64_t>(batch) * im_size;
   if (!h->wchunk.ptr || !pl::ChunkMfmaFits(h->ic, im_size) || positions * h->ic >= (1ll << 31)) return false;
+  if (h->chunk_mfma == 2) return true;
   const int cus = std::max(1, h->wg_slots_default / 2);
   if (call_algo == PL_ALGO_ROW_WALK) return h->auto_int8 && h->oc * h->ic > 8192;
   if (call_algo == PL_ALGO_IMAGE_MFMA) {
@@ -831,6 +834,12 @@ bool ChunkMfmaPays(const pl_sparse_conv_handle* h, int call_algo, int batch, int
   const int64_t block_tiles = (positions + 127) / 128 * CeilDiv(h->oc, 128);
   if (h->ic <= 128) return im_size % 4 != 0 ? block_tiles * 2 <= cus : h->ic % 16 != 0 && block_tiles * 4 <= cus;
   return block_tiles <= (im_size % 4 != 0 ? 2 * cus : cus / 2);
+}
+
+// The algorithm of one call (pl_sparse_conv_algo_for reports it).
+int AlgoForCall(const pl_sparse_conv_handle* h, int batch, int im_size, bool aligned16) {
+  const int algo = AlgoBesideChunkMfma(h, batch, im_size, aligned16);
+  return ChunkMfmaPays(h, algo, batch, im_size) ? PL_ALGO_CHUNK_MFMA : algo;
 }
 
 }  // namespace
@@ -858,12 +867,15 @@ int pl_device_count(void) {
 int pl_sparse_conv_prepare(const pl_sparse_conv_desc* desc, pl_sparse_conv_handle** out_handle) {
   if (!desc || !out_handle) return Fail(PL_ERR_BAD_ARG, "null argument");
   *out_handle = nullptr;
-  if (desc->struct_size != sizeof(pl_sparse_conv_desc) && desc->struct_size != offsetof(pl_sparse_conv_desc, tuning))
+  // callers compiled against a header without the tuning fields, or without the last ones, pass what they know
+  constexpr size_t kNoTuning = offsetof(pl_sparse_conv_desc, tuning), kNoChunkTuning = kNoTuning + offsetof(pl_sparse_conv_tuning, chunk_mfma);
+  if (desc->struct_size != sizeof(pl_sparse_conv_desc) && desc->struct_size != kNoChunkTuning && desc->struct_size != kNoTuning)
     return Fail(PL_ERR_BAD_ARG, "pl_sparse_conv_desc size mismatch (%u vs %zu)", desc->struct_size, sizeof(pl_sparse_conv_desc));
   pl_sparse_conv_tuning tune{};
-  if (desc->struct_size == sizeof(pl_sparse_conv_desc)) tune = desc->tuning;
-  for (int32_t sw : {tune.mfma_stream, tune.mfma_sub_tiles, tune.walk_tiled, tune.walk_chunked, tune.image_tr_regroup, tune.walk_pairs})
+  std::memcpy(&tune, reinterpret_cast<const char*>(desc) + kNoTuning, std::min<size_t>(desc->struct_size - kNoTuning, sizeof(tune)));
+  for (int32_t sw : {tune.mfma_stream, tune.mfma_sub_tiles, tune.walk_tiled, tune.walk_chunked, tune.image_tr_regroup, tune.walk_pairs, tune.chunk_mfma})
     if (sw < PL_TUNE_RULE || sw > PL_TUNE_ALWAYS) return Fail(PL_ERR_BAD_ARG, "a tuning switch is not PL_TUNE_RULE, PL_TUNE_NEVER or PL_TUNE_ALWAYS");
+  if (tune.chunk_positions != 0 && tune.chunk_positions != 64 && tune.chunk_positions != 128 && tune.chunk_positions != 256) return Fail(PL_ERR_BAD_ARG, "tuning.chunk_positions must be 0, 64, 128 or 256");
   if (tune.image_kernel < 0 || tune.image_kernel > 3) return Fail(PL_ERR_BAD_ARG, "tuning.image_kernel must be 0, 1, 2 or 3");
   if (desc->kind < PL_KIND_FP32 || desc->kind > PL_KIND_FP16) return Fail(PL_ERR_BAD_ARG, "unknown kind %d", desc->kind);
   if (desc->algo < PL_ALGO_AUTO || desc->algo > PL_ALGO_IMAGE_MFMA) return Fail(PL_ERR_BAD_ARG, "unknown algo %d", desc->algo);
@@ -908,6 +920,8 @@ int pl_sparse_conv_prepare(const pl_sparse_conv_desc* desc, pl_sparse_conv_handl
   h->walk_tiled = sw(tune.walk_tiled);
   h->walk_pairs = sw(tune.walk_pairs) != 0;  // the rule: pairs
   h->walk_chunked = sw(tune.walk_chunked);
+  h->chunk_mfma = sw(tune.chunk_mfma);
+  h->chunk_positions = tune.chunk_positions;
   h->mfma_i8_wide = tune.mfma_narrow_i8_stores == 0;
   if (tune.walk_split > 0) h->walk_split = std::min(kTileWalkSplits, tune.walk_split - 1);
   if (tune.mfma_tile_quads > 0) h->mfma_tile_quads = std::max(8, std::min(32, tune.mfma_tile_quads));
@@ -984,7 +998,7 @@ int pl_sparse_conv_prepare(const pl_sparse_conv_desc* desc, pl_sparse_conv_handl
     h->auto_walk = rc == PL_OK;
   }
   if (rc == PL_OK && algo == PL_ALGO_BLOCK_MFMA) rc = BuildBlockMfma(L, h);
-  if (rc == PL_OK && algo == PL_ALGO_BLOCK_MFMA && desc->ic > 64) rc = BuildChunkMfma(L, h);
+  if (rc == PL_OK && algo == PL_ALGO_BLOCK_MFMA && (h->chunk_mfma == 2 ? desc->ic >= 16 : h->chunk_mfma == 1 && desc->ic > 64)) rc = BuildChunkMfma(L, h);
   if (rc == PL_OK && (algo == PL_ALGO_IMAGE_MFMA || (h->auto_int8 && (pl::ImageMfmaFits(desc->oc, desc->ic, 16) || pl::ImageMfmaFits(desc->oc, desc->ic, 49))))) rc = BuildImageMfma(L, h);
   if (rc == PL_OK && h->wtiles.ptr && pl::ImageTrMfmaFits(desc->oc, desc->ic, 20)) rc = BuildImageTrMfma(L, h);
   if (rc == PL_OK && h->wtiles.ptr && pl::ImageMfmaRegroupsByTransposingReads(desc->ic, 196)) rc = BuildImageMfmaTrRegroup(L, h);
@@ -1191,7 +1205,7 @@ int pl_sparse_conv_run(pl_sparse_conv_handle* h, const void* x_dev, void* out_de
     p.groups_per_slice = CeilDiv(h->n_groups, slices);
     p.slices = CeilDiv(h->n_groups, p.groups_per_slice);
     e = pl::LaunchHalfWalk(h->semi ? 2 : 1, tp, threads, p, s);
-  } else if (h->int8 && ChunkMfmaPays(h, call_algo, batch, im_size)) {
+  } else if (call_algo == PL_ALGO_CHUNK_MFMA) {
     pl::ChunkMfmaParams p{};
     p.x = static_cast<const int8_t*>(x_dev);
     p.out = out_dev;
@@ -1203,7 +1217,7 @@ int pl_sparse_conv_run(pl_sparse_conv_handle* h, const void* x_dev, void* out_de
     p.hw = im_size;
     p.batch = batch;
     p.act = h->act;
-    e = pl::LaunchChunkMfma(OutKind(h->kind), std::max(1, h->wg_slots_default / 2), p, s);
+    e = pl::LaunchChunkMfma(OutKind(h->kind), std::max(1, h->wg_slots_default / 2), h->chunk_positions, p, s);
   } else if (call_algo == PL_ALGO_IMAGE_MFMA) {
     // larger maps of a multiple of 196 positions are taken slab by slab by the kernel with one row tile per wavefront
     const bool slabs = h->wtiles_rows.ptr != nullptr && (h->image_kernel == 0 || h->image_kernel == 3) && pl::ImageRowsSlabFits(h->oc, h->ic, im_size);

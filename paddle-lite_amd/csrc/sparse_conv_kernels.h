@@ -316,7 +316,8 @@ struct ChunkMfmaParams {
 
 int ChunkMfmaPaddedSteps(int K);  // 64-channel steps of the weight tiles: whole chunks of the widest kind
 bool ChunkMfmaFits(int K, int hw);
-hipError_t LaunchChunkMfma(int out_kind, int cus, const ChunkMfmaParams& p, hipStream_t stream);
+// tile_positions: positions of a tile (64, 128 or 256), 0 = chosen by the number of CUs
+hipError_t LaunchChunkMfma(int out_kind, int cus, int tile_positions, const ChunkMfmaParams& p, hipStream_t stream);
 
 // Image MFMA SpMM (int8, image_mfma_kernels.hip): one workgroup per (image,
 // 128 output rows) with the whole image's activations in LDS.

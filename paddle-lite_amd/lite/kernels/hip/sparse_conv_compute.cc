@@ -191,9 +191,9 @@ bool SparseConvCompute<P, O>::pair_endpoint(PairEndpoint* e) {
 template <PrecisionType P, PrecisionType O>
 std::string SparseConvCompute<P, O>::kernel_func_name() const {
   if (handle_ == nullptr || last_batch_ < 0) return "NotImplForSparseConv";
-  static const char* const kAlgo[] = {"auto", "row_walk", "block_mfma", "image_mfma"};
+  static const char* const kAlgo[] = {"auto", "row_walk", "block_mfma", "image_mfma", "chunk_mfma"};
   const int algo = pl_sparse_conv_algo_for(handle_, last_batch_, last_im_size_);
-  return std::string("pl_sparse_conv_run/") + (algo >= 0 && algo <= 3 ? kAlgo[algo] : "unknown");
+  return std::string("pl_sparse_conv_run/") + (algo >= 0 && algo <= 4 ? kAlgo[algo] : "unknown");
 }
 
 template class SparseConvCompute<PRECISION(kFloat), PRECISION(kFloat)>;

@@ -226,10 +226,11 @@ static void RunProblem(const Problem& p, bool run_on_device) {
     if (!p.int8) static_cast<kernels::hip::SparseConvCompute<PRECISION(kFloat), PRECISION(kFloat)>*>(k)->SetProfileRuntimeKernelInfo(&ch);
     else if (p.out_int8) static_cast<kernels::hip::SparseConvCompute<PRECISION(kInt8), PRECISION(kInt8)>*>(k)->SetProfileRuntimeKernelInfo(&ch);
     else static_cast<kernels::hip::SparseConvCompute<PRECISION(kInt8), PRECISION(kFloat)>*>(k)->SetProfileRuntimeKernelInfo(&ch);
-    // int8: the row walk for at most 256 positions in all, else the block kernel
-    // (none of these shapes is one of the image kernel's)
+    // int8: up to 256 positions in all the row walk, or the channels chunk by chunk from 8192 weights on; else the
+    // block kernel (none of these shapes is one of the image kernel's)
     const bool few_positions = p.batch * p.h * p.w <= 256;
-    EXPECT(ch.kernel_func_name == (p.int8 && !few_positions ? "pl_sparse_conv_run/block_mfma" : "pl_sparse_conv_run/row_walk"));
+    const char* int8_algo = !few_positions ? "block_mfma" : (p.oc * p.ic > 8192 ? "chunk_mfma" : "row_walk");
+    EXPECT(ch.kernel_func_name == std::string("pl_sparse_conv_run/") + (p.int8 ? int8_algo : "row_walk"));
   }
   EXPECT(y->target() == TARGET(kHIP));
   Tensor y_host;

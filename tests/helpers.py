@@ -111,7 +111,14 @@ def assert_same(case, got, want, what=""):
             raise AssertionError("%s: %d of %d elements differ, first at %s: got %r want %r" % (what, len(bad), got.size, tuple(bad[0]), got[tuple(bad[0])], want[tuple(bad[0])]))
 
 
-ALGO_NAMES = {capi.ALGO_ROW_WALK: "row_walk", capi.ALGO_BLOCK_MFMA: "block_mfma", capi.ALGO_IMAGE_MFMA: "image_mfma"}
+ALGO_NAMES = {capi.ALGO_ROW_WALK: "row_walk", capi.ALGO_BLOCK_MFMA: "block_mfma", capi.ALGO_IMAGE_MFMA: "image_mfma", capi.ALGO_CHUNK_MFMA: "chunk_mfma"}
+
+
+def forced_algo(algo):
+    """make_kernel's arguments for an int8 handle that runs `algo` on every call it can."""
+    if algo == capi.ALGO_CHUNK_MFMA:
+        return dict(algo=capi.ALGO_AUTO, tuning=capi.tuning(chunk_mfma=capi.TUNE_ALWAYS))
+    return dict(algo=algo, tuning=None if algo == capi.ALGO_AUTO else capi.tuning(chunk_mfma=capi.TUNE_NEVER))
 
 
 def algo_times(case, warm=100, steps=500, repeats=3, max_sets=24, rotation_bytes=320 << 20):
@@ -141,8 +148,10 @@ def algo_times(case, warm=100, steps=500, repeats=3, max_sets=24, rotation_bytes
     handles = {}
     for name, algo in [("auto", capi.ALGO_AUTO)] + [(n, a) for a, n in sorted(ALGO_NAMES.items())]:
         try:
-            k, _ = make_kernel(case, algo=algo)
+            k, _ = make_kernel(case, **forced_algo(algo))
         except capi.SparseConvError:
+            continue
+        if algo != capi.ALGO_AUTO and L.pl_sparse_conv_algo_for(k._handle, case.batch, case.im_size) != algo:
             continue
         outs[0].zero_()
         if L.pl_sparse_conv_run_sequence(k._handle, xp, op, n_sets, case.batch, case.im_size, 1, stream, None) < 0:

@@ -64,6 +64,26 @@ def test_struct_layout_matches_header(tmp_path):
         assert body.count(";") + body.count(",") == len(cls._fields_), cname
 
 
+def test_descriptor_sizes_of_older_headers_are_taken():
+    """A caller compiled against a header without the tuning fields, or without the last two of them, passes the size it
+    knows; any other size is refused."""
+    L = capi.lib()
+    w = pla.detect_and_pack((np.arange(8 * 16).reshape(8, 16) % 3).astype(np.float32), 4)
+    d = capi.Desc()
+    d.kind, d.first_ic, d.oc, d.ic, d.im_size = capi.KIND_FP32, w.first_ic, 8, 16, 4
+    d.nonzero_weights, d.n_weights = w.nonzero_weights.ctypes.data, w.nonzero_weights.size
+    d.oc_nonzeros, d.diffs, d.n_diffs = w.oc_nonzeros.ctypes.data, w.diffs.ctypes.data, w.diffs.size
+    d.tuning.chunk_positions = 100  # refused where it is read at all
+    tuning = capi.Desc.tuning.offset
+    for size, taken in ((tuning, True), (tuning + capi.Tuning.chunk_mfma.offset, True), (C.sizeof(capi.Desc), False), (tuning + 4, False), (C.sizeof(capi.Desc) - 4, False)):
+        d.struct_size = size
+        h = C.c_void_p()
+        rc = L.pl_sparse_conv_prepare(C.byref(d), C.byref(h))
+        assert (rc in (capi.PL_OK, capi.PL_ERR_NO_DEVICE)) == taken and (taken or rc == capi.PL_ERR_BAD_ARG), (size, rc, capi.last_error())
+        if h.value:
+            L.pl_sparse_conv_destroy(h)
+
+
 def _rand(rng, oc, ic, density, dtype, paired):
     if paired:
         m = np.repeat(rng.random_sample(((oc + 1) // 2, ic)) < density, 2, axis=0)[:oc]

@@ -7,7 +7,7 @@ import sys
 import numpy as np
 import pytest
 
-from helpers import capi, workloads, pla, oracle_pack, run_hip, run_oracle, assert_same
+from helpers import ALGO_NAMES, capi, workloads, pla, make_kernel, oracle_pack, run_hip, run_oracle, assert_same
 
 pytestmark = pytest.mark.gpu
 
@@ -44,3 +44,22 @@ def test_narrow_tiles(shape, kind):
 @pytest.mark.parametrize("shape", MIDDLE + WIDE, ids=lambda s: "x".join(map(str, s)))
 def test_wide_tiles(shape, kind):
     check(shape, kind, AP("relu"), False, shape[1])
+
+
+def test_the_choice_is_reported_and_can_be_overridden():
+    """pl_sparse_conv_algo_for names the kernel for the calls that the rule gives it out of each of the three others'
+    range, and tuning.chunk_mfma forces it and keeps it out."""
+    L = capi.lib()
+    case = workloads.make_int8("chunk", 1, 512, 512, 14, 14, 0.85, False, AP(), out_int8=False, seed=3)
+    never, _ = make_kernel(case, tuning=capi.tuning(chunk_mfma=capi.TUNE_NEVER))
+    rule, _ = make_kernel(case)
+    always, _ = make_kernel(case, tuning=capi.tuning(chunk_mfma=capi.TUNE_ALWAYS))
+    for batch, im_size, other, by_rule in ((1, 196, "image_mfma", True), (64, 196, "image_mfma", False), (4, 50, "row_walk", True), (20, 50, "block_mfma", True), (64, 784, "block_mfma", False)):
+        picked = [ALGO_NAMES[capi.check(L.pl_sparse_conv_algo_for(k._handle, batch, im_size))] for k in (never, rule, always)]
+        assert picked == [other, "chunk_mfma" if by_rule else other, "chunk_mfma"], (batch, im_size, picked)
+    assert L.pl_sparse_conv_algo_for(always._handle, 64, 3) == capi.ALGO_ROW_WALK  # no quad of positions
+    assert np.array_equal(run_hip(case, kernel=always), run_hip(case, kernel=never))
+    # a report only
+    with pytest.raises(capi.SparseConvError) as e:
+        make_kernel(case, capi.ALGO_CHUNK_MFMA)
+    assert e.value.code == capi.PL_ERR_BAD_ARG

@@ -243,7 +243,8 @@ def test_auto_picks_the_image_kernel_only_where_it_applies():
     announce("image auto")
     L = capi.lib()
     case = case_for(capi.KIND_INT8_FP32, 64, 512, 512, 14, 14, 0.85, False, ACTS["leaky"], seed=0)
-    kernel, _ = make_kernel(case, capi.ALGO_AUTO)
+    # the rule between these three kernels; the one that takes the channels chunk by chunk, kept out here, has its own
+    kernel, _ = make_kernel(case, capi.ALGO_AUTO, tuning=capi.tuning(chunk_mfma=capi.TUNE_NEVER))
     assert L.pl_sparse_conv_algo_for(kernel._handle, 64, 196) == capi.ALGO_IMAGE_MFMA
     assert L.pl_sparse_conv_algo_for(kernel._handle, 2, 196) == capi.ALGO_IMAGE_MFMA      # from two images on
     assert L.pl_sparse_conv_algo_for(kernel._handle, 1, 196) == capi.ALGO_IMAGE_MFMA      # and for a single one
@@ -253,7 +254,7 @@ def test_auto_picks_the_image_kernel_only_where_it_applies():
     assert L.pl_sparse_conv_algo_for(kernel._handle, 4, 50) == capi.ALGO_ROW_WALK         # 200 positions
     assert L.pl_sparse_conv_algo_for(kernel._handle, 64, 28 * 28) == capi.ALGO_BLOCK_MFMA  # does not fit LDS
     # tuning.image_min_items asks for more (image, 128-row group) work items before the image kernel is taken
-    picky, _ = make_kernel(case, capi.ALGO_AUTO, tuning=capi.tuning(image_min_items=128))
+    picky, _ = make_kernel(case, capi.ALGO_AUTO, tuning=capi.tuning(image_min_items=128, chunk_mfma=capi.TUNE_NEVER))
     assert L.pl_sparse_conv_algo_for(picky._handle, 64, 196) == capi.ALGO_IMAGE_MFMA
     assert L.pl_sparse_conv_algo_for(picky._handle, 2, 196) == capi.ALGO_BLOCK_MFMA
     assert L.pl_sparse_conv_algo_for(picky._handle, 1, 196) == capi.ALGO_ROW_WALK         # 196 positions in all
@@ -322,7 +323,7 @@ def test_image_rows_slabs_bit_exact(shape, kind):
         got = run_hip(case, capi.ALGO_IMAGE_MFMA)
         assert_same(case, got, want, "image slabs %s %s %s" % (kind, act, shape))
         # the automatic choice takes the slabs for these few work items and gives the same bits
-        kernel, _ = make_kernel(case, capi.ALGO_AUTO)
+        kernel, _ = make_kernel(case, capi.ALGO_AUTO, tuning=capi.tuning(chunk_mfma=capi.TUNE_NEVER))
         assert capi.lib().pl_sparse_conv_algo_for(kernel._handle, batch, h * w) == capi.ALGO_IMAGE_MFMA
         assert np.array_equal(run_hip(case, kernel=kernel), got)
         # and the block kernel agrees
