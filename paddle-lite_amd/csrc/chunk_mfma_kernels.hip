@@ -287,39 +287,63 @@ hipError_t Launch(int nw, const ChunkMfmaParams& p, dim3 grid, hipStream_t s) {
 int ChunkMfmaPaddedSteps(int K) { return (K + 511) / 512 * 8; }
 bool ChunkMfmaFits(int K, int hw) { return K >= 16 && hw >= 4; }
 
+ChunkMfmaPlan PlanChunkMfma(int out_kind, int cus, int tile_positions, int K, int M, int hw, int batch) {
+  const int qpi = (hw + 3) / 4, ksteps = (K + 63) / 64;
+  const int64_t total_quads = (int64_t)batch * qpi;
+  auto plan_for = [&](int nw) {
+    ChunkMfmaPlan p{};
+    p.nw = nw;
+    // whole images per tile where they fit: their channel rows lie back to back, so no line is fetched in parts
+    p.tile_quads = qpi <= 16 * nw ? 16 * nw / qpi * qpi : 16 * nw;
+    p.tiles = (int)((total_quads + p.tile_quads - 1) / p.tile_quads);
+    p.row_groups = ((M + 15) / 16 + 7) / 8;
+    p.chunks = (ksteps + 8 / nw - 1) / (8 / nw);
+    p.workgroups = 8ll * p.row_groups * ((p.tiles + 7) / 8);
+    return p;
+  };
+  if (tile_positions != 0) return plan_for(tile_positions / 64);
+  // The tile width: a CU holds one workgroup, a workgroup takes about 3 us and 1.35 us per chunk, so the fewest rounds
+  // times that, rounds being what the XCD with the most workgroups needs.  2048 -> 2048 @14x14 x 16: 256 positions 24.6 us
+  // (one round of 16 chunks), 128 36.6 (two of 8), 64 44.7 (four of 4); 1024 -> 256 @14x14 x 32: 14.6, 12.7 and 9.9 (one
+  // round each); 608 -> 736 @9x8 x 42: 11.4 (one round), 13.2 and 12.9 (two).
+  const ChunkMfmaPlan widest = plan_for(4);
+  ChunkMfmaPlan best{};
+  int64_t least = 0;
+  for (int nw : {1, 2, 4}) {
+    const ChunkMfmaPlan p = nw == 4 ? widest : plan_for(nw);
+    const int64_t cost = (p.workgroups + cus - 1) / cus * (300 + 135 * p.chunks);
+    if (nw == 1 || cost < least) least = cost, best = p;
+  }
+  // Over several rounds what all workgroups together read counts more than how full the last round is, and the widest
+  // tile reads the weights the fewest times: it from a round and a half of its workgroups on (with one-byte output and on
+  // ragged maps, where whole images leave up to a fifth of a tile empty, beyond two and a half).  us with the width of the
+  // formula above / the widest: 2048 -> 2048 @14x14 x 64 131 / 98 (int8 output 111 / 89), 1280 -> 2048 @14x14 x 128 195 /
+  // 149, 2048 -> 1024 @28x28 x 24 96 / 84; at two and a half rounds 768 -> 1024 @14x14 x 80 with int8 output 35.0 / 36.6,
+  // 2048 -> 1024 @7x7 x 300 101 / 112.
+  const bool few_rounds_count = out_kind == kOutI8 || hw % 4 != 0;
+  if (few_rounds_count ? 2 * widest.workgroups > 5ll * cus : 2 * widest.workgroups >= 3ll * cus) best = widest;
+  return best;
+}
+
 hipError_t LaunchChunkMfma(int out_kind, int cus, int tile_positions, const ChunkMfmaParams& p, hipStream_t stream) {
   if (p.batch <= 0 || p.M <= 0) return hipSuccess;
   if (!ChunkMfmaFits(p.K, p.hw)) return hipErrorInvalidValue;
   const int64_t positions = (int64_t)p.batch * p.hw;
   // tensor offsets are kept in 32 bits
   if (positions * p.K >= (1ll << 31) || positions >= (1ll << 31) - 512) return hipErrorInvalidValue;
+  const ChunkMfmaPlan plan = PlanChunkMfma(out_kind, cus, tile_positions, p.K, p.M, p.hw, p.batch);
   ChunkMfmaParams q = p;
   q.qpi = (p.hw + 3) / 4;
   q.quad_aligned = p.hw % 4 == 0;
   q.total_quads = (uint32_t)p.batch * (uint32_t)q.qpi;
   q.row_tiles = (p.M + 15) / 16;
-  q.ksteps = (p.K + 63) / 64;
   q.padded_ksteps = ChunkMfmaPaddedSteps(p.K);
-  q.row_groups = (q.row_tiles + 7) / 8;
-  // whole images per tile where they fit: their channel rows lie back to back, so no line is fetched in parts
-  auto tile_quads = [&](int nw) { return q.qpi <= 16 * nw ? 16 * nw / q.qpi * q.qpi : 16 * nw; };
-  auto tiles = [&](int nw) { return (int)((q.total_quads + tile_quads(nw) - 1) / tile_quads(nw)); };
-  // The tile width: a CU holds one workgroup, a workgroup takes about 3 us and 1.35 us per chunk, so the fewest rounds
-  // times that, rounds being what the XCD with the most workgroups needs.  2048 -> 2048 @14x14 x 16: 256 positions 24.6 us
-  // (one round of 16 chunks), 128 36.6 (two of 8), 64 44.7 (four of 4); 1024 -> 256 @14x14 x 32: 14.6, 12.7 and 9.9 (one
-  // round each); 608 -> 736 @9x8 x 42: 11.4 (one round), 13.2 and 12.9 (two).
-  int nw = 1;
-  int64_t best = 0;
-  for (int w : {1, 2, 4}) {
-    const int64_t rounds = ((int64_t)((tiles(w) + 7) / 8) * q.row_groups * 8 + cus - 1) / cus;
-    const int64_t cost = rounds * (300 + 135 * ((q.ksteps + 8 / w - 1) / (8 / w)));
-    if (w == 1 || cost < best) best = cost, nw = w;
-  }
-  if (tile_positions != 0) nw = tile_positions / 64;
-  q.tile_quads = tile_quads(nw);
-  q.tiles = tiles(nw);
-  q.chunks = (q.ksteps + 8 / nw - 1) / (8 / nw);
-  const int64_t wgs = 8ll * q.row_groups * ((q.tiles + 7) / 8);
+  q.row_groups = plan.row_groups;
+  q.tile_quads = plan.tile_quads;
+  q.tiles = plan.tiles;
+  q.chunks = plan.chunks;
+  const int nw = plan.nw;
+  const int64_t wgs = plan.workgroups;
   if (wgs > (1ll << 30)) return hipErrorInvalidValue;
   const dim3 grid((uint32_t)wgs);
   switch (out_kind) {

@@ -307,16 +307,24 @@ struct ChunkMfmaParams {
   int quad_aligned;      // hw % 4 == 0
   uint32_t total_quads;  // batch * qpi
   int row_tiles;         // ceil(M / 16)
-  int ksteps;            // ceil(K / 64)
   int padded_ksteps;     // steps wtiles holds, the last ones zero
   int chunks;
   int tile_quads;        // position quads of a tile
   int tiles, row_groups;
 };
 
+// How a call is divided: a tile width, the workgroups it makes (of 128 rows x one tile; a CU holds one at a time) and
+// the chunks of channels each of them takes.
+struct ChunkMfmaPlan {
+  int nw;  // position quads per tile / 16
+  int tile_quads, tiles, row_groups, chunks;
+  int64_t workgroups;
+};
+
 int ChunkMfmaPaddedSteps(int K);  // 64-channel steps of the weight tiles: whole chunks of the widest kind
 bool ChunkMfmaFits(int K, int hw);
 // tile_positions: positions of a tile (64, 128 or 256), 0 = chosen by the number of CUs
+ChunkMfmaPlan PlanChunkMfma(int out_kind, int cus, int tile_positions, int K, int M, int hw, int batch);
 hipError_t LaunchChunkMfma(int out_kind, int cus, int tile_positions, const ChunkMfmaParams& p, hipStream_t stream);
 
 // Image MFMA SpMM (int8, image_mfma_kernels.hip): one workgroup per (image,

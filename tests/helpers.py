@@ -121,10 +121,11 @@ def forced_algo(algo):
     return dict(algo=algo, tuning=None if algo == capi.ALGO_AUTO else capi.tuning(chunk_mfma=capi.TUNE_NEVER))
 
 
-def algo_times(case, warm=100, steps=500, repeats=3, max_sets=24, rotation_bytes=320 << 20):
+def algo_times(case, warm=100, steps=500, repeats=3, max_sets=24, rotation_bytes=320 << 20, chunk_positions=()):
     """Device time per launch (us, events inside pl_sparse_conv_run_sequence) of an int8 case with the
-    algorithm left to the handle ("auto") and with each algorithm forced; an algorithm the shape is outside of
-    is left out.  Every handle's output on the first two images is compared with the oracle before it is
+    algorithm left to the handle ("auto") and with each algorithm forced, the one that takes the channels chunk
+    by chunk also with each of the tile widths in `chunk_positions`; an algorithm the shape is outside of is
+    left out.  Every handle's output on the first two images is compared with the oracle before it is
     timed.  Buffer sets rotate (up to `max_sets` of them, `rotation_bytes` in all); the runs of the handles are
     interleaved `repeats` times and the smallest time of each is kept, so that a clock ramp or another
     process's burst does not land on one algorithm.  Returns (times, name of the algorithm auto picked)."""
@@ -146,9 +147,12 @@ def algo_times(case, warm=100, steps=500, repeats=3, max_sets=24, rotation_bytes
     nchk = min(case.batch, 2)
     want = run_oracle(case, x=case.x[:nchk])
     handles = {}
-    for name, algo in [("auto", capi.ALGO_AUTO)] + [(n, a) for a, n in sorted(ALGO_NAMES.items())]:
+    wanted = [("auto", capi.ALGO_AUTO, forced_algo(capi.ALGO_AUTO))] + [(n, a, forced_algo(a)) for a, n in sorted(ALGO_NAMES.items())]
+    for width in chunk_positions:
+        wanted.append(("chunk_mfma_%d" % width, capi.ALGO_CHUNK_MFMA, dict(algo=capi.ALGO_AUTO, tuning=capi.tuning(chunk_mfma=capi.TUNE_ALWAYS, chunk_positions=width))))
+    for name, algo, how in wanted:
         try:
-            k, _ = make_kernel(case, **forced_algo(algo))
+            k, _ = make_kernel(case, **how)
         except capi.SparseConvError:
             continue
         if algo != capi.ALGO_AUTO and L.pl_sparse_conv_algo_for(k._handle, case.batch, case.im_size) != algo:

@@ -6,7 +6,7 @@ automatic handle is more than 15 % (plus 0.3 us of timer resolution on these 4 t
 the best forced algorithm."""
 import pytest
 
-from helpers import algo_times, workloads
+from helpers import algo_times, pla, workloads
 
 pytestmark = pytest.mark.gpu
 
@@ -29,3 +29,24 @@ def test_auto_is_within_15_percent_of_the_best_forced_algorithm(shape):
             if times["auto"] > 1.15 * best + 0.3:
                 slow.append("batch %d: auto (%s) %.2f us, %s %.2f us" % (batch, picked, times["auto"], best_name, best))
     assert not slow, "; ".join(slow)
+
+
+# (batch, ic, oc, side, output): wide layers over several rounds of the workgroups that the device holds at once
+WIDE_LAYERS = [(64, 2048, 2048, 14, "fp32"), (64, 2048, 2048, 14, "int8"), (24, 2048, 1024, 28, "fp32")]
+
+
+@pytest.mark.parametrize("layer", WIDE_LAYERS, ids=lambda l: "%dx%dx%d_%d_%s" % l)
+def test_auto_is_within_15_percent_on_wide_layers(layer):
+    check_layer(*layer)
+
+
+def check_layer(batch, ic, oc, side, out, sparsity=0.85):
+    print("auto choice", batch, ic, oc, side, out, sparsity, flush=True)
+    case = workloads.make_int8("%dx%dx%d_%d" % (batch, ic, oc, side), batch, ic, oc, side, side, sparsity, False, pla.ActivationParam("leaky_relu", Leaky_relu_alpha=0.1), out_int8=out == "int8", seed=ic + oc,
+                               output_scale=0.2 * (ic / 64.0)**0.5 if out == "int8" else 1.0)
+    times, picked = algo_times(case, warm=30, steps=100, chunk_positions=(64, 128, 256))
+    best_name, best = min(((k, v) for k, v in times.items() if k != "auto"), key=lambda kv: kv[1])
+    if times["auto"] > 1.15 * best + 0.3:
+        times, picked = algo_times(case, warm=60, steps=200, repeats=5, chunk_positions=(64, 128, 256))
+        best_name, best = min(((k, v) for k, v in times.items() if k != "auto"), key=lambda kv: kv[1])
+    assert times["auto"] <= 1.15 * best + 0.3, "auto (%s) %.2f us, %s %.2f us" % (picked, times["auto"], best_name, best)
