@@ -797,49 +797,112 @@ int AlgoBesideChunkMfma(const pl_sparse_conv_handle* h, int batch, int im_size, 
 }
 
 // Whether the kernel that takes the channels chunk by chunk (chunk_mfma_kernels.hip) runs a call that
-// AlgoBesideChunkMfma gives to `call_algo`.  It spreads a call over the chip in workgroups of 128 rows x 64 - 256 positions, pays one short load -
-// multiply chain per 512 channels and does not care about the map's alignment.  Measured at 85 % zeros with fp32
-// output (us, it against what ran before):
-//  * more than 512 channels: 512 rows of 2048 channels on 7 x 7 maps 10.0 / 10.9 / 13.5 against 21.3 / 28.7 / 27.6 at
-//    1 / 16 / 64 images, 768 -> 768 @12x12 7.8 against 19.8 at 16, 2048 -> 2048 @14x14 24.7 against 31.5 at 16; level with
-//    the block kernel on 1024 -> 256 @14x14 at 64 (14.5 / 13.6, int8 output 12.8 / 13.4);
-//  * maps that are no multiple of four positions, which the block kernel loads with clamped addresses, up to two of its
-//    tiles per CU: 192 -> 384 @17x17 5.7 against 8.4 at 8 images, 13.4 against 14.7 at 64; 146 -> 231 @35x35 20.9 against 17.5
-//    at 36 (690 tiles); with at most 128 channels up to half a tile per CU: 96 -> 128 @13x11 5.6 against 8.3 at 23; 99 -> 143
-//    @27x24 10.4 against 6.4 at 32 (324 tiles);
-//  * channel counts that are no multiple of 16, likewise clamped there, up to a tile for every fourth CU: 117 -> 91 @8x8 4.1
-//    against 7.2 at 9; 125 -> 227 @18x18 6.2 against 5.2 at 17 (88 tiles);
-//  * up to 512 channels otherwise only where the block kernel has a tile for less than half the CUs: 512 -> 128
-//    @28x28 5.6 against 7.3 at 8 images but 10.8 against 8.2 at 32, 384 -> 96 @14x14 5.3 against 7.6 at 16, 256 -> 64
-//    @56x56 4.4 against 4.6 at 1 but 10.0 against 6.3 at 16;
-//  * calls of at most 256 positions, in place of the row walk, from 8192 weights on: 96 -> 576 @14x14 4.2 against 5.2, 160 ->
-//    960 @7x7 4.8 against 11.3, 288 -> 32 @8x8 3.7 against 3.8; the walk is ahead on 160 -> 32 @8x8 x 2, 3.2 against 3.7;
-//  * in place of the image kernels while those have work items for less than three CUs of eight: 512 -> 512 @14x14 4.2 /
-//    5.4 / 6.2 / 10.5 against 6.4 / 6.5 / 6.9 / 7.3 at 1 / 4 / 16 / 32 images, 1024 -> 1024 @7x7 6.9 / 7.6 against 7.9 / 8.9 at
-//    1 / 16; with 256 channels only up to eight items: 256 -> 512 @14x14 4.2 / 5.2 against 4.6 / 4.7 at 1 / 4.
-bool ChunkMfmaPays(const pl_sparse_conv_handle* h, int call_algo, int batch, int im_size) {
+// AlgoBesideChunkMfma gives to another kernel.  It spreads a call over the chip in workgroups of 128 rows x 64 - 256
+// positions, one per CU, pays one load - multiply chain per 512 channels and does not care about the map's alignment.
+// The rules below separate 68 000 measured calls of 65 - 2300 channels, 8 - 2300 rows, maps of 20 - 3600 positions at 1 - 128
+// images, 70 - 95 % zeros, both outputs; times are us per launch, 85 % zeros unless stated, this kernel against the other.
+
+// In place of the row walk (at most 256 positions).  On maps that are no multiple of four positions the walk moves its
+// tensors byte by byte: 96 -> 256 @7x7 4.6 / 4.7, 520 -> 64 @9x9 6.7 / 9.9, 72 -> 64 4.5 / 4.2.  Elsewhere both times in units of
+// 0.01 us, fitted to 4400 calls: the walk pays for its channels, its lists, tiles that cross images off the 16-position
+// grid and row groups behind those that run at once, this kernel for chunks of 512 channels.  384 -> 96 @14x14 4.1 / 4.4,
+// 520 -> 64 5.5 / 4.8, 768 -> 256 at 95 / 85 / 70 % zeros 5.5 / 4.6, 5.6, 6.5; 144 -> 512 4.1 / 4.6, 2048 -> 2048 9.1 / 47.
+bool ChunkMfmaBeatsWalk(const pl_sparse_conv_handle* h, int im_size, bool aligned16) {
+  if (im_size % 4 != 0 || !aligned16) return h->ic >= 96 || h->n_groups >= 512;
+  const int groups = std::max(1, h->n_groups), chunks = CeilDiv(h->ic, 512);
+  const int64_t list = h->entries / groups;
+  int64_t walk = 287 + h->ic * 23ll / 100 + list * (h->semi ? 215 : 73) / 100, chunk = 276 + 131 * chunks;
+  if (im_size % 16 != 0) walk += 35 + h->ic / 10, chunk += 18 + 16 * chunks;
+  if (im_size < 32) chunk += 22 + 40 * chunks;
+  walk += std::max(0, groups - (h->ic > 1280 ? 512 : 256)) * (115ll + h->ic / 20) / 256;
+  return walk >= chunk;
+}
+
+// In place of an image kernel, while that has work items for less than three CUs of eight: 512 -> 512 @14x14 4.2 / 5.4 /
+// 6.2 / 10.5 against 6.4 / 6.5 / 6.9 / 7.3 at 1 / 4 / 16 / 32 images, 1024 -> 1024 @7x7 6.9 / 7.6 against 7.9 / 8.9 at 1 / 16.
+// With 256 channels only on maps of 196 positions and more, for one or two images or up to eight slabs: 256 -> 512 @14x14
+// 0.91, 1.0 and 1.08 of the image kernel's time at 1, 2 and 8 images, 256 -> 128 @28x28 0.92 at one; at 8 x 8 1.12 - 1.2, at 7 x 7
+// 1.2 - 1.27 whatever the batch.  With 128 channels never (1.0 - 1.6).
+bool ChunkMfmaBeatsImage(const pl_sparse_conv_handle* h, int batch, int im_size, int cus) {
+  if (h->image_kernel != 0 || h->ic < 256) return false;
+  const bool slabs = im_size > 256;
+  const int64_t images = im_size == 49 ? (batch + 1) / 2 : static_cast<int64_t>(batch) * (slabs ? im_size / 196 : 1);
+  const int64_t items = images * (h->oc / 128);
+  if (h->ic < 512) return im_size >= 196 && items <= 8 && (slabs || batch <= 2);
+  return items * 8 < 3 * cus;
+}
+
+// In place of the block kernel, by the tiles of 128 rows x 128 positions that kernel makes, by the same as this kernel's
+// widest tiles hold (`halves`: whole images leave some of them empty) and by this kernel's workgroups, all per CU.
+bool ChunkMfmaBeatsBlock(const pl_sparse_conv_handle* h, int batch, int im_size, int cus) {
+  if (h->mfma_tile_quads != 0 || h->mfma_sub_tiles != 1 || h->mfma_stream != 1) return false;  // the block kernel in a form asked for
+  const int64_t positions = static_cast<int64_t>(batch) * im_size;
+  if (positions <= 256) return true;
+  const int ic = h->ic, oc = h->oc;
+  const bool one_byte = h->kind == PL_KIND_INT8_INT8, ragged = im_size % 4 != 0;
+  const int64_t tiles = (positions + 127) / 128 * CeilDiv(oc, 128);
+  if (ic <= 128) {
+    // Ragged maps, which the block kernel loads with clamped addresses: up to a tile for every second CU (96 -> 128 @13x11
+    // 5.6 / 8.3 at 23 images), with one row tile and four-byte output only the smallest and the largest (128 -> 16 @17x17 x 16
+    // 5.7 / 4.8).
+    if (ragged) return tiles * 2 <= cus && (oc > 16 || one_byte || im_size < 64 || im_size > 512);
+    // Channel counts that are no multiple of 16, clamped likewise, up to a tile for every fourth CU: 117 -> 91 @8x8 4.1 / 7.2 at
+    // 9 images, 65 -> 160 @12x12 5.2 / 9.0; 125 -> 227 @18x18 6.2 / 5.2 at 17 (88 tiles).
+    return ic % 16 != 0 && tiles * 4 <= cus;
+  }
+  const pl::ChunkMfmaPlan plan = pl::PlanChunkMfma(OutKind(h->kind), cus, h->chunk_positions, ic, oc, im_size, batch);
+  if (ic <= 512) {
+    if (!ragged) return tiles * 2 <= cus;  // 512 -> 128 @28x28 5.6 / 7.3 at 8 images, 10.8 / 8.2 at 32; 256 -> 64 @56x56 4.4 / 4.6 at 1
+    if (tiles <= cus) return true;         // 192 -> 384 @17x17 5.7 / 8.4 at 8 images
+    // Up to two tiles per CU: 384 channels 0.76 - 1.02.  Others while rows, not positions, make the tiles many: 192 -> 384
+    // @17x17 x 64 0.84, 192 -> 96 @35x35 x 32 1.12; with one-byte output in one round of workgroups: 192 -> 384 @13x13 x 128 (384
+    // of them) 1.24.
+    if (tiles > 2 * cus) return false;
+    if (ic > 256 && ic <= 384) return true;
+    return one_byte ? plan.workgroups <= cus && oc > 16 : positions <= 150 * cus;
+  }
+  // the block kernel skips blocks of 32 x 32 zeros and this one does not
+  const int64_t blocks = static_cast<int64_t>(h->row_blocks) * h->ksteps;
+  const bool dense = h->blocks_present * 4 >= blocks * 3;
+  // Up to 1024 channels the block kernel holds all of them in LDS, beyond 640 (512 with one-byte output, which stages its
+  // stores there) with room for one workgroup per CU: 768 -> 768 @12x12 7.8 / 19.8 at 16 images, 1024 -> 256 @28x28 x 64 39.1 /
+  // 42.6; 1024 -> 1024 @20x20 x 64 (1600 tiles) with 5 / 30 % of the blocks present 1.34 / 1.2 of its time.
+  if (ic <= 1024 && ic > (one_byte ? 512 : 640)) return one_byte || h->blocks_present * 2 >= blocks || tiles <= 4 * cus;
+  // Two workgroups of the block kernel per CU: it is ahead once there are many tiles, the sooner the more of this kernel's
+  // tiles stay empty.  With one-byte output 2048 -> 2048 @14x14 x 64 (2048 halves) 0.9, 1472 -> 812 @12x12 x 118 (1652, two
+  // fifths empty) 1.5.
+  const int64_t halves = 2ll * pl::PlanChunkMfma(OutKind(h->kind), cus, 256, ic, oc, im_size, batch).tiles * CeilDiv(oc, 128);
+  const bool full = halves * 3 <= tiles * 4;
+  if (one_byte) return dense ? halves <= (full ? 7 : 4) * cus : plan.workgroups <= 3 * cus;
+  if (ic <= 640) {
+    // 520 -> 2048 @20x20 x 32 (1600 tiles) 56.1 / 39.4, 600 -> 96 @28x28 x 64 (392) 15.7 / 13.6, 520 -> 1024 @14x14 x 32 (392) 13.2 /
+    // 16.6; half a block of rows is padding for the block kernel: 600 -> 48 @28x28 x 64 0.89
+    if (ragged) return halves <= 4 * cus || (halves <= 6 * cus && oc <= 48);
+    return tiles * 5 <= 7 * cus || (im_size <= 256 && full && dense && tiles <= 3 * cus) || (oc <= 48 && oc % 32 != 0 && tiles <= 4 * cus);
+  }
+  // 1536 -> 2048 @13x11 x 128 200 / 139, 1280 -> 512 @20x20 x 128 85.9 / 61.2
+  if (ragged) return tiles <= 2 * cus || (halves <= 4 * cus && h->blocks_present * 4 >= blocks);
+  // 2048 -> 2048 @14x14 x 16 (400 tiles) 22.4 / 31.5, @10x10 x 64 (800) 0.85; 1280 -> 256 @28x28 x 32 (392 tiles, 208 workgroups)
+  // 1.14, 1325 -> 1243 @22x22 x 11 (420, 240) 0.78; 2048 -> 256 @28x28 x 64 (784) 0.88
+  if (tiles * 2 <= 3 * cus) return true;
+  if (!dense) return false;
+  return (halves <= 4 * cus && im_size <= 256 && full) || (tiles <= 2 * cus && (ic > 1536 || (plan.workgroups * 10 >= 9 * cus && plan.workgroups <= cus))) || (ic > 1920 && oc <= 256 && tiles <= 4 * cus);
+}
+
+bool ChunkMfmaPays(const pl_sparse_conv_handle* h, int call_algo, int batch, int im_size, bool aligned16) {
   const int64_t positions = static_cast<int64_t>(batch) * im_size;
   if (!h->wchunk.ptr || !pl::ChunkMfmaFits(h->ic, im_size) || positions * h->ic >= (1ll << 31)) return false;
   if (h->chunk_mfma == 2) return true;
   const int cus = std::max(1, h->wg_slots_default / 2);
-  if (call_algo == PL_ALGO_ROW_WALK) return h->auto_int8 && h->oc * h->ic > 8192;
-  if (call_algo == PL_ALGO_IMAGE_MFMA) {
-    if (!h->auto_int8 || h->image_kernel != 0 || h->ic < 256) return false;
-    const int64_t images = im_size == 49 ? (batch + 1) / 2 : static_cast<int64_t>(batch) * (im_size > 256 ? im_size / 196 : 1);
-    const int64_t items = images * (h->oc / 128);
-    return h->ic < 512 ? items <= 8 : items * 8 < 3 * cus;
-  }
-  if (h->mfma_tile_quads != 0 || h->mfma_sub_tiles != 1 || h->mfma_stream != 1) return false;  // the block kernel in a form asked for
-  if (h->ic > 512 || positions <= 256) return true;
-  const int64_t block_tiles = (positions + 127) / 128 * CeilDiv(h->oc, 128);
-  if (h->ic <= 128) return im_size % 4 != 0 ? block_tiles * 2 <= cus : h->ic % 16 != 0 && block_tiles * 4 <= cus;
-  return block_tiles <= (im_size % 4 != 0 ? 2 * cus : cus / 2);
+  if (call_algo == PL_ALGO_ROW_WALK) return ChunkMfmaBeatsWalk(h, im_size, aligned16);
+  if (call_algo == PL_ALGO_IMAGE_MFMA) return ChunkMfmaBeatsImage(h, batch, im_size, cus);
+  return ChunkMfmaBeatsBlock(h, batch, im_size, cus);
 }
 
 // The algorithm of one call (pl_sparse_conv_algo_for reports it).
 int AlgoForCall(const pl_sparse_conv_handle* h, int batch, int im_size, bool aligned16) {
   const int algo = AlgoBesideChunkMfma(h, batch, im_size, aligned16);
-  return ChunkMfmaPays(h, algo, batch, im_size) ? PL_ALGO_CHUNK_MFMA : algo;
+  return ChunkMfmaPays(h, algo, batch, im_size, aligned16) ? PL_ALGO_CHUNK_MFMA : algo;
 }
 
 }  // namespace

@@ -4,6 +4,7 @@ launch, every algorithm the shape allows timed in the same process on the same b
 (helpers.algo_times: parity-checked handles, interleaved runs, best of three).  A cell fails when the
 automatic handle is more than 15 % (plus 0.3 us of timer resolution on these 4 to 17 us launches) slower than
 the best forced algorithm."""
+import numpy as np
 import pytest
 
 from helpers import algo_times, pla, workloads
@@ -40,10 +41,28 @@ def test_auto_is_within_15_percent_on_wide_layers(layer):
     check_layer(*layer)
 
 
-def check_layer(batch, ic, oc, side, out, sparsity=0.85):
-    print("auto choice", batch, ic, oc, side, out, sparsity, flush=True)
+# calls at the borders of the rule for the kernel that takes the channels chunk by chunk: more than 512 channels over many
+# positions, few of them through the row walk, small maps with 256 channels, channel blocks without weights
+BORDERS = [(64, 520, 96, 56, "fp32"), (32, 520, 2048, 20, "fp32"), (128, 1280, 512, 20, "fp32"), (64, 1536, 2048, 17, "fp32"), (128, 1472, 812, 12, "int8"), (2, 96, 128, 10, "int8"),
+           (32, 256, 256, 10, "fp32"), (2, 768, 256, 8, "fp32"), (128, 192, 384, 13, "int8"), (16, 2048, 2048, 14, "fp32"), (64, 192, 384, 17, "fp32"), (16, 600, 600, 12, "fp32")]
+
+
+@pytest.mark.parametrize("layer", BORDERS, ids=lambda l: "%dx%dx%d_%d_%s" % l)
+def test_auto_is_within_15_percent_at_the_borders_of_the_chunk_rule(layer):
+    check_layer(*layer)
+
+
+def test_auto_is_within_15_percent_with_empty_blocks():
+    check_layer(64, 1024, 1024, 20, "fp32", 0.95, blocked=True)
+
+
+def check_layer(batch, ic, oc, side, out, sparsity=0.85, blocked=False):
+    print("auto choice", batch, ic, oc, side, out, sparsity, blocked, flush=True)
     case = workloads.make_int8("%dx%dx%d_%d" % (batch, ic, oc, side), batch, ic, oc, side, side, sparsity, False, pla.ActivationParam("leaky_relu", Leaky_relu_alpha=0.1), out_int8=out == "int8", seed=ic + oc,
                                output_scale=0.2 * (ic / 64.0)**0.5 if out == "int8" else 1.0)
+    if blocked:  # whole 32 x 32 blocks of zeros
+        keep = np.random.RandomState(ic).random_sample((oc // 32, ic // 32)) >= sparsity
+        case.dense = (workloads._int8_nonzero(np.random.RandomState(oc), (oc, ic)) * np.kron(keep, np.ones((32, 32), dtype=bool))).astype(np.int8)
     times, picked = algo_times(case, warm=30, steps=100, chunk_positions=(64, 128, 256))
     best_name, best = min(((k, v) for k, v in times.items() if k != "auto"), key=lambda kv: kv[1])
     if times["auto"] > 1.15 * best + 0.3:
