@@ -151,7 +151,8 @@ typedef struct pl_sparse_conv_tuning {
   int32_t chunk_mfma;        /* (switch) int8 calls with the channels taken chunk
                                 by chunk (PL_ALGO_CHUNK_MFMA), PL_ALGO_AUTO and
                                 PL_ALGO_BLOCK_MFMA; it takes 16 channels and maps
-                                of 4 positions and more                       */
+                                of 4 positions and more.  By the rule, a kernel
+                                that another field names keeps its calls      */
   int32_t chunk_positions;   /* that kernel: positions per tile, 64, 128 or 256 */
 } pl_sparse_conv_tuning;
 

@@ -183,6 +183,7 @@ struct pl_sparse_conv_handle {
   DevBuf wchunk;            // dense 16x64 tiles of the kernel that takes the channels chunk by chunk
   int chunk_mfma = 1;       // that kernel: 0 never, 1 by the rule, 2 whenever the shape allows
   int chunk_positions = 0;  // positions per tile of that kernel; 0 = chosen per problem
+  bool walk_asked = false, block_asked = false, image_asked = false;  // a tuning field names a form of the plain walk / the block kernel / an image kernel
   int mfma_stream = 1;      // streaming block MFMA: 0 never, 1 when the shape suits it, 2 whenever the shape allows
   int mfma_i8_wide = 1;
   int mfma_tile_quads = 0;  // 0 = chosen per problem
@@ -824,7 +825,7 @@ bool ChunkMfmaBeatsWalk(const pl_sparse_conv_handle* h, int im_size, bool aligne
 // 0.91, 1.0 and 1.08 of the image kernel's time at 1, 2 and 8 images, 256 -> 128 @28x28 0.92 at one; at 8 x 8 1.12 - 1.2, at 7 x 7
 // 1.2 - 1.27 whatever the batch.  With 128 channels never (1.0 - 1.6).
 bool ChunkMfmaBeatsImage(const pl_sparse_conv_handle* h, int batch, int im_size, int cus) {
-  if (h->image_kernel != 0 || h->ic < 256) return false;
+  if (h->ic < 256) return false;
   const bool slabs = im_size > 256;
   const int64_t images = im_size == 49 ? (batch + 1) / 2 : static_cast<int64_t>(batch) * (slabs ? im_size / 196 : 1);
   const int64_t items = images * (h->oc / 128);
@@ -835,7 +836,6 @@ bool ChunkMfmaBeatsImage(const pl_sparse_conv_handle* h, int batch, int im_size,
 // In place of the block kernel, by the tiles of 128 rows x 128 positions that kernel makes, by the same as this kernel's
 // widest tiles hold (`halves`: whole images leave some of them empty) and by this kernel's workgroups, all per CU.
 bool ChunkMfmaBeatsBlock(const pl_sparse_conv_handle* h, int batch, int im_size, int cus) {
-  if (h->mfma_tile_quads != 0 || h->mfma_sub_tiles != 1 || h->mfma_stream != 1) return false;  // the block kernel in a form asked for
   const int64_t positions = static_cast<int64_t>(batch) * im_size;
   if (positions <= 256) return true;
   const int ic = h->ic, oc = h->oc;
@@ -894,9 +894,10 @@ bool ChunkMfmaPays(const pl_sparse_conv_handle* h, int call_algo, int batch, int
   if (!h->wchunk.ptr || !pl::ChunkMfmaFits(h->ic, im_size) || positions * h->ic >= (1ll << 31)) return false;
   if (h->chunk_mfma == 2) return true;
   const int cus = std::max(1, h->wg_slots_default / 2);
-  if (call_algo == PL_ALGO_ROW_WALK) return ChunkMfmaBeatsWalk(h, im_size, aligned16);
-  if (call_algo == PL_ALGO_IMAGE_MFMA) return ChunkMfmaBeatsImage(h, batch, im_size, cus);
-  return ChunkMfmaBeatsBlock(h, batch, im_size, cus);
+  // a kernel whose form a tuning field names keeps its calls
+  if (call_algo == PL_ALGO_ROW_WALK) return !h->walk_asked && ChunkMfmaBeatsWalk(h, im_size, aligned16);
+  if (call_algo == PL_ALGO_IMAGE_MFMA) return !h->image_asked && ChunkMfmaBeatsImage(h, batch, im_size, cus);
+  return !h->block_asked && ChunkMfmaBeatsBlock(h, batch, im_size, cus);
 }
 
 // The algorithm of one call (pl_sparse_conv_algo_for reports it).
@@ -985,6 +986,9 @@ int pl_sparse_conv_prepare(const pl_sparse_conv_desc* desc, pl_sparse_conv_handl
   h->walk_chunked = sw(tune.walk_chunked);
   h->chunk_mfma = sw(tune.chunk_mfma);
   h->chunk_positions = tune.chunk_positions;
+  h->walk_asked = tune.walk_tile != 0 || tune.walk_threads != 0 || tune.walk_slices != 0;
+  h->block_asked = tune.mfma_stream != PL_TUNE_RULE || tune.mfma_sub_tiles != PL_TUNE_RULE || tune.mfma_tile_quads != 0 || tune.mfma_narrow_i8_stores != 0 || tune.wg_slots != 0;
+  h->image_asked = tune.image_kernel != 0 || tune.image_min_items != 0 || tune.image_tr_regroup != PL_TUNE_RULE;
   h->mfma_i8_wide = tune.mfma_narrow_i8_stores == 0;
   if (tune.walk_split > 0) h->walk_split = std::min(kTileWalkSplits, tune.walk_split - 1);
   if (tune.mfma_tile_quads > 0) h->mfma_tile_quads = std::max(8, std::min(32, tune.mfma_tile_quads));

@@ -63,3 +63,15 @@ def test_the_choice_is_reported_and_can_be_overridden():
     with pytest.raises(capi.SparseConvError) as e:
         make_kernel(case, capi.ALGO_CHUNK_MFMA)
     assert e.value.code == capi.PL_ERR_BAD_ARG
+
+
+def test_a_kernel_that_a_tuning_field_names_keeps_its_calls():
+    L = capi.lib()
+    # (batch, ic, positions, the kernel without this one, fields that name its form)
+    for batch, ic, im_size, other, fields in ((1, 512, 50, "row_walk", ("walk_tile", "walk_threads", "walk_slices")), (20, 512, 50, "block_mfma", ("mfma_stream", "mfma_sub_tiles", "mfma_tile_quads", "mfma_narrow_i8_stores", "wg_slots")),
+                                              (1, 512, 196, "image_mfma", ("image_kernel", "image_min_items", "image_tr_regroup"))):
+        case = workloads.make_int8("chunk", 1, ic, 512, 1, im_size, 0.85, False, AP(), out_int8=True, seed=3)
+        for field in (None,) + fields:
+            value = {"walk_tile": 64, "walk_threads": 256, "mfma_tile_quads": 16, "wg_slots": 512}.get(field, 1)  # 1: the switches' NEVER, one item, the first image kernel
+            kernel, _ = make_kernel(case, tuning=capi.tuning(**({field: value} if field else {})))
+            assert ALGO_NAMES[capi.check(L.pl_sparse_conv_algo_for(kernel._handle, batch, im_size))] == (other if field else "chunk_mfma"), (other, field)
