@@ -1065,7 +1065,9 @@ int pl_sparse_conv_prepare(const pl_sparse_conv_desc* desc, pl_sparse_conv_handl
     h->auto_walk = rc == PL_OK;
   }
   if (rc == PL_OK && algo == PL_ALGO_BLOCK_MFMA) rc = BuildBlockMfma(L, h);
-  if (rc == PL_OK && algo == PL_ALGO_BLOCK_MFMA && (h->chunk_mfma == 2 ? desc->ic >= 16 : h->chunk_mfma == 1 && desc->ic > 64)) rc = BuildChunkMfma(L, h);
+  // the tiles of the kernel that takes the channels chunk by chunk, where some call can be given to it
+  const bool replaces_any = !h->block_asked || (h->auto_int8 && (!h->walk_asked || !h->image_asked));
+  if (rc == PL_OK && algo == PL_ALGO_BLOCK_MFMA && (h->chunk_mfma == 2 ? desc->ic >= 16 : h->chunk_mfma == 1 && desc->ic > 64 && replaces_any)) rc = BuildChunkMfma(L, h);
   if (rc == PL_OK && (algo == PL_ALGO_IMAGE_MFMA || (h->auto_int8 && (pl::ImageMfmaFits(desc->oc, desc->ic, 16) || pl::ImageMfmaFits(desc->oc, desc->ic, 49))))) rc = BuildImageMfma(L, h);
   if (rc == PL_OK && h->wtiles.ptr && pl::ImageTrMfmaFits(desc->oc, desc->ic, 20)) rc = BuildImageTrMfma(L, h);
   if (rc == PL_OK && h->wtiles.ptr && pl::ImageMfmaRegroupsByTransposingReads(desc->ic, 196)) rc = BuildImageMfmaTrRegroup(L, h);

@@ -75,3 +75,16 @@ def test_a_kernel_that_a_tuning_field_names_keeps_its_calls():
             value = {"walk_tile": 64, "walk_threads": 256, "mfma_tile_quads": 16, "wg_slots": 512}.get(field, 1)  # 1: the switches' NEVER, one item, the first image kernel
             kernel, _ = make_kernel(case, tuning=capi.tuning(**({field: value} if field else {})))
             assert ALGO_NAMES[capi.check(L.pl_sparse_conv_algo_for(kernel._handle, batch, im_size))] == (other if field else "chunk_mfma"), (other, field)
+
+
+def test_weight_tiles_are_held_where_some_call_can_use_them():
+    """Device memory of a handle: tiles of 16 rows x 64 channels in whole chunks of 512 channels, none where a tuning field
+    gives every call to another kernel."""
+    case = workloads.make_int8("chunk", 1, 520, 40, 7, 7, 0.85, False, AP(), out_int8=True, seed=3)
+
+    def size(algo, **fields):
+        return make_kernel(case, algo, tuning=capi.tuning(**fields))[0].info()["device_bytes"]
+
+    assert size(capi.ALGO_AUTO) - size(capi.ALGO_AUTO, chunk_mfma=capi.TUNE_NEVER) == 3 * 16 * 1024  # 40 rows: three tiles
+    assert size(capi.ALGO_BLOCK_MFMA, mfma_tile_quads=16) == size(capi.ALGO_BLOCK_MFMA, mfma_tile_quads=16, chunk_mfma=capi.TUNE_NEVER)
+    assert size(capi.ALGO_AUTO, mfma_tile_quads=16) == size(capi.ALGO_AUTO)  # few positions: in place of the walk
