@@ -808,7 +808,10 @@ int AlgoBesideChunkMfma(const pl_sparse_conv_handle* h, int batch, int im_size, 
 // 0.01 us, fitted to 4400 calls: the walk pays for its channels, its lists, tiles that cross images off the 16-position
 // grid and row groups behind those that run at once, this kernel for chunks of 512 channels.  384 -> 96 @14x14 4.1 / 4.4,
 // 520 -> 64 5.5 / 4.8, 768 -> 256 at 95 / 85 / 70 % zeros 5.5 / 4.6, 5.6, 6.5; 144 -> 512 4.1 / 4.6, 2048 -> 2048 9.1 / 47.
+// From 8192 weights on only.  Below, this kernel is mostly level or behind (160 -> 32 @8x8 x 2 3.7 / 3.2); few rows of many
+// channels on ragged maps would gain there (1000 -> 8 @7x7 5.5 / 11).
 bool ChunkMfmaBeatsWalk(const pl_sparse_conv_handle* h, int im_size, bool aligned16) {
+  if (static_cast<int64_t>(h->oc) * h->ic <= 8192) return false;
   if (im_size % 4 != 0 || !aligned16) return h->ic >= 96 || h->n_groups >= 512;
   const int groups = std::max(1, h->n_groups), chunks = CeilDiv(h->ic, 512);
   const int64_t list = h->entries / groups;
