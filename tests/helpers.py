@@ -74,6 +74,10 @@ _PREC = {capi.KIND_FP32: ("float32", "float32"), capi.KIND_INT8_FP32: ("int8", "
 
 
 def make_kernel(case, algo=capi.ALGO_AUTO, force_semi=None, quirks=False, im_size=None, tuning=None):
+    """ALGO_BLOCK_MFMA without tuning fields means the block kernel on every call: the one that takes the channels chunk by
+    chunk, to which such a handle gives some of them, is kept out."""
+    if algo == capi.ALGO_BLOCK_MFMA and tuning is None:
+        tuning = capi.tuning(chunk_mfma=capi.TUNE_NEVER)
     weights = pla.detect_and_pack(case.dense, im_size or case.im_size, force_semi=force_semi)
     param = pla.SparseConvParam(weights, bias=case.bias, activation_param=case.act, enable_int8=case.kind not in (capi.KIND_FP32, capi.KIND_FP16), input_scale=case.input_scale,
                                 weight_scale=case.weight_scale if case.weight_scale is not None else (), output_scale=case.output_scale)

@@ -1,7 +1,7 @@
 """The int8 kernel that takes the input channels chunk by chunk, against the CPU oracle through the C ABI, bit for
-bit: channel counts around a group of 16, a step of 64 and a chunk, one to seven chunks (each way the loop over the
-chunks can end), rows around a tile of 16 and a group of 128, maps of four positions and more with every remainder
-modulo four, tiles of whole images and tiles that cross images, and each of the three tile widths."""
+bit, at each of its three tile widths: channel counts around a group of 16, a step of 64 and a chunk, one to 25 chunks
+(each way the loop over the chunks can end), rows around a tile of 16 and a group of 128, maps of four positions and more
+with every remainder modulo four, tiles of whole images and tiles that cross images; tensors off the 16-byte grid."""
 import sys
 
 import numpy as np
@@ -13,37 +13,77 @@ pytestmark = pytest.mark.gpu
 
 AP = pla.ActivationParam
 KINDS = {"acc32": capi.KIND_INT8_ACC32, "fp32out": capi.KIND_INT8_FP32, "int8out": capi.KIND_INT8_INT8}
+WIDTHS = (64, 128, 256)
 # (batch, ic, oc, h, w).  64-position tiles hold chunks of 512 channels, 128: 256, 256: 128.
-NARROW = [(1, 513, 17, 2, 2), (3, 520, 1, 1, 5), (5, 527, 127, 2, 3), (2, 600, 129, 7, 7), (1, 1024, 16, 14, 14), (1, 1025, 40, 9, 11), (9, 1536, 33, 3, 3),
-          (1, 2049, 130, 5, 13), (2, 2561, 20, 8, 8), (1, 3100, 24, 1, 7), (4, 79, 140, 5, 9), (2, 65, 200, 3, 5), (1, 512, 512, 14, 14), (1, 200, 72, 12, 12)]
-MIDDLE = [(16, 520, 4096, 8, 8), (3, 1030, 2200, 17, 17)]
-WIDE = [(2, 130, 4096, 31, 33), (2, 330, 4096, 31, 33), (2, 900, 4096, 32, 32)]
+SMALL = [(1, 513, 17, 2, 2), (3, 520, 1, 1, 5), (5, 527, 127, 2, 3), (2, 600, 129, 7, 7), (1, 1024, 16, 14, 14), (1, 1025, 40, 9, 11), (9, 1536, 33, 3, 3), (1, 1900, 24, 5, 6),
+         (1, 2049, 130, 5, 13), (2, 2561, 20, 8, 8), (1, 3100, 24, 1, 7), (4, 79, 140, 5, 9), (2, 65, 200, 3, 5), (1, 512, 512, 14, 14), (1, 200, 72, 12, 12)]
+LARGE = [(16, 520, 4096, 8, 8), (3, 1030, 2200, 17, 17), (2, 130, 4096, 31, 33), (2, 330, 4096, 31, 33), (2, 900, 4096, 32, 32)]
+
+
+def chunk_case(shape, kind, act, paired, seed):
+    batch, ic, oc, h, w = shape
+    case = workloads.make_int8("chunk", batch, ic, oc, h, w, 0.8, paired, AP() if kind == "acc32" else act, out_int8=(kind == "int8out"), seed=seed,
+                               output_scale=0.2 * float(np.sqrt(ic / 64.0)) if kind == "int8out" else 1.0)
+    case.kind = KINDS[kind]
+    return case
+
+
+def chunk_kernel(case, width):
+    """A kernel that runs chunk by chunk on tiles of `width` positions (0: the rule's), which the library confirms."""
+    kernel, _ = make_kernel(case, tuning=capi.tuning(chunk_mfma=capi.TUNE_ALWAYS, chunk_positions=width))
+    assert capi.lib().pl_sparse_conv_algo_for(kernel._handle, case.batch, case.im_size) == capi.ALGO_CHUNK_MFMA
+    return kernel
 
 
 def check(shape, kind, act, paired, seed):
     print("CASE chunk", shape, kind, file=sys.stderr, flush=True)
-    batch, ic, oc, h, w = shape
-    k = KINDS[kind]
-    case = workloads.make_int8("chunk", batch, ic, oc, h, w, 0.8, paired, AP() if kind == "acc32" else act, out_int8=(kind == "int8out"), seed=seed,
-                               output_scale=0.2 * float(np.sqrt(ic / 64.0)) if kind == "int8out" else 1.0)
-    case.kind = k
-    got = run_hip(case, capi.ALGO_BLOCK_MFMA)
+    batch, _, _, h, w = shape
+    case = chunk_case(shape, kind, act, paired, seed)
     few = case.x[:1] if batch * h * w > 1000 else case.x
-    assert_same(case, got[:len(few)], run_oracle(case, oracle_pack(case), x=few), "chunk %s %s" % (shape, kind))
-    if len(few) != batch:  # the last image too: it ends the last tile
-        assert_same(case, got[-1:], run_oracle(case, oracle_pack(case), x=case.x[-1:]), "chunk %s %s, last image" % (shape, kind))
+    want = run_oracle(case, oracle_pack(case), x=few)
+    last = run_oracle(case, oracle_pack(case), x=case.x[-1:]) if len(few) != batch else None
+    for width in (0,) + WIDTHS:
+        got = run_hip(case, kernel=chunk_kernel(case, width))
+        assert_same(case, got[:len(few)], want, "chunk %s %s, width %d" % (shape, kind, width))
+        if last is not None:  # it ends the last tile
+            assert_same(case, got[-1:], last, "chunk %s %s, width %d, last image" % (shape, kind, width))
 
 
 @pytest.mark.parametrize("kind", sorted(KINDS))
-@pytest.mark.parametrize("shape", NARROW, ids=lambda s: "x".join(map(str, s)))
-def test_narrow_tiles(shape, kind):
+@pytest.mark.parametrize("shape", SMALL, ids=lambda s: "x".join(map(str, s)))
+def test_small_calls(shape, kind):
     check(shape, kind, [AP("relu"), AP("hard_swish"), AP("leaky_relu", Leaky_relu_alpha=0.1), AP("relu6")][shape[1] % 4], shape[2] % 2 == 0, shape[1])
 
 
 @pytest.mark.parametrize("kind", sorted(KINDS))
-@pytest.mark.parametrize("shape", MIDDLE + WIDE, ids=lambda s: "x".join(map(str, s)))
-def test_wide_tiles(shape, kind):
+@pytest.mark.parametrize("shape", LARGE, ids=lambda s: "x".join(map(str, s)))
+def test_large_calls(shape, kind):
     check(shape, kind, AP("relu"), False, shape[1])
+
+
+# maps with every remainder modulo four, a last tile that is not full and rows that end inside a tile
+@pytest.mark.parametrize("kind", sorted(KINDS))
+@pytest.mark.parametrize("shape", [(3, 130, 37, 6, 6), (2, 200, 20, 5, 9), (3, 520, 129, 3, 6), (2, 77, 30, 3, 13)], ids=lambda s: "x".join(map(str, s)))
+def test_tensors_off_the_grid_and_their_surroundings(shape, kind):
+    """x and out start 1 - 3 elements behind a 16-byte boundary; the bytes around out stay as they were."""
+    import torch
+
+    print("CASE chunk off the grid", shape, kind, file=sys.stderr, flush=True)
+    case = chunk_case(shape, kind, AP("relu"), False, shape[1])
+    want = run_oracle(case, oracle_pack(case))
+    batch, ic, oc, h, w = shape
+    fill, dtype = (77, torch.int8) if kind == "int8out" else (77, torch.int32) if kind == "acc32" else (77.0, torch.float32)
+    for width in WIDTHS:
+        kernel = chunk_kernel(case, width)
+        for shift in (1, 2, 3):
+            guard = 64 + shift
+            x = torch.randint(-127, 128, (case.x.size + 2 * guard,), dtype=torch.int8, device="cuda")
+            x[guard:guard + case.x.size] = torch.from_numpy(case.x.reshape(-1)).cuda()
+            out = torch.full((want.size + 2 * guard,), fill, dtype=dtype, device="cuda")
+            kernel.Run(x[guard:guard + case.x.size].view(case.x.shape), out[guard:guard + want.size].view(want.shape))
+            host = out.cpu().numpy()
+            assert (host[:guard] == fill).all() and (host[guard + want.size:] == fill).all(), (width, shift)
+            assert_same(case, host[guard:guard + want.size].reshape(want.shape), want, "chunk off the grid %s %s %d %d" % (shape, kind, width, shift))
 
 
 def test_the_choice_is_reported_and_can_be_overridden():

@@ -114,8 +114,8 @@ def test_tile_widths_bit_exact(shape, tq, kind):
 # more than 1024 input channels: the block MFMA kernel takes the k-steps a
 # chunk at a time through one LDS tile.  Aligned and odd images, a channel
 # count off the 32 grid, images smaller than a quad, a chunk count of one
-# plus a remainder.
-MANY_CHANNEL_SHAPES = [(2, 2048, 64, 4, 4), (1, 1100, 40, 6, 6), (1, 1030, 33, 7, 7), (3, 1500, 20, 1, 2), (1, 1056, 128, 8, 8)]
+# plus a remainder; 513 - 1024 channels, which fit LDS at once.
+MANY_CHANNEL_SHAPES = [(2, 2048, 64, 4, 4), (1, 1100, 40, 6, 6), (1, 1030, 33, 7, 7), (3, 1500, 20, 1, 2), (1, 1056, 128, 8, 8), (2, 1024, 72, 10, 10), (3, 700, 33, 9, 9)]
 
 
 @pytest.mark.parametrize("kind", ["acc32", "fp32out", "int8out"])
@@ -128,7 +128,7 @@ def test_many_channels_bit_exact(shape, kind):
     got = run_hip(case, capi.ALGO_BLOCK_MFMA)
     want = run_oracle(case, oracle_pack(case))
     assert_same(case, got, want, "many-channel %s %s" % (kind, shape))
-    # the default choice for int8 is the same kernel now
+    # the automatic choice (the kernel that takes the channels chunk by chunk, or the row walk) gives the same bits
     got_auto = run_hip(case, capi.ALGO_AUTO)
     assert np.array_equal(got_auto, got)
 
