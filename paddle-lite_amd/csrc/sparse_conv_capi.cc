@@ -809,7 +809,7 @@ int AlgoBesideChunkMfma(const pl_sparse_conv_handle* h, int batch, int im_size, 
 // grid and row groups behind those that run at once, this kernel for chunks of 512 channels.  384 -> 96 @14x14 4.1 / 4.4,
 // 520 -> 64 5.5 / 4.8, 768 -> 256 at 95 / 85 / 70 % zeros 5.5 / 4.6, 5.6, 6.5; 144 -> 512 4.1 / 4.6, 2048 -> 2048 9.1 / 47.
 // From 8192 weights on only.  Below, this kernel is mostly level or behind (160 -> 32 @8x8 x 2 3.7 / 3.2); few rows of many
-// channels on ragged maps would gain there (1000 -> 8 @7x7 5.5 / 11).
+// channels on ragged maps would gain there (512 -> 16 @9x9 4.8 / 9.9).
 bool ChunkMfmaBeatsWalk(const pl_sparse_conv_handle* h, int im_size, bool aligned16) {
   if (static_cast<int64_t>(h->oc) * h->ic <= 8192) return false;
   if (im_size % 4 != 0 || !aligned16) return h->ic >= 96 || h->n_groups >= 512;
@@ -885,11 +885,13 @@ bool ChunkMfmaBeatsBlock(const pl_sparse_conv_handle* h, int batch, int im_size,
   }
   // 1536 -> 2048 @13x11 x 128 200 / 139, 1280 -> 512 @20x20 x 128 85.9 / 61.2
   if (ragged) return tiles <= 2 * cus || (halves <= 4 * cus && h->blocks_present * 4 >= blocks);
-  // 2048 -> 2048 @14x14 x 16 (400 tiles) 22.4 / 31.5, @10x10 x 64 (800) 0.85; 1280 -> 256 @28x28 x 32 (392 tiles, 208 workgroups)
-  // 1.14, 1325 -> 1243 @22x22 x 11 (420, 240) 0.78; 2048 -> 256 @28x28 x 64 (784) 0.88
-  if (tiles * 2 <= 3 * cus) return true;
+  // Small maps whose images fill this kernel's tiles, though not the grid of 64 positions that the block kernel's end on:
+  // 2048 -> 2048 @14x14 x 16 (400 tiles) 24.7 / 31.5, with 10 % of the blocks present 24.8 / 29.0, @10x10 x 64 (800) 0.85, but
+  // @8x8 x 128 1.13.  Elsewhere 1280 -> 256 @28x28 x 32 (392 tiles, 208 workgroups) 1.14, 1325 -> 1243 @22x22 x 11 (420, 240) 0.78,
+  // 2048 -> 256 @28x28 x 64 (784) 0.88.
+  if (tiles * 2 <= 3 * cus || (halves <= 4 * cus && im_size <= 256 && im_size % 64 != 0 && full)) return true;
   if (!dense) return false;
-  return (halves <= 4 * cus && im_size <= 256 && full) || (tiles <= 2 * cus && (ic > 1536 || (plan.workgroups * 10 >= 9 * cus && plan.workgroups <= cus))) || (ic > 1920 && oc <= 256 && tiles <= 4 * cus);
+  return (tiles <= 2 * cus && (ic > 1536 || (plan.workgroups * 10 >= 9 * cus && plan.workgroups <= cus))) || (ic > 1920 && oc <= 256 && tiles <= 4 * cus);
 }
 
 bool ChunkMfmaPays(const pl_sparse_conv_handle* h, int call_algo, int batch, int im_size, bool aligned16) {

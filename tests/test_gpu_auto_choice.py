@@ -52,8 +52,9 @@ def test_auto_is_within_15_percent_at_the_borders_of_the_chunk_rule(layer):
     check_layer(*layer)
 
 
-def test_auto_is_within_15_percent_with_empty_blocks():
-    check_layer(64, 1024, 1024, 20, "fp32", 0.95, blocked=True)
+@pytest.mark.parametrize("layer", [(64, 1024, 1024, 20, "fp32"), (16, 2048, 2048, 14, "fp32"), (128, 2048, 2048, 8, "fp32")], ids=lambda l: "%dx%dx%d_%d_%s" % l)
+def test_auto_is_within_15_percent_with_empty_blocks(layer):
+    check_layer(*layer, sparsity=0.95, blocked=True)
 
 
 def check_layer(batch, ic, oc, side, out, sparsity=0.85, blocked=False):
