@@ -10,13 +10,15 @@
 // ahead are issued; the weights (dense tiles in operand order, straight into registers: every wavefront needs its own
 // rows only) are requested one chunk ahead.  One barrier per chunk.
 //
-// What bounds it: the operand reads from LDS.  Every wavefront reads the whole chunk (32 KB at 128 bytes per clock and
-// CU: 2048 clocks for the eight of them, and about 500 for the writes), while the chunk's 256 matrix instructions take
-// 1024 clocks of each SIMD.  A chunk takes 2500 - 3300 clocks with everything in L2; a workgroup whose wavefronts own
-// two or four row tiles and split the channels halves the reads but was no faster on a full chip (25.4 us on
-// 2048 -> 2048 @14x14 x 16 against 24.6: there L2, which serves 170 - 220 MB per launch, limits both).
-// 31.4 -> 24.6 us on that layer (128-position tiles of the block kernel, one 8-step chunk at a time, before), 512 -> 512
-// @14x14 on one image 6.4 -> 4.2, 2048 -> 512 @7x7 on 16 images 28.7 -> 10.9.
+// What bounds it: on a full chip no unit by itself.  2048 -> 2048 @14x14 x 16 (one workgroup per CU, 16 chunks) takes 51 K clocks,
+// 3.2 K per chunk, of which by counters and device rates LDS is busy for 1.6 K (every wavefront reads the whole chunk, 256 KB at
+// 235 bytes per clock and CU; 32 KB of writes at 71), the matrix cores of a SIMD for 1.0 K and its vector ALU for 0.6 K; L2 serves
+// 176 MB of reads per launch, 73 % of its requests from its own lines.  With two wavefronts per SIMD and a barrier per chunk these
+// overlap in part only.  A workgroup whose wavefronts own two or four row tiles and split the channels halves the LDS reads and was
+// no faster there (25.4 us against 24.6).  A call of one chunk is its chain of one load, transpose, multiply and store.
+// us per launch, buffers rotating over 320 MB, the kernel that ran before / this one: that layer (the block kernel) 31.5 / 24.7,
+// on buffers that stay in the last-level cache 31.4 / 22.5; 512 -> 512 @14x14 on one image 6.4 / 4.4; 2048 -> 512 @7x7 on 16 images
+// 30.0 / 10.9.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -303,7 +305,7 @@ ChunkMfmaPlan PlanChunkMfma(int out_kind, int cus, int tile_positions, int K, in
   };
   if (tile_positions != 0) return plan_for(tile_positions / 64);
   // The tile width: a CU holds one workgroup, a workgroup takes about 3 us and 1.35 us per chunk, so the fewest rounds
-  // times that, rounds being what the XCD with the most workgroups needs.  2048 -> 2048 @14x14 x 16: 256 positions 24.6 us
+  // times that, rounds being what the XCD with the most workgroups needs.  2048 -> 2048 @14x14 x 16: 256 positions 24.7 us
   // (one round of 16 chunks), 128 36.6 (two of 8), 64 44.7 (four of 4); 1024 -> 256 @14x14 x 32: 14.6, 12.7 and 9.9 (one
   // round each); 608 -> 736 @9x8 x 42: 11.4 (one round), 13.2 and 12.9 (two).
   const ChunkMfmaPlan widest = plan_for(4);

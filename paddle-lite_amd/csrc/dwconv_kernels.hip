@@ -48,10 +48,10 @@ __device__ __forceinline__ uint32_t LoadBytes4(const int8_t* ptr, const int8_t* 
   return d == 0 ? v : (d < 0 ? up : down);
 }
 
-// The K dwords from `ptr` on, lo - 4 <= ptr < hi, for a tensor of at least 4 * K bytes: the loads are moved inside the
-// tensor as one piece and the bytes shifted into place, those outside [lo, hi) being zero.  A dword at a time, each
-// with its own bounds, the workgroups of the first and the last plane took 1.5 - 2 us longer than the others, and every
-// launch as much longer (us with bounds per dword / per piece: stride 1, 32 planes of 112x112 on 64 images 18.3 / 16.0,
+// The K dwords from `ptr` on, lo - 4 <= ptr < hi - 4 (the bytes are shifted by at most 4 * K - 1), for a tensor of at least
+// 4 * K bytes: the loads are moved inside the tensor as one piece and the bytes shifted into place, those outside [lo, hi)
+// being zero.  A dword at a time, each with its own bounds, the workgroups of the first and the last plane took 1.5 - 2 us
+// longer than the others, and every launch as much longer (us with bounds per dword / per piece: stride 1, 32 planes of 112x112 on 64 images 18.3 / 16.0,
 // on one 4.9 / 3.2; stride 2, 256 of 28x28 7.2 / 5.6 and 4.5 / 3.3).
 template <int K>
 __device__ __forceinline__ void LoadInside(const int8_t* ptr, const int8_t* lo, const int8_t* hi, uint32_t (&D)[K]) {

@@ -1755,10 +1755,12 @@ int pl_sparse_conv_dwconv3x3_fits(const pl_sparse_conv_handle* conv, const pl_dw
 
 int pl_sparse_conv_dwconv3x3_pays(const pl_sparse_conv_handle* conv, const pl_dwconv_handle* dw, int32_t batch, int32_t height, int32_t width) {
   if (!pl_sparse_conv_dwconv3x3_fits(conv, dw, height, width) || batch <= 0) return 0;
-  // Measured on 512 -> 512 @14x14 (us, two launches against one, at 1 / 16 / 32 / 48 / 64 images): stride 2: 9.3 / 8.2,
-  // 9.8 / 8.4, 10.3 / 8.5, 11.0 / 8.6, 11.9 / 8.8; stride 1: 9.6 / 10.7, 10.4 / 11.1, 11.4 / 11.3, 12.7 / 11.5, 13.8 / 11.8.
-  // The one launch does the depthwise work of 128 planes on the CU that made them, whatever the batch; the
-  // depthwise kernel spreads a small batch over the chip.
+  // us, two launches against one, replayed from a graph, at 1 / 4 / 16 / 32 / 64 images @14x14.  Stride 2: 512 -> 512 7.4 / 8.4,
+  // 8.3 / 8.5, 9.4 / 8.5, 10.7 / 8.8, 12.0 / 8.9; 256 -> 512 7.4 / 6.8, 8.0 / 6.9, 8.5 / 6.9, 8.9 / 7.0, 10.3 / 7.4; 128 -> 128 7.2 / 6.0 ...
+  // 7.9 / 6.3.  Stride 1: 512 -> 512 7.7 / 11.0, 8.5 / 11.1, 10.1 / 11.2, 11.8 / 11.6, 14.1 / 12.1; 256 -> 512 7.7 / 9.4, 8.3 / 9.6, 9.2 / 9.7,
+  // 10.2 / 9.9, 12.3 / 10.6.  The one launch does the depthwise work of 128 planes on the CU that made them, whatever the batch;
+  // the depthwise kernel spreads a small batch over the chip.  512 channels at stride 2 would be better off in two launches at
+  // up to four images there, but not where the host paces the calls: from the Python classes two take 10.0 us and one 8.3.
   if (dw->stride == 2) return 1;
   const int64_t workgroups = static_cast<int64_t>(batch) * (conv->oc / 128);
   const int cus = std::max(1, conv->wg_slots_default / 2);
