@@ -853,7 +853,7 @@ bool ChunkMfmaBeatsBlock(const pl_sparse_conv_handle* h, int batch, int im_size,
     // 9 images, 65 -> 160 @12x12 5.2 / 9.0; 125 -> 227 @18x18 6.2 / 5.2 at 17 (88 tiles).
     return ic % 16 != 0 && tiles * 4 <= cus;
   }
-  const pl::ChunkMfmaPlan plan = pl::PlanChunkMfma(OutKind(h->kind), cus, h->chunk_positions, ic, oc, im_size, batch);
+  const auto workgroups = [&] { return pl::PlanChunkMfma(OutKind(h->kind), cus, h->chunk_positions, ic, oc, im_size, batch).workgroups; };
   if (ic <= 512) {
     if (!ragged) return tiles * 2 <= cus;  // 512 -> 128 @28x28 5.6 / 7.3 at 8 images, 10.8 / 8.2 at 32; 256 -> 64 @56x56 4.4 / 4.6 at 1
     if (tiles <= cus) return true;         // 192 -> 384 @17x17 5.7 / 8.4 at 8 images
@@ -862,7 +862,7 @@ bool ChunkMfmaBeatsBlock(const pl_sparse_conv_handle* h, int batch, int im_size,
     // of them) 1.24.
     if (tiles > 2 * cus) return false;
     if (ic > 256 && ic <= 384) return true;
-    return one_byte ? plan.workgroups <= cus && oc > 16 : positions <= 150 * cus;
+    return one_byte ? oc > 16 && workgroups() <= cus : positions <= 150 * cus;
   }
   // the block kernel skips blocks of 32 x 32 zeros and this one does not
   const int64_t blocks = static_cast<int64_t>(h->row_blocks) * h->ksteps;
@@ -876,7 +876,7 @@ bool ChunkMfmaBeatsBlock(const pl_sparse_conv_handle* h, int batch, int im_size,
   // fifths empty) 1.5.
   const int64_t halves = 2ll * pl::PlanChunkMfma(OutKind(h->kind), cus, 256, ic, oc, im_size, batch).tiles * CeilDiv(oc, 128);
   const bool full = halves * 3 <= tiles * 4;
-  if (one_byte) return dense ? halves <= (full ? 7 : 4) * cus : plan.workgroups <= 3 * cus;
+  if (one_byte) return dense ? halves <= (full ? 7 : 4) * cus : workgroups() <= 3 * cus;
   if (ic <= 640) {
     // 520 -> 2048 @20x20 x 32 (1600 tiles) 56.1 / 39.4, 600 -> 96 @28x28 x 64 (392) 15.7 / 13.6, 520 -> 1024 @14x14 x 32 (392) 13.2 /
     // 16.6; half a block of rows is padding for the block kernel: 600 -> 48 @28x28 x 64 0.89
@@ -891,7 +891,10 @@ bool ChunkMfmaBeatsBlock(const pl_sparse_conv_handle* h, int batch, int im_size,
   // 2048 -> 256 @28x28 x 64 (784) 0.88.
   if (tiles * 2 <= 3 * cus || (halves <= 4 * cus && im_size <= 256 && im_size % 64 != 0 && full)) return true;
   if (!dense) return false;
-  return (tiles <= 2 * cus && (ic > 1536 || (plan.workgroups * 10 >= 9 * cus && plan.workgroups <= cus))) || (ic > 1920 && oc <= 256 && tiles <= 4 * cus);
+  if (ic > 1920 && oc <= 256 && tiles <= 4 * cus) return true;
+  if (tiles > 2 * cus || ic > 1536) return tiles <= 2 * cus;
+  const int64_t own = workgroups();
+  return own * 10 >= 9 * cus && own <= cus;  // they fill the chip once
 }
 
 bool ChunkMfmaPays(const pl_sparse_conv_handle* h, int call_algo, int batch, int im_size, bool aligned16) {
