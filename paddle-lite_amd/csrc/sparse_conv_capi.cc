@@ -871,12 +871,12 @@ bool ChunkMfmaBeatsBlock(const pl_sparse_conv_handle* h, int batch, int im_size,
   // stores there) with room for one workgroup per CU: 768 -> 768 @12x12 7.8 / 19.8 at 16 images, 1024 -> 256 @28x28 x 64 39.1 /
   // 42.6; 1024 -> 1024 @20x20 x 64 (1600 tiles) with 5 / 30 % of the blocks present 1.34 / 1.2 of its time.
   if (ic <= 1024 && ic > (one_byte ? 512 : 640)) return one_byte || h->blocks_present * 2 >= blocks || tiles <= 4 * cus;
-  // Two workgroups of the block kernel per CU: it is ahead once there are many tiles, the sooner the more of this kernel's
-  // tiles stay empty.  With one-byte output 2048 -> 2048 @14x14 x 64 (2048 halves) 0.9, 1472 -> 812 @12x12 x 118 (1652, two
-  // fifths empty) 1.5.
+  // Two workgroups of the block kernel per CU: with four-byte output it is ahead once there are many tiles, with one-byte output
+  // where many are met by tiles of this kernel that stay empty: 2048 -> 2048 @14x14 x 64 (2048 halves) 87.6 / 96.6, 1472 -> 812
+  // @12x12 x 118 (1652, two fifths empty) 1.5; over 250 calls of 1024 halves and more without that 0.92 at the median, 1.23 at most.
   const int64_t halves = 2ll * pl::PlanChunkMfma(OutKind(h->kind), cus, 256, ic, oc, im_size, batch).tiles * CeilDiv(oc, 128);
   const bool full = halves * 3 <= tiles * 4;
-  if (one_byte) return dense ? halves <= (full ? 7 : 4) * cus : workgroups() <= 3 * cus;
+  if (one_byte) return dense ? full || halves <= 4 * cus : workgroups() <= 3 * cus;
   if (ic <= 640) {
     // 520 -> 2048 @20x20 x 32 (1600 tiles) 56.1 / 39.4, 600 -> 96 @28x28 x 64 (392) 15.7 / 13.6, 520 -> 1024 @14x14 x 32 (392) 13.2 /
     // 16.6; half a block of rows is padding for the block kernel: 600 -> 48 @28x28 x 64 0.89
