@@ -43,8 +43,10 @@ enum {
  * lite/backends/arm/math/fp16/sparse_conv_fp16.cc, sparse_semi_conv_fp16.cc):
  * the descriptor carries the fp32 sparse tensors and the fp32 bias of the
  * pass, which prepare converts to binary16 like that kernel's PrepareForRun;
- * x_dev / out_dev are binary16, and accumulation and activation run in
- * half precision. */
+ * x_dev / out_dev are binary16 and the activation runs in half precision.
+ * Accumulation runs in half precision in the walks, and in fp32 with one
+ * rounding to binary16 before the activation on the matrix cores
+ * (tuning.float_mfma). */
 enum {
   PL_KIND_FP32 = 0,
   PL_KIND_INT8_FP32 = 1,
@@ -88,7 +90,14 @@ enum {
  * positions among these run as dense 16x64 weight tiles with the channels
  * taken chunk by chunk instead, and so do such calls of a handle prepared
  * for PL_ALGO_BLOCK_MFMA; tuning.chunk_mfma forces or forbids it.
- * pl_sparse_conv_algo_for() reports the choice, that kernel as
+ * A floating-point handle prepared with PL_ALGO_AUTO runs calls whose
+ * nonzeros would take a walk longer as a dense product, too (fp16 beyond
+ * 4e7 weight x position products, fp32 by the expected times of both);
+ * tuning.float_mfma forces or forbids it, and PL_ALGO_ROW_WALK or a walk_*
+ * field keeps every call with the walks.  Positions whose inputs hold an
+ * infinity or a NaN are walked there, so these reach the rows that read them
+ * and no others.
+ * pl_sparse_conv_algo_for() reports the choice, these dense products as
  *   PL_ALGO_CHUNK_MFMA (a report only: pl_sparse_conv_desc.algo takes the
  *                     others). */
 enum { PL_ALGO_AUTO = 0, PL_ALGO_ROW_WALK = 1, PL_ALGO_BLOCK_MFMA = 2, PL_ALGO_IMAGE_MFMA = 3, PL_ALGO_CHUNK_MFMA = 4 };
@@ -154,6 +163,12 @@ typedef struct pl_sparse_conv_tuning {
                                 of 4 positions and more.  By the rule, a kernel
                                 that another field names keeps its calls      */
   int32_t chunk_positions;   /* that kernel: positions per tile, 64, 128 or 256 */
+  int32_t float_mfma;        /* (switch) fp32 / fp16 calls on the matrix cores
+                                (PL_ALGO_CHUNK_MFMA), PL_ALGO_AUTO only; it takes
+                                8 channels and maps of 4 positions and more.  By
+                                the rule, a handle with a walk_* field keeps its
+                                calls with the walks                           */
+  int32_t float_mfma_rows;   /* that kernel: rows per workgroup, 64, 128, 256  */
 } pl_sparse_conv_tuning;
 
 /* Everything PrepareForRun() knows.  All pointers are HOST pointers and are

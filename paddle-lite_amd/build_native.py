@@ -37,6 +37,7 @@ SOURCES = [
     ("chunk_walk_kernels.hip", "chunk_walk_kernels.o", []),
     ("tile_walk_kernels.hip", "tile_walk_kernels.o", []),
     ("fp16_walk_kernels.hip", "fp16_walk_kernels.o", []),
+    ("float_mfma_kernels.hip", "float_mfma_kernels.o", []),
     ("dwconv_kernels.hip", "dwconv_kernels.o", []),
     ("chunk_mfma_kernels.hip", "chunk_mfma_kernels.o", []),
     ("image_mfma_kernels.hip", "image_mfma_kernels.o", []),

@@ -73,6 +73,8 @@ class Tuning(C.Structure):
         ("walk_pairs", C.c_int32),
         ("chunk_mfma", C.c_int32),
         ("chunk_positions", C.c_int32),
+        ("float_mfma", C.c_int32),
+        ("float_mfma_rows", C.c_int32),
     ]
 
 

@@ -1,0 +1,567 @@
+// Floating-point sparse 1x1 convolution as a dense product on the matrix cores (v_mfma_f32_32x32x16_f16), the channels
+// taken chunk by chunk, for the calls whose nonzeros cost a walk more than all weights cost here.
+//
+// One workgroup of eight wavefronts makes a tile of WR x 32 output rows x 128 positions (32 quads).  Per chunk of 64
+// channels a thread loads four channels of one position quad, turns them into operand cells (eight channels of one
+// position, 16 bytes) and writes these to one of two LDS buffers while the other one is multiplied; a wavefront owns 32
+// rows (WR = 8), or shares them with KH - 1 others that take the other channels of every chunk (WR = 4, 2).  Weights
+// come straight into registers, a chunk ahead.  One barrier per chunk.  The vector ALU's share of a step is spread
+// between its matrix instructions: wavefronts issue in order, and both of a SIMD are at the same place.
+//
+// fp16: products and sums are exact to fp32, rounded to half precision once before the activation, which runs in half
+// precision as in the walks (against 64 bits 2.1e-4 in 2-norm, the walks, whose sums are binary16, 8e-4 .. 2.6e-3).
+// fp32: inputs and weights as two binary16 pieces each (22 - 23 bits), three of the four products.  A row's weights are
+// scaled by a power of two at prepare, a position's inputs by one that follows the largest of them seen so far, so
+// pieces keep their bits whatever the magnitudes (a value 2^-12 of its position's largest still has 22).  The products
+// with a low piece have sums of their own: the matrix cores cut sums off instead of rounding them, and every addition
+// to the large sum costs up to an ulp of it (512 channels, 85 % zeros, against 64 bits: 2.2e-7 in 2-norm with one sum, 1.4e-7
+// with two; the walks 1.6e-7).  Positions whose inputs hold an infinity or a NaN, which a dense product spreads through
+// its zero weights, are walked nonzero by nonzero at the end.
+//
+// What bounds it: the way from L2 into a CU.  A chunk of the widest form takes 96 KB in fp32 (64 KB weights, 32 KB inputs;
+// half in fp16) and 2.0 us (0.9), 47 - 53 KB per us and CU, which no depth of prefetch raised (four chunks ahead instead of two:
+// fp16 15.0 -> 16.9 us, the first chunk only arrives later); the matrix instructions of a chunk alone take 1.35 us (0.45).
+// Hence 256 rows x 128 positions (128 x 256 has every weight fetched by two wavefronts: fp16 20.0 against 17.1 us at the
+// time), hence nothing staged twice.  us per launch, buffers rotating over 320 MB, the walk that ran before / this one:
+// fp16 64 x 512 -> 512 @14x14, 85 % zeros 29.4 / 14.5; fp16 8 x 128 -> 256 @55x55, row pairs, 70 % 20.3 / 9.4; fp32 64 x 512 -> 512
+// @14x14, 85 % 34.7 / 25.9; fp32 64 x 1024 -> 1024 @7x7, row pairs, 70 % 60.6 / 29.4.
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+#include <type_traits>
+
+#include "epilogue.h"
+#include "half_act.h"
+#include "kernarg_head.h"
+#include "launch_lds.h"
+#include "sparse_conv_kernels.h"
+
+namespace pl {
+namespace {
+
+using epilogue::ActivateT;
+using epilogue::DispatchAct;
+using half_act::ActivateH;
+using half_act::h1;
+using half_act::h2;
+
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+
+constexpr int kChunk = kFloatMfmaChunk;  // channels of a chunk
+constexpr int kSteps = kChunk / 16;      // matrix instructions' channel steps of a chunk
+constexpr int kQuads = 32;               // position quads of a tile
+constexpr int kThreads = 512;
+constexpr int kGroups = kChunk / 8;      // operand cells of a position and chunk (eight channels each)
+
+// what the first loads need arrives in registers
+PL_IN_HEAD(FloatMfmaParams, x);
+PL_IN_HEAD(FloatMfmaParams, wtiles);
+PL_IN_HEAD(FloatMfmaParams, K);
+PL_IN_HEAD(FloatMfmaParams, hw);
+PL_IN_HEAD(FloatMfmaParams, batch);
+PL_IN_HEAD(FloatMfmaParams, qpi);
+PL_IN_HEAD(FloatMfmaParams, total_quads);
+PL_IN_HEAD(FloatMfmaParams, chunks);
+PL_IN_HEAD(FloatMfmaParams, tiles);
+PL_IN_HEAD(FloatMfmaParams, row_groups);
+PL_IN_HEAD(FloatMfmaParams, row_blocks);
+
+// Four neighbouring positions of one channel.
+template <bool F32>
+using Quad = std::conditional_t<F32, u4, u2>;
+
+// One value of a call whose input holds infinities or NaNs: the nonzeros in index order, as the walks take them.
+__device__ __forceinline__ float WalkF32(const FloatMfmaParams& p, const float* x, int row, float bias) {
+  const DevGroup g = p.groups[p.nr == 2 ? row >> 1 : row];
+  const int r = row - g.row0;
+  float acc = bias;
+  for (uint32_t e = 0; e < g.count; ++e) {
+    const uint32_t k = p.kidx[g.first + e];
+    if (k < (uint32_t)p.K) acc = __builtin_fmaf(x[(size_t)k * p.hw], __uint_as_float(p.wts[(size_t)(g.first + e) * p.nr + r]), acc);
+  }
+  return acc;
+}
+__device__ __forceinline__ h1 WalkF16(const FloatMfmaParams& p, const h1* x, int row, h1 bias) {
+  const DevGroup g = p.groups[p.nr == 2 ? row >> 1 : row];
+  const int shift = 16 * (row - g.row0);
+  h1 acc = bias;
+  for (uint32_t e = 0; e < g.count; ++e) {
+    const uint32_t k = p.kidx[g.first + e];
+    if (k < (uint32_t)p.K) acc = __builtin_fmaf16(x[(size_t)k * p.hw], __builtin_bit_cast(h1, (uint16_t)(p.wts[g.first + e] >> shift)), acc);
+  }
+  return acc;
+}
+
+// LDS: two buffers of operand cells, or what the wavefronts of a row block hand to each other at the end; behind either
+// (a wavefront may still look at the flag when another has begun to hand over), for fp32, the positions' maxima and the
+// flag.
+constexpr int LdsTables(int wr, bool f32) {
+  const int cells = 2 * (f32 ? 2 : 1) * kGroups * 4 * kQuads * 16, trade = 8 * (64 - 8 * wr) * 64 * 4;
+  return cells > trade ? cells : trade;
+}
+
+template <int WR, bool F32, bool RAGGED>
+__device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* xt) {
+  constexpr int QT = kQuads;               // position quads of a tile
+  constexpr int UC = 4;                    // channels a thread brings in of a chunk: half a cell
+  constexpr int KH = 8 / WR;               // wavefronts that share a row block, each with its part of a chunk's steps
+  constexpr int STEPS = kSteps / KH;       // steps of one of them
+  constexpr int FIN = 16 / KH;             // rows per lane that a wavefront finishes
+  constexpr int PIECES = F32 ? 2 : 1;      // binary16 pieces of a value
+  constexpr int DEPTH = 2;                 // chunks of activations in registers
+  constexpr int ADEPTH = 1;                // chunks of weights in registers
+  constexpr int kCells = kGroups * 4 * QT; // cells of a chunk and piece
+  constexpr int kBuf = PIECES * kCells;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // each XCD owns a contiguous range of tiles, the row groups of one tile follow each other there
+  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+  const int first_tile = (xcd * p.tiles) >> 3, last_tile = ((xcd + 1) * p.tiles) >> 3;
+  const int tile = first_tile + slot / p.row_groups, rg = slot % p.row_groups;
+  if (tile >= last_tile) return;
+
+  // the thread's part of a chunk: UC channels of quad j; a partial quad (the end of an image whose size is not a multiple
+  // of 4) is read from the last four positions of its channel row and shifted, threads behind the tensor's last quad
+  // repeat that one
+  const int part = (tid / QT) & 1, j = tid & (QT - 1), kg = tid / (QT * 2);
+  const uint32_t tile_quad0 = (uint32_t)tile * (uint32_t)QT;
+  const uint32_t quad = min(tile_quad0 + (uint32_t)j, p.total_quads - 1u);
+  const uint32_t img = quad / (uint32_t)p.qpi;
+  const int pp = 4 * (int)(quad - img * (uint32_t)p.qpi);
+  const int first = min(pp, p.hw - 4), shift = pp - first;
+  constexpr uint32_t kElem = F32 ? 4u : 2u;
+  const uint32_t vbase = img * (uint32_t)p.K * (uint32_t)p.hw + (uint32_t)first;
+  Quad<F32> r[DEPTH][UC];
+  // Loads of one chunk.  The last group of a channel count that is no multiple of 8 holds the last eight channels,
+  // groups behind it repeat it against weights of zero.  Chunks behind the last one lie outside the buffer: nothing is
+  // fetched for them, and no condition around the loads makes the wait for older ones wait for these too.
+  const __amdgpu_buffer_rsrc_t xbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.x), 0, (int)((uint32_t)p.batch * (uint32_t)p.K * (uint32_t)p.hw * kElem), 0x00020000);
+  const int pitch_in = p.hw * (int)kElem;
+  auto issue = [&](Quad<F32> (&rd)[UC], int chunk) {
+    const uint32_t k = (uint32_t)(min(chunk * kChunk + 8 * kg, p.K - 8) + UC * part);
+    const uint32_t voff = chunk < p.chunks ? (vbase + k * (uint32_t)p.hw) * kElem : 0x80000000u;
+#pragma unroll
+    for (int i = 0; i < UC; ++i) {
+      if constexpr (F32) {
+        rd[i] = __builtin_amdgcn_raw_buffer_load_b128(xbuf, (int)voff, i * pitch_in, 0);
+      } else {
+        rd[i] = __builtin_amdgcn_raw_buffer_load_b64(xbuf, (int)voff, i * pitch_in, 0);
+      }
+    }
+  };
+  auto align_quad = [&](Quad<F32> (&rd)[UC]) {
+    if (!RAGGED) return;
+#pragma unroll
+    for (int i = 0; i < UC; ++i) {
+      if constexpr (F32) {
+        if (shift & 1) rd[i] = u4{rd[i].y, rd[i].z, rd[i].w, rd[i].w};
+        if (shift & 2) rd[i] = u4{rd[i].z, rd[i].w, rd[i].w, rd[i].w};
+      } else {
+        const uint64_t v = (((uint64_t)rd[i].y << 32) | rd[i].x) >> (16 * shift);
+        rd[i] = u2{(uint32_t)v, (uint32_t)(v >> 32)};
+      }
+    }
+  };
+  // the operand cells of position c of the quad: eight channels
+  char* const cells = reinterpret_cast<char*>(xt + kg * (4 * QT) + j) + 2 * UC * part;
+  // fp32: every position's inputs are scaled by a power of two that follows the largest of them seen so far (below)
+  [[maybe_unused]] float scale[4];
+  [[maybe_unused]] float peak = 0.0f;
+  auto put = [](char* dst, const uint32_t (&d)[UC / 2]) {
+    *reinterpret_cast<u2*>(dst) = u2{d[0], d[1]};
+  };
+  auto commit = [&](Quad<F32> (&rd)[UC], int buf, int c) {
+    char* dst = cells + (buf * kBuf + c * QT) * 16;
+    if constexpr (F32) {
+      uint32_t hi[UC / 2], lo[UC / 2];
+#pragma unroll
+      for (int i = 0; i < UC / 2; ++i) {
+        const float a = __uint_as_float(rd[2 * i][c]) * scale[c], b = __uint_as_float(rd[2 * i + 1][c]) * scale[c];
+        peak = fmaxf(peak, fmaxf(fabsf(a), fabsf(b)));
+        const h2 h = __builtin_convertvector((v2f{a, b}), h2);
+        const h2 l = __builtin_convertvector((v2f{a - (float)h.x, b - (float)h.y}), h2);
+        hi[i] = __builtin_bit_cast(uint32_t, h), lo[i] = __builtin_bit_cast(uint32_t, l);
+      }
+      put(dst, hi);
+      put(dst + kCells * 16, lo);
+    } else {
+      const uint32_t sel = c & 1 ? 0x07060302u : 0x05040100u;
+      uint32_t d[UC / 2];
+#pragma unroll
+      for (int i = 0; i < UC / 2; ++i) d[i] = __builtin_amdgcn_perm(rd[2 * i + 1][c >> 1], rd[2 * i][c >> 1], sel);
+      put(dst, d);
+    }
+  };
+
+  // the wavefront's row block (past the last one: the last one again, not stored) and window of 32 quads
+  const int rb = rg * WR + wave % WR, kh = wave / WR;
+  const int n = lane & 31, half = lane >> 5;
+  const int wsteps = p.chunks * kSteps;
+  const __amdgpu_buffer_rsrc_t wbuf =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(static_cast<const char*>(p.wtiles)) + (size_t)min(rb, p.row_blocks - 1) * p.padded_ksteps * (1024 * PIECES), 0, wsteps * (1024 * PIECES), 0x00020000);
+  h8 a[ADEPTH][STEPS][PIECES];
+  auto load_weights = [&](h8 (&dst)[PIECES], int chunk, int ks) {
+#pragma unroll
+    for (int q = 0; q < PIECES; ++q) dst[q] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(wbuf, lane * 16, ((chunk * kSteps + kh * STEPS + ks) * PIECES + q) * 1024, 0));
+  };
+  const uint4* const operand = xt + (2 * STEPS * kh + half) * (4 * QT) + n;
+  // fp32: the products of two high pieces, and those of a high and a low one, which would otherwise each round the sum
+  // of the former (the matrix cores cut sums off rather than round them)
+  v16f acc[4];
+  [[maybe_unused]] v16f rest[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[c][i] = 0.0f, rest[c][i] = 0.0f;
+
+  // The scales of fp32.  colmax holds the bits of the largest magnitude of every position; its exponent gives the scale
+  // that takes it to [2^12, 2^13).  A chunk with a value beyond 2^15 after scaling raises the flag; then everyone takes
+  // the new maxima, brings the sums so far to the new scales and writes that chunk's cells again.
+  uint32_t* const colmax = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(xt) + LdsTables(WR, F32));
+  uint32_t* const flag = colmax + 4 * QT;
+  const uint32_t* const own_max = colmax + 4 * n;  // of the positions whose sums the lane holds
+  [[maybe_unused]] int own_exp[4];
+  auto scale_exp = [](uint32_t bits) { return max(1, min(254, 266 - (int)(bits >> 23))); };
+  auto collect = [&](Quad<F32> (&rd)[UC]) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      float m = 0.0f;
+#pragma unroll
+      for (int i = 0; i < UC; ++i) m = fmaxf(m, fabsf(__uint_as_float(rd[i][c])));
+      atomicMax(&colmax[4 * j + c], __float_as_uint(m));
+    }
+  };
+  auto rescale = [&](Quad<F32> (&rd)[UC], int buf) {
+    collect(rd);
+    __syncthreads();
+    if (tid == 0) *flag = 0;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const uint32_t m = colmax[4 * j + c], om = own_max[c];
+      if (__uint_as_float(m) * scale[c] >= 0x1p15f) scale[c] = __uint_as_float((uint32_t)scale_exp(m) << 23);
+      if (__uint_as_float(om) * __uint_as_float((uint32_t)own_exp[c] << 23) >= 0x1p15f) {
+        const int e = scale_exp(om);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[c][i] = __builtin_amdgcn_ldexpf(acc[c][i], e - own_exp[c]), rest[c][i] = __builtin_amdgcn_ldexpf(rest[c][i], e - own_exp[c]);
+        own_exp[c] = e;
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) commit(rd, buf, c);
+    __syncthreads();
+  };
+
+  // One chunk: kSteps x 4 cells.  Behind the multiplies of a step the next chunk's cells of one position go to the
+  // other buffer; then the loads of the chunk DEPTH behind that one are issued into the registers this frees.
+  constexpr int PF = F32 ? 2 : 3;
+  auto run_chunk = [&](auto slot_c, auto last_c, int chunk) {
+    constexpr bool LAST = decltype(last_c)::value;  // no chunk is left to load
+    constexpr int S = decltype(slot_c)::value, NEXT = (S + 1) % DEPTH, AS = S % ADEPTH;
+    const uint4* const cells_in = operand + (S & 1) * kBuf;
+    uint4 b[PF + 1][PIECES];
+    auto read = [&](int v) {
+#pragma unroll
+      for (int q = 0; q < PIECES; ++q) b[v % (PF + 1)][q] = cells_in[q * kCells + (v >> 2) * 2 * (4 * QT) + (v & 3) * QT];
+    };
+#pragma unroll
+    for (int d = 0; d < PF; ++d) read(d);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ks = 0; ks < STEPS; ++ks) {
+      if (ks == 0) align_quad(r[NEXT]);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int v = 4 * ks + c;
+        if (v + PF < 4 * STEPS) read(v + PF);
+        const h8 xh = __builtin_bit_cast(h8, b[v % (PF + 1)][0]);
+        acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[AS][ks][0], xh, acc[c], 0, 0, 0);
+        if constexpr (F32) {
+          const h8 xl = __builtin_bit_cast(h8, b[v % (PF + 1)][PIECES - 1]);
+          rest[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[AS][ks][PIECES - 1], xh, rest[c], 0, 0, 0);
+          rest[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[AS][ks][0], xl, rest[c], 0, 0, 0);
+        }
+      }
+      if (!LAST || ADEPTH < DEPTH) load_weights(a[AS][ks], chunk + ADEPTH, ks);
+#pragma unroll
+      for (int c = 0; c < KH; ++c) commit(r[NEXT], (S + 1) & 1, KH * ks + c);
+      // the vector ALU's share of a step goes between its matrix instructions: a wavefront issues in order
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        if (4 * ks + c + PF < 4 * STEPS) __builtin_amdgcn_sched_group_barrier(0x100, PIECES, 0);
+#pragma unroll
+        for (int q = 0; q < (F32 ? 3 : 1); ++q) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, F32 ? 2 * KH : KH, 0);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (F32) {
+      if (peak >= 0x1p15f) *flag = 1;
+      peak = 0.0f;
+      __syncthreads();
+      if (__builtin_amdgcn_readfirstlane(*flag) != 0) rescale(r[NEXT], (S + 1) & 1);
+      if (!LAST) issue(r[NEXT], chunk + 1 + DEPTH);
+    } else {
+      if (!LAST) issue(r[NEXT], chunk + 1 + DEPTH);
+      __syncthreads();
+    }
+  };
+  static_assert(kSteps == 4 && STEPS >= 1, "KH positions of the quads are written per step");
+  static_assert(DEPTH % 2 == 0 && DEPTH % ADEPTH == 0, "the buffer and the weights' registers follow from the slot");
+#pragma unroll
+  for (int d = 0; d < DEPTH; ++d) {
+    issue(r[d], d);
+    __builtin_amdgcn_sched_barrier(0);
+    if (d < ADEPTH) {
+#pragma unroll
+      for (int ks = 0; ks < STEPS; ++ks) load_weights(a[d % ADEPTH][ks], d, ks);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  if constexpr (!F32) align_quad(r[0]);
+  if constexpr (F32) {
+    for (int i = tid; i <= 4 * QT; i += kThreads) colmax[i] = 0;  // and the flag
+    __syncthreads();
+    align_quad(r[0]);
+    collect(r[0]);
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      scale[c] = __uint_as_float((uint32_t)scale_exp(colmax[4 * j + c]) << 23);
+      own_exp[c] = scale_exp(own_max[c]);
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < 4; ++c) commit(r[0], 0, c);
+  if constexpr (F32) peak = 0.0f;
+  issue(r[0], DEPTH);
+  __syncthreads();
+  using More = std::false_type;
+  using Last = std::true_type;
+  int chunk = 0;
+  for (; chunk + DEPTH <= p.chunks; chunk += DEPTH) {
+    run_chunk(std::integral_constant<int, 0>(), More(), chunk);
+    run_chunk(std::integral_constant<int, 1>(), More(), chunk + 1);
+    if constexpr (DEPTH == 4) {
+      run_chunk(std::integral_constant<int, 2>(), More(), chunk + 2);
+      run_chunk(std::integral_constant<int, 3>(), More(), chunk + 3);
+    }
+  }
+  if (chunk < p.chunks) {
+    run_chunk(std::integral_constant<int, 0>(), Last(), chunk);
+    if constexpr (DEPTH == 4) {
+      if (chunk + 1 < p.chunks) {
+        run_chunk(std::integral_constant<int, 1>(), Last(), chunk + 1);
+        if (chunk + 2 < p.chunks) run_chunk(std::integral_constant<int, 2>(), Last(), chunk + 2);
+      }
+    }
+  }
+
+  // Lane (n, half) holds rows 8 (i / 4) + 4 half + i % 4 (i = 0 .. 15) of the row block at the four positions of quad n.
+  // Wavefronts that share a row block finish FIN of the sixteen each, from what the others hand over through LDS.
+  float fin[4][FIN];
+  if constexpr (KH == 1) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) fin[c][i] = F32 ? acc[c][i] + rest[c][i] : acc[c][i];
+  } else {
+    // [row block][finishing part][part it comes from, without its own][value][lane]
+    float* const trade = reinterpret_cast<float*>(xt) + (wave % WR) * (KH * (KH - 1) * 4 * FIN * 64) + lane;
+    auto slot_of = [](int to, int from) { return (to * (KH - 1) + (from < to ? from : from - 1)) * (4 * FIN * 64); };
+#pragma unroll
+    for (int to = 0; to < KH; ++to) {
+      if (to == kh) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+          for (int i = 0; i < FIN; ++i) fin[c][i] = F32 ? acc[c][to * FIN + i] + rest[c][to * FIN + i] : acc[c][to * FIN + i];
+      } else {
+        float* const dst = trade + slot_of(to, kh);
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+          for (int i = 0; i < FIN; ++i) dst[(c * FIN + i) * 64] = F32 ? acc[c][to * FIN + i] + rest[c][to * FIN + i] : acc[c][to * FIN + i];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < KH - 1; ++k) {
+      const float* const src = trade + (kh * (KH - 1) + k) * (4 * FIN * 64);
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int i = 0; i < FIN; ++i) fin[c][i] += src[(c * FIN + i) * 64];
+    }
+  }
+  // An infinity or a NaN among the inputs of a position reaches every row of the product through the zero weights: such
+  // quads are left to the walk below.
+  float poison = 0.0f;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) poison = __builtin_fmaf(fin[c][0], 0.0f, poison);
+  const int row_in_block = 4 * half + (32 / KH) * kh, row0 = rb * 32 + row_in_block;
+  const uint32_t oq = tile_quad0 + (uint32_t)n;
+  const uint32_t on = oq / (uint32_t)p.qpi;
+  const int opp = 4 * (int)(oq - on * (uint32_t)p.qpi);
+  int valid = oq >= p.total_quads ? 0 : min(4, p.hw - opp);
+  const bool bad = valid != 0 && poison != poison;
+  const int walked = bad ? valid : 0;
+  if (bad) valid = 0;
+  float bias[FIN];
+  [[maybe_unused]] int row_exp[FIN];
+  const int table = min(rb, p.row_blocks - 1) * 32 + row_in_block;
+  auto bias_of = [&](int row) { return F32 ? static_cast<const float*>(p.bias)[row] : (float)static_cast<const h1*>(p.bias)[row]; };
+#pragma unroll
+  for (int b = 0; b < FIN / 4; ++b) {
+    if constexpr (F32) {
+      const v4f v = p.bias ? *reinterpret_cast<const v4f*>(static_cast<const float*>(p.bias) + table + 8 * b) : v4f{0.0f, 0.0f, 0.0f, 0.0f};
+      const int4 e = *reinterpret_cast<const int4*>(p.row_exp + table + 8 * b);
+      bias[4 * b] = v.x, bias[4 * b + 1] = v.y, bias[4 * b + 2] = v.z, bias[4 * b + 3] = v.w;
+      row_exp[4 * b] = e.x, row_exp[4 * b + 1] = e.y, row_exp[4 * b + 2] = e.z, row_exp[4 * b + 3] = e.w;
+    } else {
+      const u2 v = p.bias ? *reinterpret_cast<const u2*>(static_cast<const h1*>(p.bias) + table + 8 * b) : u2{0u, 0u};
+      const uint32_t d0 = v.x, d1 = v.y;
+      const h2 lo = __builtin_bit_cast(h2, d0), hi = __builtin_bit_cast(h2, d1);
+      bias[4 * b] = (float)lo.x, bias[4 * b + 1] = (float)lo.y, bias[4 * b + 2] = (float)hi.x, bias[4 * b + 3] = (float)hi.y;
+    }
+  }
+  // Stores past the end of the buffer are dropped, so lanes and rows without an output need no branch.
+  constexpr uint32_t kOutside = 0x80000000u;
+  const __amdgpu_buffer_rsrc_t obuf = __builtin_amdgcn_make_buffer_rsrc(p.out, 0, (int)((uint32_t)p.batch * (uint32_t)p.M * (uint32_t)p.hw * kElem), 0x00020000);
+  const uint32_t pitch = (uint32_t)p.hw * kElem;
+  const uint32_t obase = ((on * (uint32_t)p.M + (uint32_t)row0) * (uint32_t)p.hw + (uint32_t)opp) * kElem;
+  auto finish = [&](auto act_c) {
+    constexpr int ACT = decltype(act_c)::value;
+    const uint32_t h0 = p.act_h_words[0], h1w = p.act_h_words[1];
+    const DevActH act_h = {ACT, (uint16_t)h0, (uint16_t)(h0 >> 16), (uint16_t)h1w, (uint16_t)(h1w >> 16)};
+#pragma unroll
+    for (int i = 0; i < FIN; ++i) {
+      const int rr = 8 * (i >> 2) + (i & 3);
+      const uint32_t at = row0 + rr < p.M && valid != 0 ? obase + (uint32_t)rr * pitch : kOutside;
+      const int whole = (int)(valid == 4 ? at : kOutside);
+      if constexpr (F32) {
+        u4 o;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) o[c] = __float_as_uint(ActivateT<ACT>(__builtin_amdgcn_ldexpf(fin[c][i], row_exp[i] + 127 - own_exp[c]) + bias[i], p.act));
+        __builtin_amdgcn_raw_buffer_store_b128(o, obuf, whole, 0, 0);
+        if constexpr (RAGGED) {
+#pragma unroll
+          for (int c = 0; c < 3; ++c) __builtin_amdgcn_raw_buffer_store_b32(o[c], obuf, (int)(valid != 4 && c < valid ? at + 4 * c : kOutside), 0, 0);
+        }
+      } else {
+        const h2 o0 = ActivateH<ACT>(__builtin_convertvector((v2f{fin[0][i] + bias[i], fin[1][i] + bias[i]}), h2), act_h);
+        const h2 o1 = ActivateH<ACT>(__builtin_convertvector((v2f{fin[2][i] + bias[i], fin[3][i] + bias[i]}), h2), act_h);
+        const u2 o = {__builtin_bit_cast(uint32_t, o0), __builtin_bit_cast(uint32_t, o1)};
+        __builtin_amdgcn_raw_buffer_store_b64(o, obuf, whole, 0, 0);
+        if constexpr (RAGGED) {
+#pragma unroll
+          for (int c = 0; c < 3; ++c) __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(o[c >> 1] >> (16 * (c & 1))), obuf, (int)(valid != 4 && c < valid ? at + 2 * c : kOutside), 0, 0);
+        }
+      }
+    }
+    if (walked != 0) {
+      const size_t xat = (size_t)on * p.K * p.hw + opp;
+#pragma unroll 1
+      for (int at = 0; at < FIN * walked; ++at) {
+        const int i = at / walked, c = at - i * walked, rr = 8 * (i >> 2) + (i & 3);
+        if (row0 + rr >= p.M) break;
+        char* dst = static_cast<char*>(p.out) + obase + (size_t)rr * pitch;
+        if constexpr (F32) {
+          reinterpret_cast<float*>(dst)[c] = ActivateT<ACT>(WalkF32(p, static_cast<const float*>(p.x) + xat + c, row0 + rr, p.bias ? bias_of(row0 + rr) : 0.0f), p.act);
+        } else {
+          const h1 v = WalkF16(p, static_cast<const h1*>(p.x) + xat + c, row0 + rr, (h1)(p.bias ? bias_of(row0 + rr) : 0.0f));
+          reinterpret_cast<h1*>(dst)[c] = ActivateH<ACT>(h2{v, v}, act_h).x;
+        }
+      }
+    }
+  };
+  if (row0 < p.M) DispatchAct(p.act.type, finish);
+}
+
+template <int WR, bool F32, bool RAGGED>
+__global__ void __launch_bounds__(kThreads, F32 ? 2 : 4) FloatMfmaKernel(PL_HEAD_PARAMS, const FloatMfmaParams block) {
+  const FloatMfmaParams p = WithHead(block, PL_HEAD_ARGS);
+  extern __shared__ uint4 xt[];
+  FloatMfmaBody<WR, F32, RAGGED>(p, xt);
+}
+
+template <int WR, bool F32>
+hipError_t Launch(const FloatMfmaParams& p, dim3 grid, hipStream_t s) {
+  const dim3 block(kThreads);
+  constexpr size_t lds = LdsTables(WR, F32) + (F32 ? (4 * kQuads + 4) * 4 : 0);
+  return p.quad_aligned ? LaunchWithHead(FloatMfmaKernel<WR, F32, false>, grid, block, lds, s, p) : LaunchWithHead(FloatMfmaKernel<WR, F32, true>, grid, block, lds, s, p);
+}
+
+}  // namespace
+
+int FloatMfmaPaddedSteps(int K) { return (K + kChunk - 1) / kChunk * kSteps; }
+bool FloatMfmaFits(bool f32, int K, int M, int hw, int64_t positions) {
+  // offsets are kept in 32 bits, and the half above 2^31 stands for what is left out
+  const int64_t values = (1ll << 31) / (f32 ? 4 : 2);
+  return K >= 8 && hw >= 4 && positions * K < values && positions * M < values && ((int64_t)K + kChunk) * (M + 31) * 2 < values;
+}
+
+// The rows a workgroup takes: the least of the times fitted to 5600 random calls in fp32 and 4600 in fp16 (32 - 2048
+// channels and rows, 50 - 100 000 positions, 256 CUs); picks the fastest form in all but 5 % of them.  Many rows per workgroup fetch the
+// inputs the fewest times, few rows let small calls fill the chip and halve the chain of a chunk: 64 x 1024 -> 1024 @7x7
+// fp32 256 rows 37.3, 128 rows 29.4, 64 rows 40.9; 64 x 512 -> 512 @14x14 25.9, 34.1, 47.7; one image 96 -> 192 @56x56 8.0, 6.9, 6.4.
+FloatMfmaPlan PlanFloatMfma(bool f32, int cus, int row_blocks, int K, int M, int hw, int batch) {
+  const int64_t tiles = ((int64_t)batch * ((hw + 3) / 4) + kQuads - 1) / kQuads;
+  const int chunks = (K + kChunk - 1) / kChunk;
+  // us: a launch, a chunk of it; full chip (fp32) and every further round of workgroups (fp16: beyond one per CU, two fit)
+  struct Cost {
+    double launch, chunk, full, full_chunk, round, round_chunk;
+  };
+  static constexpr Cost kF32[3] = {{4.5, 1.56, 2.9, 0.89, 4.8, 2.1}, {4.6, 0.98, 2.0, 0.56, 5.0, 1.22}, {4.5, 0.74, 1.2, 0.4, 4.4, 0.82}};
+  static constexpr Cost kF16[3] = {{3.9, 0.67, 0.0, 0.0, 2.5, 1.6}, {4.2, 0.48, 0.0, 0.0, 2.2, 1.14}, {4.0, 0.4, 0.0, 0.0, 3.2, 0.75}};
+  FloatMfmaPlan best{};
+  for (int i = 0; i < 3; ++i) {
+    const int wr = 8 >> i;
+    if (row_blocks != 0 && wr != row_blocks) continue;
+    FloatMfmaPlan p{};
+    p.wr = wr;
+    p.row_groups = ((M + 31) / 32 + wr - 1) / wr;
+    p.workgroups = 8ll * p.row_groups * ((tiles + 7) / 8);
+    const double per_cu = (double)p.workgroups / cus;
+    const Cost& c = f32 ? kF32[i] : kF16[i];
+    double rounds = per_cu > 1.0 ? per_cu - 1.0 : 0.0;
+    if (f32) rounds = (double)((p.workgroups + cus - 1) / cus - 1);
+    p.us = c.launch + c.chunk * chunks + (per_cu < 1.0 ? per_cu : 1.0) * (c.full + c.full_chunk * chunks) + rounds * (c.round + c.round_chunk * chunks);
+    if (best.wr == 0 || p.us < best.us) best = p;
+  }
+  return best;
+}
+
+hipError_t LaunchFloatMfma(bool f32, int cus, int row_blocks, const FloatMfmaParams& p, hipStream_t stream) {
+  if (p.batch <= 0 || p.M <= 0) return hipSuccess;
+  if (!FloatMfmaFits(f32, p.K, p.M, p.hw, (int64_t)p.batch * p.hw)) return hipErrorInvalidValue;
+  const FloatMfmaPlan plan = PlanFloatMfma(f32, cus, row_blocks, p.K, p.M, p.hw, p.batch);
+  FloatMfmaParams q = p;
+  q.qpi = (p.hw + 3) / 4;
+  q.quad_aligned = p.hw % 4 == 0;
+  q.total_quads = (uint32_t)p.batch * (uint32_t)q.qpi;
+  q.row_blocks = (p.M + 31) / 32;
+  q.row_groups = plan.row_groups;
+  q.chunks = (p.K + kChunk - 1) / kChunk;
+  q.padded_ksteps = FloatMfmaPaddedSteps(p.K);
+  q.tiles = (int)((q.total_quads + kQuads - 1) / kQuads);
+  if (plan.workgroups > (1ll << 30)) return hipErrorInvalidValue;
+  const dim3 grid((uint32_t)plan.workgroups);
+  switch (plan.wr) {
+    case 8:
+      return f32 ? Launch<8, true>(q, grid, stream) : Launch<8, false>(q, grid, stream);
+    case 4:
+      return f32 ? Launch<4, true>(q, grid, stream) : Launch<4, false>(q, grid, stream);
+    case 2:
+      return f32 ? Launch<2, true>(q, grid, stream) : Launch<2, false>(q, grid, stream);
+    default:
+      return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace pl

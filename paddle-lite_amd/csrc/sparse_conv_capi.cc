@@ -109,6 +109,28 @@ uint16_t HalfBits(double f) {
   return static_cast<uint16_t>(sign | r);  // subnormal; r == 1024 is the smallest normal number
 }
 
+// binary16 bit pattern -> the same value
+float HalfValue(uint16_t h) {
+  const int e = (h >> 10) & 31, m = h & 1023;
+  if (e != 0 && e != 31) {
+    const uint32_t u = (static_cast<uint32_t>(h & 0x8000u) << 16) | (static_cast<uint32_t>(h & 0x7fffu) << 13) + (112u << 23);
+    float f;
+    std::memcpy(&f, &u, 4);
+    return f;
+  }
+  const float mag = e == 31 ? (m ? NAN : INFINITY) : std::ldexp(static_cast<float>(m), -24);
+  return h & 0x8000u ? -mag : mag;
+}
+
+// HalfBits for the values that are most of a weight matrix: floats that are normal numbers in half precision too
+uint16_t FastHalfBits(float f) {
+  uint32_t u;
+  std::memcpy(&u, &f, 4);
+  const uint32_t a = u & 0x7fffffffu;
+  if (a < 0x38800000u || a >= 0x477fe000u) return HalfBits(f);  // below 2^-14, or may round to infinity
+  return static_cast<uint16_t>(((u >> 16) & 0x8000u) | ((a + 0xfffu + ((a >> 13) & 1u) - (112u << 23)) >> 13));
+}
+
 pl::DevActH ToDevActH(const pl_activation& a) {
   pl::DevActH d{};
   d.type = a.type;
@@ -174,6 +196,11 @@ struct pl_sparse_conv_handle {
   bool half = false;
   pl::DevActH act_h{};
   DevBuf hw_kidx, hw_wts, hw_bias;
+  // fp32 / fp16 on the matrix cores: dense 32x16 tiles, in fp32 the exponents of the rows' scales behind them
+  DevBuf wfloat;
+  size_t float_row_exp = 0;      // where these begin
+  int float_mfma = 1;            // 0 never, 1 by the rule, 2 whenever the shape allows
+  int float_mfma_rows = 0;  // positions per tile; 0 = chosen per problem
   // block MFMA
   int row_blocks = 0, ksteps = 0, kmask_words = 1;
   int64_t blocks_present = 0;
@@ -206,7 +233,7 @@ struct pl_sparse_conv_handle {
   int padded_rows = 0;
 
   int64_t DeviceBytes() const {
-    return static_cast<int64_t>(groups.bytes + kidx.bytes + wts.bytes + cw_desc.bytes + cw_idx.bytes + cw_wts.bytes + hw_kidx.bytes + hw_wts.bytes + hw_bias.bytes + wblocks.bytes + kmask.bytes + wchunk.bytes + wtiles.bytes + wtiles_rg.bytes + wtiles_tr.bytes + wtiles_rows.bytes + tw.DeviceBytes() + tw_narrow.DeviceBytes() + scale.bytes + bias.bytes);
+    return static_cast<int64_t>(groups.bytes + kidx.bytes + wts.bytes + cw_desc.bytes + cw_idx.bytes + cw_wts.bytes + hw_kidx.bytes + hw_wts.bytes + hw_bias.bytes + wfloat.bytes + wblocks.bytes + kmask.bytes + wchunk.bytes + wtiles.bytes + wtiles_rg.bytes + wtiles_tr.bytes + wtiles_rows.bytes + tw.DeviceBytes() + tw_narrow.DeviceBytes() + scale.bytes + bias.bytes);
   }
 };
 
@@ -315,7 +342,7 @@ int BuildHalfWalk(const pl::DecodedLayout& L, pl_sparse_conv_handle* h) {
 
 int UploadHalfBias(pl_sparse_conv_handle* h, const float* bias) {
   if (!bias) return PL_OK;
-  std::vector<uint16_t> b(static_cast<size_t>(h->oc));
+  std::vector<uint16_t> b(static_cast<size_t>(h->padded_rows), 0);
   for (int i = 0; i < h->oc; ++i) b[i] = HalfBits(bias[i]);
   const hipError_t e = h->hw_bias.Upload(b.data(), b.size() * sizeof(uint16_t));
   if (e != hipSuccess) return FailHip(e, "uploading biases");
@@ -599,6 +626,64 @@ int BuildChunkMfma(const pl::DecodedLayout& L, pl_sparse_conv_handle* h) {
     }
   }
   const hipError_t e = h->wchunk.Upload(tiles.data(), tiles.size());
+  if (e != hipSuccess) return FailHip(e, "uploading the weight tiles");
+  return PL_OK;
+}
+
+// Dense tiles take 2 or 4 bytes per weight: not for handles whose nonzeros are fewer than one in 32, which no call was
+// measured with and whose lists are far smaller.
+bool FloatMfmaWanted(const pl_sparse_conv_handle* h) {
+  return h->float_mfma != 0 && h->ic >= 8 && (h->float_mfma == 2 || h->nnz * 32 >= static_cast<int64_t>(h->oc) * h->ic);
+}
+
+// Dense 32x16 binary16 tiles for the floating-point product (FloatMfmaParams::wtiles).
+int BuildFloatMfma(const pl::DecodedLayout& L, pl_sparse_conv_handle* h) {
+  const int blocks = CeilDiv(L.oc, 32), kss = pl::FloatMfmaPaddedSteps(L.ic), pieces = h->half ? 1 : 2;
+  const size_t tile_values = static_cast<size_t>(blocks) * kss * pieces * 512;
+  std::vector<uint16_t> tiles(tile_values + (h->half ? 0 : static_cast<size_t>(blocks) * 64), 0);
+  const uint32_t whole = static_cast<uint32_t>(L.ic) / 8u * 8u;  // channels in whole groups of eight
+  // fp32: a row's weights are scaled by a power of two that takes the largest of them to [2^14, 2^15)
+  std::vector<int32_t> row_exp(static_cast<size_t>(blocks) * 32, 0);
+  bool finite = true;
+  auto value = [](uint32_t bits) {
+    float w;
+    std::memcpy(&w, &bits, 4);
+    return w;
+  };
+  for (const pl::RowGroup& g : L.groups) {
+    float top[2] = {0.0f, 0.0f};
+    for (uint32_t j = 0; j < g.count; ++j) {
+      const float w0 = value(L.w0[g.first + j]), w1 = g.nrows == 2 ? value(L.w1[g.first + j]) : 0.0f;
+      finite = finite && std::isfinite(w0) && std::isfinite(w1);
+      top[0] = std::max(top[0], std::fabs(w0));
+      top[1] = std::max(top[1], std::fabs(w1));
+    }
+    for (int i = 0; i < g.nrows; ++i) row_exp[g.row0 + i] = top[i] > 0.0f ? std::max(-127, std::min(126, std::ilogb(top[i]) - 14)) : 0;
+  }
+  auto put = [&](int row, uint32_t c, float w) {
+    const uint32_t t = c < whole ? c & 7u : 8u - (static_cast<uint32_t>(L.ic) - c);
+    const size_t lane = (static_cast<size_t>(row) & 31u) + 32u * ((c >> 3) & 1u);
+    uint16_t* at = &tiles[((static_cast<size_t>(row >> 5) * kss + (c >> 4)) * pieces * 64 + lane) * 8 + t];
+    at[0] = FastHalfBits(w);
+    if (h->half) {
+      finite = finite && (at[0] & 0x7c00u) != 0x7c00u;
+    } else {
+      at[512] = FastHalfBits(w - HalfValue(at[0]));
+    }
+  };
+  for (const pl::RowGroup& g : L.groups) {
+    float scale[2] = {1.0f, 1.0f};
+    for (int i = 0; !h->half && i < g.nrows; ++i) scale[i] = std::ldexp(1.0f, std::max(-126, std::min(127, -row_exp[g.row0 + i])));
+    for (uint32_t j = 0; j < g.count; ++j) {
+      put(g.row0, L.ic_index[g.first + j], value(L.w0[g.first + j]) * scale[0]);
+      if (g.nrows == 2) put(g.row0 + 1, L.ic_index[g.first + j], value(L.w1[g.first + j]) * scale[1]);
+    }
+  }
+  // an infinite weight would reach every position through the zeros among the inputs
+  if (!finite) return PL_OK;
+  h->float_row_exp = tile_values * sizeof(uint16_t);
+  if (!h->half) std::memcpy(&tiles[tile_values], row_exp.data(), row_exp.size() * sizeof(int32_t));
+  const hipError_t e = h->wfloat.Upload(tiles.data(), tiles.size() * sizeof(uint16_t));
   if (e != hipSuccess) return FailHip(e, "uploading the weight tiles");
   return PL_OK;
 }
@@ -908,8 +993,39 @@ bool ChunkMfmaPays(const pl_sparse_conv_handle* h, int call_algo, int batch, int
   return !h->block_asked && ChunkMfmaBeatsBlock(h, batch, im_size, cus);
 }
 
+// Whether a floating-point call runs on the matrix cores (float_mfma_kernels.hip).  The rules were fitted to 5600 random
+// calls in fp32 and 4600 in fp16, every form and the walk timed (32 - 2048 channels and rows, 50 - 100 000 positions,
+// 70 - 95 % zeros).
+bool FloatMfmaPays(const pl_sparse_conv_handle* h, int batch, int im_size, bool aligned16) {
+  const int64_t positions = static_cast<int64_t>(batch) * im_size;
+  if (!h->wfloat.ptr || !pl::FloatMfmaFits(!h->half, h->ic, h->oc, im_size, positions)) return false;
+  if (!h->walk_plain_fits && !(im_size % 4 == 0 && aligned16)) return false;  // refused by the walks
+  if (h->float_mfma == 2) return true;
+  const int cus = std::max(1, h->wg_slots_default / 2);
+  const double P = static_cast<double>(positions);
+  if (h->half) {
+    // Ahead almost everywhere (1.7 times on average).  Calls of few products keep the walks, whose sums follow the
+    // reference's half precision value for value; either way takes 4 - 9 us.  A call that fills the chip with few nonzeros per row on
+    // maps the walk loads 16 bytes at a time is memory's: 16 x 32 -> 384 @48x48, 93 % zeros 8.1 against 13.0 us here; 102 x 96 -> 200
+    // @20x20, 86 % 9.6 against 11.9.  Of 3260 calls taken 51 are more than 10 % slower than before, by up to 1.55 times.
+    if (P * h->ic * h->oc <= 4e7) return false;
+    return !(im_size % 8 == 0 && aligned16 && h->nnz < 32ll * h->oc && pl::PlanFloatMfma(false, cus, 8, h->ic, h->oc, im_size, batch).workgroups >= cus);
+  }
+  // fp32: where the walk is expected to take 1.1 times as long.  Its time by the form its channels allow (tiles of 128, 64,
+  // 32 and 16 positions): launch and first tile, entries of the index lists, inputs staged and outputs stored (element by
+  // element on ragged maps); within -20 .. +7 % for half of the calls.  Of 1940 calls taken 74 are more than 10 % slower than before, by
+  // up to 1.35 times; 683 others would have gained more than that.
+  const bool vec = im_size % 4 == 0 && aligned16;
+  const int form = h->ic <= 271 ? 0 : (h->ic <= 543 ? 1 : (h->ic <= 1087 ? 2 : 3));
+  static constexpr double kFirst[4] = {0.0, 2.0, 4.0, 8.0}, kEntry[2][4] = {{5.0e-8, 5.0e-8, 7.5e-8, 10.0e-8}, {6.0e-8, 6.0e-8, 9.0e-8, 12.5e-8}};
+  const double walk = (vec ? 3.9 : 5.5) + kFirst[form] + P * (static_cast<double>(h->entries) * kEntry[h->semi][form] + h->ic * (vec ? 6.5e-7 : 8e-7) + h->oc * (vec ? 5.5e-7 : 15e-7)) * 256.0 / cus;
+  if (walk < 1.1 * 5.2) return false;  // less than any form takes
+  return 1.1 * pl::PlanFloatMfma(true, cus, h->float_mfma_rows / 32, h->ic, h->oc, im_size, batch).us < walk;
+}
+
 // The algorithm of one call (pl_sparse_conv_algo_for reports it).
 int AlgoForCall(const pl_sparse_conv_handle* h, int batch, int im_size, bool aligned16) {
+  if (!h->int8) return FloatMfmaPays(h, batch, im_size, aligned16) ? PL_ALGO_CHUNK_MFMA : h->algo;
   const int algo = AlgoBesideChunkMfma(h, batch, im_size, aligned16);
   return ChunkMfmaPays(h, algo, batch, im_size, aligned16) ? PL_ALGO_CHUNK_MFMA : algo;
 }
@@ -940,14 +1056,16 @@ int pl_sparse_conv_prepare(const pl_sparse_conv_desc* desc, pl_sparse_conv_handl
   if (!desc || !out_handle) return Fail(PL_ERR_BAD_ARG, "null argument");
   *out_handle = nullptr;
   // callers compiled against a header without the tuning fields, or without the last ones, pass what they know
-  constexpr size_t kNoTuning = offsetof(pl_sparse_conv_desc, tuning), kNoChunkTuning = kNoTuning + offsetof(pl_sparse_conv_tuning, chunk_mfma);
-  if (desc->struct_size != sizeof(pl_sparse_conv_desc) && desc->struct_size != kNoChunkTuning && desc->struct_size != kNoTuning)
+  constexpr size_t kNoTuning = offsetof(pl_sparse_conv_desc, tuning), kNoChunkTuning = kNoTuning + offsetof(pl_sparse_conv_tuning, chunk_mfma),
+                   kNoFloatTuning = kNoTuning + offsetof(pl_sparse_conv_tuning, float_mfma);
+  if (desc->struct_size != sizeof(pl_sparse_conv_desc) && desc->struct_size != kNoFloatTuning && desc->struct_size != kNoChunkTuning && desc->struct_size != kNoTuning)
     return Fail(PL_ERR_BAD_ARG, "pl_sparse_conv_desc size mismatch (%u vs %zu)", desc->struct_size, sizeof(pl_sparse_conv_desc));
   pl_sparse_conv_tuning tune{};
   std::memcpy(&tune, reinterpret_cast<const char*>(desc) + kNoTuning, std::min<size_t>(desc->struct_size - kNoTuning, sizeof(tune)));
-  for (int32_t sw : {tune.mfma_stream, tune.mfma_sub_tiles, tune.walk_tiled, tune.walk_chunked, tune.image_tr_regroup, tune.walk_pairs, tune.chunk_mfma})
+  for (int32_t sw : {tune.mfma_stream, tune.mfma_sub_tiles, tune.walk_tiled, tune.walk_chunked, tune.image_tr_regroup, tune.walk_pairs, tune.chunk_mfma, tune.float_mfma})
     if (sw < PL_TUNE_RULE || sw > PL_TUNE_ALWAYS) return Fail(PL_ERR_BAD_ARG, "a tuning switch is not PL_TUNE_RULE, PL_TUNE_NEVER or PL_TUNE_ALWAYS");
   if (tune.chunk_positions != 0 && tune.chunk_positions != 64 && tune.chunk_positions != 128 && tune.chunk_positions != 256) return Fail(PL_ERR_BAD_ARG, "tuning.chunk_positions must be 0, 64, 128 or 256");
+  if (tune.float_mfma_rows != 0 && tune.float_mfma_rows != 64 && tune.float_mfma_rows != 128 && tune.float_mfma_rows != 256) return Fail(PL_ERR_BAD_ARG, "tuning.float_mfma_rows must be 0, 64, 128 or 256");
   if (tune.image_kernel < 0 || tune.image_kernel > 3) return Fail(PL_ERR_BAD_ARG, "tuning.image_kernel must be 0, 1, 2 or 3");
   if (desc->kind < PL_KIND_FP32 || desc->kind > PL_KIND_FP16) return Fail(PL_ERR_BAD_ARG, "unknown kind %d", desc->kind);
   if (desc->algo < PL_ALGO_AUTO || desc->algo > PL_ALGO_IMAGE_MFMA) return Fail(PL_ERR_BAD_ARG, "unknown algo %d", desc->algo);
@@ -994,6 +1112,11 @@ int pl_sparse_conv_prepare(const pl_sparse_conv_desc* desc, pl_sparse_conv_handl
   h->walk_chunked = sw(tune.walk_chunked);
   h->chunk_mfma = sw(tune.chunk_mfma);
   h->chunk_positions = tune.chunk_positions;
+  // a handle that asks for a walk, or for a form of one, keeps its calls there
+  const bool float_walk_asked = desc->algo != PL_ALGO_AUTO || tune.walk_tiled != PL_TUNE_RULE || tune.walk_split != 0 || tune.walk_chunked != PL_TUNE_RULE || tune.chunk_walk_groups != 0 || tune.walk_tile != 0 ||
+                                tune.walk_threads != 0 || tune.walk_slices != 0 || tune.walk_pairs != PL_TUNE_RULE;
+  h->float_mfma = float_walk_asked && tune.float_mfma != PL_TUNE_ALWAYS ? 0 : sw(tune.float_mfma);
+  h->float_mfma_rows = tune.float_mfma_rows;
   h->walk_asked = tune.walk_tile != 0 || tune.walk_threads != 0 || tune.walk_slices != 0;
   h->block_asked = tune.mfma_stream != PL_TUNE_RULE || tune.mfma_sub_tiles != PL_TUNE_RULE || tune.mfma_tile_quads != 0 || tune.mfma_narrow_i8_stores != 0 || tune.wg_slots != 0;
   h->image_asked = tune.image_kernel != 0 || tune.image_min_items != 0 || tune.image_tr_regroup != PL_TUNE_RULE;
@@ -1043,6 +1166,7 @@ int pl_sparse_conv_prepare(const pl_sparse_conv_desc* desc, pl_sparse_conv_handl
     h->tw_narrow.form = pl::kHalfTileWalkNarrowForm;
     if (hrc == PL_OK) hrc = BuildTileWalk(L, desc->bias, h, &h->tw_narrow, true, pl::kHalfTileWalkNarrowTile * 2, 2);
     if (hrc == PL_OK) hrc = UploadHalfBias(h, desc->bias);
+    if (hrc == PL_OK && FloatMfmaWanted(h)) hrc = BuildFloatMfma(L, h);
     if (hrc != PL_OK) {
       delete h;
       return hrc;
@@ -1081,6 +1205,7 @@ int pl_sparse_conv_prepare(const pl_sparse_conv_desc* desc, pl_sparse_conv_handl
   if (rc == PL_OK && h->wtiles.ptr && pl::ImageMfmaRegroupsByTransposingReads(desc->ic, 196)) rc = BuildImageMfmaTrRegroup(L, h);
   if (rc == PL_OK && h->wtiles.ptr && pl::ImageRowsMfmaFits(desc->oc, desc->ic, 16)) rc = BuildImageRowsMfma(L, h);
   if (rc == PL_OK && algo == PL_ALGO_ROW_WALK && !int8) rc = BuildChunkWalk(L, h);
+  if (rc == PL_OK && algo == PL_ALGO_ROW_WALK && !int8 && FloatMfmaWanted(h)) rc = BuildFloatMfma(L, h);
   if (rc == PL_OK && algo == PL_ALGO_ROW_WALK && !int8 && !half) {
     // the form with the largest tile that holds all channels in LDS: 128 positions (pairs of row groups, or single
     // ones on request), else 64 / 32 / 16 positions with 4 / 8 / 16 row groups per step
@@ -1188,7 +1313,9 @@ int pl_sparse_conv_run(pl_sparse_conv_handle* h, const void* x_dev, void* out_de
   const bool aligned16 = reinterpret_cast<uintptr_t>(x_dev) % 16 == 0 && reinterpret_cast<uintptr_t>(out_dev) % 16 == 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
   hipError_t e;
-  const int call_algo = AlgoForCall(h, batch, im_size, aligned16);
+  int call_algo = AlgoForCall(h, batch, im_size, aligned16);
+  // the floating-point product takes whole elements
+  if (!h->int8 && ((reinterpret_cast<uintptr_t>(x_dev) | reinterpret_cast<uintptr_t>(out_dev)) & (h->half ? 1u : 3u)) != 0) call_algo = h->algo;
   // Half precision: the walk with the tile and the lists in LDS, from 7 tiles on (13 with row pairs, whose plain
   // walk is twice as efficient per list entry) on 256 CUs: measured against the other half-precision walks at
   // 1 - 784 tiles, it is 1.3 - 2.5 times as fast from there on and slower below.  Tiles of 256 positions where
@@ -1197,7 +1324,7 @@ int pl_sparse_conv_run(pl_sparse_conv_handle* h, const void* x_dev, void* out_de
   const TileWalkStreams* half_tw = nullptr;
   int half_tile = 0;
   bool half_ragged = false;
-  if (h->half && h->walk_tiled > 0) {
+  if (h->half && h->walk_tiled > 0 && call_algo != PL_ALGO_CHUNK_MFMA) {
     if (h->tw.built != 0 && im_size % 8 == 0 && aligned16) {
       half_tw = &h->tw;
     } else if (h->tw_narrow.built != 0 && im_size % 4 == 0 && aligned8) {
@@ -1213,7 +1340,26 @@ int pl_sparse_conv_run(pl_sparse_conv_handle* h, const void* x_dev, void* out_de
       if (!pays) half_tw = nullptr;
     }
   }
-  if (half_tw) {
+  if (!h->int8 && call_algo == PL_ALGO_CHUNK_MFMA) {
+    pl::FloatMfmaParams p{};
+    p.x = x_dev;
+    p.out = out_dev;
+    p.wtiles = h->wfloat.ptr;
+    p.bias = !h->has_bias ? nullptr : (h->half ? h->hw_bias.ptr : h->bias.ptr);
+    p.row_exp = reinterpret_cast<const int32_t*>(static_cast<const char*>(h->wfloat.ptr) + h->float_row_exp);
+    p.groups = static_cast<const pl::DevGroup*>(h->groups.ptr);
+    p.kidx = static_cast<const uint32_t*>(h->half ? h->hw_kidx.ptr : h->kidx.ptr);
+    p.wts = static_cast<const uint32_t*>(h->half ? h->hw_wts.ptr : h->wts.ptr);
+    p.nr = h->semi ? 2 : 1;
+    p.K = h->ic;
+    p.M = h->oc;
+    p.hw = im_size;
+    p.batch = batch;
+    p.act = h->act;
+    p.act_h_words[0] = h->act_h.alpha | static_cast<uint32_t>(h->act_h.hs_offset) << 16;
+    p.act_h_words[1] = h->act_h.hs_inv_scale | static_cast<uint32_t>(h->act_h.hs_threshold) << 16;
+    e = pl::LaunchFloatMfma(!h->half, std::max(1, h->wg_slots_default / 2), h->float_mfma_rows / 32, p, s);
+  } else if (half_tw) {
     const TileWalkDivision d = DivideTileWalk(h, *half_tw, CeilDiv(static_cast<int>(P), half_tile));
     pl::HalfTileWalkParams p{};
     p.x = static_cast<const uint16_t*>(x_dev);

@@ -243,6 +243,59 @@ struct HalfWalkParams {
 // tile_pos: 128, 64, 32 or 16 positions with (K + 1) * tile_pos * 2 bytes of LDS.
 hipError_t LaunchHalfWalk(int nrows, int tile_pos, int threads, const HalfWalkParams& p, hipStream_t stream);
 
+// Floating-point SpMM on the matrix cores (float_mfma_kernels.hip): dense 32x16 weight tiles, the channels taken chunk by
+// chunk.
+constexpr int kFloatMfmaChunk = 64;
+
+struct FloatMfmaParams {
+  // the first 56 bytes: what the first loads of a kernel need (kernarg_head.h)
+  const void* x;
+  // [row block of 32][16-channel step][64 lanes][8 x binary16]; lane l of a tile holds row l % 32, value t channel
+  // 16 step + 8 (l / 32) + t; in the last, partial group of eight channels value t is channel K - 8 + t (zero where
+  // that channel belongs to the group before)
+  const void* wtiles;
+  int K;
+  int hw;
+  int batch;
+  // filled in by the launcher
+  int qpi;               // position quads per image = ceil(hw / 4)
+  uint32_t total_quads;  // batch * qpi
+  int chunks;
+  int tiles, row_groups;
+  int row_blocks;        // ceil(M / 32)
+  // behind the head
+  int padded_ksteps;     // steps wtiles holds, the last ones zero
+  int quad_aligned;      // hw % 4 == 0
+  // from the caller again
+  int M;
+  int nr;                // rows per list of the plain walk, 1 or 2
+  void* out;
+  const void* bias;      // fp32 or binary16, padded to a multiple of 32 rows; may be null
+  // fp32, padded to a multiple of 32 rows: the tiles of a row hold w 2^-row_exp in two binary16 pieces, [step][piece][64 lanes][8]
+  const int32_t* row_exp;
+  // the plain walk's lists, for the positions whose inputs are not finite
+  const DevGroup* groups;
+  const uint32_t* kidx;
+  const uint32_t* wts;
+  DevAct act;
+  uint32_t act_h_words[2];  // alpha and hs_offset, hs_inv_scale and hs_threshold of DevActH (16-bit members would go through scratch memory)
+};
+
+// How a call is divided (workgroups of wr x 32 rows x 128 positions) and what it is expected to take.
+struct FloatMfmaPlan {
+  int wr;
+  int row_groups;
+  int64_t workgroups;
+  double us;
+};
+
+int FloatMfmaPaddedSteps(int K);  // 16-channel steps of the weight tiles: whole chunks
+bool FloatMfmaFits(bool f32, int K, int M, int hw, int64_t positions);
+// row_blocks: blocks of 32 rows per workgroup, 8, 4 or 2; 0 = chosen by the call
+FloatMfmaPlan PlanFloatMfma(bool f32, int cus, int row_blocks, int K, int M, int hw, int batch);
+// x and out on whole elements
+hipError_t LaunchFloatMfma(bool f32, int cus, int row_blocks, const FloatMfmaParams& p, hipStream_t stream);
+
 // Block MFMA SpMM (int8): dense 32x32 weight blocks pre-arranged in operand
 // order, empty blocks skipped through a per-row-block bit mask.
 struct MfmaParams {

@@ -1,0 +1,188 @@
+"""fp32 / fp16 sparse_conv2d on the matrix cores (tuning.float_mfma) against the same sums in 64 bits, and the rule that
+gives calls to it."""
+import numpy as np
+import pytest
+
+from helpers import capi, workloads, pla, make_kernel, run_hip, run_oracle, oracle_pack
+
+pytestmark = pytest.mark.gpu
+
+AP = pla.ActivationParam
+ACTS = {"none": AP(), "relu": AP("relu"), "relu6": AP("relu6", Relu_clipped_coef=6.0), "leaky": AP("leaky_relu", Leaky_relu_alpha=0.1), "hswish": AP("hard_swish")}
+KINDS = {"fp32": capi.KIND_FP32, "fp16": capi.KIND_FP16}
+ROWS = (64, 128, 256)
+
+
+def make_case(kind, batch, ic, oc, h, w, paired=False, act="none", sparsity=0.75, seed=0):
+    c = workloads.make_fp32("t", batch, ic, oc, h, w, sparsity, paired, ACTS[act], seed=seed + ic + 3 * oc)
+    c.kind = KINDS[kind]
+    if kind == "fp16":
+        c.x = c.x.astype(np.float16)
+    return c
+
+
+def forced(case, rows, paired=False):
+    kernel = make_kernel(case, force_semi=paired, tuning=capi.tuning(float_mfma=capi.TUNE_ALWAYS, float_mfma_rows=rows))[0]
+    assert capi.lib().pl_sparse_conv_algo_for(kernel._handle, case.batch, case.im_size) == capi.ALGO_CHUNK_MFMA
+    return kernel
+
+
+def sums(case):
+    """Sums before the activation in 64 bits, and the same with every term's magnitude."""
+    to = np.float16 if case.kind == capi.KIND_FP16 else np.float32
+    w = case.dense.astype(to).astype(np.float64)
+    bias = np.zeros(w.shape[0]) if case.bias is None else case.bias.astype(to).astype(np.float64)
+    x = case.x.astype(np.float64).reshape(case.batch, w.shape[1], -1)
+    shape = (case.batch, w.shape[0]) + tuple(case.x.shape[2:])
+    return (np.matmul(w, x) + bias[:, None]).reshape(shape), (np.matmul(np.abs(w), np.abs(x)) + np.abs(bias)[:, None]).reshape(shape)
+
+
+def activate(v, act, dtype):
+    one = lambda t: np.asarray(t).astype(dtype)  # noqa: E731
+    v = one(v)
+    if act == "relu":
+        return np.maximum(v, one(0))
+    if act == "relu6":
+        return np.minimum(np.maximum(v, one(0)), one(6))
+    if act == "leaky":
+        return np.where(v >= 0, v, one(v * one(0.1)))
+    if act == "hswish":
+        return one(one(v * one(1.0 / 6.0)) * np.minimum(np.maximum(one(v + one(3)), one(0)), one(6)))
+    return v
+
+
+def check(case, act, got):
+    """fp32: pieces of 22 bits of both factors and of three of four products (4 units of 2^-23 of every term), and one
+    cut sum per 16 channels.  fp16: one rounding of a sum that is fp32's, so at most the neighbouring binary16 value,
+    then the activation's own roundings (hard_swish: two factors that follow the sum and three roundings)."""
+    ref, mag = sums(case)
+    assert got.shape == ref.shape
+    if case.kind == capi.KIND_FP32:
+        tol = (6 + case.x.shape[1] / 16.0) * 2.0 ** -23 * mag
+        if act == "hswish":
+            tol = 2 * tol + np.abs(ref) * tol
+        assert (np.abs(got - activate(ref, act, np.float64)) <= tol + 1e-30).all()
+        return
+    assert got.dtype == np.float16
+    tol = 2.0 ** -10 * np.abs(ref) + 2.0 ** -19 * mag + 1e-7
+    if act == "hswish":
+        tol = (3 + 2 * np.abs(ref)) * tol
+    assert (np.abs(got.astype(np.float64) - activate(ref.astype(np.float16), act, np.float16).astype(np.float64)) <= tol).all()
+
+
+# (batch, ic, oc, h, w): one quad; a single row; channels off the groups of eight and chunks of 64 (fewer than one, one more than a
+# chunk, odd numbers of chunks); rows off the blocks of 32 and the workgroups' 64 / 128 / 256; maps off the quads
+# (partial quads of 1, 2 and 3 positions, several images per tile); exactly one tile and one position more
+SHAPES = [(1, 8, 1, 2, 2), (3, 9, 33, 5, 1), (2, 63, 31, 3, 3), (1, 65, 64, 9, 6), (5, 130, 65, 7, 7), (2, 203, 129, 11, 5), (1, 256, 257, 8, 16), (1, 64, 96, 3, 43), (2, 320, 40, 14, 14), (9, 100, 300, 1, 7)]
+
+
+@pytest.mark.parametrize("rows", ROWS)
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("paired", [False, True], ids=["unstructured", "semi"])
+@pytest.mark.parametrize("kind", sorted(KINDS))
+def test_against_64_bits(kind, paired, shape, rows):
+    act = sorted(ACTS)[(sum(shape) + rows // 64) % len(ACTS)]
+    case = make_case(kind, *shape, paired=paired, act=act)
+    check(case, act, run_hip(case, kernel=forced(case, rows, paired)))
+
+
+@pytest.mark.parametrize("act", sorted(ACTS))
+@pytest.mark.parametrize("kind", sorted(KINDS))
+def test_activations_and_a_new_bias(kind, act):
+    case = make_case(kind, 3, 96, 70, 6, 7, act=act)
+    case.bias = None
+    kernel = forced(case, 128)
+    check(case, act, run_hip(case, kernel=kernel))
+    case.bias = np.linspace(-0.7, 0.9, 70).astype(np.float32)
+    capi.check(capi.lib().pl_sparse_conv_set_epilogue(kernel._handle, None, case.bias.ctypes.data, None))
+    check(case, act, run_hip(case, kernel=kernel))
+
+
+@pytest.mark.parametrize("rows", ROWS)
+@pytest.mark.parametrize("how", ["images", "late", "grow", "tails", "small", "large"])
+def test_fp32_magnitudes(how, rows):
+    """The scales follow the inputs: images of very different size in one tile, positions that begin with a chunk of
+    zeros, channels that grow from chunk to chunk (new scales in the middle of a sum), heavy tails, both ends of the
+    exponent range."""
+    case = make_case("fp32", 6, 330, 40, 5, 7)
+    rng = np.random.RandomState(1)
+    if how == "images":
+        case.x *= (10.0 ** np.linspace(-9, 9, 6)).astype(np.float32)[:, None, None, None]
+    elif how == "late":
+        case.x[:, :64] = 0
+        case.x[2, :200] = 0
+    elif how == "grow":
+        case.x *= (2.0 ** (np.arange(330) // 8 % 20 - 10)).astype(np.float32)[None, :, None, None]
+    elif how == "tails":
+        case.x *= np.exp(2 * rng.standard_normal(case.x.shape)).astype(np.float32)
+    else:
+        case.bias = None
+        case.x *= np.float32(1e-30 if how == "small" else 1e30)
+    check(case, "none", run_hip(case, kernel=forced(case, rows)))
+
+
+@pytest.mark.parametrize("rows", ROWS)
+@pytest.mark.parametrize("paired", [False, True], ids=["unstructured", "semi"])
+@pytest.mark.parametrize("kind", sorted(KINDS))
+def test_infinities_and_nans_reach_only_the_rows_that_read_them(kind, paired, rows):
+    """A dense product would spread them through its zero weights.  Partial quads and every part of the channels."""
+    case = make_case(kind, 3, 200, 70, 9, 5, paired=paired, act="leaky", sparsity=0.9)
+    case.x[0, 3, 2, 1] = np.inf
+    case.x[0, 150, 8, 4] = np.nan
+    case.x[1, 70, 0, 0] = -np.inf
+    case.x[2, 199, 4, 4] = np.inf
+    got, want = run_hip(case, kernel=forced(case, rows, paired)), run_oracle(case, oracle_pack(case, force_semi=paired))
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.isnan(want).any() and not np.isnan(want).all()
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)]) and np.isinf(want).any()
+    rest = np.isfinite(want)
+    case.x[~np.isfinite(case.x)] = 0
+    ref, mag = sums(case)
+    tol = 2.0 ** -7 if kind == "fp16" else 2.0 ** -18  # the walk's own sums among them
+    assert (np.abs(got.astype(np.float64) - np.where(ref >= 0, ref, 0.1 * ref))[rest] <= (tol * mag)[rest]).all()
+
+
+@pytest.mark.parametrize("kind", sorted(KINDS))
+def test_tensors_off_the_16_byte_grid(kind):
+    """Tensors that start one element behind a 16-byte boundary: the same bits as the aligned call, nothing written
+    outside the output."""
+    import torch
+
+    case = make_case(kind, 3, 96, 40, 9, 7)
+    kernel = forced(case, 64)
+    want = run_hip(case, kernel=kernel)
+    dtype = torch.float32 if kind == "fp32" else torch.float16
+    flat_x = torch.zeros(case.x.size + 16, dtype=dtype, device="cuda")
+    x = flat_x[1:1 + case.x.size].view(case.x.shape)
+    x.copy_(torch.from_numpy(case.x))
+    flat_o = torch.full((want.size + 16,), 77.0, dtype=dtype, device="cuda")
+    out = flat_o[1:1 + want.size].view(want.shape)
+    kernel.Run(x, out)
+    torch.cuda.synchronize()
+    assert np.array_equal(out.cpu().numpy(), want)
+    host = flat_o.cpu().numpy()
+    assert host[0] == 77.0 and (host[1 + want.size:] == 77.0).all()
+
+
+def test_the_rule():
+    """Which calls leave the walks: many nonzeros per row, not calls of few products, never those of a handle that asks for
+    a walk; a layer with hardly any nonzeros holds no dense tiles."""
+    L = capi.lib()
+
+    def algo(case, batch, im_size, **tuning):
+        kernel = make_kernel(case, tuning=capi.tuning(**tuning) if tuning else None)[0]
+        return L.pl_sparse_conv_algo_for(kernel._handle, batch, im_size), kernel.info()["device_bytes"]
+
+    for kind in KINDS:
+        deep = make_case(kind, 1, 512, 512, 14, 14, sparsity=0.8)
+        taken, size = algo(deep, 64, 196)
+        assert taken == capi.ALGO_CHUNK_MFMA
+        assert algo(deep, 1, 16)[0] == capi.ALGO_ROW_WALK
+        assert algo(deep, 64, 196, walk_tiled=capi.TUNE_RULE, walk_pairs=capi.TUNE_ALWAYS)[0] == capi.ALGO_ROW_WALK
+        never, walk_size = algo(deep, 64, 196, float_mfma=capi.TUNE_NEVER)
+        assert never == capi.ALGO_ROW_WALK and walk_size < size
+        assert algo(make_case(kind, 1, 512, 512, 4, 4, sparsity=0.98), 64, 196)[0] == capi.ALGO_ROW_WALK
+    # few nonzeros per row
+    assert algo(make_case("fp32", 1, 96, 192, 8, 8, sparsity=0.9), 1, 3136)[0] == capi.ALGO_ROW_WALK
+    assert algo(make_case("fp16", 1, 96, 200, 8, 8, sparsity=0.86), 102, 400)[0] == capi.ALGO_ROW_WALK
+    with pytest.raises(capi.SparseConvError):
+        make_kernel(make_case("fp32", 1, 16, 16, 4, 4), tuning=capi.tuning(float_mfma_rows=96))
