@@ -92,6 +92,28 @@ def build_library(verbose=False):
     return LIB_PATH
 
 
+PYTHON_RUN_PATH = os.path.join(LIB_DIR, "pl_python_run.so")
+
+
+def build_python_run(verbose=False):
+    """The native part of the Python classes' Run (csrc/python_run.cc): a CPython module over torch's C++ tensors, host
+    code only.  Calls the entry points of the library by address, so it does not link against it."""
+    import sysconfig
+
+    from torch.utils import cpp_extension
+    import torch
+
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-Wno-sign-compare", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI)]
+    for path in cpp_extension.include_paths() + ["/opt/rocm/include", sysconfig.get_paths()["include"]]:
+        cmd += ["-isystem", path]
+    cmd += [os.path.join(CSRC, "python_run.cc"), "-o", PYTHON_RUN_PATH, "-L" + torch_lib, "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath," + torch_lib]
+    os.makedirs(LIB_DIR, exist_ok=True)
+    _run(cmd, verbose)
+    return PYTHON_RUN_PATH
+
+
 LITE_DIR = os.path.join(PKG, "lite")
 LITE_LIB_PATH = os.path.join(LIB_DIR, "libpl_lite_hip.so")
 ROOT = os.path.dirname(PKG)
@@ -186,4 +208,5 @@ def build_sanitized(out_dir):
 
 if __name__ == "__main__":
     print(build_library(verbose=True))
+    print(build_python_run(verbose=True))
     print(build_host_mirror(verbose=True))

@@ -228,6 +228,53 @@ def current_stream(device):
     return _raw_stream(device.index)
 
 
+NATIVE_RUN_PATH = os.path.join(PKG, "lib", "pl_python_run.so")
+_native_run = False  # not looked for yet
+
+
+def native_run():
+    """The module with the native part of the Python classes' Run (csrc/python_run.cc), or None where it was not built or
+    does not load beside this torch: the classes then take the same steps in Python."""
+    global _native_run
+    if _native_run is False:
+        import torch  # noqa: F401  (the module is linked against its libraries)
+        from importlib.machinery import ExtensionFileLoader
+        from importlib.util import module_from_spec, spec_from_loader
+
+        try:
+            loader = ExtensionFileLoader("pl_python_run", NATIVE_RUN_PATH)
+            module = module_from_spec(spec_from_loader("pl_python_run", loader))
+            loader.exec_module(module)
+            _native_run = module
+        except ImportError:
+            _native_run = None
+    return _native_run
+
+
+_type_codes = {}
+
+
+def type_code(dtype):
+    """The number by which the native part of Run knows a torch element type."""
+    code = _type_codes.get(dtype)
+    if code is None:
+        import torch
+
+        code = _type_codes[dtype] = native_run().type_code(torch.empty(0, dtype=dtype))
+    return code
+
+
+_addresses = {}
+
+
+def entry_address(name):
+    """Address of an entry point of the library, as the native part of Run takes it."""
+    address = _addresses.get(name)
+    if address is None:
+        address = _addresses[name] = C.cast(getattr(lib(), name), C.c_void_p).value
+    return address
+
+
 def last_error():
     return lib().pl_last_error().decode("utf-8", "replace")
 

@@ -6,6 +6,8 @@ with the HIP library behind it.  It is the layer between two pointwise
 convolutions of a MobileNet, which is why it sits beside sparse_conv2d here.
 """
 import ctypes as C
+import functools
+import sys
 
 import numpy as np
 
@@ -55,6 +57,7 @@ class DepthwiseConv(object):
         self.param = param
         self._handle = None
         self._bound = None  # what Run looks up once (_bind)
+        self._native = None  # its native form and torch.cuda (SparseConvKernel.Run)
         self._first_epoch = True
         self.w_scale_ = None
         self.bias_ = None
@@ -122,6 +125,8 @@ class DepthwiseConv(object):
         self._handle = h
         self._bound = None
         self._first_epoch = False
+        if "torch" in sys.modules:  # else at the first Run
+            self._bind()
 
     def out_shape(self, x_shape):
         n, c, h, w = x_shape
@@ -133,9 +138,17 @@ class DepthwiseConv(object):
             self.PrepareForRun()
         return self.Run(x, out, stream)
 
-    # What surrounds the launch is kept short, as in SparseConvKernel.Run: the current device is only changed when it is
-    # not the tensor's (9.6 -> 5.6 us of host time per call with `out`).
+    # The common call is one native function, as in SparseConvKernel.Run; the current device is only changed when it is not
+    # the tensor's.
     def Run(self, x, out=None, stream=None):
+        if self._native is not None:
+            native, cuda = self._native
+            done = native(cuda.current_device(), x, out, stream)
+            if done is not None:
+                return done
+        return self._run(x, out, stream)
+
+    def _run(self, x, out, stream):
         if self._handle is None:
             raise RuntimeError("PrepareForRun has not been called")
         int8, out_dtype, c, stride, pad, torch, run = self._bound or self._bind()
@@ -164,9 +177,14 @@ class DepthwiseConv(object):
 
         self._bound = (torch.int8, torch.int8 if self.kind == capi.KIND_INT8_INT8 else torch.float32, self.param.filter.shape[0], self.param.strides[0], self.param.paddings[0], torch,
                        capi.lib().pl_dwconv3x3_run)
+        native = capi.native_run()
+        if native is not None:
+            out_type = capi.type_code(self._bound[1])
+            self._native = (functools.partial(native.depthwise, capi.entry_address("pl_dwconv3x3_run"), self._handle.value, out_type, int(self._bound[2]), int(self._bound[3]), int(self._bound[4])), torch.cuda)
         return self._bound
 
     def _release(self):
+        self._native = None
         if self._handle is not None:
             capi.lib().pl_dwconv3x3_destroy(self._handle)
             self._handle = None
@@ -193,6 +211,11 @@ def run_conv_dw(conv, dw, x, out=None, stream=None):
         raise RuntimeError("PrepareForRun has not been called")
     int8, _, _, stride, pad, torch, _ = dw._bound or dw._bind()
     weights = conv.param.weights
+    native = capi.native_run()
+    if native is not None:
+        done = native.pair(capi.entry_address("pl_sparse_conv_dwconv3x3_run"), conv._handle.value, dw._handle.value, weights.ic, weights.oc, stride, pad, torch.cuda.current_device(), x, out, stream)
+        if done is not None:
+            return done
     shape = x.shape
     if not x.is_cuda or not x.is_contiguous() or x.dtype != int8 or len(shape) != 4 or shape[1] != weights.ic:
         raise ValueError("x must be a contiguous int8 NCHW device tensor with %d channels" % weights.ic)
