@@ -98,8 +98,8 @@ __device__ __forceinline__ h1 WalkF16(const FloatMfmaParams& p, const h1* x, int
 }
 
 // LDS: two buffers of operand cells, or what the wavefronts of a row block hand to each other at the end; behind either
-// (a wavefront may still look at the flag when another has begun to hand over), for fp32, the positions' maxima and the
-// flag.
+// (a wavefront may still look at a flag when another has begun to hand over), for fp32, the positions' maxima and the two
+// flags.
 constexpr int LdsTables(int wr, bool f32) {
   const int cells = 2 * (f32 ? 2 : 1) * kGroups * 4 * kQuads * 16, trade = 8 * (64 - 8 * wr) * 64 * 4;
   return cells > trade ? cells : trade;
@@ -219,10 +219,12 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
     for (int i = 0; i < 16; ++i) acc[c][i] = 0.0f, rest[c][i] = 0.0f;
 
   // The scales of fp32.  colmax holds the bits of the largest magnitude of every position; its exponent gives the scale
-  // that takes it to [2^12, 2^13).  A chunk with a value beyond 2^15 after scaling raises the flag; then everyone takes
-  // the new maxima, brings the sums so far to the new scales and writes that chunk's cells again.
+  // that takes it to [2^12, 2^13).  A chunk with a value beyond 2^15 after scaling raises its flag; then everyone
+  // takes the new maxima, brings the sums so far to the new scales and writes that chunk's cells again.  Even and odd
+  // chunks have a flag each: a wavefront may be behind the barrier of one chunk and at its look at that chunk's flag
+  // while another is through the next chunk's values.
   uint32_t* const colmax = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(xt) + LdsTables(WR, F32));
-  uint32_t* const flag = colmax + 4 * QT;
+  uint32_t* const flags = colmax + 4 * QT;
   const uint32_t* const own_max = colmax + 4 * n;  // of the positions whose sums the lane holds
   [[maybe_unused]] int own_exp[4];
   auto scale_exp = [](uint32_t bits) { return max(1, min(254, 266 - (int)(bits >> 23))); };
@@ -238,7 +240,7 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
   auto rescale = [&](Quad<F32> (&rd)[UC], int buf) {
     collect(rd);
     __syncthreads();
-    if (tid == 0) *flag = 0;
+    if (tid == 0) flags[buf] = 0;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       const uint32_t m = colmax[4 * j + c], om = own_max[c];
@@ -301,10 +303,10 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
       __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (F32) {
-      if (peak >= 0x1p15f) *flag = 1;
+      if (peak >= 0x1p15f) flags[(S + 1) & 1] = 1;
       peak = 0.0f;
       __syncthreads();
-      if (__builtin_amdgcn_readfirstlane(*flag) != 0) rescale(r[NEXT], (S + 1) & 1);
+      if (__builtin_amdgcn_readfirstlane(flags[(S + 1) & 1]) != 0) rescale(r[NEXT], (S + 1) & 1);
       if (!LAST) issue(r[NEXT], chunk + 1 + DEPTH);
     } else {
       if (!LAST) issue(r[NEXT], chunk + 1 + DEPTH);
@@ -325,7 +327,7 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
   }
   if constexpr (!F32) align_quad(r[0]);
   if constexpr (F32) {
-    for (int i = tid; i <= 4 * QT; i += kThreads) colmax[i] = 0;  // and the flag
+    for (int i = tid; i < 4 * QT + 2; i += kThreads) colmax[i] = 0;  // and the flags
     __syncthreads();
     align_quad(r[0]);
     collect(r[0]);
