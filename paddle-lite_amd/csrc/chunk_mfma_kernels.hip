@@ -25,6 +25,7 @@
 #include <type_traits>
 
 #include "epilogue.h"
+#include "kernarg_head.h"
 #include "launch_lds.h"
 #include "sparse_conv_kernels.h"
 
@@ -38,6 +39,20 @@ using epilogue::TruncPackI8x4;
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+
+// what the first loads need arrives in registers
+PL_IN_HEAD(ChunkMfmaParams, x);
+PL_IN_HEAD(ChunkMfmaParams, wtiles);
+PL_IN_HEAD(ChunkMfmaParams, K);
+PL_IN_HEAD(ChunkMfmaParams, hw);
+PL_IN_HEAD(ChunkMfmaParams, qpi);
+PL_IN_HEAD(ChunkMfmaParams, total_quads);
+PL_IN_HEAD(ChunkMfmaParams, tile_quads);
+PL_IN_HEAD(ChunkMfmaParams, tiles);
+PL_IN_HEAD(ChunkMfmaParams, row_groups);
+PL_IN_HEAD(ChunkMfmaParams, row_tiles);
+PL_IN_HEAD(ChunkMfmaParams, padded_ksteps);
+PL_IN_HEAD(ChunkMfmaParams, chunks);
 
 constexpr int kBufCells = 2048;  // 16-byte cells of one chunk: (channel group of 16, position of the tile)
 
@@ -167,6 +182,17 @@ __device__ __forceinline__ void ChunkBody(const ChunkMfmaParams& p, uint4* xt) {
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) load_weights(0, ks);
   __builtin_amdgcn_sched_barrier(0);
+  // scales and biases behind the first loads: the epilogue of a small call would begin with a wait for memory
+  const int row0 = rt * 16 + 4 * kq;
+  float sc[4], bi[4];
+  if (OUT != kOutAcc32) {
+    // arrays are padded to a multiple of 32 rows
+    const int row = min(rt, p.row_tiles - 1) * 16 + 4 * kq;
+    const float4 s4 = *reinterpret_cast<const float4*>(p.scale + row), b4 = *reinterpret_cast<const float4*>(p.bias + row);
+    sc[0] = s4.x, sc[1] = s4.y, sc[2] = s4.z, sc[3] = s4.w;
+    bi[0] = b4.x, bi[1] = b4.y, bi[2] = b4.z, bi[3] = b4.w;
+  }
+  __builtin_amdgcn_sched_barrier(0);
   if (p.chunks >= 3) {
     issue_all(r[1], 1);
     __builtin_amdgcn_sched_barrier(0);
@@ -196,15 +222,7 @@ __device__ __forceinline__ void ChunkBody(const ChunkMfmaParams& p, uint4* xt) {
   }
 
   // epilogue: lane (n, kq) holds rows 4 kq .. 4 kq + 3 of the row tile at the four positions of quad 16 w + n
-  const int row0 = rt * 16 + 4 * kq;
   if (row0 >= p.M) return;
-  float sc[4], bi[4];
-  if (OUT != kOutAcc32) {
-    // arrays are padded to a multiple of 32 rows
-    const float4 s4 = *reinterpret_cast<const float4*>(p.scale + row0), b4 = *reinterpret_cast<const float4*>(p.bias + row0);
-    sc[0] = s4.x, sc[1] = s4.y, sc[2] = s4.z, sc[3] = s4.w;
-    bi[0] = b4.x, bi[1] = b4.y, bi[2] = b4.z, bi[3] = b4.w;
-  }
   constexpr uint32_t kElem = OUT == kOutI8 ? 1u : 4u;
   // output rows that start on 64-byte boundaries are stored as streaming data; others share sectors with their
   // neighbours, which merge in L2 only if stored plainly (384 -> 384 @28x28 x 16, fp32: 9.2 against 12.2 us;
@@ -270,7 +288,8 @@ __device__ __forceinline__ void ChunkBody(const ChunkMfmaParams& p, uint4* xt) {
 }
 
 template <int NW, int OUT>
-__global__ void __launch_bounds__(512, 2) ChunkMfmaKernel(const ChunkMfmaParams p) {
+__global__ void __launch_bounds__(512, 2) ChunkMfmaKernel(PL_HEAD_PARAMS, const ChunkMfmaParams block) {
+  const ChunkMfmaParams p = WithHead(block, PL_HEAD_ARGS);
   extern __shared__ uint4 xt[];
   ChunkBody<NW, OUT>(p, xt);
 }
@@ -279,9 +298,9 @@ template <int OUT>
 hipError_t Launch(int nw, const ChunkMfmaParams& p, dim3 grid, hipStream_t s) {
   const dim3 block(512);
   const size_t lds = 2 * kBufCells * 16;
-  if (nw == 4) return LaunchWithLds(ChunkMfmaKernel<4, OUT>, grid, block, lds, s, p);
-  if (nw == 2) return LaunchWithLds(ChunkMfmaKernel<2, OUT>, grid, block, lds, s, p);
-  return LaunchWithLds(ChunkMfmaKernel<1, OUT>, grid, block, lds, s, p);
+  if (nw == 4) return LaunchWithHead(ChunkMfmaKernel<4, OUT>, grid, block, lds, s, p);
+  if (nw == 2) return LaunchWithHead(ChunkMfmaKernel<2, OUT>, grid, block, lds, s, p);
+  return LaunchWithHead(ChunkMfmaKernel<1, OUT>, grid, block, lds, s, p);
 }
 
 }  // namespace

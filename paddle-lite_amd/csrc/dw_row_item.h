@@ -104,20 +104,5 @@ __device__ __forceinline__ void DwRowItemWith(const DwConvParams& p, const DwRow
   }
 }
 
-// The same with the channel's filter rows, scale and bias loaded here (channel c).
-template <int STRIDE, int NOUT, int OUT, int ACT>
-__device__ __forceinline__ void DwRowItem(const DwConvParams& p, const DwRowStage& st, uint32_t plane, int c, int oy, bool live, char* dst_i8) {
-  uint32_t wrow[3] = {0u, 0u, 0u};
-  float s = 0.f, b = 0.f;
-  if (live) {
-    wrow[0] = p.wpack[4 * c];
-    wrow[1] = p.wpack[4 * c + 1];
-    wrow[2] = p.wpack[4 * c + 2];
-    s = p.scale[c];
-    b = p.bias[c];
-  }
-  DwRowItemWith<STRIDE, NOUT, OUT, ACT>(p, st, plane, wrow, s, b, oy, live, dst_i8);
-}
-
 }  // namespace dwrow
 }  // namespace pl

@@ -15,6 +15,7 @@
 #include "dw_row_item.h"
 #include "dwconv_kernels.h"
 #include "epilogue.h"
+#include "kernarg_head.h"
 #include "launch_lds.h"
 
 namespace pl {
@@ -23,6 +24,23 @@ namespace {
 using namespace epilogue;
 
 typedef float v4f __attribute__((ext_vector_type(4)));
+
+// what the first loads need arrives in registers
+PL_IN_HEAD(DwConvParams, x);
+PL_IN_HEAD(DwConvParams, planes);
+PL_IN_HEAD(DwConvParams, h);
+PL_IN_HEAD(DwConvParams, w);
+PL_IN_HEAD(DwConvParams, items);
+PL_IN_HEAD(DwConvParams, magic_items);
+PL_IN_HEAD(DwConvParams, blocks_per_group);
+PL_IN_HEAD(DwConvParams, magic_blocks);
+PL_IN_HEAD(DwConvParams, groups_w);
+PL_IN_HEAD(DwConvParams, magic_groups);
+PL_IN_HEAD(DwConvParams, planes_per_group);
+PL_IN_HEAD(DwConvParams, planes_per_block);
+PL_IN_HEAD(DwConvParams, pad);
+PL_IN_HEAD(DwConvParams, act_type);
+PL_IN_HEAD(DwConvParams, lanes_shared);
 
 // Dword at `ptr` (any alignment).  SAFE: the caller knows that the four
 // bytes lie inside the tensor.  Otherwise bytes outside [lo, hi) read as zero
@@ -114,7 +132,7 @@ __device__ __forceinline__ void DwItem(const DwConvParams& p, uint32_t plane, in
     // a row outside [0, h) is zero padding: it reads its neighbour and meets a zero filter row below
     rows[r] = plane_ptr + (uint32_t)(min(max(iy0 + r, 0), p.h - 1) * p.w) + cb;
   }
-  if (CG == 1 && p.share_lanes) {
+  if (CG == 1 && p.lanes_shared) {
     // Neighbouring lanes hold neighbouring column groups of the same rows, and
     // the dwords a lane needs beside its own STRIDE dwords are its
     // neighbours' own: each lane loads only its own bytes (the wavefront's
@@ -300,8 +318,9 @@ __device__ __forceinline__ void DwBody(const DwConvParams& p) {
 // R output rows by 4 * CG columns per item (the per-item address and mask
 // arithmetic is shared by all of them).
 template <int STRIDE, int R, int CG, int OUT>
-__global__ void __launch_bounds__(256) DwConv3x3Kernel(const DwConvParams p) {
-  DispatchAct(p.act.type, [&](auto act_c) {
+__global__ void __launch_bounds__(256) DwConv3x3Kernel(PL_HEAD_PARAMS, const DwConvParams block) {
+  const DwConvParams p = WithHead(block, PL_HEAD_ARGS);
+  DispatchAct(p.act_type, [&](auto act_c) {
     constexpr int ACT = decltype(act_c)::value;
     DwBody<STRIDE, R, CG, OUT, ACT>(p);
   });
@@ -324,11 +343,11 @@ __global__ void __launch_bounds__(256) DwConv3x3Kernel(const DwConvParams p) {
 //   * int8 outputs go to LDS byte by byte (the workgroup's output rows are
 //     one contiguous range too) and leave as aligned 16-byte pieces; fp32
 //     outputs are stored directly (dword aligned).
-using dwrow::DwRowItem;
 using dwrow::DwRowStage;
 
 template <int STRIDE, int NOUT, int OUT>
-__global__ void __launch_bounds__(256) DwRowKernel(const DwConvParams p) {
+__global__ void __launch_bounds__(256) DwRowKernel(PL_HEAD_PARAMS, const DwConvParams block) {
+  const DwConvParams p = WithHead(block, PL_HEAD_ARGS);
   extern __shared__ uint4 dw_lds[];
   const int tid = (int)threadIdx.x;
   const uint32_t total = p.planes * (uint32_t)p.oh;  // items
@@ -361,20 +380,25 @@ __global__ void __launch_bounds__(256) DwRowKernel(const DwConvParams p) {
       }
     }
   }
+  const uint32_t item = first + (uint32_t)tid;
+  const bool live = item < total;
+  const uint32_t plane = live ? DivMagic(item, (uint32_t)p.oh, p.magic_items) : plane_b;
+  const int oy = live ? (int)(item - plane * (uint32_t)p.oh) : oy_b;
+  const int c = (int)(plane - DivMagic(plane, (uint32_t)p.channels, p.magic_channels) * (uint32_t)p.channels);
+  // the channel's filter rows, scale and bias beside the input, not behind the barrier
+  uint32_t wrow[3];
+#pragma unroll
+  for (int r = 0; r < 3; ++r) wrow[r] = p.wpack[4 * c + r];
+  const float s = p.scale[c], b = p.bias[c];
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     const int j = tid + 256 * u;
     if (j < pieces) *reinterpret_cast<uint4*>(st.lds_in + 16 + 16 * j) = piece[u];
   }
   __syncthreads();
-  const uint32_t item = first + (uint32_t)tid;
-  const bool live = item < total;
-  const uint32_t plane = live ? DivMagic(item, (uint32_t)p.oh, p.magic_items) : plane_b;
-  const int oy = live ? (int)(item - plane * (uint32_t)p.oh) : oy_b;
-  const int c = (int)(plane - DivMagic(plane, (uint32_t)p.channels, p.magic_channels) * (uint32_t)p.channels);
-  DispatchAct(p.act.type, [&](auto act_c) {
+  DispatchAct(p.act_type, [&](auto act_c) {
     constexpr int ACT = decltype(act_c)::value;
-    DwRowItem<STRIDE, NOUT, OUT, ACT>(p, st, plane, c, oy, live, lds_out + (uint32_t)tid * (uint32_t)p.ow);
+    dwrow::DwRowItemWith<STRIDE, NOUT, OUT, ACT>(p, st, plane, wrow, s, b, oy, live, lds_out + (uint32_t)tid * (uint32_t)p.ow);
   });
   if (OUT == kOutI8) {
     __syncthreads();
@@ -397,17 +421,14 @@ __global__ void __launch_bounds__(256) DwRowKernel(const DwConvParams p) {
 
 template <int STRIDE, int NOUT>
 hipError_t LaunchRows(int out_kind, dim3 grid, size_t lds, hipStream_t stream, const DwConvParams& q) {
-  if (out_kind == kOutI8) return LaunchWithLds(DwRowKernel<STRIDE, NOUT, kOutI8>, grid, dim3(256), lds, stream, q);
-  return LaunchWithLds(DwRowKernel<STRIDE, NOUT, kOutF32>, grid, dim3(256), lds, stream, q);
+  if (out_kind == kOutI8) return LaunchWithHead(DwRowKernel<STRIDE, NOUT, kOutI8>, grid, dim3(256), lds, stream, q);
+  return LaunchWithHead(DwRowKernel<STRIDE, NOUT, kOutF32>, grid, dim3(256), lds, stream, q);
 }
 
 template <int STRIDE, int R, int CG>
-void LaunchShape(int out_kind, dim3 grid, hipStream_t stream, const DwConvParams& q) {
-  if (out_kind == kOutI8) {
-    hipLaunchKernelGGL((DwConv3x3Kernel<STRIDE, R, CG, kOutI8>), grid, dim3(256), 0, stream, q);
-  } else {
-    hipLaunchKernelGGL((DwConv3x3Kernel<STRIDE, R, CG, kOutF32>), grid, dim3(256), 0, stream, q);
-  }
+hipError_t LaunchShape(int out_kind, dim3 grid, hipStream_t stream, const DwConvParams& q) {
+  if (out_kind == kOutI8) return LaunchWithHead(DwConv3x3Kernel<STRIDE, R, CG, kOutI8>, grid, dim3(256), 0, stream, q);
+  return LaunchWithHead(DwConv3x3Kernel<STRIDE, R, CG, kOutF32>, grid, dim3(256), 0, stream, q);
 }
 
 // ceil(2^32 / d) for d >= 2 (a divisor of 1 is handled by the kernel: its magic would need 33 bits)
@@ -419,6 +440,7 @@ hipError_t LaunchDwConv3x3(int stride, int out_kind, const DwConvParams& p, hipS
   if (p.planes == 0 || p.oh <= 0 || p.ow <= 0) return hipSuccess;
   if ((stride != 1 && stride != 2) || (p.pad != 0 && p.pad != 1) || (out_kind != kOutF32 && out_kind != kOutI8)) return hipErrorInvalidValue;
   DwConvParams q = p;
+  q.act_type = (int8_t)p.act.type;
   // Item shape: output rows by groups of four output columns per thread.
   // More outputs per thread lower the instruction count per output, fewer
   // leave more wavefronts to hide the load latency.  Measured on the MobileNet
@@ -455,7 +477,7 @@ hipError_t LaunchDwConv3x3(int stride, int out_kind, const DwConvParams& p, hipS
   // Rows that are not 4-byte aligned make the overlapping per-lane loads
   // slow; there the lanes share their dwords instead (measured: 14x14 planes
   // 12.7 -> 10.4 us, 112x112 planes 28.3 -> 31.5 us with sharing).
-  q.share_lanes = cg != 1 ? 0 : (p.share_lanes >= 0 ? p.share_lanes : (p.w % 4 != 0 ? 1 : 0));
+  q.lanes_shared = cg != 1 ? 0 : (p.share_lanes >= 0 ? p.share_lanes : (p.w % 4 != 0 ? 1 : 0));
   q.groups_w = (p.ow + 4 * cg - 1) / (4 * cg);
   const int64_t items = (int64_t)((p.oh + rows - 1) / rows) * q.groups_w;
   // 256 * items (the span of a group of planes) must fit 32 bits
@@ -468,9 +490,9 @@ hipError_t LaunchDwConv3x3(int stride, int out_kind, const DwConvParams& p, hipS
     gcd = a;
     a = t;
   }
-  q.planes_per_group = 256 / gcd;
+  q.planes_per_group = (int16_t)(256 / gcd);
   q.blocks_per_group = (int)((int64_t)q.planes_per_group * q.items / 256);
-  q.planes_per_block = 256 / q.items + 2;  // bound on the planes one workgroup touches
+  q.planes_per_block = (int16_t)(256 / q.items + 2);  // bound on the planes one workgroup touches
   q.magic_items = Magic(q.items);
   q.magic_groups = Magic(q.groups_w);
   q.magic_blocks = Magic(q.blocks_per_group);
@@ -482,42 +504,30 @@ hipError_t LaunchDwConv3x3(int stride, int out_kind, const DwConvParams& p, hipS
   const int shape = 100 * stride + 10 * rows + cg;
   switch (shape) {
     case 121:
-      LaunchShape<1, 2, 1>(out_kind, grid, stream, q);
-      break;
+      return LaunchShape<1, 2, 1>(out_kind, grid, stream, q);
     case 141:
-      LaunchShape<1, 4, 1>(out_kind, grid, stream, q);
-      break;
+      return LaunchShape<1, 4, 1>(out_kind, grid, stream, q);
     case 112:
-      LaunchShape<1, 1, 2>(out_kind, grid, stream, q);
-      break;
+      return LaunchShape<1, 1, 2>(out_kind, grid, stream, q);
     case 122:
-      LaunchShape<1, 2, 2>(out_kind, grid, stream, q);
-      break;
+      return LaunchShape<1, 2, 2>(out_kind, grid, stream, q);
     case 142:
-      LaunchShape<1, 4, 2>(out_kind, grid, stream, q);
-      break;
+      return LaunchShape<1, 4, 2>(out_kind, grid, stream, q);
     case 114:
-      LaunchShape<1, 1, 4>(out_kind, grid, stream, q);
-      break;
+      return LaunchShape<1, 1, 4>(out_kind, grid, stream, q);
     case 124:
-      LaunchShape<1, 2, 4>(out_kind, grid, stream, q);
-      break;
+      return LaunchShape<1, 2, 4>(out_kind, grid, stream, q);
     case 221:
-      LaunchShape<2, 2, 1>(out_kind, grid, stream, q);
-      break;
+      return LaunchShape<2, 2, 1>(out_kind, grid, stream, q);
     case 212:
-      LaunchShape<2, 1, 2>(out_kind, grid, stream, q);
-      break;
+      return LaunchShape<2, 1, 2>(out_kind, grid, stream, q);
     case 222:
-      LaunchShape<2, 2, 2>(out_kind, grid, stream, q);
-      break;
+      return LaunchShape<2, 2, 2>(out_kind, grid, stream, q);
     case 214:
-      LaunchShape<2, 1, 4>(out_kind, grid, stream, q);
-      break;
+      return LaunchShape<2, 1, 4>(out_kind, grid, stream, q);
     default:
       return hipErrorInvalidValue;
   }
-  return hipGetLastError();
 }
 
 }  // namespace pl

@@ -343,27 +343,31 @@ hipError_t LaunchBlockMfma(const MfmaConfig& cfg, const MfmaParams& p, hipStream
 
 // Chunk MFMA SpMM (int8, chunk_mfma_kernels.hip): dense 16x64 weight tiles, the channels taken chunk by chunk.
 struct ChunkMfmaParams {
+  // the first 56 bytes: what the first loads of the kernel need (kernarg_head.h)
   const int8_t* x;
-  void* out;
   // [row tile of 16][64-channel step][64 lanes][16 bytes]; lane l of a tile holds row l % 16, byte t channel
   // 64 step + 16 (l / 16) + t; in the last, partial group of 16 channels byte t is channel K - 16 + t (zero where
   // that channel belongs to the group before)
   const void* wtiles;
-  const float* scale;  // padded to a multiple of 32 rows
-  const float* bias;   // likewise (zeros when the op has no bias)
-  int K, M;
+  int K;
   int hw;
-  int batch;
-  DevAct act;
   // filled in by the launcher
   int qpi;               // position quads per image = ceil(hw / 4)
-  int quad_aligned;      // hw % 4 == 0
   uint32_t total_quads;  // batch * qpi
+  int tile_quads;        // position quads of a tile
+  int tiles, row_groups;
   int row_tiles;         // ceil(M / 16)
   int padded_ksteps;     // steps wtiles holds, the last ones zero
   int chunks;
-  int tile_quads;        // position quads of a tile
-  int tiles, row_groups;
+  // behind the head
+  int quad_aligned;      // hw % 4 == 0
+  // from the caller again
+  int M;
+  int batch;
+  void* out;
+  const float* scale;  // padded to a multiple of 32 rows
+  const float* bias;   // likewise (zeros when the op has no bias)
+  DevAct act;
 };
 
 // How a call is divided: a tile width, the workgroups it makes (of 128 rows x one tile; a CU holds one at a time) and
