@@ -509,18 +509,25 @@ bool FloatMfmaFits(bool f32, int K, int M, int hw, int64_t positions) {
 }
 
 // The rows a workgroup takes: the least of the times fitted to 5600 random calls in fp32 and 4600 in fp16 (32 - 2048
-// channels and rows, 50 - 100 000 positions, 256 CUs); picks the fastest form in all but 5 % of them.  Many rows per workgroup fetch the
-// inputs the fewest times, few rows let small calls fill the chip and halve the chain of a chunk: 64 x 1024 -> 1024 @7x7
+// channels and rows, 50 - 100 000 positions, 256 CUs); the form picked takes 0.1 % (fp32) and 1.2 % (fp16) longer than the
+// fastest on average.  Many rows per workgroup fetch the inputs the fewest times, few rows let small calls fill the chip
+// and halve the chain of a chunk: 64 x 1024 -> 1024 @7x7
 // fp32 256 rows 37.3, 128 rows 29.4, 64 rows 40.9; 64 x 512 -> 512 @14x14 25.9, 34.1, 47.7; one image 96 -> 192 @56x56 8.0, 6.9, 6.4.
 FloatMfmaPlan PlanFloatMfma(bool f32, int cus, int row_blocks, int K, int M, int hw, int batch) {
   const int64_t tiles = ((int64_t)batch * ((hw + 3) / 4) + kQuads - 1) / kQuads;
   const int chunks = (K + kChunk - 1) / kChunk;
-  // us: a launch, a chunk of it; full chip (fp32) and every further round of workgroups (fp16: beyond one per CU, two fit)
+  // us: a launch, a chunk of it; a full chip and a chunk of it; every workgroup beyond one per CU and a chunk of it (fp16,
+  // where two share a CU); every further round of workgroups and a chunk of it; outputs
   struct Cost {
-    double launch, chunk, full, full_chunk, round, round_chunk;
+    double launch, chunk, full, full_chunk, over, over_chunk, round, round_chunk, out;
   };
-  static constexpr Cost kF32[3] = {{4.5, 1.56, 2.9, 0.89, 4.8, 2.1}, {4.6, 0.98, 2.0, 0.56, 5.0, 1.22}, {4.5, 0.74, 1.2, 0.4, 4.4, 0.82}};
-  static constexpr Cost kF16[3] = {{3.9, 0.67, 0.0, 0.0, 2.5, 1.6}, {4.2, 0.48, 0.0, 0.0, 2.2, 1.14}, {4.0, 0.4, 0.0, 0.0, 3.2, 0.75}};
+  static constexpr Cost kF32[3] = {
+      {4.5, 1.56, 2.9, 0.89, 0, 0, 4.8, 2.1, 0}, {4.6, 0.98, 2.0, 0.56, 0, 0, 5.0, 1.22, 0}, {4.5, 0.74, 1.2, 0.4, 0, 0, 4.4, 0.82, 0}};
+  // maps of whole and of ragged quads
+  static constexpr Cost kF16[2][3] = {
+      {{3.1, 0.57, 0, 0.34, 0.57, 0.27, 0.023, 0.79, 0.4}, {3.7, 0.38, 0, 0.33, 0.43, 0.41, 0.74, 0.36, 0.31}, {3.6, 0.31, 0.8, 0.21, 0.84, 0.23, 2.1, 0.32, 0}},
+      {{3.8, 0.66, 0, 0.28, 0.13, 0.34, 0, 0.91, 0.59}, {4.1, 0.47, 0, 0.3, 0.4, 0.33, 0.68, 0.5, 0.43}, {3.8, 0.39, 0.42, 0.26, 0.52, 0.25, 2.5, 0.32, 0.13}}};
+  const double positions = (double)batch * hw;
   FloatMfmaPlan best{};
   for (int i = 0; i < 3; ++i) {
     const int wr = 8 >> i;
@@ -529,11 +536,11 @@ FloatMfmaPlan PlanFloatMfma(bool f32, int cus, int row_blocks, int K, int M, int
     p.wr = wr;
     p.row_groups = ((M + 31) / 32 + wr - 1) / wr;
     p.workgroups = 8ll * p.row_groups * ((tiles + 7) / 8);
-    const double per_cu = (double)p.workgroups / cus;
-    const Cost& c = f32 ? kF32[i] : kF16[i];
-    double rounds = per_cu > 1.0 ? per_cu - 1.0 : 0.0;
-    if (f32) rounds = (double)((p.workgroups + cus - 1) / cus - 1);
-    p.us = c.launch + c.chunk * chunks + (per_cu < 1.0 ? per_cu : 1.0) * (c.full + c.full_chunk * chunks) + rounds * (c.round + c.round_chunk * chunks);
+    const Cost& c = f32 ? kF32[i] : kF16[hw % 4 != 0][i];
+    const int64_t used = f32 ? p.workgroups : p.row_groups * tiles;  // fp16: without those of the last eight tiles that return at once
+    const double per_cu = (double)used / cus, over = per_cu > 1.0 ? per_cu - 1.0 : 0.0, rounds = (double)((used + cus - 1) / cus - 1);
+    p.us = c.launch + c.chunk * chunks + (per_cu < 1.0 ? per_cu : 1.0) * (c.full + c.full_chunk * chunks) + over * (c.over + c.over_chunk * chunks) + rounds * (c.round + c.round_chunk * chunks) +
+           1e-6 * c.out * positions * M * 256.0 / cus;
     if (best.wr == 0 || p.us < best.us) best = p;
   }
   return best;

@@ -993,34 +993,44 @@ bool ChunkMfmaPays(const pl_sparse_conv_handle* h, int call_algo, int batch, int
   return !h->block_asked && ChunkMfmaBeatsBlock(h, batch, im_size, cus);
 }
 
-// Whether a floating-point call runs on the matrix cores (float_mfma_kernels.hip).  The rules were fitted to 5600 random
-// calls in fp32 and 4600 in fp16, every form and the walk timed (32 - 2048 channels and rows, 50 - 100 000 positions,
-// 70 - 95 % zeros).
+// What the float walks are expected to take, by the positions a lane can load at a time and by the tile their channels
+// allow (128, 64, 32 and 16 positions): launch, entries of the index lists over all positions (single rows; pairs of
+// rows), inputs staged, outputs stored, filling the first tile, the entries of a single position's lists.  Fitted to
+// 4600 random calls in half precision and 5600 in fp32 (32 - 2048 channels and rows, 50 - 100 000 positions, 70 - 95 % zeros, 256
+// CUs); within -16 .. +9 % for half of them.
+double WalkMicroseconds(const pl_sparse_conv_handle* h, int cus, double positions, int im_size, bool aligned16) {
+  struct Cost {
+    double launch, entry, pair_entry, in, out, tile, list;
+  };
+  static constexpr Cost kHalf[3][4] = {
+      {{3.7, 1.1, 2.4, 3.7, 2.9, 9, 1.5}, {4, 2, 4.7, 4.4, 0, 5.6, 0.74}, {4.3, 2.9, 5.4, 4.9, 0, 4.3, 0.56}, {6.8, 2.6, 5.3, 7.4, 0, 3.2, 0.49}},
+      {{3.8, 2.2, 2.9, 3.2, 5.2, 7.8, 1.1}, {4.3, 3.2, 5.7, 3.8, 1.3, 6.4, 0.66}, {4.6, 3.3, 7.2, 8.1, 1.8, 7.2, 0.6}, {5.4, 2.4, 7.9, 12, 0, 5.2, 0.52}},
+      {{5.2, 0, 0.11, 6.7, 17, 18, 1.4}, {7, 1.5, 3.9, 5.9, 13, 6.6, 0.85}, {5.9, 2.2, 5.2, 7.2, 7.4, 7.5, 0.74}, {6.5, 1.9, 5.8, 12, 0, 5.6, 0.87}}};
+  static constexpr Cost kSingle[2][4] = {
+      {{3.3, 3.1, 3.9, 7.6, 6.8, 4, 1.3}, {4.1, 4.8, 7.9, 7.5, 0.24, 3.3, 0.54}, {3.9, 5.8, 8.3, 10, 0, 4.2, 0.55}, {4.9, 6, 9.3, 16, 0, 2.6, 0.63}},
+      {{4.5, 1.4, 2.9, 9.2, 17, 8.4, 1.3}, {5, 3.9, 6.4, 9.5, 12, 6.2, 0.57}, {5.7, 6.1, 12, 11, 1.6, 4.5, 0.55}, {6.9, 6.1, 12, 20, 0, 4.2, 0.52}}};
+  const int loads = !aligned16 || im_size % 4 != 0 ? 2 : (im_size % 8 != 0 ? 1 : 0);
+  const int form = h->ic <= 271 ? 0 : (h->ic <= 543 ? 1 : (h->ic <= 1087 ? 2 : 3));
+  const Cost& c = h->half ? kHalf[loads][form] : kSingle[loads / 2][form];
+  const double entries = static_cast<double>(h->entries), work = positions * 256.0 / cus;
+  return c.launch + 1e-3 * c.tile * h->ic + 1e-4 * c.list * entries + work * (1e-8 * (h->semi ? c.pair_entry : c.entry) * entries + 1e-7 * (c.in * h->ic + c.out * h->oc));
+}
+
+// Where the walk is expected to take 1.2 times (half precision: 1.15 times) as long: of the calls above 1570 of 5600 in fp32 and
+// 3070 of 4600 in half precision are taken, 18 and 13 of these are more than 10 % slower than the walk (by up to 1.29 and 1.38
+// times), 830 and 96 others would have gained more than 10 %.  Of 3100 and 2900 other calls 15 and 9 are more than 10 %
+// slower than by the walk alone; on average the rule makes fp32 1.11 and half precision 1.49 times as fast.
 bool FloatMfmaPays(const pl_sparse_conv_handle* h, int batch, int im_size, bool aligned16) {
   const int64_t positions = static_cast<int64_t>(batch) * im_size;
   if (!h->wfloat.ptr || !pl::FloatMfmaFits(!h->half, h->ic, h->oc, im_size, positions)) return false;
   if (!h->walk_plain_fits && !(im_size % 4 == 0 && aligned16)) return false;  // refused by the walks
   if (h->float_mfma == 2) return true;
-  const int cus = std::max(1, h->wg_slots_default / 2);
+  // Calls of few products in half precision keep the walks, whose sums follow the reference's value for value; either way
+  // takes 4 - 9 us.
   const double P = static_cast<double>(positions);
-  if (h->half) {
-    // Ahead almost everywhere (1.7 times on average).  Calls of few products keep the walks, whose sums follow the
-    // reference's half precision value for value; either way takes 4 - 9 us.  A call that fills the chip with few nonzeros per row on
-    // maps the walk loads 16 bytes at a time is memory's: 16 x 32 -> 384 @48x48, 93 % zeros 8.1 against 13.0 us here; 102 x 96 -> 200
-    // @20x20, 86 % 9.6 against 11.9.  Of 3260 calls taken 51 are more than 10 % slower than before, by up to 1.55 times.
-    if (P * h->ic * h->oc <= 4e7) return false;
-    return !(im_size % 8 == 0 && aligned16 && h->nnz < 32ll * h->oc && pl::PlanFloatMfma(false, cus, 8, h->ic, h->oc, im_size, batch).workgroups >= cus);
-  }
-  // fp32: where the walk is expected to take 1.1 times as long.  Its time by the form its channels allow (tiles of 128, 64,
-  // 32 and 16 positions): launch and first tile, entries of the index lists, inputs staged and outputs stored (element by
-  // element on ragged maps); within -20 .. +7 % for half of the calls.  Of 1940 calls taken 74 are more than 10 % slower than before, by
-  // up to 1.35 times; 683 others would have gained more than that.
-  const bool vec = im_size % 4 == 0 && aligned16;
-  const int form = h->ic <= 271 ? 0 : (h->ic <= 543 ? 1 : (h->ic <= 1087 ? 2 : 3));
-  static constexpr double kFirst[4] = {0.0, 2.0, 4.0, 8.0}, kEntry[2][4] = {{5.0e-8, 5.0e-8, 7.5e-8, 10.0e-8}, {6.0e-8, 6.0e-8, 9.0e-8, 12.5e-8}};
-  const double walk = (vec ? 3.9 : 5.5) + kFirst[form] + P * (static_cast<double>(h->entries) * kEntry[h->semi][form] + h->ic * (vec ? 6.5e-7 : 8e-7) + h->oc * (vec ? 5.5e-7 : 15e-7)) * 256.0 / cus;
-  if (walk < 1.1 * 5.2) return false;  // less than any form takes
-  return 1.1 * pl::PlanFloatMfma(true, cus, h->float_mfma_rows / 32, h->ic, h->oc, im_size, batch).us < walk;
+  if (h->half && P * h->ic * h->oc <= 4e7) return false;
+  const int cus = std::max(1, h->wg_slots_default / 2);
+  return (h->half ? 1.15 : 1.2) * pl::PlanFloatMfma(!h->half, cus, h->float_mfma_rows / 32, h->ic, h->oc, im_size, batch).us < WalkMicroseconds(h, cus, P, im_size, aligned16);
 }
 
 // The algorithm of one call (pl_sparse_conv_algo_for reports it).
