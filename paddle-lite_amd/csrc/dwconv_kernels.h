@@ -26,9 +26,9 @@ struct DwConvParams {
   int8_t pad;              // 0 or 1, all four sides
   int8_t act_type;         // act.type
   int8_t lanes_shared;     // share_lanes as it was chosen
-  int8_t reserved;
+  int8_t quads;            // items on the matrix cores
+  uint32_t magic_channels; // ceil(2^32 / channels) likewise
   // behind the head
-  uint32_t magic_channels; // likewise for channels
   int row_lds_in;          // row items: bytes of LDS for the staged input
   // from the caller again
   void* out;               // NCHW [batch, channels, oh, ow], fp32 or int8

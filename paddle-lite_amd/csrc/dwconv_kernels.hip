@@ -24,6 +24,8 @@ namespace {
 using namespace epilogue;
 
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 
 // what the first loads need arrives in registers
 PL_IN_HEAD(DwConvParams, x);
@@ -41,6 +43,8 @@ PL_IN_HEAD(DwConvParams, planes_per_block);
 PL_IN_HEAD(DwConvParams, pad);
 PL_IN_HEAD(DwConvParams, act_type);
 PL_IN_HEAD(DwConvParams, lanes_shared);
+PL_IN_HEAD(DwConvParams, quads);
+PL_IN_HEAD(DwConvParams, magic_channels);
 
 // Dword at `ptr` (any alignment).  SAFE: the caller knows that the four
 // bytes lie inside the tensor.  Otherwise bytes outside [lo, hi) read as zero
@@ -87,6 +91,65 @@ __device__ __forceinline__ void LoadInside(const int8_t* ptr, const int8_t* lo, 
   }
 #pragma unroll
   for (int k = 0; k < K; ++k) D[k] = __builtin_amdgcn_alignbyte(e[k + 1], e[k], d & 3u);
+}
+
+// Activation, quantisation and stores of the R rows from oy0 on of 4 * CG outputs; at(o): where row oy0 + o starts.
+template <int R, int CG, int OUT, int ACT, typename At>
+__device__ __forceinline__ void DwStore(const DwConvParams& p, const int (&acc)[R][4 * CG], float s, float b, int oy0, int ox0, At&& at) {
+#pragma unroll
+  for (int o = 0; o < R; ++o) {
+    if (o > 0 && oy0 + o >= p.oh) break;
+    if (OUT == kOutI8) {
+      uint32_t packed[CG];
+#pragma unroll
+      for (int q4 = 0; q4 < CG; ++q4) {
+        float q[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) q[k] = ActQuantF<ACT>(__builtin_fmaf((float)acc[o][4 * q4 + k], s, b), p.act);
+        packed[q4] = TruncPackI8x4(q[0], q[1], q[2], q[3]);
+      }
+      int8_t* dst = reinterpret_cast<int8_t*>(at(o));
+      // global memory takes dword and short stores at any byte address
+      if (CG > 1 && ox0 + 4 * CG <= p.ow) {
+        // the whole item in one store: the wavefront's stores are then contiguous
+        if (CG == 2) {
+          *reinterpret_cast<uint2*>(dst) = make_uint2(packed[0], packed[CG - 1]);
+        } else {
+          *reinterpret_cast<uint4*>(dst) = make_uint4(packed[0], packed[1 % CG], packed[2 % CG], packed[3 % CG]);
+        }
+      } else {
+#pragma unroll
+        for (int q4 = 0; q4 < CG; ++q4) {
+          const int n_out = min(4, p.ow - (ox0 + 4 * q4));
+          if (n_out <= 0) break;
+          if (n_out == 4) {
+            *reinterpret_cast<uint32_t*>(dst + 4 * q4) = packed[q4];
+          } else {
+            if (n_out >= 2) *reinterpret_cast<uint16_t*>(dst + 4 * q4) = (uint16_t)packed[q4];
+            if (n_out == 1) dst[4 * q4] = (int8_t)packed[q4];
+            if (n_out == 3) dst[4 * q4 + 2] = (int8_t)(packed[q4] >> 16);
+          }
+        }
+      }
+    } else {
+#pragma unroll
+      for (int q4 = 0; q4 < CG; ++q4) {
+        const int n_out = min(4, p.ow - (ox0 + 4 * q4));
+        if (n_out <= 0) break;
+        float v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = ActivateT<ACT>(__builtin_fmaf((float)acc[o][4 * q4 + k], s, b), p.act);
+        float* dst = reinterpret_cast<float*>(at(o)) + 4 * q4;
+        if (n_out == 4) {  // a four-dword store needs dword alignment only
+          *reinterpret_cast<v4f*>(dst) = v4f{v[0], v[1], v[2], v[3]};
+        } else {
+#pragma unroll
+          for (int k = 0; k < 4; ++k)
+            if (k < n_out) dst[k] = v[k];
+        }
+      }
+    }
+  }
 }
 
 // One item: 4 * CG neighbouring outputs (from column ox0 = 4 * CG * g) of the
@@ -207,62 +270,9 @@ __device__ __forceinline__ void DwItem(const DwConvParams& p, uint32_t plane, in
     }
   }
   const float s = p.scale[c], b = p.bias[c];
-#pragma unroll
-  for (int o = 0; o < R; ++o) {
-    const int oy = R * oyr + o;
-    if (oy >= p.oh) break;
-    const size_t row_at = ((size_t)plane * (uint32_t)p.oh + (uint32_t)oy) * (uint32_t)p.ow + (uint32_t)ox0;
-    if (OUT == kOutI8) {
-      uint32_t packed[CG];
-#pragma unroll
-      for (int q4 = 0; q4 < CG; ++q4) {
-        float q[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) q[k] = ActQuantF<ACT>(__builtin_fmaf((float)acc[o][4 * q4 + k], s, b), p.act);
-        packed[q4] = TruncPackI8x4(q[0], q[1], q[2], q[3]);
-      }
-      int8_t* dst = static_cast<int8_t*>(p.out) + row_at;
-      // global memory takes dword and short stores at any byte address
-      if (CG > 1 && ox0 + 4 * CG <= p.ow) {
-        // the whole item in one store: the wavefront's stores are then contiguous
-        if (CG == 2) {
-          *reinterpret_cast<uint2*>(dst) = make_uint2(packed[0], packed[CG - 1]);
-        } else {
-          *reinterpret_cast<uint4*>(dst) = make_uint4(packed[0], packed[1 % CG], packed[2 % CG], packed[3 % CG]);
-        }
-      } else {
-#pragma unroll
-        for (int q4 = 0; q4 < CG; ++q4) {
-          const int n_out = min(4, p.ow - (ox0 + 4 * q4));
-          if (n_out <= 0) break;
-          if (n_out == 4) {
-            *reinterpret_cast<uint32_t*>(dst + 4 * q4) = packed[q4];
-          } else {
-            if (n_out >= 2) *reinterpret_cast<uint16_t*>(dst + 4 * q4) = (uint16_t)packed[q4];
-            if (n_out == 1) dst[4 * q4] = (int8_t)packed[q4];
-            if (n_out == 3) dst[4 * q4 + 2] = (int8_t)(packed[q4] >> 16);
-          }
-        }
-      }
-    } else {
-#pragma unroll
-      for (int q4 = 0; q4 < CG; ++q4) {
-        const int n_out = min(4, p.ow - (ox0 + 4 * q4));
-        if (n_out <= 0) break;
-        float v[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) v[k] = ActivateT<ACT>(__builtin_fmaf((float)acc[o][4 * q4 + k], s, b), p.act);
-        float* dst = static_cast<float*>(p.out) + row_at + 4 * q4;
-        if (n_out == 4) {  // a four-dword store needs dword alignment only
-          *reinterpret_cast<v4f*>(dst) = v4f{v[0], v[1], v[2], v[3]};
-        } else {
-#pragma unroll
-          for (int k = 0; k < 4; ++k)
-            if (k < n_out) dst[k] = v[k];
-        }
-      }
-    }
-  }
+  DwStore<R, CG, OUT, ACT>(p, acc, s, b, R * oyr, ox0, [&](int o) {
+    return static_cast<char*>(p.out) + (((size_t)plane * (uint32_t)p.oh + (uint32_t)(R * oyr + o)) * (uint32_t)p.ow + (uint32_t)ox0) * (OUT == kOutI8 ? 1 : 4);
+  });
 }
 
 // x / d for any 32-bit x with magic = ceil(2^32 / d), d >= 2: the multiply-high
@@ -271,6 +281,124 @@ __device__ __forceinline__ uint32_t DivMagic(uint32_t x, uint32_t d, uint32_t ma
   if (d == 1) return x;
   const uint32_t q = __umulhi(x, magic);
   return q * d > x ? q - 1 : q;
+}
+
+// The channel of plane plane0 + pl, plane0 uniform: plane0 % channels + pl, less channels past the last one.
+__device__ __forceinline__ int DwChannel(const DwConvParams& p, uint32_t plane0, int pl) {
+  int c = (int)(plane0 - DivMagic(plane0, (uint32_t)p.channels, p.magic_channels) * (uint32_t)p.channels) + pl;
+  if (c >= p.channels) c = p.channels > p.planes_per_block ? c - p.channels : c % p.channels;
+  return c;
+}
+
+// The same item on the matrix cores, for rows of whole aligned dwords and padding 1.  What bounds the item above is its
+// instruction count (300 for 16 outputs at stride 1, 2/3 of the kernel's time on 112x112 planes).  The products of a
+// dword of an input row with the four outputs about it are one 4 x 4 x 4 product here: its four columns are four lanes'
+// dwords, its four rows the filter row at the four outputs' places, so that neither windows are cut out of the dwords
+// nor sums set to zero, and each lane ends with its own outputs (175 instructions and 24 products).  At stride 1 the one
+// byte on either side of the dword under the outputs is a product of both neighbours at once.  The four lanes
+// of a product must belong to one plane: items % 4 == 0.  Rows outside the plane are loads outside the buffer, which
+// are zero; offsets count from 16 bytes before plane0, so that they stay positive (SAFE workgroups only).  64 images,
+// us before / three products per row and quad / two: 32 planes of 112x112 16.8 / 16.1 / 14.9, 128 of 56x56
+// 15.7 / 15.7 / 14.6, 256 of 28x28 10.4 / 10.1 / 9.7; stride 2, 256 of 28x28 5.6 / 5.3; a copy of the bytes takes 11.6, 11.6
+// and 7.0.
+template <int STRIDE, int R, int CG, int OUT, int ACT>
+__device__ __forceinline__ void DwItemQuads(const DwConvParams& p, uint32_t plane0, int pl, int oyr, int g) {
+  constexpr int kRows = 3 + STRIDE * (R - 1), K = STRIDE * (CG - 1) + 3;
+  constexpr uint32_t kOutside = 0x80000000u;
+  const uint32_t hw = (uint32_t)(p.h * p.w);
+  const int ox0 = 4 * CG * g, cb = STRIDE * ox0, iy0 = STRIDE * R * oyr - 1;
+  const int64_t front = (int64_t)plane0 * hw - 16;
+  const int64_t rest = (int64_t)p.planes * hw - front;
+  const __amdgpu_buffer_rsrc_t xbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(p.x) + front, 0, (int)(rest < 0x7fffffff ? rest : 0x7fffffff), 0x00020000);
+  const uint32_t at = (uint32_t)pl * hw + (uint32_t)(iy0 * p.w + cb + 12);  // dword 0: four bytes before column cb
+  uint32_t d[kRows][K];
+#pragma unroll
+  for (int r = 0; r < kRows; ++r) {
+    // the row below the first is always inside: an output has at least one row of its window beside that of the padding
+    uint32_t off = at + (uint32_t)(r * p.w);
+    if (r == 0) off = oyr > 0 ? off : kOutside;
+    if (r >= 2) off = iy0 + r < p.h ? off : kOutside;
+#pragma unroll
+    for (int k = 0; k < K; k += 4) {
+      if (K - k >= 4) {
+        const v4u v = __builtin_amdgcn_raw_buffer_load_b128(xbuf, (int)off, 4 * k, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) d[r][k + i < K ? k + i : 0] = v[i];
+      } else {
+#pragma unroll
+        for (int i = k; i < K; ++i) d[r][i] = __builtin_amdgcn_raw_buffer_load_b32(xbuf, (int)off, 4 * i, 0);
+      }
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  const int c = DwChannel(p, plane0, pl);
+  const uint32_t wrow[3] = {p.wpack[4 * c], p.wpack[4 * c + 1], p.wpack[4 * c + 2]};
+  const float s = p.scale[c], b = p.bias[c];
+  // columns outside [0, w): dword 0 lies before column 0 or is inside, a later one is inside or past the last column
+  uint32_t mask[K];
+  mask[0] = g == 0 ? 0u : 0xffffffffu;
+#pragma unroll
+  for (int k = 1; k < K; ++k) mask[k] = cb + 4 * (k - 1) < p.w ? 0xffffffffu : 0u;
+  // row j of a product: lane % 4 == j holds the filter row where output j meets a dword: bytes STRIDE j + 3 .. + 2 of the
+  // twelve of three dwords (selector 0x0c is a zero byte).  Stride 1: the middle one, then byte 3 of the first as
+  // byte 3 and byte 0 of the last as byte 0; stride 2: each of them.
+  constexpr int T = STRIDE == 1 ? 2 : 3;
+  const int j = (int)(threadIdx.x & 3);
+  uint32_t sel[T];
+  if (STRIDE == 1) {
+    sel[0] = __builtin_amdgcn_alignbyte(0x0c0c0c02u, 0x01000c0cu, (uint32_t)(3 - j));
+    sel[1] = j == 0 ? 0x000c0c0cu : (j == 3 ? 0x0c0c0c02u : 0x0c0c0c0cu);
+  } else {
+    const uint32_t two = (j & 1) ? 0x0201000cu : 0x0c0c0201u;
+    sel[0] = j == 0 ? 0x000c0c0cu : 0x0c0c0c0cu;
+    sel[1] = j < 2 ? two : (j == 2 ? 0x000c0c0cu : 0x0c0c0c0cu);
+    sel[T - 1] = j < 2 ? 0x0c0c0c0cu : two;
+  }
+  int A[3][T];
+#pragma unroll
+  for (int fr = 0; fr < 3; ++fr)
+#pragma unroll
+    for (int t = 0; t < T; ++t) A[fr][t] = (int)__builtin_amdgcn_perm(0u, wrow[fr], sel[t]);
+  v4i sums[R][CG];
+#pragma unroll
+  for (int o = 0; o < R; ++o)
+#pragma unroll
+    for (int q = 0; q < CG; ++q) sums[o][q] = v4i{0, 0, 0, 0};
+#pragma unroll
+  for (int r = 0; r < kRows; ++r) {
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+      if (k != 1) d[r][k] &= mask[k];
+    int in[T][CG];
+#pragma unroll
+    for (int q = 0; q < CG; ++q) {
+      if (STRIDE == 1) {
+        in[0][q] = (int)d[r][q + 1];
+        in[1][q] = (int)__builtin_amdgcn_perm(d[r][q + 2], d[r][q], 0x03020104u);  // bytes 1 and 2 meet zeros
+      } else {
+#pragma unroll
+        for (int t = 0; t < T; ++t) in[t][q] = (int)d[r][2 * q + t];
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int o = 0; o < R; ++o) {
+        const int fr = r - STRIDE * o;
+        if (fr < 0 || fr > 2) continue;
+#pragma unroll
+        for (int q = 0; q < CG; ++q) sums[o][q] = __builtin_amdgcn_mfma_i32_4x4x4i8(A[fr][t], in[t][q], sums[o][q], 0, 0, 0);
+      }
+  }
+  int acc[R][4 * CG];
+#pragma unroll
+  for (int o = 0; o < R; ++o)
+#pragma unroll
+    for (int i = 0; i < 4 * CG; ++i) acc[o][i] = sums[o][i / 4][i % 4];
+  // offsets in 32 bits from the workgroup's first plane
+  char* const out0 = static_cast<char*>(p.out) + (int64_t)plane0 * (uint32_t)(p.oh * p.ow) * (OUT == kOutI8 ? 1 : 4);
+  const uint32_t row0 = ((uint32_t)pl * (uint32_t)p.oh + (uint32_t)(R * oyr)) * (uint32_t)p.ow + (uint32_t)ox0;
+  DwStore<R, CG, OUT, ACT>(p, acc, s, b, R * oyr, ox0, [&](int o) { return out0 + (row0 + (uint32_t)o * (uint32_t)p.ow) * (OUT == kOutI8 ? 1u : 4u); });
 }
 
 // One item per thread and no loop: a wavefront that has stores in flight can
@@ -288,9 +416,11 @@ __device__ __forceinline__ void DwItems(const DwConvParams& p, uint32_t plane0, 
   if (plane >= p.planes) return;
   const int oyr = (int)DivMagic((uint32_t)item, (uint32_t)p.groups_w, p.magic_groups);  // item / groups_w
   const int g = item - oyr * p.groups_w;
-  int c = (int)(plane0 - DivMagic(plane0, (uint32_t)p.channels, p.magic_channels) * (uint32_t)p.channels) + pl;  // plane0 % channels (uniform) + pl
-  if (c >= p.channels) c = p.channels > p.planes_per_block ? c - p.channels : c % p.channels;
-  DwItem<STRIDE, R, CG, OUT, ACT, SAFE>(p, plane, c, oyr, g);
+  if (SAFE && CG == 2 && p.quads) {
+    DwItemQuads<STRIDE, R, CG, OUT, ACT>(p, plane0, pl, oyr, g);
+  } else {
+    DwItem<STRIDE, R, CG, OUT, ACT, SAFE>(p, plane, DwChannel(p, plane0, pl), oyr, g);
+  }
 }
 
 template <int STRIDE, int R, int CG, int OUT, int ACT>
@@ -318,7 +448,7 @@ __device__ __forceinline__ void DwBody(const DwConvParams& p) {
 // R output rows by 4 * CG columns per item (the per-item address and mask
 // arithmetic is shared by all of them).
 template <int STRIDE, int R, int CG, int OUT>
-__global__ void __launch_bounds__(256) DwConv3x3Kernel(PL_HEAD_PARAMS, const DwConvParams block) {
+__global__ void __launch_bounds__(256, 4) DwConv3x3Kernel(PL_HEAD_PARAMS, const DwConvParams block) {
   const DwConvParams p = WithHead(block, PL_HEAD_ARGS);
   DispatchAct(p.act_type, [&](auto act_c) {
     constexpr int ACT = decltype(act_c)::value;
@@ -448,7 +578,8 @@ hipError_t LaunchDwConv3x3(int stride, int out_kind, const DwConvParams& p, hipS
   // 1x4): stride 1: 112x112 28.0 / - / - / 19.7 / 20.1, 56x56 26.5 / 24.4 /
   // - / 19.4 / 22.6, 28x28 14.2 / 14.1 / - / 12.9 / 13.3, 14x14 9.7 / 9.8 /
   // - / 9.8 / -; stride 2 (output size): 56x56 20.5 / - / 16.4 / 19.9 / 21.3,
-  // 28x28 11.2 / - / 10.2 / 11.8 / 12.0.
+  // 28x28 11.2 / - / 10.2 / 11.8 / 12.0.  With items on the matrix cores (2x2 / 4x2 / 1x4, per launch): 112x112 14.9 /
+  // 15.1 / 15.9, 56x56 14.6 / 17.1 / 17.8, 28x28 9.7 / 11.3 / 10.8; stride 2 (1x2 / 2x2): 56x56 13.8 / 15.0, 28x28 8.8 / 10.1.
   int rows = p.item_rows, cg = p.item_cols;
   const bool rows_given = rows == 1 || rows == 2 || rows == 4, cols_given = cg == 1 || cg == 2 || cg == 4;
   // Narrow planes of 16-byte aligned tensors: one output row per thread, global memory touched in aligned
@@ -493,6 +624,8 @@ hipError_t LaunchDwConv3x3(int stride, int out_kind, const DwConvParams& p, hipS
   q.planes_per_group = (int16_t)(256 / gcd);
   q.blocks_per_group = (int)((int64_t)q.planes_per_group * q.items / 256);
   q.planes_per_block = (int16_t)(256 / q.items + 2);  // bound on the planes one workgroup touches
+  // the matrix cores: rows of whole aligned dwords, four lanes of one plane, offsets within the planes of a workgroup in 32 bits
+  q.quads = cg == 2 && p.pad == 1 && p.w % 4 == 0 && reinterpret_cast<uintptr_t>(p.x) % 4 == 0 && q.items % 4 == 0 && (int64_t)(q.planes_per_block + 1) * p.h * p.w < (1ll << 29);
   q.magic_items = Magic(q.items);
   q.magic_groups = Magic(q.groups_w);
   q.magic_blocks = Magic(q.blocks_per_group);

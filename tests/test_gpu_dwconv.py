@@ -127,6 +127,20 @@ def test_item_shapes(stride, rows, cols, out):
             run_case(n, c, h, w, stride, pad, out, ACTS["relu6"](), True, seed=1000 * rows + 100 * cols + 10 * i + pad + stride, item_rows=rows, item_cols=cols)
 
 
+# items of two column groups on rows of whole aligned dwords go to the matrix cores, four lanes of one plane at a time, but
+# for the workgroups at the ends of the tensor: planes that share a workgroup and that take several, odd heights (the
+# last item has a row too many), a last group of four columns, the narrowest planes; the second tensor starts off a dword
+QUADS = {1: [(2, 2), (4, 2), (1, 2)], 2: [(1, 2), (2, 2)]}
+
+
+@pytest.mark.parametrize("stride,rows,cols", [(s, r, c) for s in (1, 2) for (r, c) in QUADS[s]])
+@pytest.mark.parametrize("out", ["int8", "fp32"])
+def test_matrix_core_items(stride, rows, cols, out):
+    for i, (n, c, h, w) in enumerate([(2, 40, 28, 28), (1, 300, 8, 4), (2, 150, 7, 8), (3, 30, 16, 24), (1, 40, 31, 52), (1, 9, 112, 112), (2, 700, 4, 8), (1, 7, 15, 236), (1, 2, 56, 56)]):
+        for guard in (64, 65):
+            run_case(n, c, h, w, stride, 1, out, ACTS["relu" if i % 2 else "none"](), True, seed=500 * rows + 10 * i + stride, guard=guard, item_rows=rows, item_cols=cols)
+
+
 # narrow planes (w + 2 * pad <= 16) take one whole output row per thread by
 # default; both that kernel and the general one, on every width it covers
 @pytest.mark.parametrize("row_items", [capi.TUNE_NEVER, capi.TUNE_ALWAYS], ids=["general", "row-items"])
