@@ -299,39 +299,34 @@ hipError_t LaunchFloatMfma(bool f32, int cus, int row_blocks, const FloatMfmaPar
 // Block MFMA SpMM (int8): dense 32x32 weight blocks pre-arranged in operand
 // order, empty blocks skipped through a per-row-block bit mask.
 struct MfmaParams {
-  // the first 56 bytes: what the first loads of the block kernel need (kernarg_head.h); from qpi on all but row_blocks,
-  // ksteps and small is filled in by the launcher
   const int8_t* x;
+  void* out;
   const void* wblocks;     // [row_blocks][ksteps][64 lanes][16 bytes]
-  int K;
+  const uint32_t* kmask;   // [row_blocks][kmask_words] bit ks set = block (rb, ks) has a nonzero
+  int kmask_words;         // ceil(ksteps / 32)
+  const float* scale;      // padded to 32 * row_blocks
+  const float* bias;       // padded likewise (zeros when the op has no bias)
+  int row_blocks;
+  int ksteps;              // ceil(K / 32)
+  int M, K;
   int hw;
+  uint32_t P;              // batch * hw
+  int small;               // 1: input and output tensors are each below 2 GB
+  DevAct act;
+  // filled in by the launcher
+  int vec;                 // hw >= 4: positions are handled four at a time by dword access
+  int quad_aligned;        // hw % 4 == 0: every quad is complete
   int qpi;                 // quads per image = ceil(hw / 4)
   uint32_t total_quads;    // batch * qpi
   int tiles;               // tiles of tile_quads quads
+  int tile_quads;
+  int sub_tiles;           // tiles per workgroup (1, 2 or 4)
   int row_groups;          // groups of four row blocks
-  int row_blocks;
-  int ksteps;              // ceil(K / 32)
-  int8_t vec;              // hw >= 4: positions are handled four at a time by dword access
-  int8_t quad_aligned;     // hw % 4 == 0: every quad is complete
-  int8_t small;            // 1: input and output tensors are each below 2 GB
-  int8_t sub_tiles;        // tiles per workgroup (1, 2 or 4)
-  int8_t tile_quads;
-  int8_t act_type;         // act.type
-  int8_t i8_stage;         // int8 output is regrouped through LDS for 16-byte stores
-  int8_t reserved;
-  // behind the head
-  void* out;
-  const uint32_t* kmask;   // [row_blocks][kmask_words] bit ks set = block (rb, ks) has a nonzero
-  int kmask_words;         // ceil(ksteps / 32)
-  int M;
-  const float* scale;      // padded to 32 * row_blocks
-  const float* bias;       // padded likewise (zeros when the op has no bias)
-  uint32_t P;              // batch * hw
+  int i8_stage;            // int8 output is regrouped through LDS for 16-byte stores
   // streaming variant (tiles cut per image, workgroups walk over tiles)
   int stream_tpi;          // tiles per image
   int stream_tiles;        // batch * stream_tpi
   int stream_lanes;        // workgroups per XCD and row group = tile stride of a workgroup
-  DevAct act;
 };
 
 struct MfmaConfig {

@@ -22,7 +22,6 @@
 // Positions are the flattened (image, pixel) index g = n*hw + p, so tiles do
 // not care about image boundaries.
 #include "epilogue.h"
-#include "kernarg_head.h"
 #include "launch_lds.h"
 #include "sparse_conv_kernels.h"
 
@@ -381,25 +380,6 @@ __global__ void __launch_bounds__(1024) RowWalkKernel(const WalkParams p) {
 // tile's quad j, so a lane ends up with the four consecutive positions of
 // each of its rows (one 16-byte fp32 store or one dword int8 store).
 // LDS: xt[kg][c*32 + j], 16-byte cells, kg = group of 16 input channels.
-// what the first loads of the block kernel need arrives in registers
-PL_IN_HEAD(MfmaParams, x);
-PL_IN_HEAD(MfmaParams, wblocks);
-PL_IN_HEAD(MfmaParams, K);
-PL_IN_HEAD(MfmaParams, hw);
-PL_IN_HEAD(MfmaParams, qpi);
-PL_IN_HEAD(MfmaParams, total_quads);
-PL_IN_HEAD(MfmaParams, tiles);
-PL_IN_HEAD(MfmaParams, row_groups);
-PL_IN_HEAD(MfmaParams, row_blocks);
-PL_IN_HEAD(MfmaParams, ksteps);
-PL_IN_HEAD(MfmaParams, vec);
-PL_IN_HEAD(MfmaParams, quad_aligned);
-PL_IN_HEAD(MfmaParams, small);
-PL_IN_HEAD(MfmaParams, sub_tiles);
-PL_IN_HEAD(MfmaParams, tile_quads);
-PL_IN_HEAD(MfmaParams, act_type);
-PL_IN_HEAD(MfmaParams, i8_stage);
-
 struct QuadInfo {
   uint32_t n;    // image
   uint32_t pp;   // first position of the quad in its image
@@ -1063,14 +1043,13 @@ __global__ void __launch_bounds__(256, (KSMAX == 4 ? 3 : 2)) StreamMfmaKernel(co
 // At least two workgroups per CU (two wavefronts per SIMD): caps the kernel
 // at 256 VGPRs.
 template <int KSMAX, int OUT>
-__global__ void __launch_bounds__(256, (KSMAX == 4 ? 4 : 2)) BlockMfmaKernel(PL_HEAD_PARAMS, const MfmaParams head_block) {
-  const MfmaParams p = WithHead(head_block, PL_HEAD_ARGS);
+__global__ void __launch_bounds__(256, (KSMAX == 4 ? 4 : 2)) BlockMfmaKernel(const MfmaParams p) {
   extern __shared__ uint4 xt[];
   if (!p.vec) {
     MfmaBody<KSMAX, OUT, -1, false>(p, xt);
     return;
   }
-  DispatchAct(OUT == kOutAcc32 ? 0 : p.act_type, [&](auto act_c) {
+  DispatchAct(OUT == kOutAcc32 ? 0 : p.act.type, [&](auto act_c) {
     constexpr int ACT = decltype(act_c)::value;
     MfmaBody<KSMAX, OUT, ACT, true>(p, xt);
   });
@@ -1113,17 +1092,17 @@ template <int OUT>
 hipError_t MfmaByKs(int ks_max, const MfmaParams& p, dim3 grid, dim3 block, size_t lds, hipStream_t s) {
   switch (ks_max) {
     case 2:
-      return LaunchWithHead(BlockMfmaKernel<2, OUT>, grid, block, lds, s, p);
+      return LaunchWithLds(BlockMfmaKernel<2, OUT>, grid, block, lds, s, p);
     case 4:
-      return LaunchWithHead(BlockMfmaKernel<4, OUT>, grid, block, lds, s, p);
+      return LaunchWithLds(BlockMfmaKernel<4, OUT>, grid, block, lds, s, p);
     case 8:
-      return LaunchWithHead(BlockMfmaKernel<8, OUT>, grid, block, lds, s, p);
+      return LaunchWithLds(BlockMfmaKernel<8, OUT>, grid, block, lds, s, p);
     case 16:
-      return LaunchWithHead(BlockMfmaKernel<16, OUT>, grid, block, lds, s, p);
+      return LaunchWithLds(BlockMfmaKernel<16, OUT>, grid, block, lds, s, p);
     case 32:
-      return LaunchWithHead(BlockMfmaKernel<32, OUT>, grid, block, lds, s, p);
+      return LaunchWithLds(BlockMfmaKernel<32, OUT>, grid, block, lds, s, p);
     case 64:
-      return LaunchWithHead(BlockMfmaKernel<64, OUT>, grid, block, lds, s, p);
+      return LaunchWithLds(BlockMfmaKernel<64, OUT>, grid, block, lds, s, p);
     default:
       return hipErrorInvalidValue;
   }
@@ -1195,8 +1174,7 @@ hipError_t LaunchBlockMfma(const MfmaConfig& cfg, const MfmaParams& p, hipStream
   q.total_quads = (p.P / (uint32_t)p.hw) * (uint32_t)q.qpi;
   q.vec = p.hw >= 4;
   q.quad_aligned = p.hw % 4 == 0;
-  q.tile_quads = (int8_t)cfg.tile_quads;
-  q.act_type = (int8_t)p.act.type;
+  q.tile_quads = cfg.tile_quads;
   uint32_t tiles = (q.total_quads + cfg.tile_quads - 1) / cfg.tile_quads;
   q.row_groups = (p.row_blocks + 3) / 4;
   // Streaming variant: large maps with 128 or 256 channels, whole row groups,
@@ -1225,7 +1203,7 @@ hipError_t LaunchBlockMfma(const MfmaConfig& cfg, const MfmaParams& p, hipStream
   q.sub_tiles = 1;
   if (cfg.ks_max == 2 && cfg.sub_tiles && q.vec && cfg.tile_quads == 32 && (p.row_blocks % 4 == 0 || p.row_blocks <= 2)) {
     const uint32_t t = 4u / (uint32_t)p.ksteps;
-    if (cfg.sub_tiles == 2 || (tiles / t) * q.row_groups >= 1024u) q.sub_tiles = (int8_t)t;
+    if (cfg.sub_tiles == 2 || (tiles / t) * q.row_groups >= 1024u) q.sub_tiles = (int)t;
   }
   tiles = (tiles + q.sub_tiles - 1) / q.sub_tiles;
   q.tiles = (int)tiles;  // workgroup-level tiles
