@@ -143,7 +143,7 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
   const int pitch_in = p.hw * (int)kElem;
   auto issue = [&](Quad<F32> (&rd)[UC], int chunk) {
     const uint32_t k = (uint32_t)(min(chunk * kChunk + 8 * kg, p.K - 8) + UC * part);
-    const uint32_t voff = chunk < p.chunks ? (vbase + k * (uint32_t)p.hw) * kElem : 0x80000000u;
+    const uint32_t voff = chunk < p.chunks ? (vbase + k * (uint32_t)p.hw) * kElem : kFloatMfmaOutside;
 #pragma unroll
     for (int i = 0; i < UC; ++i) {
       if constexpr (F32) {
@@ -200,13 +200,12 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
   // the wavefront's row block (past the last one: the last one again, not stored) and window of 32 quads
   const int rb = rg * WR + wave % WR, kh = wave / WR;
   const int n = lane & 31, half = lane >> 5;
-  const int wsteps = p.chunks * kSteps;
-  const __amdgpu_buffer_rsrc_t wbuf =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(static_cast<const char*>(p.wtiles)) + (size_t)min(rb, p.row_blocks - 1) * p.padded_ksteps * (1024 * PIECES), 0, wsteps * (1024 * PIECES), 0x00020000);
+  char* const wblock = const_cast<char*>(static_cast<const char*>(p.wtiles)) + (size_t)min(rb, p.row_blocks - 1) * p.padded_ksteps * (1024 * PIECES);
   h8 a[ADEPTH][STEPS][PIECES];
   auto load_weights = [&](h8 (&dst)[PIECES], int chunk, int ks) {
+    const __amdgpu_buffer_rsrc_t wbuf = __builtin_amdgcn_make_buffer_rsrc(wblock, 0, (int)FloatMfmaWeightBytes(chunk, p.chunks, PIECES), 0x00020000);
 #pragma unroll
-    for (int q = 0; q < PIECES; ++q) dst[q] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(wbuf, lane * 16, ((chunk * kSteps + kh * STEPS + ks) * PIECES + q) * 1024, 0));
+    for (int q = 0; q < PIECES; ++q) dst[q] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(wbuf, lane * 16, (int)FloatMfmaWeightTile(chunk, p.chunks, kh * STEPS + ks, PIECES, q), 0));
   };
   const uint4* const operand = xt + (2 * STEPS * kh + half) * (4 * QT) + n;
   // fp32: the products of two high pieces, and those of a high and a low one, which would otherwise each round the sum
@@ -259,7 +258,7 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
 
   // One chunk: kSteps x 4 cells.  Behind the multiplies of a step the next chunk's cells of one position go to the
   // other buffer; then the loads of the chunk DEPTH behind that one are issued into the registers this frees.
-  constexpr int PF = F32 ? 2 : 3;
+  constexpr int PF = F32 || (RAGGED && WR == 8) ? 2 : 3;  // operand cells in flight; the ragged form of 128 registers has room for two
   auto run_chunk = [&](auto slot_c, auto last_c, int chunk) {
     constexpr bool LAST = decltype(last_c)::value;  // no chunk is left to load
     constexpr int S = decltype(slot_c)::value, NEXT = (S + 1) % DEPTH, AS = S % ADEPTH;
@@ -287,7 +286,7 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
           rest[c] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[AS][ks][0], xl, rest[c], 0, 0, 0);
         }
       }
-      if (!LAST || ADEPTH < DEPTH) load_weights(a[AS][ks], chunk + ADEPTH, ks);
+      if (!LAST) load_weights(a[AS][ks], chunk + ADEPTH, ks);
 #pragma unroll
       for (int c = 0; c < KH; ++c) commit(r[NEXT], (S + 1) & 1, KH * ks + c);
       // the vector ALU's share of a step goes between its matrix instructions: a wavefront issues in order
@@ -433,7 +432,7 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
     }
   }
   // Stores past the end of the buffer are dropped, so lanes and rows without an output need no branch.
-  constexpr uint32_t kOutside = 0x80000000u;
+  constexpr uint32_t kOutside = kFloatMfmaOutside;
   const __amdgpu_buffer_rsrc_t obuf = __builtin_amdgcn_make_buffer_rsrc(p.out, 0, (int)((uint32_t)p.batch * (uint32_t)p.M * (uint32_t)p.hw * kElem), 0x00020000);
   const uint32_t pitch = (uint32_t)p.hw * kElem;
   const uint32_t obase = ((on * (uint32_t)p.M + (uint32_t)row0) * (uint32_t)p.hw + (uint32_t)opp) * kElem;
