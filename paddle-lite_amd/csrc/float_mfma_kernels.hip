@@ -10,13 +10,18 @@
 //
 // fp16: products and sums are exact to fp32, rounded to half precision once before the activation, which runs in half
 // precision as in the walks (against 64 bits 2.1e-4 in 2-norm, the walks, whose sums are binary16, 8e-4 .. 2.6e-3).
-// fp32: inputs and weights as two binary16 pieces each (22 - 23 bits), three of the four products.  A row's weights are
-// scaled by a power of two at prepare, a position's inputs by one that follows the largest of them seen so far, so
-// pieces keep their bits whatever the magnitudes (a value 2^-12 of its position's largest still has 22).  The products
-// with a low piece have sums of their own: the matrix cores cut sums off instead of rounding them, and every addition
-// to the large sum costs up to an ulp of it (512 channels, 85 % zeros, against 64 bits: 2.2e-7 in 2-norm with one sum, 1.4e-7
-// with two; the walks 1.6e-7).  Positions whose inputs hold an infinity or a NaN, which a dense product spreads through
-// its zero weights, are walked nonzero by nonzero at the end.
+// fp32: inputs and weights as two binary16 pieces each, the second one times 2^11, and three of the four products.  A
+// row's weights are scaled by a power of two at prepare, a position's inputs by one that follows the largest of them seen
+// so far.  A scaled value of 2^-13 and more is within 2^-23 of its pieces' sum, which is 2^-25 of its position's largest; a smaller one
+// keeps an absolute error of 2^-36.  The products with a low piece have sums of their own: the matrix cores cut sums off instead
+// of rounding them, and every addition to the large sum costs up to an ulp of it (512 channels, 85 % zeros, against 64
+// bits: 2.2e-7 in 2-norm with one sum, 1.4e-7 with two; the walks 1.6e-7).  Products with a zero weight add nothing, whatever the
+// input (a sum is cut off below its largest product that is not zero).
+//
+// What a dense product would get wrong is walked nonzero by nonzero at the end: outputs that an infinity or a NaN reached
+// through a zero weight, and in fp32 outputs too small for the absolute error of the small inputs of their position.  The quads
+// that hold such an input are marked; the error of a row there is at most 2^-36 of the sum of its scaled weights'
+// magnitudes, so a result of 2^-13 of that sum and more is within 2^-23, and anything less is walked.
 //
 // What bounds it: the way from L2 into a CU.  A chunk of the widest form takes 96 KB in fp32 (64 KB weights, 32 KB inputs;
 // half in fp16) and 2.0 us (0.9), 47 - 53 KB per us and CU, which no depth of prefetch raised (four chunks ahead instead of two:
@@ -57,6 +62,11 @@ constexpr int kSteps = kChunk / 16;      // matrix instructions' channel steps o
 constexpr int kQuads = 32;               // position quads of a tile
 constexpr int kThreads = 512;
 constexpr int kGroups = kChunk / 8;      // operand cells of a position and chunk (eight channels each)
+// A scaled input is kept times kFloatMfmaLow.  A new scale from kPeak on; a mark below kSmallBits, which is kFloatMfmaSmall
+// as the inputs are compared: bits without the sign, less one, so that zero is the largest.
+constexpr float kPeak = 0x1p15f * kFloatMfmaLow;
+constexpr uint32_t kSmallBits = (125u << 24) - 1u;
+static_assert(kFloatMfmaSmall * kFloatMfmaLow == 0x1p-2f, "kSmallBits");
 
 // what the first loads need arrives in registers
 PL_IN_HEAD(FloatMfmaParams, x);
@@ -75,7 +85,7 @@ PL_IN_HEAD(FloatMfmaParams, row_blocks);
 template <bool F32>
 using Quad = std::conditional_t<F32, u4, u2>;
 
-// One value of a call whose input holds infinities or NaNs: the nonzeros in index order, as the walks take them.
+// One value that the product cannot give: the nonzeros in index order, as the walks take them.
 __device__ __forceinline__ float WalkF32(const FloatMfmaParams& p, const float* x, int row, float bias) {
   const DevGroup g = p.groups[p.nr == 2 ? row >> 1 : row];
   const int r = row - g.row0;
@@ -98,8 +108,9 @@ __device__ __forceinline__ h1 WalkF16(const FloatMfmaParams& p, const h1* x, int
 }
 
 // LDS: two buffers of operand cells, or what the wavefronts of a row block hand to each other at the end; behind either
-// (a wavefront may still look at a flag when another has begun to hand over), for fp32, the positions' maxima and the two
-// flags.
+// (a wavefront may still look at a flag when another has begun to hand over), for fp32, the positions' maxima, the two
+// flags and the marks of the quads.
+constexpr int kF32Tables = (4 * kQuads + 4 + kQuads) * 4;
 constexpr int LdsTables(int wr, bool f32) {
   const int cells = 2 * (f32 ? 2 : 1) * kGroups * 4 * kQuads * 16, trade = 8 * (64 - 8 * wr) * 64 * 4;
   return cells > trade ? cells : trade;
@@ -168,9 +179,11 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
   };
   // the operand cells of position c of the quad: eight channels
   char* const cells = reinterpret_cast<char*>(xt + kg * (4 * QT) + j) + 2 * UC * part;
-  // fp32: every position's inputs are scaled by a power of two that follows the largest of them seen so far (below)
+  // fp32: every position's inputs are scaled by a power of two that follows the largest of them seen so far (below); this is
+  // kFloatMfmaLow times that
   [[maybe_unused]] float scale[4];
   [[maybe_unused]] float peak = 0.0f;
+  [[maybe_unused]] uint32_t low = 0xffffffffu;  // the smallest magnitude but zero, as kSmallBits
   auto put = [](char* dst, const uint32_t (&d)[UC / 2]) {
     *reinterpret_cast<u2*>(dst) = u2{d[0], d[1]};
   };
@@ -180,10 +193,15 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
       uint32_t hi[UC / 2], lo[UC / 2];
 #pragma unroll
       for (int i = 0; i < UC / 2; ++i) {
+        // the first pieces are one mixed-precision multiply-add each
         const float a = __uint_as_float(rd[2 * i][c]) * scale[c], b = __uint_as_float(rd[2 * i + 1][c]) * scale[c];
-        peak = fmaxf(peak, fmaxf(fabsf(a), fabsf(b)));
-        const h2 h = __builtin_convertvector((v2f{a, b}), h2);
-        const h2 l = __builtin_convertvector((v2f{a - (float)h.x, b - (float)h.y}), h2);
+        peak = fmaxf(fmaxf(peak, fabsf(a)), fabsf(b));
+        low = min(min(low, (__float_as_uint(a) << 1) - 1u), (__float_as_uint(b) << 1) - 1u);
+        const h2 both = {(h1)__builtin_fmaf(a, 1.0f / kFloatMfmaLow, 0.0f), (h1)__builtin_fmaf(b, 1.0f / kFloatMfmaLow, 0.0f)};
+        uint32_t word = __builtin_bit_cast(uint32_t, both);
+        asm("" : "+v"(word));  // the second value is taken from the word, not converted again
+        const h2 h = __builtin_bit_cast(h2, word);
+        const h2 l = __builtin_convertvector((v2f{__builtin_fmaf((float)h.x, -kFloatMfmaLow, a), __builtin_fmaf((float)h.y, -kFloatMfmaLow, b)}), h2);
         hi[i] = __builtin_bit_cast(uint32_t, h), lo[i] = __builtin_bit_cast(uint32_t, l);
       }
       put(dst, hi);
@@ -224,9 +242,11 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
   // while another is through the next chunk's values.
   uint32_t* const colmax = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(xt) + LdsTables(WR, F32));
   uint32_t* const flags = colmax + 4 * QT;
+  uint32_t* const marks = flags + 4;
   const uint32_t* const own_max = colmax + 4 * n;  // of the positions whose sums the lane holds
-  [[maybe_unused]] int own_exp[4];
-  auto scale_exp = [](uint32_t bits) { return max(1, min(254, 266 - (int)(bits >> 23))); };
+  [[maybe_unused]] uint32_t own_exps = 0;  // a byte each: four registers do not fit beside the sums
+  auto own_exp = [&](int c) { return (int)(own_exps >> (8 * c) & 0xffu); };
+  auto scale_exp = [](uint32_t bits) { return max(1, min(243, 266 - (int)(bits >> 23))); };
   auto collect = [&](Quad<F32> (&rd)[UC]) {
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
@@ -243,12 +263,16 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       const uint32_t m = colmax[4 * j + c], om = own_max[c];
-      if (__uint_as_float(m) * scale[c] >= 0x1p15f) scale[c] = __uint_as_float((uint32_t)scale_exp(m) << 23);
-      if (__uint_as_float(om) * __uint_as_float((uint32_t)own_exp[c] << 23) >= 0x1p15f) {
+      if (__uint_as_float(m) * scale[c] >= kPeak) {
+        scale[c] = __uint_as_float((uint32_t)(scale_exp(m) + 11) << 23);
+        marks[j] = 1;  // sums may lose bits, too
+      }
+      const int before = own_exp(c);
+      if (__uint_as_float(om) * __uint_as_float((uint32_t)before << 23) >= 0x1p15f) {
         const int e = scale_exp(om);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[c][i] = __builtin_amdgcn_ldexpf(acc[c][i], e - own_exp[c]), rest[c][i] = __builtin_amdgcn_ldexpf(rest[c][i], e - own_exp[c]);
-        own_exp[c] = e;
+        for (int i = 0; i < 16; ++i) acc[c][i] = __builtin_amdgcn_ldexpf(acc[c][i], e - before), rest[c][i] = __builtin_amdgcn_ldexpf(rest[c][i], e - before);
+        own_exps = (own_exps & ~(0xffu << (8 * c))) | (uint32_t)e << (8 * c);
       }
     }
 #pragma unroll
@@ -302,7 +326,10 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
       __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (F32) {
-      if (peak >= 0x1p15f) flags[(S + 1) & 1] = 1;
+      if (peak >= kPeak || low < kSmallBits) {  // one branch for both
+        if (peak >= kPeak) flags[(S + 1) & 1] = 1;
+        if (low < kSmallBits) marks[j] = 1;
+      }
       peak = 0.0f;
       __syncthreads();
       if (__builtin_amdgcn_readfirstlane(flags[(S + 1) & 1]) != 0) rescale(r[NEXT], (S + 1) & 1);
@@ -326,20 +353,23 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
   }
   if constexpr (!F32) align_quad(r[0]);
   if constexpr (F32) {
-    for (int i = tid; i < 4 * QT + 2; i += kThreads) colmax[i] = 0;  // and the flags
+    for (int i = tid; i < kF32Tables / 4; i += kThreads) colmax[i] = 0;  // and the flags and marks
     __syncthreads();
     align_quad(r[0]);
     collect(r[0]);
     __syncthreads();
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      scale[c] = __uint_as_float((uint32_t)scale_exp(colmax[4 * j + c]) << 23);
-      own_exp[c] = scale_exp(own_max[c]);
+      scale[c] = __uint_as_float((uint32_t)(scale_exp(colmax[4 * j + c]) + 11) << 23);
+      own_exps |= (uint32_t)scale_exp(own_max[c]) << (8 * c);
     }
   }
 #pragma unroll
   for (int c = 0; c < 4; ++c) commit(r[0], 0, c);
-  if constexpr (F32) peak = 0.0f;
+  if constexpr (F32) {
+    if (low < kSmallBits) marks[j] = 1;
+    peak = 0.0f;
+  }
   issue(r[0], DEPTH);
   __syncthreads();
   using More = std::false_type;
@@ -366,11 +396,12 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
   // Lane (n, half) holds rows 8 (i / 4) + 4 half + i % 4 (i = 0 .. 15) of the row block at the four positions of quad n.
   // Wavefronts that share a row block finish FIN of the sixteen each, from what the others hand over through LDS.
   float fin[4][FIN];
+  auto total = [&](int c, int i) { return F32 ? __builtin_fmaf(rest[c][i], 1.0f / kFloatMfmaLow, acc[c][i]) : acc[c][i]; };
   if constexpr (KH == 1) {
 #pragma unroll
     for (int c = 0; c < 4; ++c)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) fin[c][i] = F32 ? acc[c][i] + rest[c][i] : acc[c][i];
+      for (int i = 0; i < 16; ++i) fin[c][i] = total(c, i);
   } else {
     // [row block][finishing part][part it comes from, without its own][value][lane]
     float* const trade = reinterpret_cast<float*>(xt) + (wave % WR) * (KH * (KH - 1) * 4 * FIN * 64) + lane;
@@ -381,13 +412,13 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
 #pragma unroll
         for (int c = 0; c < 4; ++c)
 #pragma unroll
-          for (int i = 0; i < FIN; ++i) fin[c][i] = F32 ? acc[c][to * FIN + i] + rest[c][to * FIN + i] : acc[c][to * FIN + i];
+          for (int i = 0; i < FIN; ++i) fin[c][i] = total(c, to * FIN + i);
       } else {
         float* const dst = trade + slot_of(to, kh);
 #pragma unroll
         for (int c = 0; c < 4; ++c)
 #pragma unroll
-          for (int i = 0; i < FIN; ++i) dst[(c * FIN + i) * 64] = F32 ? acc[c][to * FIN + i] + rest[c][to * FIN + i] : acc[c][to * FIN + i];
+          for (int i = 0; i < FIN; ++i) dst[(c * FIN + i) * 64] = total(c, to * FIN + i);
       }
     }
     __syncthreads();
@@ -400,8 +431,8 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
         for (int i = 0; i < FIN; ++i) fin[c][i] += src[(c * FIN + i) * 64];
     }
   }
-  // An infinity or a NaN among the inputs of a position reaches every row of the product through the zero weights: such
-  // quads are left to the walk below.
+  // An infinity or a NaN among the inputs of a position reaches every row of the product through the zero weights.  Such
+  // quads are walked below, in fp32 those and the marked ones output by output.
   float poison = 0.0f;
 #pragma unroll
   for (int c = 0; c < 4; ++c) poison = __builtin_fmaf(fin[c][0], 0.0f, poison);
@@ -410,9 +441,10 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
   const uint32_t on = oq / (uint32_t)p.qpi;
   const int opp = 4 * (int)(oq - on * (uint32_t)p.qpi);
   int valid = oq >= p.total_quads ? 0 : min(4, p.hw - opp);
-  const bool bad = valid != 0 && poison != poison;
-  const int walked = bad ? valid : 0;
-  if (bad) valid = 0;
+  bool suspect = poison != poison;
+  if constexpr (F32) suspect = suspect || marks[n] != 0;
+  const int looked_at = suspect ? valid : 0;
+  if (suspect) valid = 0;
   float bias[FIN];
   [[maybe_unused]] int row_exp[FIN];
   const int table = min(rb, p.row_blocks - 1) * 32 + row_in_block;
@@ -448,7 +480,7 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
       if constexpr (F32) {
         u4 o;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) o[c] = __float_as_uint(ActivateT<ACT>(__builtin_amdgcn_ldexpf(fin[c][i], row_exp[i] + 127 - own_exp[c]) + bias[i], p.act));
+        for (int c = 0; c < 4; ++c) o[c] = __float_as_uint(ActivateT<ACT>(__builtin_amdgcn_ldexpf(fin[c][i], row_exp[i] + 127 - own_exp(c)) + bias[i], p.act));
         __builtin_amdgcn_raw_buffer_store_b128(o, obuf, whole, 0, 0);
         if constexpr (RAGGED) {
 #pragma unroll
@@ -465,12 +497,32 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
         }
       }
     }
-    if (walked != 0) {
+    if (looked_at != 0) {
+      uint64_t walk = 0;
+#pragma unroll
+      for (int i = 0; i < FIN; ++i) {
+        const int rr = 8 * (i >> 2) + (i & 3);
+        if (row0 + rr >= p.M) break;
+        if constexpr (F32) {
+          const float reach = reinterpret_cast<const float*>(p.row_exp + 32 * p.row_blocks)[table + rr];
+          float* dst = reinterpret_cast<float*>(static_cast<char*>(p.out) + obase + (size_t)rr * pitch);
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            if (c >= looked_at) break;
+            if (!(fabsf(fin[c][i]) >= reach)) {
+              walk |= 1ull << (4 * i + c);
+            } else {
+              dst[c] = ActivateT<ACT>(__builtin_amdgcn_ldexpf(fin[c][i], row_exp[i] + 127 - own_exp(c)) + bias[i], p.act);
+            }
+          }
+        } else {
+          walk |= (uint64_t)((1u << looked_at) - 1u) << (4 * i);
+        }
+      }
       const size_t xat = (size_t)on * p.K * p.hw + opp;
 #pragma unroll 1
-      for (int at = 0; at < FIN * walked; ++at) {
-        const int i = at / walked, c = at - i * walked, rr = 8 * (i >> 2) + (i & 3);
-        if (row0 + rr >= p.M) break;
+      for (; walk != 0; walk &= walk - 1) {
+        const int bit = __builtin_ctzll(walk), i = bit >> 2, c = bit & 3, rr = 8 * (i >> 2) + (i & 3);
         char* dst = static_cast<char*>(p.out) + obase + (size_t)rr * pitch;
         if constexpr (F32) {
           reinterpret_cast<float*>(dst)[c] = ActivateT<ACT>(WalkF32(p, static_cast<const float*>(p.x) + xat + c, row0 + rr, p.bias ? bias_of(row0 + rr) : 0.0f), p.act);
@@ -494,7 +546,7 @@ __global__ void __launch_bounds__(kThreads, F32 ? 2 : 4) FloatMfmaKernel(PL_HEAD
 template <int WR, bool F32>
 hipError_t Launch(const FloatMfmaParams& p, dim3 grid, hipStream_t s) {
   const dim3 block(kThreads);
-  constexpr size_t lds = LdsTables(WR, F32) + (F32 ? (4 * kQuads + 4) * 4 : 0);
+  constexpr size_t lds = LdsTables(WR, F32) + (F32 ? kF32Tables : 0);
   return p.quad_aligned ? LaunchWithHead(FloatMfmaKernel<WR, F32, false>, grid, block, lds, s, p) : LaunchWithHead(FloatMfmaKernel<WR, F32, true>, grid, block, lds, s, p);
 }
 

@@ -196,7 +196,7 @@ struct pl_sparse_conv_handle {
   bool half = false;
   pl::DevActH act_h{};
   DevBuf hw_kidx, hw_wts, hw_bias;
-  // fp32 / fp16 on the matrix cores: dense 32x16 tiles, in fp32 the exponents of the rows' scales behind them
+  // fp32 / fp16 on the matrix cores: dense 32x16 tiles, in fp32 what is kept per row behind them
   DevBuf wfloat;
   size_t float_row_exp = 0;      // where these begin
   int float_mfma = 1;            // 0 never, 1 by the rule, 2 whenever the shape allows
@@ -640,10 +640,11 @@ bool FloatMfmaWanted(const pl_sparse_conv_handle* h) {
 int BuildFloatMfma(const pl::DecodedLayout& L, pl_sparse_conv_handle* h) {
   const int blocks = CeilDiv(L.oc, 32), kss = pl::FloatMfmaPaddedSteps(L.ic), pieces = h->half ? 1 : 2;
   const size_t tile_values = static_cast<size_t>(blocks) * kss * pieces * 512;
-  std::vector<uint16_t> tiles(tile_values + (h->half ? 0 : static_cast<size_t>(blocks) * 64), 0);
+  std::vector<uint16_t> tiles(tile_values + (h->half ? 0 : static_cast<size_t>(blocks) * 128), 0);
   const uint32_t whole = static_cast<uint32_t>(L.ic) / 8u * 8u;  // channels in whole groups of eight
   // fp32: a row's weights are scaled by a power of two that takes the largest of them to [2^14, 2^15)
   std::vector<int32_t> row_exp(static_cast<size_t>(blocks) * 32, 0);
+  std::vector<double> row_sum(static_cast<size_t>(blocks) * 32, 0.0);
   bool finite = true;
   auto value = [](uint32_t bits) {
     float w;
@@ -668,7 +669,8 @@ int BuildFloatMfma(const pl::DecodedLayout& L, pl_sparse_conv_handle* h) {
     if (h->half) {
       finite = finite && (at[0] & 0x7c00u) != 0x7c00u;
     } else {
-      at[512] = FastHalfBits(w - HalfValue(at[0]));
+      at[512] = FastHalfBits((w - HalfValue(at[0])) * pl::kFloatMfmaLow);
+      row_sum[row] += std::fabs(w);
     }
   };
   for (const pl::RowGroup& g : L.groups) {
@@ -682,7 +684,12 @@ int BuildFloatMfma(const pl::DecodedLayout& L, pl_sparse_conv_handle* h) {
   // an infinite weight would reach every position through the zeros among the inputs
   if (!finite) return PL_OK;
   h->float_row_exp = tile_values * sizeof(uint16_t);
-  if (!h->half) std::memcpy(&tiles[tile_values], row_exp.data(), row_exp.size() * sizeof(int32_t));
+  if (!h->half) {
+    std::vector<float> reach(row_sum.size());
+    for (size_t i = 0; i < reach.size(); ++i) reach[i] = static_cast<float>(row_sum[i] * pl::kFloatMfmaSmall);
+    std::memcpy(&tiles[tile_values], row_exp.data(), row_exp.size() * sizeof(int32_t));
+    std::memcpy(&tiles[tile_values + 2 * row_exp.size()], reach.data(), reach.size() * sizeof(float));
+  }
   const hipError_t e = h->wfloat.Upload(tiles.data(), tiles.size() * sizeof(uint16_t));
   if (e != hipSuccess) return FailHip(e, "uploading the weight tiles");
   return PL_OK;

@@ -246,6 +246,9 @@ hipError_t LaunchHalfWalk(int nrows, int tile_pos, int threads, const HalfWalkPa
 // Floating-point SpMM on the matrix cores (float_mfma_kernels.hip): dense 32x16 weight tiles, the channels taken chunk by
 // chunk.
 constexpr int kFloatMfmaChunk = 64;
+// fp32: the second binary16 piece of a scaled value is what the first one leaves, times kFloatMfmaLow.  Values of kFloatMfmaSmall
+// and more have a relative error of at most 2^-23 in their pieces; below it the error stays at 2^-36 or less.
+constexpr float kFloatMfmaLow = 2048.0f, kFloatMfmaSmall = 0x1p-13f;
 
 struct FloatMfmaParams {
   // the first 56 bytes: what the first loads of a kernel need (kernarg_head.h)
@@ -271,9 +274,10 @@ struct FloatMfmaParams {
   int nr;                // rows per list of the plain walk, 1 or 2
   void* out;
   const void* bias;      // fp32 or binary16, padded to a multiple of 32 rows; may be null
-  // fp32, padded to a multiple of 32 rows: the tiles of a row hold w 2^-row_exp in two binary16 pieces, [step][piece][64 lanes][8]
+  // fp32, padded to a multiple of 32 rows: the tiles of a row hold w 2^-row_exp in two binary16 pieces, [step][piece][64 lanes][8];
+  // behind these, as floats: 2^-13 of the sum of a row's |w| 2^-row_exp
   const int32_t* row_exp;
-  // the plain walk's lists, for the positions whose inputs are not finite
+  // the plain walk's lists, for the outputs that the product cannot give
   const DevGroup* groups;
   const uint32_t* kidx;
   const uint32_t* wts;

@@ -122,6 +122,44 @@ def test_fp32_magnitudes(how, rows):
 
 
 @pytest.mark.parametrize("rows", ROWS)
+@pytest.mark.parametrize("channels", [[5], [150], [329], list(range(3, 330, 9))], ids=["first", "middle", "last", "many"])
+@pytest.mark.parametrize("size", [1e4, 1e6, 1e8, 1e12, 1e30])
+def test_fp32_large_inputs_stay_with_the_rows_that_read_them(size, channels, rows):
+    """Every output against the magnitudes of its own row: one that reads none of the large channels must be as exact as
+    without them.  Half of the inputs are zero, some positions have no other input than a large one."""
+    case = make_case("fp32", 2, 330, 70, 9, 7, act="none", sparsity=0.9)
+    case.bias = None
+    case.x = np.maximum(case.x, 0)
+    case.x[1, :, 3:5] = 0
+    case.x[:, channels] = np.where(case.x[:, channels] > 0.5, -size, size)
+    case.x[0, channels, 2] = 0.25
+    reads = (case.dense[:, channels] != 0).any(axis=1)
+    assert not reads.all() and reads.any()
+    check(case, "none", run_hip(case, kernel=forced(case, rows)))
+
+
+@pytest.mark.parametrize("rows", ROWS)
+@pytest.mark.parametrize("binades", [24, 60, 230])
+def test_fp32_inputs_of_all_magnitudes(binades, rows):
+    """Exponents spread evenly, so every position holds values that its largest one leaves few bits."""
+    case = make_case("fp32", 3, 200, 40, 5, 9, act="none", sparsity=0.95)
+    case.bias = None
+    rng = np.random.RandomState(2)
+    case.x = np.ldexp(case.x, rng.randint(-binades, 1, size=case.x.shape) + (100 if binades > 100 else 0)).astype(np.float32)
+    check(case, "none", run_hip(case, kernel=forced(case, rows)))
+
+
+def test_fp32_error_is_not_above_the_walks():
+    """2-norm against 64 bits of a deep layer (one sum for all products, which the matrix cores cut off, would be 1.4 times
+    the walk's)."""
+    case = make_case("fp32", 16, 512, 512, 14, 14, act="none", sparsity=0.85)
+    ref, _ = sums(case)
+    walk = make_kernel(case, tuning=capi.tuning(float_mfma=capi.TUNE_NEVER))[0]
+    off = [np.linalg.norm((run_hip(case, kernel=k) - ref).ravel()) for k in [walk] + [forced(case, rows) for rows in ROWS]]
+    assert max(off[1:]) <= off[0]
+
+
+@pytest.mark.parametrize("rows", ROWS)
 @pytest.mark.parametrize("paired", [False, True], ids=["unstructured", "semi"])
 @pytest.mark.parametrize("kind", sorted(KINDS))
 def test_infinities_and_nans_reach_only_the_rows_that_read_them(kind, paired, rows):
