@@ -636,7 +636,8 @@ bool FloatMfmaWanted(const pl_sparse_conv_handle* h) {
   return h->float_mfma != 0 && h->ic >= 8 && (h->float_mfma == 2 || h->nnz * 32 >= static_cast<int64_t>(h->oc) * h->ic);
 }
 
-// Dense 32x16 binary16 tiles for the floating-point product (FloatMfmaParams::wtiles).
+// Dense 32x16 binary16 tiles for the floating-point product (FloatMfmaParams::wtiles); none where a weight does not survive
+// in them.
 int BuildFloatMfma(const pl::DecodedLayout& L, pl_sparse_conv_handle* h) {
   const int blocks = CeilDiv(L.oc, 32), kss = pl::FloatMfmaPaddedSteps(L.ic), pieces = h->half ? 1 : 2;
   const size_t tile_values = static_cast<size_t>(blocks) * kss * pieces * 512;
@@ -645,7 +646,7 @@ int BuildFloatMfma(const pl::DecodedLayout& L, pl_sparse_conv_handle* h) {
   // fp32: a row's weights are scaled by a power of two that takes the largest of them to [2^14, 2^15)
   std::vector<int32_t> row_exp(static_cast<size_t>(blocks) * 32, 0);
   std::vector<double> row_sum(static_cast<size_t>(blocks) * 32, 0.0);
-  bool finite = true;
+  bool exact = true;
   auto value = [](uint32_t bits) {
     float w;
     std::memcpy(&w, &bits, 4);
@@ -655,34 +656,36 @@ int BuildFloatMfma(const pl::DecodedLayout& L, pl_sparse_conv_handle* h) {
     float top[2] = {0.0f, 0.0f};
     for (uint32_t j = 0; j < g.count; ++j) {
       const float w0 = value(L.w0[g.first + j]), w1 = g.nrows == 2 ? value(L.w1[g.first + j]) : 0.0f;
-      finite = finite && std::isfinite(w0) && std::isfinite(w1);
+      exact = exact && std::isfinite(w0) && std::isfinite(w1);
       top[0] = std::max(top[0], std::fabs(w0));
       top[1] = std::max(top[1], std::fabs(w1));
     }
     for (int i = 0; i < g.nrows; ++i) row_exp[g.row0 + i] = top[i] > 0.0f ? std::max(-127, std::min(126, std::ilogb(top[i]) - 14)) : 0;
   }
-  auto put = [&](int row, uint32_t c, float w) {
+  auto put = [&](int row, uint32_t c, float weight) {
     const uint32_t t = c < whole ? c & 7u : 8u - (static_cast<uint32_t>(L.ic) - c);
     const size_t lane = (static_cast<size_t>(row) & 31u) + 32u * ((c >> 3) & 1u);
     uint16_t* at = &tiles[((static_cast<size_t>(row >> 5) * kss + (c >> 4)) * pieces * 64 + lane) * 8 + t];
-    at[0] = FastHalfBits(w);
     if (h->half) {
-      finite = finite && (at[0] & 0x7c00u) != 0x7c00u;
-    } else {
-      at[512] = FastHalfBits((w - HalfValue(at[0])) * pl::kFloatMfmaLow);
-      row_sum[row] += std::fabs(w);
+      at[0] = FastHalfBits(weight);
+      exact = exact && (at[0] & 0x7c00u) != 0x7c00u;
+      return;
     }
+    const double w = std::ldexp(static_cast<double>(weight), -row_exp[row]);
+    at[0] = FastHalfBits(static_cast<float>(w));
+    at[512] = FastHalfBits(static_cast<float>((w - HalfValue(at[0])) * pl::kFloatMfmaLow));
+    // a weight far below its row's largest has lost its bits, which shows where the input of that one is zero
+    exact = exact && std::fabs(w - HalfValue(at[0]) - HalfValue(at[512]) / static_cast<double>(pl::kFloatMfmaLow)) <= std::fabs(w) * 0x1p-22;
+    row_sum[row] += std::fabs(w);
   };
   for (const pl::RowGroup& g : L.groups) {
-    float scale[2] = {1.0f, 1.0f};
-    for (int i = 0; !h->half && i < g.nrows; ++i) scale[i] = std::ldexp(1.0f, std::max(-126, std::min(127, -row_exp[g.row0 + i])));
     for (uint32_t j = 0; j < g.count; ++j) {
-      put(g.row0, L.ic_index[g.first + j], value(L.w0[g.first + j]) * scale[0]);
-      if (g.nrows == 2) put(g.row0 + 1, L.ic_index[g.first + j], value(L.w1[g.first + j]) * scale[1]);
+      put(g.row0, L.ic_index[g.first + j], value(L.w0[g.first + j]));
+      if (g.nrows == 2) put(g.row0 + 1, L.ic_index[g.first + j], value(L.w1[g.first + j]));
     }
   }
   // an infinite weight would reach every position through the zeros among the inputs
-  if (!finite) return PL_OK;
+  if (!exact) return PL_OK;
   h->float_row_exp = tile_values * sizeof(uint16_t);
   if (!h->half) {
     std::vector<float> reach(row_sum.size());

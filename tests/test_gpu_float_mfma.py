@@ -149,6 +149,35 @@ def test_fp32_inputs_of_all_magnitudes(binades, rows):
     check(case, "none", run_hip(case, kernel=forced(case, rows)))
 
 
+@pytest.mark.parametrize("paired", [False, True], ids=["unstructured", "semi"])
+@pytest.mark.parametrize("size", [1.0, 1e4, 1e6, 1e8, 1e12, 1e30])
+def test_fp32_weights_far_below_their_rows_largest(size, paired):
+    """One weight of every row is large and meets zeros: what is left are the small ones.  Where the tiles would not hold
+    these, the calls stay with the walks."""
+    case = make_case("fp32", 2, 330, 70, 9, 7, paired=paired, act="none", sparsity=0.9)
+    case.bias = None
+    case.dense[:, 100] = size
+    case.x[:, 100] = 0
+    case.x[1, 100, ::2] = 1
+    kernel = make_kernel(case, force_semi=paired, tuning=capi.tuning(float_mfma=capi.TUNE_ALWAYS))[0]
+    check(case, "none", run_hip(case, kernel=kernel))
+    taken = capi.lib().pl_sparse_conv_algo_for(kernel._handle, case.batch, case.im_size) == capi.ALGO_CHUNK_MFMA
+    assert taken == (size <= 1e4)
+
+
+def test_fp32_the_smallest_weights():
+    """Rows of subnormal weights, rows that reach from the smallest to the largest number."""
+    case = make_case("fp32", 1, 64, 40, 6, 6, act="none", sparsity=0.5)
+    case.bias = None
+    case.dense[:20] = np.where(case.dense[:20] != 0, np.float32(2.0 ** -140) * np.sign(case.dense[:20]), 0)
+    kernel = forced(case, 64)
+    case.x *= np.float32(1e30)
+    check(case, "none", run_hip(case, kernel=kernel))
+    case.dense[20, :2] = 3e38, 2.0 ** -149
+    kernel = make_kernel(case, tuning=capi.tuning(float_mfma=capi.TUNE_ALWAYS))[0]
+    assert capi.lib().pl_sparse_conv_algo_for(kernel._handle, 1, 36) == capi.ALGO_ROW_WALK
+
+
 def test_fp32_error_is_not_above_the_walks():
     """2-norm against 64 bits of a deep layer (one sum for all products, which the matrix cores cut off, would be 1.4 times
     the walk's)."""
