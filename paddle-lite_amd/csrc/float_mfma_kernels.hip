@@ -85,26 +85,42 @@ PL_IN_HEAD(FloatMfmaParams, row_blocks);
 template <bool F32>
 using Quad = std::conditional_t<F32, u4, u2>;
 
-// One value that the product cannot give: the nonzeros in index order, as the walks take them.
-__device__ __forceinline__ float WalkF32(const FloatMfmaParams& p, const float* x, int row, float bias) {
+// What the nonzeros at .. of a row's list (every step-th from there on) add to four neighbouring positions of x.
+// Eight entries at a time: their channels and weights first, then the inputs; the list's padding reads channel 0 and adds nothing.
+template <bool F32>
+__device__ __forceinline__ void WalkRow(const FloatMfmaParams& p, const char* x, int row, uint32_t at, uint32_t step, float (&acc)[4]) {
+  constexpr int kBatch = 8;
+  constexpr uint32_t kElem = F32 ? 4u : 2u;
   const DevGroup g = p.groups[p.nr == 2 ? row >> 1 : row];
   const int r = row - g.row0;
-  float acc = bias;
-  for (uint32_t e = 0; e < g.count; ++e) {
-    const uint32_t k = p.kidx[g.first + e];
-    if (k < (uint32_t)p.K) acc = __builtin_fmaf(x[(size_t)k * p.hw], __uint_as_float(p.wts[(size_t)(g.first + e) * p.nr + r]), acc);
+  for (uint32_t e = at; e < g.count; e += kBatch * step) {
+    uint32_t k[kBatch], w[kBatch];
+    Quad<F32> v[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const uint32_t from = g.first + min(e + (uint32_t)u * step, g.count - 1u);
+      k[u] = p.kidx[from];
+      w[u] = F32 ? p.wts[(size_t)from * p.nr + r] : p.wts[from] >> (16 * r);
+    }
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      if (e + (uint32_t)u * step >= g.count) k[u] = (uint32_t)p.K;
+      __builtin_memcpy(&v[u], x + (size_t)(k[u] < (uint32_t)p.K ? k[u] : 0u) * ((uint32_t)p.hw * kElem), sizeof(v[u]));
+    }
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      if (k[u] >= (uint32_t)p.K) continue;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        if constexpr (F32) {
+          acc[c] = __builtin_fmaf(__uint_as_float(v[u][c]), __uint_as_float(w[u]), acc[c]);
+        } else {
+          const uint32_t word = v[u][c >> 1];
+          acc[c] = __builtin_fmaf((float)half_act::HalfBits((uint16_t)(word >> (16 * (c & 1)))), (float)half_act::HalfBits((uint16_t)w[u]), acc[c]);
+        }
+      }
+    }
   }
-  return acc;
-}
-__device__ __forceinline__ h1 WalkF16(const FloatMfmaParams& p, const h1* x, int row, h1 bias) {
-  const DevGroup g = p.groups[p.nr == 2 ? row >> 1 : row];
-  const int shift = 16 * (row - g.row0);
-  h1 acc = bias;
-  for (uint32_t e = 0; e < g.count; ++e) {
-    const uint32_t k = p.kidx[g.first + e];
-    if (k < (uint32_t)p.K) acc = __builtin_fmaf16(x[(size_t)k * p.hw], __builtin_bit_cast(h1, (uint16_t)(p.wts[g.first + e] >> shift)), acc);
-  }
-  return acc;
 }
 
 // LDS: two buffers of operand cells, or what the wavefronts of a row block hand to each other at the end; behind either
@@ -114,6 +130,87 @@ constexpr int kF32Tables = (4 * kQuads + 4 + kQuads) * 4;
 constexpr int LdsTables(int wr, bool f32) {
   const int cells = 2 * (f32 ? 2 : 1) * kGroups * 4 * kQuads * 16, trade = 8 * (64 - 8 * wr) * 64 * 4;
   return cells > trade ? cells : trade;
+}
+
+// The outputs that the product could not give, by the whole wavefront: lane (n, half) brings the bits of its own (4 i + c: row
+// first_row + 8 (i / 4) + 4 half + i % 4, position c of quad n).  A row with many such quads
+// is walked by two lanes per quad, others by sixteen lanes per row and quad, four of these at a time.
+// What bounds it: with few quads two memory round trips per sixteen lanes' entries, with all of them the inputs, which every
+// row's nonzeros fetch again from L1 and L2.  fp32 16 x 512 -> 512 @14x14, 85 % zeros, one NaN / a NaN in every position: every lane
+// its own outputs, one value after the other, 108 / 436 us; this 23 / 70 (without any 14, the walk 15).
+template <bool F32>
+__device__ __forceinline__ void WalkOutputs(const FloatMfmaParams& p, uint64_t walk, int fin, int first_row, uint32_t first_quad) {
+  constexpr uint32_t kElem = F32 ? 4u : 2u;
+  constexpr int kManyQuads = 8;
+  const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), n = lane & 31, half = lane >> 5;  // not held in a register meanwhile
+  // four positions inside the map
+  const uint32_t image = (first_quad + (uint32_t)n) / (uint32_t)p.qpi;
+  const int position = 4 * (int)(first_quad + (uint32_t)n - image * (uint32_t)p.qpi);
+  const uint32_t inside = (uint32_t)min(position, p.hw - 4), past = (uint32_t)position - inside;
+  const uint32_t from_own = image * (uint32_t)p.K * (uint32_t)p.hw + inside, to_own = image * (uint32_t)p.M * (uint32_t)p.hw + inside;
+  int next = 0, row = 0, half_of = 0;
+  uint32_t quads = 0, bits = 0;  // of the present row: quads left; the lane's own four bits
+  for (;;) {
+    int taken = 0, quad = 0, item_row = 0;
+    uint32_t item_bits = 0;
+    bool many = false;
+    while (taken < 4) {
+      if (quads == 0) {
+        if (next == 2 * fin) break;
+        const int i = next >> 1;
+        half_of = next & 1;
+        ++next;
+        bits = half == half_of ? (uint32_t)(walk >> (4 * i)) & 15u : 0u;
+        quads = (uint32_t)(__ballot(bits != 0) >> (32 * half_of));
+        row = first_row + 8 * (i >> 2) + 4 * half_of + (i & 3);
+        continue;
+      }
+      if (__popc(quads) > kManyQuads) {
+        if (taken != 0) break;  // the next time
+        many = true;
+        quads = 0;
+        quad = n, item_row = row, item_bits = (uint32_t)__shfl((int)bits, n + 32 * half_of);
+        break;
+      }
+      const int q = __ffs(quads) - 1;
+      quads &= quads - 1;
+      const uint32_t b = (uint32_t)__shfl((int)bits, q + 32 * half_of);
+      if (lane >> 4 == taken) quad = q, item_row = row, item_bits = b;
+      ++taken;
+    }
+    if (taken == 0 && !many) break;
+    const uint32_t from = (uint32_t)__shfl((int)from_own, quad), to = (uint32_t)__shfl((int)to_own, quad);
+    item_bits <<= (uint32_t)__shfl((int)past, quad);
+    const uint32_t at = many ? half : lane & 15;
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (item_bits != 0) WalkRow<F32>(p, static_cast<const char*>(p.x) + (size_t)from * kElem, item_row, at, many ? 2 : 16, acc);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      if (many) {
+        acc[c] += __shfl_xor(acc[c], 32);
+      } else {
+#pragma unroll
+        for (int m = 8; m >= 1; m >>= 1) acc[c] += __shfl_xor(acc[c], m);
+      }
+    }
+    if (item_bits == 0 || at != 0) continue;
+    char* const dst = static_cast<char*>(p.out) + ((size_t)to + (size_t)(uint32_t)item_row * (uint32_t)p.hw) * kElem;
+    DispatchAct(p.act.type, [&](auto act_c) {
+      constexpr int ACT = decltype(act_c)::value;
+      const uint32_t h0 = p.act_h_words[0], h1w = p.act_h_words[1];
+      const DevActH act_h = {ACT, (uint16_t)h0, (uint16_t)(h0 >> 16), (uint16_t)h1w, (uint16_t)(h1w >> 16)};
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        if ((item_bits >> c & 1u) == 0) continue;
+        if constexpr (F32) {
+          reinterpret_cast<float*>(dst)[c] = ActivateT<ACT>(acc[c] + (p.bias ? static_cast<const float*>(p.bias)[item_row] : 0.0f), p.act);
+        } else {
+          const h1 v = (h1)(acc[c] + (p.bias ? (float)static_cast<const h1*>(p.bias)[item_row] : 0.0f));
+          reinterpret_cast<h1*>(dst)[c] = ActivateH<ACT>(h2{v, v}, act_h).x;
+        }
+      }
+    });
+  }
 }
 
 template <int WR, bool F32, bool RAGGED>
@@ -443,12 +540,10 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
   int valid = oq >= p.total_quads ? 0 : min(4, p.hw - opp);
   bool suspect = poison != poison;
   if constexpr (F32) suspect = suspect || marks[n] != 0;
-  const int looked_at = suspect ? valid : 0;
-  if (suspect) valid = 0;
+  if (suspect) valid = -valid;  // positions to be looked at
   float bias[FIN];
   [[maybe_unused]] int row_exp[FIN];
   const int table = min(rb, p.row_blocks - 1) * 32 + row_in_block;
-  auto bias_of = [&](int row) { return F32 ? static_cast<const float*>(p.bias)[row] : (float)static_cast<const h1*>(p.bias)[row]; };
 #pragma unroll
   for (int b = 0; b < FIN / 4; ++b) {
     if constexpr (F32) {
@@ -468,6 +563,7 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
   const __amdgpu_buffer_rsrc_t obuf = __builtin_amdgcn_make_buffer_rsrc(p.out, 0, (int)((uint32_t)p.batch * (uint32_t)p.M * (uint32_t)p.hw * kElem), 0x00020000);
   const uint32_t pitch = (uint32_t)p.hw * kElem;
   const uint32_t obase = ((on * (uint32_t)p.M + (uint32_t)row0) * (uint32_t)p.hw + (uint32_t)opp) * kElem;
+  uint64_t walk = 0;  // bit 4 i + c: the output of row i at position c is left to the walk
   auto finish = [&](auto act_c) {
     constexpr int ACT = decltype(act_c)::value;
     const uint32_t h0 = p.act_h_words[0], h1w = p.act_h_words[1];
@@ -475,7 +571,7 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
 #pragma unroll
     for (int i = 0; i < FIN; ++i) {
       const int rr = 8 * (i >> 2) + (i & 3);
-      const uint32_t at = row0 + rr < p.M && valid != 0 ? obase + (uint32_t)rr * pitch : kOutside;
+      const uint32_t at = row0 + rr < p.M && valid > 0 ? obase + (uint32_t)rr * pitch : kOutside;
       const int whole = (int)(valid == 4 ? at : kOutside);
       if constexpr (F32) {
         u4 o;
@@ -497,43 +593,32 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
         }
       }
     }
-    if (looked_at != 0) {
-      uint64_t walk = 0;
+    if (F32 && valid < 0) {
 #pragma unroll
       for (int i = 0; i < FIN; ++i) {
         const int rr = 8 * (i >> 2) + (i & 3);
         if (row0 + rr >= p.M) break;
-        if constexpr (F32) {
-          const float reach = reinterpret_cast<const float*>(p.row_exp + 32 * p.row_blocks)[table + rr];
-          float* dst = reinterpret_cast<float*>(static_cast<char*>(p.out) + obase + (size_t)rr * pitch);
+        const float reach = reinterpret_cast<const float*>(p.row_exp + 32 * p.row_blocks)[table + rr];
+        float* dst = reinterpret_cast<float*>(static_cast<char*>(p.out) + obase + (size_t)rr * pitch);
 #pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            if (c >= looked_at) break;
-            if (!(fabsf(fin[c][i]) >= reach)) {
-              walk |= 1ull << (4 * i + c);
-            } else {
-              dst[c] = ActivateT<ACT>(__builtin_amdgcn_ldexpf(fin[c][i], row_exp[i] + 127 - own_exp(c)) + bias[i], p.act);
-            }
+        for (int c = 0; c < 4; ++c) {
+          if (c >= -valid) break;
+          if (!(fabsf(fin[c][i]) >= reach)) {
+            walk |= 1ull << (4 * i + c);
+          } else {
+            dst[c] = ActivateT<ACT>(__builtin_amdgcn_ldexpf(fin[c][i], row_exp[i] + 127 - own_exp(c)) + bias[i], p.act);
           }
-        } else {
-          walk |= (uint64_t)((1u << looked_at) - 1u) << (4 * i);
-        }
-      }
-      const size_t xat = (size_t)on * p.K * p.hw + opp;
-#pragma unroll 1
-      for (; walk != 0; walk &= walk - 1) {
-        const int bit = __builtin_ctzll(walk), i = bit >> 2, c = bit & 3, rr = 8 * (i >> 2) + (i & 3);
-        char* dst = static_cast<char*>(p.out) + obase + (size_t)rr * pitch;
-        if constexpr (F32) {
-          reinterpret_cast<float*>(dst)[c] = ActivateT<ACT>(WalkF32(p, static_cast<const float*>(p.x) + xat + c, row0 + rr, p.bias ? bias_of(row0 + rr) : 0.0f), p.act);
-        } else {
-          const h1 v = WalkF16(p, static_cast<const h1*>(p.x) + xat + c, row0 + rr, (h1)(p.bias ? bias_of(row0 + rr) : 0.0f));
-          reinterpret_cast<h1*>(dst)[c] = ActivateH<ACT>(h2{v, v}, act_h).x;
         }
       }
     }
   };
   if (row0 < p.M) DispatchAct(p.act.type, finish);
+  if (__ballot(valid < 0) == 0) return;
+  if constexpr (!F32) {
+    for (int i = 0; i < FIN; ++i)
+      if (valid < 0 && row0 + 8 * (i >> 2) + (i & 3) < p.M) walk |= (uint64_t)((1u << -valid) - 1u) << (4 * i);
+  }
+  WalkOutputs<F32>(p, walk, FIN, rb * 32 + (32 / KH) * kh, tile_quad0);
 }
 
 template <int WR, bool F32, bool RAGGED>

@@ -645,7 +645,7 @@ int BuildFloatMfma(const pl::DecodedLayout& L, pl_sparse_conv_handle* h) {
   const uint32_t whole = static_cast<uint32_t>(L.ic) / 8u * 8u;  // channels in whole groups of eight
   // fp32: a row's weights are scaled by a power of two that takes the largest of them to [2^14, 2^15)
   std::vector<int32_t> row_exp(static_cast<size_t>(blocks) * 32, 0);
-  std::vector<double> row_sum(static_cast<size_t>(blocks) * 32, 0.0);
+  std::vector<double> row_sum(row_exp.size(), 0.0), row_scale(row_exp.size(), 1.0);
   bool exact = true;
   auto value = [](uint32_t bits) {
     float w;
@@ -660,7 +660,10 @@ int BuildFloatMfma(const pl::DecodedLayout& L, pl_sparse_conv_handle* h) {
       top[0] = std::max(top[0], std::fabs(w0));
       top[1] = std::max(top[1], std::fabs(w1));
     }
-    for (int i = 0; i < g.nrows; ++i) row_exp[g.row0 + i] = top[i] > 0.0f ? std::max(-127, std::min(126, std::ilogb(top[i]) - 14)) : 0;
+    for (int i = 0; i < g.nrows; ++i) {
+      row_exp[g.row0 + i] = top[i] > 0.0f ? std::max(-127, std::min(126, std::ilogb(top[i]) - 14)) : 0;
+      row_scale[g.row0 + i] = std::ldexp(1.0, -row_exp[g.row0 + i]);
+    }
   }
   auto put = [&](int row, uint32_t c, float weight) {
     const uint32_t t = c < whole ? c & 7u : 8u - (static_cast<uint32_t>(L.ic) - c);
@@ -671,7 +674,7 @@ int BuildFloatMfma(const pl::DecodedLayout& L, pl_sparse_conv_handle* h) {
       exact = exact && (at[0] & 0x7c00u) != 0x7c00u;
       return;
     }
-    const double w = std::ldexp(static_cast<double>(weight), -row_exp[row]);
+    const double w = weight * row_scale[row];
     at[0] = FastHalfBits(static_cast<float>(w));
     at[512] = FastHalfBits(static_cast<float>((w - HalfValue(at[0])) * pl::kFloatMfmaLow));
     // a weight far below its row's largest has lost its bits, which shows where the input of that one is zero

@@ -208,6 +208,66 @@ def test_infinities_and_nans_reach_only_the_rows_that_read_them(kind, paired, ro
     assert (np.abs(got.astype(np.float64) - np.where(ref >= 0, ref, 0.1 * ref))[rest] <= (tol * mag)[rest]).all()
 
 
+@pytest.mark.parametrize("paired", [False, True], ids=["unstructured", "semi"])
+@pytest.mark.parametrize("kind", sorted(KINDS))
+def test_every_number_of_quads_to_walk(kind, paired):
+    """Positions with a NaN from one to all of a tile, partial quads among them: rows with few quads and with many take
+    different ways.  The other positions keep the bits of a call without any."""
+    case = make_case(kind, 2, 200, 70, 9, 9, paired=paired, act="relu", sparsity=0.8)
+    kernel = forced(case, 128, paired)
+    clean = run_hip(case, kernel=kernel)
+    reads = case.dense[:, 3] != 0
+    if paired:
+        reads = np.repeat(reads.reshape(-1, 2).any(axis=1), 2)  # the walk of a pair of rows multiplies both of its weights
+    whole = case.x.copy()
+    for count in (1, 2, 5, 30, 36, 40, 80, 162):
+        case.x = whole.copy()
+        spoiled = np.zeros((2, 81), bool)
+        spoiled.reshape(-1)[np.random.RandomState(count).permutation(162)[:count]] = True
+        case.x[:, 3][spoiled.reshape(2, 9, 9)] = np.nan
+        got = run_hip(case, kernel=kernel)
+        hit = spoiled.reshape(2, 1, 9, 9) & reads[None, :, None, None]
+        assert np.isfinite(got[~hit]).all()
+        near = np.abs(got.astype(np.float64) - clean)[~hit]
+        assert near.max() <= (2e-2 if kind == "fp16" else 2e-5)
+        if kind == "fp32":
+            quads = np.repeat(np.pad(spoiled, ((0, 0), (0, 3))).reshape(2, 21, 4).any(axis=2), 4, axis=1)[:, :81].reshape(2, 1, 9, 9)
+            assert np.array_equal(got[np.broadcast_to(~quads, got.shape)], clean[np.broadcast_to(~quads, got.shape)])
+
+
+@pytest.mark.parametrize("kind", sorted(KINDS))
+def test_time_with_nans(kind):
+    """One NaN, and one in every position: at most 4 and 10 times a call without (fp32 1.7 and 5 times; every lane for itself
+    it was 8 and 31)."""
+    import torch
+
+    case = make_case(kind, 16, 512, 512, 14, 14, act="none", sparsity=0.85)
+    kernel = forced(case, 0)
+    x = torch.from_numpy(case.x).cuda()
+    one, every = x.clone(), x.clone()
+    one[3, 77, 4, 4] = float("nan")
+    every[:, 77] = float("nan")
+    out = kernel.Run(x)
+
+    def us(tensor):
+        best = 1e9
+        for _ in range(6):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(20):
+                kernel.Run(tensor, out)
+            end.record()
+            end.synchronize()
+            best = min(best, start.elapsed_time(end) * 50)
+        return best
+
+    us(x)
+    clean = us(x)
+    times = us(one), us(every)
+    print("clean %.1f us, one NaN %.1f, all %.1f" % ((clean,) + times))
+    assert times[0] <= 4 * clean and times[1] <= 10 * clean, (clean, times)
+
+
 @pytest.mark.parametrize("kind", sorted(KINDS))
 def test_tensors_off_the_16_byte_grid(kind):
     """Tensors that start one element behind a 16-byte boundary: the same bits as the aligned call, nothing written
