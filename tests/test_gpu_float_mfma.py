@@ -308,6 +308,10 @@ def test_the_rule():
         never, walk_size = algo(deep, 64, 196, float_mfma=capi.TUNE_NEVER)
         assert never == capi.ALGO_ROW_WALK and walk_size < size
         assert algo(make_case(kind, 1, 512, 512, 4, 4, sparsity=0.98), 64, 196)[0] == capi.ALGO_ROW_WALK
+    # few rows: the product takes longer than its times for more rows say
+    assert algo(make_case("fp32", 1, 1184, 62, 9, 11, sparsity=0.82), 38, 99)[0] == capi.ALGO_ROW_WALK
+    assert algo(make_case("fp32", 1, 800, 64, 33, 33, sparsity=0.88), 7, 1089)[0] == capi.ALGO_ROW_WALK
+    assert algo(make_case("fp32", 1, 1624, 40, 8, 8, sparsity=0.76), 10, 2209)[0] == capi.ALGO_CHUNK_MFMA
     # few nonzeros per row
     assert algo(make_case("fp32", 1, 96, 192, 8, 8, sparsity=0.9), 1, 3136)[0] == capi.ALGO_ROW_WALK
     assert algo(make_case("fp16", 1, 96, 200, 8, 8, sparsity=0.86), 102, 400)[0] == capi.ALGO_ROW_WALK
