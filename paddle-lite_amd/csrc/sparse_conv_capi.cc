@@ -200,7 +200,7 @@ struct pl_sparse_conv_handle {
   DevBuf wfloat;
   size_t float_row_exp = 0;      // where these begin
   int float_mfma = 1;            // 0 never, 1 by the rule, 2 whenever the shape allows
-  int float_mfma_rows = 0;  // positions per tile; 0 = chosen per problem
+  int float_mfma_rows = 0;       // rows per workgroup; 0 = chosen per problem
   // block MFMA
   int row_blocks = 0, ksteps = 0, kmask_words = 1;
   int64_t blocks_present = 0;
@@ -630,10 +630,11 @@ int BuildChunkMfma(const pl::DecodedLayout& L, pl_sparse_conv_handle* h) {
   return PL_OK;
 }
 
-// Dense tiles take 2 or 4 bytes per weight: not for handles whose nonzeros are fewer than one in 32, which no call was
-// measured with and whose lists are far smaller.
+// Dense tiles take 2 or 4 bytes per weight (2048 -> 2048 8.4 and 16.8 MB): not for layers of more weights than a call can take, and
+// not for handles whose nonzeros are fewer than one in 32, whose lists are far smaller (5 % was the least among the layers that
+// the rule below was fitted to, which leaves the few between the two to the fit).
 bool FloatMfmaWanted(const pl_sparse_conv_handle* h) {
-  return h->float_mfma != 0 && h->ic >= 8 && (h->float_mfma == 2 || h->nnz * 32 >= static_cast<int64_t>(h->oc) * h->ic);
+  return h->float_mfma != 0 && pl::FloatMfmaFits(!h->half, h->ic, h->oc, 4, 4) && (h->float_mfma == 2 || h->nnz * 32 >= static_cast<int64_t>(h->oc) * h->ic);
 }
 
 // Dense 32x16 binary16 tiles for the floating-point product (FloatMfmaParams::wtiles); none where a weight does not survive

@@ -317,3 +317,13 @@ def test_the_rule():
     assert algo(make_case("fp16", 1, 96, 200, 8, 8, sparsity=0.86), 102, 400)[0] == capi.ALGO_ROW_WALK
     with pytest.raises(capi.SparseConvError):
         make_kernel(make_case("fp32", 1, 16, 16, 4, 4), tuning=capi.tuning(float_mfma_rows=96))
+
+
+def test_no_tiles_for_layers_that_no_call_can_use_them_with():
+    """20000 x 14000 weights are beyond the kernel's 32-bit offsets: 1.1 GB of tiles otherwise."""
+    oc, ic = 14000, 20000
+    weights = pla.SparseWeights(np.zeros(0, np.float32), np.zeros(oc, np.uint32), np.zeros(0, np.int32), 0, 0, oc, ic, 49)
+    kernel = pla.SparseConvKernel(pla.SparseConvParam(weights), tuning=capi.tuning(float_mfma=capi.TUNE_ALWAYS))
+    kernel.PrepareForRun()
+    assert kernel.info()["device_bytes"] < 2 ** 27  # the lists of 14000 empty rows take 35 MB
+    assert capi.lib().pl_sparse_conv_algo_for(kernel._handle, 1, 49) == capi.ALGO_ROW_WALK
