@@ -118,6 +118,33 @@ def assert_same(case, got, want, what=""):
 ALGO_NAMES = {capi.ALGO_ROW_WALK: "row_walk", capi.ALGO_BLOCK_MFMA: "block_mfma", capi.ALGO_IMAGE_MFMA: "image_mfma", capi.ALGO_CHUNK_MFMA: "chunk_mfma"}
 
 
+def assert_dense_product(case, got, what=""):
+    """Outputs of the floating-point dense product against the same sums in 64 bits.  fp16: one rounding of a sum that is
+    fp32's, so at most the neighbouring binary16 value; fp32: what two pieces of every factor and one cut sum per 16 channels
+    leave.  Then the activation's own roundings (hard_swish: two factors that follow the sum and three roundings)."""
+    half = case.kind == capi.KIND_FP16
+    to, out = (np.float16, np.float16) if half else (np.float32, np.float64)
+    w = case.dense.astype(to).astype(np.float64)
+    bias = np.zeros(w.shape[0]) if case.bias is None else case.bias.astype(to).astype(np.float64)
+    x = case.x[:got.shape[0]].astype(np.float64).reshape(got.shape[0], w.shape[1], -1)
+    ref, mag = (np.matmul(w, x) + bias[:, None]).reshape(got.shape), (np.matmul(np.abs(w), np.abs(x)) + np.abs(bias)[:, None]).reshape(got.shape)
+    tol = 2.0 ** -10 * np.abs(ref) + 2.0 ** -19 * mag + 1e-7 if half else (6 + w.shape[1] / 16.0) * 2.0 ** -23 * mag + 1e-30
+    one = lambda t: np.asarray(t).astype(out)  # noqa: E731
+    v, act = one(ref), case.act
+    kind = act.active_type if act.has_active else capi.ACT_NONE
+    if kind == capi.ACT_RELU:
+        v = np.maximum(v, one(0))
+    elif kind == capi.ACT_RELU6:
+        v = np.minimum(np.maximum(v, one(0)), one(act.Relu_clipped_coef))
+    elif kind == capi.ACT_LEAKY_RELU:
+        v = np.where(v >= 0, v, one(v * one(act.Leaky_relu_alpha)))
+    elif kind == capi.ACT_HARD_SWISH:
+        v = one(one(v * one(1.0 / act.hard_swish_scale)) * np.minimum(np.maximum(one(v + one(act.hard_swish_offset)), one(0)), one(act.hard_swish_threshold)))
+        tol = (3 + 2 * np.abs(ref)) * tol
+    off = np.abs(got.astype(np.float64) - v.astype(np.float64))
+    assert got.shape == ref.shape and (off <= tol).all(), "%s: off by up to %g of the bound" % (what, float((off / tol).max()))
+
+
 def forced_algo(algo):
     """make_kernel's arguments for an int8 handle that runs `algo` on every call it can."""
     if algo == capi.ALGO_CHUNK_MFMA:
