@@ -437,7 +437,7 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
     }
   };
   static_assert(kSteps == 4 && STEPS >= 1, "KH positions of the quads are written per step");
-  static_assert(DEPTH % 2 == 0 && DEPTH % ADEPTH == 0, "the buffer and the weights' registers follow from the slot");
+  static_assert(DEPTH == 2 && DEPTH % ADEPTH == 0, "the buffer and the weights' registers follow from the slot");
 #pragma unroll
   for (int d = 0; d < DEPTH; ++d) {
     issue(r[d], d);
@@ -475,20 +475,8 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
   for (; chunk + DEPTH <= p.chunks; chunk += DEPTH) {
     run_chunk(std::integral_constant<int, 0>(), More(), chunk);
     run_chunk(std::integral_constant<int, 1>(), More(), chunk + 1);
-    if constexpr (DEPTH == 4) {
-      run_chunk(std::integral_constant<int, 2>(), More(), chunk + 2);
-      run_chunk(std::integral_constant<int, 3>(), More(), chunk + 3);
-    }
   }
-  if (chunk < p.chunks) {
-    run_chunk(std::integral_constant<int, 0>(), Last(), chunk);
-    if constexpr (DEPTH == 4) {
-      if (chunk + 1 < p.chunks) {
-        run_chunk(std::integral_constant<int, 1>(), Last(), chunk + 1);
-        if (chunk + 2 < p.chunks) run_chunk(std::integral_constant<int, 2>(), Last(), chunk + 2);
-      }
-    }
-  }
+  if (chunk < p.chunks) run_chunk(std::integral_constant<int, 0>(), Last(), chunk);
 
   // Lane (n, half) holds rows 8 (i / 4) + 4 half + i % 4 (i = 0 .. 15) of the row block at the four positions of quad n.
   // Wavefronts that share a row block finish FIN of the sixteen each, from what the others hand over through LDS.
