@@ -645,8 +645,10 @@ FloatMfmaPlan PlanFloatMfma(bool f32, int cus, int row_blocks, int K, int M, int
   struct Cost {
     double launch, chunk, full, full_chunk, over, over_chunk, round, round_chunk, out;
   };
-  static constexpr Cost kF32[3] = {
-      {4.5, 1.56, 2.9, 0.89, 0, 0, 4.8, 2.1, 0}, {4.6, 0.98, 2.0, 0.56, 0, 0, 5.0, 1.22, 0}, {4.5, 0.74, 1.2, 0.4, 0, 0, 4.4, 0.82, 0}};
+  // the last one for layers of at most 64 rows, of which there were hardly any among those calls (1802 of 8 - 64 rows; another
+  // 884 take 0.91 .. 1.08 of what it says, and by the one before 1.13 times as long in the middle)
+  static constexpr Cost kF32[4] = {
+      {4.5, 1.56, 2.9, 0.89, 0, 0, 4.8, 2.1, 0}, {4.6, 0.98, 2.0, 0.56, 0, 0, 5.0, 1.22, 0}, {4.5, 0.74, 1.2, 0.4, 0, 0, 4.4, 0.82, 0}, {3.9, 0.91, 1.65, 0.58, 0, 0, 5.0, 1.02, 0}};
   // maps of whole and of ragged quads
   static constexpr Cost kF16[2][3] = {
       {{3.1, 0.57, 0, 0.34, 0.57, 0.27, 0.023, 0.79, 0.4}, {3.7, 0.38, 0, 0.33, 0.43, 0.41, 0.74, 0.36, 0.31}, {3.6, 0.31, 0.8, 0.21, 0.84, 0.23, 2.1, 0.32, 0}},
@@ -655,22 +657,18 @@ FloatMfmaPlan PlanFloatMfma(bool f32, int cus, int row_blocks, int K, int M, int
   FloatMfmaPlan best{};
   for (int i = 0; i < 3; ++i) {
     const int wr = 8 >> i;
-    if (row_blocks != 0 && wr != row_blocks) continue;
+    if (row_blocks != 0 ? wr != row_blocks : wr > 2 && f32 && M <= 64) continue;
     FloatMfmaPlan p{};
     p.wr = wr;
     p.row_groups = ((M + 31) / 32 + wr - 1) / wr;
     p.workgroups = 8ll * p.row_groups * ((tiles + 7) / 8);
-    const Cost& c = f32 ? kF32[i] : kF16[hw % 4 != 0][i];
+    const Cost& c = f32 ? kF32[M <= 64 && wr == 2 ? 3 : i] : kF16[hw % 4 != 0][i];
     const int64_t used = f32 ? p.workgroups : p.row_groups * tiles;  // fp16: without those of the last eight tiles that return at once
     const double per_cu = (double)used / cus, over = per_cu > 1.0 ? per_cu - 1.0 : 0.0, rounds = (double)((used + cus - 1) / cus - 1);
     p.us = c.launch + c.chunk * chunks + (per_cu < 1.0 ? per_cu : 1.0) * (c.full + c.full_chunk * chunks) + over * (c.over + c.over_chunk * chunks) + rounds * (c.round + c.round_chunk * chunks) +
            1e-6 * c.out * positions * M * 256.0 / cus;
     if (best.wr == 0 || p.us < best.us) best = p;
   }
-  // Few rows, of which there were hardly any among the calls above: 1.18 times the fitted time (median of 371 calls that the
-  // rule took, 1.07 .. 1.3).  Without this 32 of them were more than 5 % slower than the walk, by up to 1.47 times; with it 220 are
-  // taken, none behind by more than 4 %.
-  if (f32 && M <= 64) best.us *= 1.18;
   return best;
 }
 

@@ -1027,13 +1027,19 @@ double WalkMicroseconds(const pl_sparse_conv_handle* h, int cus, double position
   const int form = h->ic <= 271 ? 0 : (h->ic <= 543 ? 1 : (h->ic <= 1087 ? 2 : 3));
   const Cost& c = h->half ? kHalf[loads][form] : kSingle[loads / 2][form];
   const double entries = static_cast<double>(h->entries), work = positions * 256.0 / cus;
-  return c.launch + 1e-3 * c.tile * h->ic + 1e-4 * c.list * entries + work * (1e-8 * (h->semi ? c.pair_entry : c.entry) * entries + 1e-7 * (c.in * h->ic + c.out * h->oc));
+  const double us = c.launch + 1e-3 * c.tile * h->ic + 1e-4 * c.list * entries + work * (1e-8 * (h->semi ? c.pair_entry : c.entry) * entries + 1e-7 * (c.in * h->ic + c.out * h->oc));
+  if (h->half || h->oc > 64) return us;
+  // fp32, few rows: a tile is mostly staging, so that whole rounds of tiles count: 0.85 of the above in the first round, 1.08
+  // times behind it (medians of 1802 calls of 8 - 64 rows)
+  return us * (positions / (128 >> form) / cus < 1.0 ? 0.85 : 1.08);
 }
 
 // Where the walk is expected to take 1.2 times (half precision: 1.15 times) as long: of the calls above 1570 of 5600 in fp32 and
-// 3070 of 4600 in half precision are taken, 18 and 13 of these are more than 10 % slower than the walk (by up to 1.29 and 1.38
-// times), 830 and 96 others would have gained more than 10 %.  Of 3100 and 2900 other calls 15 and 9 are more than 10 %
-// slower than by the walk alone; on average the rule makes fp32 1.11 and half precision 1.49 times as fast.
+// 3070 of 4600 in half precision are taken, 18 and 13 of these are more than 10 % slower than the walk, 830 and 96 others would have
+// gained more than 10 %.  On 2567 and 1980 other calls 15 and 13 are more than 5 % slower, by up to 1.28 and 1.44 times; on
+// average the rule makes fp32 1.10 and half precision 1.49 times as fast.
+// fp32 layers of at most 64 rows: 1.05 times, by their own times of both.  On 3615 calls 1575 are taken, 48 more than 5 % slower, by up
+// to 1.26 times, and they are 1.21 times as fast on average; by the times for all rows 1646, 156, 1.47 and 1.20.
 bool FloatMfmaPays(const pl_sparse_conv_handle* h, int batch, int im_size, bool aligned16) {
   const int64_t positions = static_cast<int64_t>(batch) * im_size;
   if (!h->wfloat.ptr || !pl::FloatMfmaFits(!h->half, h->ic, h->oc, im_size, positions)) return false;
@@ -1044,7 +1050,7 @@ bool FloatMfmaPays(const pl_sparse_conv_handle* h, int batch, int im_size, bool 
   const double P = static_cast<double>(positions);
   if (h->half && P * h->ic * h->oc <= 4e7) return false;
   const int cus = std::max(1, h->wg_slots_default / 2);
-  return (h->half ? 1.15 : 1.2) * pl::PlanFloatMfma(!h->half, cus, h->float_mfma_rows / 32, h->ic, h->oc, im_size, batch).us < WalkMicroseconds(h, cus, P, im_size, aligned16);
+  return (h->half ? 1.15 : (h->oc <= 64 ? 1.05 : 1.2)) * pl::PlanFloatMfma(!h->half, cus, h->float_mfma_rows / 32, h->ic, h->oc, im_size, batch).us < WalkMicroseconds(h, cus, P, im_size, aligned16);
 }
 
 // The algorithm of one call (pl_sparse_conv_algo_for reports it).
