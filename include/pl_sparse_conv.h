@@ -94,9 +94,16 @@ enum {
  * nonzeros would take a walk longer as a dense product, too (fp16 beyond
  * 4e7 weight x position products, fp32 by the expected times of both);
  * tuning.float_mfma forces or forbids it, and PL_ALGO_ROW_WALK or a walk_*
- * field keeps every call with the walks.  Positions whose inputs hold an
- * infinity or a NaN are walked there, so these reach the rows that read them
- * and no others.
+ * field keeps every call with the walks.  The three walks give the same bits;
+ * the dense product adds in another order (and in fp16 in fp32), so an image
+ * alone and the same image in a batch, or aligned and unaligned tensors, can
+ * differ in the last bits where one of the two calls runs there.  In fp32 the
+ * error of an output stays in proportion to the sum of its own row's
+ * |weight * input| (tested: (6 + ic / 16) 2^-23 of it), whatever else the
+ * input holds: outputs that the product cannot give to that, and those that
+ * an infinity or a NaN reached through a zero weight, are walked there
+ * (a call with many of them takes up to five times as long), and a layer with
+ * a weight below about 2^-28 of its row's largest stays with the walks.
  * pl_sparse_conv_algo_for() reports the choice, these dense products as
  *   PL_ALGO_CHUNK_MFMA (a report only: pl_sparse_conv_desc.algo takes the
  *                     others). */

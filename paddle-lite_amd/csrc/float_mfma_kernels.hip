@@ -23,13 +23,16 @@
 // that hold such an input are marked; the error of a row there is at most 2^-36 of the sum of its scaled weights'
 // magnitudes, so a result of 2^-13 of that sum and more is within 2^-23, and anything less is walked.
 //
-// What bounds it: the way from L2 into a CU.  A chunk of the widest form takes 96 KB in fp32 (64 KB weights, 32 KB inputs;
-// half in fp16) and 2.0 us (0.9), 47 - 53 KB per us and CU, which no depth of prefetch raised (four chunks ahead instead of two:
-// fp16 15.0 -> 16.9 us, the first chunk only arrives later); the matrix instructions of a chunk alone take 1.35 us (0.45).
+// What bounds it: no unit alone.  64 x 512 -> 512 @14x14 in fp32, per CU (counters): matrix cores busy 49 % of the time, vector ALU 24 %
+// beside the matrix instructions' issue, LDS 26 %, 36 KB per us from L2 (47 - 53 inside the loop: a chunk of the widest form is 96 KB in
+// fp32, 64 of them weights, and half in fp16, and takes 2.0 and 0.9 us, its matrix instructions alone 1.35 and 0.45).  One barrier per chunk
+// keeps the wavefronts in step, so that the vector ALU's work adds to the rest: the search for small inputs, three of
+// eleven instructions per pair of values, costs 2 - 3 % with 256 rows and 4 % with 64 (13 % there at 32 chunks).  More chunks
+// in flight gain nothing (four instead of two: fp16 15.0 -> 16.9 us, the first chunk only arrives later).
 // Hence 256 rows x 128 positions (128 x 256 has every weight fetched by two wavefronts: fp16 20.0 against 17.1 us at the
 // time), hence nothing staged twice.  us per launch, buffers rotating over 320 MB, the walk that ran before / this one:
-// fp16 64 x 512 -> 512 @14x14, 85 % zeros 29.4 / 14.5; fp16 8 x 128 -> 256 @55x55, row pairs, 70 % 20.3 / 9.4; fp32 64 x 512 -> 512
-// @14x14, 85 % 34.7 / 25.9; fp32 64 x 1024 -> 1024 @7x7, row pairs, 70 % 60.6 / 29.4.
+// fp16 64 x 512 -> 512 @14x14, 85 % zeros 29.3 / 14.5; fp16 8 x 128 -> 256 @55x55, row pairs, 70 % 20.8 / 9.6; fp32 64 x 512 -> 512
+// @14x14, 85 % 34.1 / 26.8; fp32 64 x 1024 -> 1024 @7x7, row pairs, 70 % 61.3 / 30.3.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>

@@ -1011,7 +1011,8 @@ bool ChunkMfmaPays(const pl_sparse_conv_handle* h, int call_algo, int batch, int
 // allow (128, 64, 32 and 16 positions): launch, entries of the index lists over all positions (single rows; pairs of
 // rows), inputs staged, outputs stored, filling the first tile, the entries of a single position's lists.  Fitted to
 // 4600 random calls in half precision and 5600 in fp32 (32 - 2048 channels and rows, 50 - 100 000 positions, 70 - 95 % zeros, 256
-// CUs); within -16 .. +9 % for half of them.
+// CUs), least squares with no term below zero, so that a term may be 0 where others of a form stand in for it (ragged maps in half
+// precision of up to 271 channels: what is moved value by value hides the entries); within -16 .. +9 % for half of them.
 double WalkMicroseconds(const pl_sparse_conv_handle* h, int cus, double positions, int im_size, bool aligned16) {
   struct Cost {
     double launch, entry, pair_entry, in, out, tile, list;
@@ -1938,8 +1939,9 @@ int pl_sparse_conv_dwconv3x3_pays(const pl_sparse_conv_handle* conv, const pl_dw
   // 8.3 / 8.5, 9.4 / 8.5, 10.7 / 8.8, 12.0 / 8.9; 256 -> 512 7.4 / 6.8, 8.0 / 6.9, 8.5 / 6.9, 8.9 / 7.0, 10.3 / 7.4; 128 -> 128 7.2 / 6.0 ...
   // 7.9 / 6.3.  Stride 1: 512 -> 512 7.7 / 11.0, 8.5 / 11.1, 10.1 / 11.2, 11.8 / 11.6, 14.1 / 12.1; 256 -> 512 7.7 / 9.4, 8.3 / 9.6, 9.2 / 9.7,
   // 10.2 / 9.9, 12.3 / 10.6.  The one launch does the depthwise work of 128 planes on the CU that made them, whatever the batch;
-  // the depthwise kernel spreads a small batch over the chip.  512 channels at stride 2 would be better off in two launches at
-  // up to four images there, but not where the host paces the calls: from the Python classes two take 10.0 us and one 8.3.
+  // the depthwise kernel spreads a small batch over the chip.  At stride 2 one launch is kept at any batch: from the Python
+  // classes 256 and 128 channels gain from one image on, and 512 channels (two / one, 1 / 4 / 8 images: 7.5 / 8.2, 8.3 / 8.4, 8.6 / 8.4)
+  // would gain from two launches below six images only.
   if (dw->stride == 2) return 1;
   const int64_t workgroups = static_cast<int64_t>(batch) * (conv->oc / 128);
   const int cus = std::max(1, conv->wg_slots_default / 2);
