@@ -20,7 +20,7 @@
 //
 // What a dense product would get wrong is walked nonzero by nonzero at the end: outputs that an infinity or a NaN reached
 // through a zero weight, and in fp32 outputs too small for the absolute error of the small inputs of their position.  The quads
-// that hold such an input are marked; the error of a row there is at most 2^-36 of the sum of its scaled weights'
+// that hold such an input, or whose scale went down by more than 2^64, are marked; the error of a row there is at most 2^-36 of the sum of its scaled weights'
 // magnitudes, so a result of 2^-13 of that sum and more is within 2^-23, and anything less is walked.
 //
 // What bounds it: no unit alone.  64 x 512 -> 512 @14x14 in fp32, per CU (counters): matrix cores busy 49 % of the time, vector ALU 24 %
@@ -128,8 +128,8 @@ __device__ __forceinline__ void WalkRow(const FloatMfmaParams& p, const char* x,
 
 // LDS: two buffers of operand cells, or what the wavefronts of a row block hand to each other at the end; behind either
 // (a wavefront may still look at a flag when another has begun to hand over), for fp32, the positions' maxima, the two
-// flags and the marks of the quads.
-constexpr int kF32Tables = (4 * kQuads + 4 + kQuads) * 4;
+// flags, the marks of the quads and the positions' first scales.
+constexpr int kF32Tables = (4 * kQuads + 4 + kQuads + 4 * kQuads) * 4;
 constexpr int LdsTables(int wr, bool f32) {
   const int cells = 2 * (f32 ? 2 : 1) * kGroups * 4 * kQuads * 16, trade = 8 * (64 - 8 * wr) * 64 * 4;
   return cells > trade ? cells : trade;
@@ -343,6 +343,7 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
   uint32_t* const colmax = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(xt) + LdsTables(WR, F32));
   uint32_t* const flags = colmax + 4 * QT;
   uint32_t* const marks = flags + 4;
+  uint32_t* const first_exp = marks + QT;  // of the positions' first scales
   const uint32_t* const own_max = colmax + 4 * n;  // of the positions whose sums the lane holds
   [[maybe_unused]] uint32_t own_exps = 0;  // a byte each: four registers do not fit beside the sums
   auto own_exp = [&](int c) { return (int)(own_exps >> (8 * c) & 0xffu); };
@@ -363,16 +364,15 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       const uint32_t m = colmax[4 * j + c], om = own_max[c];
-      if (__uint_as_float(m) * scale[c] >= kPeak) {
-        scale[c] = __uint_as_float((uint32_t)(scale_exp(m) + 11) << 23);
-        marks[j] = 1;  // sums may lose bits, too
-      }
+      if (__uint_as_float(m) * scale[c] >= kPeak) scale[c] = __uint_as_float((uint32_t)(scale_exp(m) + 11) << 23);
       const int before = own_exp(c);
       if (__uint_as_float(om) * __uint_as_float((uint32_t)before << 23) >= 0x1p15f) {
         const int e = scale_exp(om);
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[c][i] = __builtin_amdgcn_ldexpf(acc[c][i], e - before), rest[c][i] = __builtin_amdgcn_ldexpf(rest[c][i], e - before);
         own_exps = (own_exps & ~(0xffu << (8 * c))) | (uint32_t)e << (8 * c);
+        // unmarked, every term of a sum was 2^-48 or more when it was added: 2^64 less is far from the subnormal numbers
+        if ((int)first_exp[4 * n + c] - e > 64) marks[n] = 1;
       }
     }
 #pragma unroll
@@ -463,6 +463,7 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
       scale[c] = __uint_as_float((uint32_t)(scale_exp(colmax[4 * j + c]) + 11) << 23);
       own_exps |= (uint32_t)scale_exp(own_max[c]) << (8 * c);
     }
+    if (tid < 4 * QT) first_exp[tid] = (uint32_t)scale_exp(colmax[tid]);
   }
 #pragma unroll
   for (int c = 0; c < 4; ++c) commit(r[0], 0, c);
@@ -530,11 +531,22 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
   const int opp = 4 * (int)(oq - on * (uint32_t)p.qpi);
   int valid = oq >= p.total_quads ? 0 : min(4, p.hw - opp);
   bool suspect = poison != poison;
-  if constexpr (F32) suspect = suspect || marks[n] != 0;
+  const int table = min(rb, p.row_blocks - 1) * 32 + row_in_block;
+  if constexpr (F32) {
+    if (marks[n] != 0) {  // most marked quads hold no output that is too small
+#pragma unroll
+      for (int b = 0; b < FIN / 4; ++b) {
+        const v4f reach = *reinterpret_cast<const v4f*>(p.row_exp + 32 * p.row_blocks + table + 8 * b);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int c = 0; c < 4; ++c) suspect = suspect || fabsf(fin[c][4 * b + i]) < reach[i];
+      }
+    }
+  }
   if (suspect) valid = -valid;  // positions to be looked at
   float bias[FIN];
   [[maybe_unused]] int row_exp[FIN];
-  const int table = min(rb, p.row_blocks - 1) * 32 + row_in_block;
 #pragma unroll
   for (int b = 0; b < FIN / 4; ++b) {
     if constexpr (F32) {

@@ -235,6 +235,21 @@ def test_every_number_of_quads_to_walk(kind, paired):
             assert np.array_equal(got[np.broadcast_to(~quads, got.shape)], clean[np.broadcast_to(~quads, got.shape)])
 
 
+def microseconds(kernel, x, out):
+    import torch
+
+    best = 1e9
+    for _ in range(7):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        for _ in range(20):
+            kernel.Run(x, out)
+        end.record()
+        end.synchronize()
+        best = min(best, start.elapsed_time(end) * 50)
+    return best
+
+
 @pytest.mark.parametrize("kind", sorted(KINDS))
 def test_time_with_nans(kind):
     """One NaN, and one in every position: at most 4 and 10 times a call without (fp32 1.7 and 5 times; every lane for itself
@@ -248,24 +263,30 @@ def test_time_with_nans(kind):
     one[3, 77, 4, 4] = float("nan")
     every[:, 77] = float("nan")
     out = kernel.Run(x)
-
-    def us(tensor):
-        best = 1e9
-        for _ in range(6):
-            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            start.record()
-            for _ in range(20):
-                kernel.Run(tensor, out)
-            end.record()
-            end.synchronize()
-            best = min(best, start.elapsed_time(end) * 50)
-        return best
-
-    us(x)
-    clean = us(x)
-    times = us(one), us(every)
+    microseconds(kernel, x, out)
+    clean = microseconds(kernel, x, out)
+    times = microseconds(kernel, one, out), microseconds(kernel, every, out)
     print("clean %.1f us, one NaN %.1f, all %.1f" % ((clean,) + times))
     assert times[0] <= 4 * clean and times[1] <= 10 * clean, (clean, times)
+
+
+def test_time_with_channels_of_different_size():
+    """New scales in every position, but no output that is too small: at most 1.25 times a call without (1.03; with every marked
+    quad looked at output by output it was 1.4 and 1.5)."""
+    import torch
+
+    case = make_case("fp32", 64, 512, 512, 14, 14, act="none", sparsity=0.85)
+    kernel = forced(case, 256)
+    x = torch.from_numpy(case.x).cuda()
+    gains = torch.from_numpy(np.exp(1.5 * np.random.RandomState(0).standard_normal((1, 512, 1, 1))).astype(np.float32)).cuda()
+    late = x.clone()
+    late[:, :64] *= 1e-3
+    out = kernel.Run(x)
+    microseconds(kernel, x, out)
+    clean = microseconds(kernel, x, out)
+    times = microseconds(kernel, x * gains, out), microseconds(kernel, late, out)
+    print("clean %.1f us, channel gains %.1f, first chunk small %.1f" % ((clean,) + times))
+    assert max(times) <= 1.25 * clean, (clean, times)
 
 
 @pytest.mark.parametrize("kind", sorted(KINDS))
