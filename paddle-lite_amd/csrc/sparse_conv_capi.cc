@@ -646,7 +646,7 @@ int BuildFloatMfma(const pl::DecodedLayout& L, pl_sparse_conv_handle* h) {
   const uint32_t whole = static_cast<uint32_t>(L.ic) / 8u * 8u;  // channels in whole groups of eight
   // fp32: a row's weights are scaled by a power of two that takes the largest of them to [2^14, 2^15)
   std::vector<int32_t> row_exp(static_cast<size_t>(blocks) * 32, 0);
-  std::vector<double> row_sum(row_exp.size(), 0.0), row_scale(row_exp.size(), 1.0);
+  std::vector<float> row_sum(row_exp.size(), 0.0f), row_scale(row_exp.size(), 1.0f);
   bool exact = true;
   auto value = [](uint32_t bits) {
     float w;
@@ -663,7 +663,7 @@ int BuildFloatMfma(const pl::DecodedLayout& L, pl_sparse_conv_handle* h) {
     }
     for (int i = 0; i < g.nrows; ++i) {
       row_exp[g.row0 + i] = top[i] > 0.0f ? std::max(-127, std::min(126, std::ilogb(top[i]) - 14)) : 0;
-      row_scale[g.row0 + i] = std::ldexp(1.0, -row_exp[g.row0 + i]);
+      row_scale[g.row0 + i] = std::ldexp(1.0f, -row_exp[g.row0 + i]);
     }
   }
   auto put = [&](int row, uint32_t c, float weight) {
@@ -675,11 +675,12 @@ int BuildFloatMfma(const pl::DecodedLayout& L, pl_sparse_conv_handle* h) {
       exact = exact && (at[0] & 0x7c00u) != 0x7c00u;
       return;
     }
-    const double w = weight * row_scale[row];
-    at[0] = FastHalfBits(static_cast<float>(w));
-    at[512] = FastHalfBits(static_cast<float>((w - HalfValue(at[0])) * pl::kFloatMfmaLow));
+    const float w = weight * row_scale[row];  // a power of two: exact, or so small that it is found out below
+    at[0] = FastHalfBits(w);
+    const float rest = (w - HalfValue(at[0])) * pl::kFloatMfmaLow;
+    at[512] = FastHalfBits(rest);
     // a weight far below its row's largest has lost its bits, which shows where the input of that one is zero
-    exact = exact && std::fabs(w - HalfValue(at[0]) - HalfValue(at[512]) / static_cast<double>(pl::kFloatMfmaLow)) <= std::fabs(w) * 0x1p-22;
+    exact = exact && std::fabs(rest - HalfValue(at[512])) <= std::fabs(w) * (0x1p-22f * pl::kFloatMfmaLow) && (w != 0.0f || weight == 0.0f);
     row_sum[row] += std::fabs(w);
   };
   for (const pl::RowGroup& g : L.groups) {
@@ -693,7 +694,7 @@ int BuildFloatMfma(const pl::DecodedLayout& L, pl_sparse_conv_handle* h) {
   h->float_row_exp = tile_values * sizeof(uint16_t);
   if (!h->half) {
     std::vector<float> reach(row_sum.size());
-    for (size_t i = 0; i < reach.size(); ++i) reach[i] = static_cast<float>(row_sum[i] * pl::kFloatMfmaSmall);
+    for (size_t i = 0; i < reach.size(); ++i) reach[i] = row_sum[i] * pl::kFloatMfmaSmall;
     std::memcpy(&tiles[tile_values], row_exp.data(), row_exp.size() * sizeof(int32_t));
     std::memcpy(&tiles[tile_values + 2 * row_exp.size()], reach.data(), reach.size() * sizeof(float));
   }
