@@ -139,6 +139,20 @@ def test_fp32_large_inputs_stay_with_the_rows_that_read_them(size, channels, row
 
 
 @pytest.mark.parametrize("rows", ROWS)
+@pytest.mark.parametrize("channels", [[5], [329], list(range(3, 330, 9))], ids=["first", "last", "many"])
+def test_fp16_large_inputs_stay_with_the_rows_that_read_them(channels, rows):
+    """The largest numbers beside ordinary and subnormal ones: a product with a zero weight takes no bits from the others."""
+    case = make_case("fp16", 2, 330, 70, 9, 7, act="none", sparsity=0.9)
+    case.bias = None
+    case.x[1] *= np.float16(1e-4)
+    case.x[:, channels] = np.where(case.x[:, channels] > 0, np.float16(-65504), np.float16(65504))
+    reads = (case.dense[:, channels] != 0).any(axis=1)
+    case.dense[reads] *= np.float32(1e-3)  # sums of these stay below the largest number
+    assert not reads.all() and reads.any()
+    check(case, "none", run_hip(case, kernel=forced(case, rows)))
+
+
+@pytest.mark.parametrize("rows", ROWS)
 @pytest.mark.parametrize("binades", [24, 60, 230])
 def test_fp32_inputs_of_all_magnitudes(binades, rows):
     """Exponents spread evenly, so every position holds values that its largest one leaves few bits."""
