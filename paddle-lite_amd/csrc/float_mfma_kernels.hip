@@ -529,7 +529,7 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
   const uint32_t oq = tile_quad0 + (uint32_t)n;
   const uint32_t on = oq / (uint32_t)p.qpi;
   const int opp = 4 * (int)(oq - on * (uint32_t)p.qpi);
-  int valid = oq >= p.total_quads ? 0 : min(4, p.hw - opp);
+  const int valid = oq >= p.total_quads ? 0 : min(4, p.hw - opp);
   bool suspect = poison != poison;
   const int table = min(rb, p.row_blocks - 1) * 32 + row_in_block;
   if constexpr (F32) {
@@ -544,7 +544,7 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
       }
     }
   }
-  if (suspect) valid = -valid;  // positions to be looked at
+  suspect = suspect && valid != 0;
   float bias[FIN];
   [[maybe_unused]] int row_exp[FIN];
 #pragma unroll
@@ -566,7 +566,6 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
   const __amdgpu_buffer_rsrc_t obuf = __builtin_amdgcn_make_buffer_rsrc(p.out, 0, (int)((uint32_t)p.batch * (uint32_t)p.M * (uint32_t)p.hw * kElem), 0x00020000);
   const uint32_t pitch = (uint32_t)p.hw * kElem;
   const uint32_t obase = ((on * (uint32_t)p.M + (uint32_t)row0) * (uint32_t)p.hw + (uint32_t)opp) * kElem;
-  uint64_t walk = 0;  // bit 4 i + c: the output of row i at position c is left to the walk
   auto finish = [&](auto act_c) {
     constexpr int ACT = decltype(act_c)::value;
     const uint32_t h0 = p.act_h_words[0], h1w = p.act_h_words[1];
@@ -574,7 +573,7 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
 #pragma unroll
     for (int i = 0; i < FIN; ++i) {
       const int rr = 8 * (i >> 2) + (i & 3);
-      const uint32_t at = row0 + rr < p.M && valid > 0 ? obase + (uint32_t)rr * pitch : kOutside;
+      const uint32_t at = row0 + rr < p.M && valid != 0 ? obase + (uint32_t)rr * pitch : kOutside;
       const int whole = (int)(valid == 4 ? at : kOutside);
       if constexpr (F32) {
         u4 o;
@@ -596,31 +595,23 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
         }
       }
     }
-    if (F32 && valid < 0) {
-#pragma unroll
-      for (int i = 0; i < FIN; ++i) {
-        const int rr = 8 * (i >> 2) + (i & 3);
-        if (row0 + rr >= p.M) break;
-        const float reach = reinterpret_cast<const float*>(p.row_exp + 32 * p.row_blocks)[table + rr];
-        float* dst = reinterpret_cast<float*>(static_cast<char*>(p.out) + obase + (size_t)rr * pitch);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          if (c >= -valid) break;
-          if (!(fabsf(fin[c][i]) >= reach)) {
-            walk |= 1ull << (4 * i + c);
-          } else {
-            dst[c] = ActivateT<ACT>(__builtin_amdgcn_ldexpf(fin[c][i], row_exp[i] + 127 - own_exp(c)) + bias[i], p.act);
-          }
-        }
-      }
-    }
   };
   if (row0 < p.M) DispatchAct(p.act.type, finish);
-  if (__ballot(valid < 0) == 0) return;
-  if constexpr (!F32) {
-    for (int i = 0; i < FIN; ++i)
-      if (valid < 0 && row0 + 8 * (i >> 2) + (i & 3) < p.M) walk |= (uint64_t)((1u << -valid) - 1u) << (4 * i);
+  if (__ballot(suspect) == 0) return;
+  uint64_t walk = 0;  // bit 4 i + c: the output of row i at position c is walked
+  if (suspect) {
+#pragma unroll
+    for (int i = 0; i < FIN; ++i) {
+      const int rr = 8 * (i >> 2) + (i & 3);
+      if (row0 + rr >= p.M) break;
+      const float reach = F32 ? reinterpret_cast<const float*>(p.row_exp + 32 * p.row_blocks)[table + rr] : 0.0f;
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (c < valid && (!F32 || !(fabsf(fin[c][i]) >= reach))) walk |= 1ull << (4 * i + c);
+    }
   }
+  // other lanes write these outputs again: what this wavefront has stored must have arrived
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   WalkOutputs<F32>(p, walk, FIN, rb * 32 + (32 / KH) * kh, tile_quad0);
 }
 
