@@ -146,10 +146,9 @@ __device__ __forceinline__ void WalkOutputs(const FloatMfmaParams& p, uint64_t w
   constexpr uint32_t kElem = F32 ? 4u : 2u;
   constexpr int kManyQuads = 8;
   const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), n = lane & 31, half = lane >> 5;  // not held in a register meanwhile
-  // four positions inside the map
   const uint32_t image = (first_quad + (uint32_t)n) / (uint32_t)p.qpi;
   const int position = 4 * (int)(first_quad + (uint32_t)n - image * (uint32_t)p.qpi);
-  const uint32_t inside = (uint32_t)min(position, p.hw - 4), past = (uint32_t)position - inside;
+  const uint32_t inside = (uint32_t)min(position, p.hw - 4);
   const uint32_t from_own = image * (uint32_t)p.K * (uint32_t)p.hw + inside, to_own = image * (uint32_t)p.M * (uint32_t)p.hw + inside;
   int next = 0, row = 0, half_of = 0;
   uint32_t quads = 0, bits = 0;  // of the present row: quads left; the lane's own four bits
@@ -183,7 +182,6 @@ __device__ __forceinline__ void WalkOutputs(const FloatMfmaParams& p, uint64_t w
     }
     if (taken == 0 && !many) break;
     const uint32_t from = (uint32_t)__shfl((int)from_own, quad), to = (uint32_t)__shfl((int)to_own, quad);
-    item_bits <<= (uint32_t)__shfl((int)past, quad);
     const uint32_t at = many ? half : lane & 15;
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     if (item_bits != 0) WalkRow<F32>(p, static_cast<const char*>(p.x) + (size_t)from * kElem, item_row, at, many ? 2 : 16, acc);
@@ -236,14 +234,14 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
   if (tile >= last_tile) return;
 
   // the thread's part of a chunk: UC channels of quad j; a partial quad (the end of an image whose size is not a multiple
-  // of 4) is read from the last four positions of its channel row and shifted, threads behind the tensor's last quad
+  // of 4) is the last four positions of its channel row, the first of which belong to the quad before; threads behind the tensor's last quad
   // repeat that one
   const int part = (tid / QT) & 1, j = tid & (QT - 1), kg = tid / (QT * 2);
   const uint32_t tile_quad0 = (uint32_t)tile * (uint32_t)QT;
   const uint32_t quad = min(tile_quad0 + (uint32_t)j, p.total_quads - 1u);
   const uint32_t img = quad / (uint32_t)p.qpi;
   const int pp = 4 * (int)(quad - img * (uint32_t)p.qpi);
-  const int first = min(pp, p.hw - 4), shift = pp - first;
+  const int first = min(pp, p.hw - 4);
   constexpr uint32_t kElem = F32 ? 4u : 2u;
   const uint32_t vbase = img * (uint32_t)p.K * (uint32_t)p.hw + (uint32_t)first;
   Quad<F32> r[DEPTH][UC];
@@ -261,19 +259,6 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
         rd[i] = __builtin_amdgcn_raw_buffer_load_b128(xbuf, (int)voff, i * pitch_in, 0);
       } else {
         rd[i] = __builtin_amdgcn_raw_buffer_load_b64(xbuf, (int)voff, i * pitch_in, 0);
-      }
-    }
-  };
-  auto align_quad = [&](Quad<F32> (&rd)[UC]) {
-    if (!RAGGED) return;
-#pragma unroll
-    for (int i = 0; i < UC; ++i) {
-      if constexpr (F32) {
-        if (shift & 1) rd[i] = u4{rd[i].y, rd[i].z, rd[i].w, rd[i].w};
-        if (shift & 2) rd[i] = u4{rd[i].z, rd[i].w, rd[i].w, rd[i].w};
-      } else {
-        const uint64_t v = (((uint64_t)rd[i].y << 32) | rd[i].x) >> (16 * shift);
-        rd[i] = u2{(uint32_t)v, (uint32_t)(v >> 32)};
       }
     }
   };
@@ -382,7 +367,7 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
 
   // One chunk: kSteps x 4 cells.  Behind the multiplies of a step the next chunk's cells of one position go to the
   // other buffer; then the loads of the chunk DEPTH behind that one are issued into the registers this frees.
-  constexpr int PF = F32 || (RAGGED && WR == 8) ? 2 : 3;  // operand cells in flight; the ragged form of 128 registers has room for two
+  constexpr int PF = F32 ? 2 : 3;  // operand cells in flight
   auto run_chunk = [&](auto slot_c, auto last_c, int chunk) {
     constexpr bool LAST = decltype(last_c)::value;  // no chunk is left to load
     constexpr int S = decltype(slot_c)::value, NEXT = (S + 1) % DEPTH, AS = S % ADEPTH;
@@ -397,7 +382,6 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int ks = 0; ks < STEPS; ++ks) {
-      if (ks == 0) align_quad(r[NEXT]);
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         const int v = 4 * ks + c;
@@ -451,11 +435,9 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
       __builtin_amdgcn_sched_barrier(0);
     }
   }
-  if constexpr (!F32) align_quad(r[0]);
   if constexpr (F32) {
     for (int i = tid; i < kF32Tables / 4; i += kThreads) colmax[i] = 0;  // and the flags and marks
     __syncthreads();
-    align_quad(r[0]);
     collect(r[0]);
     __syncthreads();
 #pragma unroll
@@ -528,8 +510,9 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
   const int row_in_block = 4 * half + (32 / KH) * kh, row0 = rb * 32 + row_in_block;
   const uint32_t oq = tile_quad0 + (uint32_t)n;
   const uint32_t on = oq / (uint32_t)p.qpi;
-  const int opp = 4 * (int)(oq - on * (uint32_t)p.qpi);
-  const int valid = oq >= p.total_quads ? 0 : min(4, p.hw - opp);
+  const int opp = 4 * (int)(oq - on * (uint32_t)p.qpi), ofirst = min(opp, p.hw - 4);
+  const bool present = oq < p.total_quads;
+  const int own = RAGGED ? opp - ofirst : 0;  // the first position of the quad that is not one of the quad before
   bool suspect = poison != poison;
   const int table = min(rb, p.row_blocks - 1) * 32 + row_in_block;
   if constexpr (F32) {
@@ -544,7 +527,7 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
       }
     }
   }
-  suspect = suspect && valid != 0;
+  suspect = suspect && present;
   float bias[FIN];
   [[maybe_unused]] int row_exp[FIN];
 #pragma unroll
@@ -565,7 +548,7 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
   constexpr uint32_t kOutside = kFloatMfmaOutside;
   const __amdgpu_buffer_rsrc_t obuf = __builtin_amdgcn_make_buffer_rsrc(p.out, 0, (int)((uint32_t)p.batch * (uint32_t)p.M * (uint32_t)p.hw * kElem), 0x00020000);
   const uint32_t pitch = (uint32_t)p.hw * kElem;
-  const uint32_t obase = ((on * (uint32_t)p.M + (uint32_t)row0) * (uint32_t)p.hw + (uint32_t)opp) * kElem;
+  const uint32_t obase = ((on * (uint32_t)p.M + (uint32_t)row0) * (uint32_t)p.hw + (uint32_t)ofirst) * kElem;
   auto finish = [&](auto act_c) {
     constexpr int ACT = decltype(act_c)::value;
     const uint32_t h0 = p.act_h_words[0], h1w = p.act_h_words[1];
@@ -573,8 +556,8 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
 #pragma unroll
     for (int i = 0; i < FIN; ++i) {
       const int rr = 8 * (i >> 2) + (i & 3);
-      const uint32_t at = row0 + rr < p.M && valid != 0 ? obase + (uint32_t)rr * pitch : kOutside;
-      const int whole = (int)(valid == 4 ? at : kOutside);
+      const uint32_t at = row0 + rr < p.M && present ? obase + (uint32_t)rr * pitch : kOutside;
+      const int whole = (int)(own == 0 ? at : kOutside);
       if constexpr (F32) {
         u4 o;
 #pragma unroll
@@ -582,7 +565,7 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
         __builtin_amdgcn_raw_buffer_store_b128(o, obuf, whole, 0, 0);
         if constexpr (RAGGED) {
 #pragma unroll
-          for (int c = 0; c < 3; ++c) __builtin_amdgcn_raw_buffer_store_b32(o[c], obuf, (int)(valid != 4 && c < valid ? at + 4 * c : kOutside), 0, 0);
+          for (int c = 1; c < 4; ++c) __builtin_amdgcn_raw_buffer_store_b32(o[c], obuf, (int)(own != 0 && c >= own ? at + 4 * c : kOutside), 0, 0);
         }
       } else {
         const h2 o0 = ActivateH<ACT>(__builtin_convertvector((v2f{fin[0][i] + bias[i], fin[1][i] + bias[i]}), h2), act_h);
@@ -591,7 +574,7 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
         __builtin_amdgcn_raw_buffer_store_b64(o, obuf, whole, 0, 0);
         if constexpr (RAGGED) {
 #pragma unroll
-          for (int c = 0; c < 3; ++c) __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(o[c >> 1] >> (16 * (c & 1))), obuf, (int)(valid != 4 && c < valid ? at + 2 * c : kOutside), 0, 0);
+          for (int c = 1; c < 4; ++c) __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(o[c >> 1] >> (16 * (c & 1))), obuf, (int)(own != 0 && c >= own ? at + 2 * c : kOutside), 0, 0);
         }
       }
     }
@@ -607,7 +590,7 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
       const float reach = F32 ? reinterpret_cast<const float*>(p.row_exp + 32 * p.row_blocks)[table + rr] : 0.0f;
 #pragma unroll
       for (int c = 0; c < 4; ++c)
-        if (c < valid && (!F32 || !(fabsf(fin[c][i]) >= reach))) walk |= 1ull << (4 * i + c);
+        if (c >= own && (!F32 || !(fabsf(fin[c][i]) >= reach))) walk |= 1ull << (4 * i + c);
     }
   }
   // other lanes write these outputs again: what this wavefront has stored must have arrived
