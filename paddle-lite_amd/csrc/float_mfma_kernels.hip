@@ -303,12 +303,12 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
   // the wavefront's row block (past the last one: the last one again, not stored) and window of 32 quads
   const int rb = rg * WR + wave % WR, kh = wave / WR;
   const int n = lane & 31, half = lane >> 5;
-  char* const wblock = const_cast<char*>(static_cast<const char*>(p.wtiles)) + (size_t)min(rb, p.row_blocks - 1) * p.padded_ksteps * (1024 * PIECES);
+  const __amdgpu_buffer_rsrc_t wbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(static_cast<const char*>(p.wtiles)) + (size_t)min(rb, p.row_blocks - 1) * p.padded_ksteps * (1024 * PIECES), 0,
+                                                                        (int)(FloatMfmaWeightTile(p.chunks, 0, PIECES, 0) + FloatMfmaWeightTail(PIECES)), 0x00020000);
   h8 a[ADEPTH][STEPS][PIECES];
   auto load_weights = [&](h8 (&dst)[PIECES], int chunk, int ks) {
-    const __amdgpu_buffer_rsrc_t wbuf = __builtin_amdgcn_make_buffer_rsrc(wblock, 0, (int)FloatMfmaWeightBytes(chunk, p.chunks, PIECES), 0x00020000);
 #pragma unroll
-    for (int q = 0; q < PIECES; ++q) dst[q] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(wbuf, lane * 16, (int)FloatMfmaWeightTile(chunk, p.chunks, kh * STEPS + ks, PIECES, q), 0));
+    for (int q = 0; q < PIECES; ++q) dst[q] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(wbuf, lane * 16, (int)FloatMfmaWeightTile(chunk, kh * STEPS + ks, PIECES, q), 0));
   };
   const uint4* const operand = xt + (2 * STEPS * kh + half) * (4 * QT) + n;
   // fp32: the products of two high pieces, and those of a high and a low one, which would otherwise each round the sum

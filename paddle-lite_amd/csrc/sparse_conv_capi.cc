@@ -641,7 +641,7 @@ bool FloatMfmaWanted(const pl_sparse_conv_handle* h) {
 // in them.
 int BuildFloatMfma(const pl::DecodedLayout& L, pl_sparse_conv_handle* h) {
   const int blocks = CeilDiv(L.oc, 32), kss = pl::FloatMfmaPaddedSteps(L.ic), pieces = h->half ? 1 : 2;
-  const size_t tile_values = static_cast<size_t>(blocks) * kss * pieces * 512;
+  const size_t tile_values = static_cast<size_t>(blocks) * kss * pieces * 512 + pl::FloatMfmaWeightTail(pieces) / 2;
   std::vector<uint16_t> tiles(tile_values + (h->half ? 0 : static_cast<size_t>(blocks) * 128), 0);
   const uint32_t whole = static_cast<uint32_t>(L.ic) / 8u * 8u;  // channels in whole groups of eight
   // fp32: a row's weights are scaled by a power of two that takes the largest of them to [2^14, 2^15)

@@ -288,14 +288,10 @@ struct FloatMfmaParams {
 // A lane's offset that lies outside every buffer of that kernel: nothing is fetched or stored there.
 constexpr uint32_t kFloatMfmaOutside = 0x80000000u;
 
-// Size of the buffer of a row block's weight tiles as the loads of a chunk see it, and where the tile of a piece of a step of
-// that chunk begins.  A chunk behind the last one, which the loop asks for ahead of time, sees an empty buffer from its
-// start on: a scalar offset at or past the size would leave it to the bounds check to compare with the size less that
-// offset.  (Both in scalar registers: a lane's offset outside the buffer costs the form of 128 registers one too many.)
-constexpr uint32_t FloatMfmaWeightBytes(int chunk, int chunks, int pieces) { return chunk < chunks ? (uint32_t)(chunks * (kFloatMfmaChunk / 16) * pieces) * 1024u : 0u; }
-constexpr uint32_t FloatMfmaWeightTile(int chunk, int chunks, int step, int pieces, int piece) {
-  return chunk < chunks ? (uint32_t)((chunk * (kFloatMfmaChunk / 16) + step) * pieces + piece) * 1024u : 0u;
-}
+// Where the weight tile of a piece of a step of a chunk begins in a row block.  The loop asks for a chunk behind the last one, too, where
+// their number is even: that is the next block's first, and behind the last block's tiles there are FloatMfmaWeightTail bytes.
+constexpr uint32_t FloatMfmaWeightTile(int chunk, int step, int pieces, int piece) { return (uint32_t)((chunk * (kFloatMfmaChunk / 16) + step) * pieces + piece) * 1024u; }
+constexpr uint32_t FloatMfmaWeightTail(int pieces) { return FloatMfmaWeightTile(1, 0, pieces, 0); }
 
 // How a call is divided (workgroups of wr x 32 rows x 128 positions) and what it is expected to take.
 struct FloatMfmaPlan {

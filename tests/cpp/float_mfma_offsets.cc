@@ -1,36 +1,42 @@
 // The loads that the floating-point dense product makes of its weight tiles, by the loop of its kernel: every chunk's weights
-// are asked for while the chunk before is multiplied, so those behind the last chunk too where the loop does not know yet that it
-// ends.  A lane's bytes must lie inside its row block's tiles, or outside a buffer whose size is not below the scalar offset.
-// Prints "ok", or what lies elsewhere.
+// are asked for while the chunk before is multiplied, and with an even number of chunks those behind the last one, too.  All of
+// them must lie inside the tiles as prepare lays them out, and a row block's own must be read once each.
+// Prints "ok", or what does not.
 #include <cstdio>
+#include <vector>
 
 #include "sparse_conv_kernels.h"
 
 int main() {
   for (int pieces = 1; pieces <= 2; ++pieces)
-    for (int chunks = 1; chunks <= 9; ++chunks) {
-      const uint32_t steps = pl::kFloatMfmaChunk / 16, size = (uint32_t)chunks * steps * (uint32_t)pieces * 1024u;
-      uint64_t seen = 0;
-      // chunk 0 before the loop, in the loop the one behind a chunk; pairs of chunks, then one
-      const int last_asked = chunks % 2 == 0 ? chunks : chunks - 1;
-      for (int chunk = 0; chunk <= last_asked; ++chunk)
-        for (int step = 0; step < (int)steps; ++step)
-          for (int piece = 0; piece < pieces; ++piece)
-            for (uint32_t lane = 0; lane < 64; ++lane) {
-              const uint64_t own = 16 * lane, tile = pl::FloatMfmaWeightTile(chunk, chunks, step, pieces, piece), bytes = pl::FloatMfmaWeightBytes(chunk, chunks, pieces);
-              const bool inside = bytes == size && own + tile + 16 <= bytes;
-              const bool outside = tile <= bytes && own >= bytes - tile;
-              if (inside == outside || inside != (chunk < chunks)) {
-                std::printf("chunk %d of %d, step %d, piece %d, lane %u: %llu + %llu of %u\n", chunk, chunks, step, piece, lane, (unsigned long long)own, (unsigned long long)tile, size);
-                return 1;
+    for (int blocks = 1; blocks <= 3; ++blocks)
+      for (int chunks = 1; chunks <= 9; ++chunks) {
+        const int steps = pl::kFloatMfmaChunk / 16;
+        const uint64_t block_bytes = static_cast<uint64_t>(chunks) * steps * pieces * 1024, all = blocks * block_bytes + pl::FloatMfmaWeightTail(pieces);
+        std::vector<int> asked = {0};  // before the loop; in it pairs of chunks, behind it the last one, which asks for nothing
+        for (int chunk = 0; chunk + 2 <= chunks; chunk += 2) {
+          asked.push_back(chunk + 1);
+          asked.push_back(chunk + 2);
+        }
+        for (int block = 0; block < blocks; ++block) {
+          std::vector<int> reads(block_bytes / 1024, 0);
+          for (int c : asked)
+            for (int step = 0; step < steps; ++step)
+              for (int piece = 0; piece < pieces; ++piece) {
+                const uint64_t tile = pl::FloatMfmaWeightTile(c, step, pieces, piece);
+                if (tile < block_bytes) ++reads[tile / 1024];
+                if (block * block_bytes + tile + 64 * 16 > all) {
+                  std::printf("chunk %d of %d, block %d of %d, step %d, piece %d: %llu of %llu\n", c, chunks, block, blocks, step, piece, (unsigned long long)(block * block_bytes + tile), (unsigned long long)all);
+                  return 1;
+                }
               }
-              if (inside) seen += 16;
+          for (int r : reads)
+            if (r != 1) {
+              std::printf("%d chunks: a tile is read %d times\n", chunks, r);
+              return 1;
             }
-      if (seen != size) {
-        std::printf("%llu of %u bytes read\n", (unsigned long long)seen, size);
-        return 1;
+        }
       }
-    }
   std::printf("ok\n");
   return 0;
 }

@@ -5,7 +5,7 @@ import subprocess
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-def test_weight_loads_stay_inside_their_row_block_or_outside_the_buffer(tmp_path):
+def test_weight_loads_stay_inside_the_tiles(tmp_path):
     exe = str(tmp_path / "offsets")
     subprocess.check_call(["g++", "-std=c++17", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-isystem", "/opt/rocm/include", "-I", os.path.join(ROOT, "paddle-lite_amd", "csrc"), "-I", os.path.join(ROOT, "include"),
                            os.path.join(ROOT, "tests", "cpp", "float_mfma_offsets.cc"), "-o", exe])
