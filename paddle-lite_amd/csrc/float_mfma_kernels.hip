@@ -31,8 +31,8 @@
 // in flight gain nothing (four instead of two: fp16 15.0 -> 16.9 us, the first chunk only arrives later).
 // Hence 256 rows x 128 positions (128 x 256 has every weight fetched by two wavefronts: fp16 20.0 against 17.1 us at the
 // time), hence nothing staged twice.  us per launch, buffers rotating over 320 MB, the walk that ran before / this one:
-// fp16 64 x 512 -> 512 @14x14, 85 % zeros 29.3 / 14.5; fp16 8 x 128 -> 256 @55x55, row pairs, 70 % 20.8 / 9.6; fp32 64 x 512 -> 512
-// @14x14, 85 % 34.1 / 26.8; fp32 64 x 1024 -> 1024 @7x7, row pairs, 70 % 61.3 / 30.3.
+// fp16 64 x 512 -> 512 @14x14, 85 % zeros 29.1 / 14.4; fp16 8 x 128 -> 256 @55x55, row pairs, 70 % 20.7 / 9.5; fp32 64 x 512 -> 512
+// @14x14, 85 % 33.0 / 25.4; fp32 64 x 1024 -> 1024 @7x7, row pairs, 70 % 61.0 / 28.8.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
