@@ -285,7 +285,7 @@ def test_time_with_nans(kind):
 
 
 def test_time_with_channels_of_different_size():
-    """New scales in every position, but no output that is too small: at most 1.25 times a call without (1.03; with every marked
+    """New scales in every position, but no output that is too small: at most 1.3 times a call without (1.03; with every marked
     quad looked at output by output it was 1.4 and 1.5)."""
     import torch
 
@@ -300,7 +300,7 @@ def test_time_with_channels_of_different_size():
     clean = microseconds(kernel, x, out)
     times = microseconds(kernel, x * gains, out), microseconds(kernel, late, out)
     print("clean %.1f us, channel gains %.1f, first chunk small %.1f" % ((clean,) + times))
-    assert max(times) <= 1.25 * clean, (clean, times)
+    assert max(times) <= 1.3 * clean, (clean, times)
 
 
 @pytest.mark.parametrize("kind", sorted(KINDS))
