@@ -288,6 +288,246 @@ __device__ __forceinline__ void ChunkBody(const ChunkMfmaParams& p, uint4* xt) {
   });
 }
 
+// The form for many channels: 256 rows x eight blocks of 16 positions, 256 channels a chunk, twelve wavefronts.  Eight multiply, two row
+// tiles with all positions each, so that nobody else loads their weights and an operand cell feeds two matrix instructions.  Four bring in
+// the activations: a thread loads 16 positions of eight channels with 16-byte loads (a block behind the last whole one of a channel row is
+// the row's last 16 positions; what the block before it holds as well is computed twice and stored once), two chunks ahead of
+// the one that it turns into cells.
+//
+// Why twelve: wavefronts issue in order and loads return in order, so a wavefront that does everything waits for its activations, which
+// come from memory, before it gets at weights that L2 has had for long, and a full queue of loads holds its matrix instructions
+// back.  2048 -> 2048 @14x14 x 16 with eight wavefronts that do both, in this shape, 21.6 us, in 128 x 256 21.1; this 19.1; the kernel above
+// 21.9 (128 x 256 in this form 22.6).  A 16-byte load takes a CU 7.0 ns, as long as an 8-byte one and less than two 4-byte
+// ones (3.7), so bytes come in twice as fast as dword by dword.
+// What bounds it: the matrix instructions, 0.85 of 1.2 us a chunk, beside 0.9 us in which the 96 KB of a chunk come in; around the
+// chunks 9.9 us (launch, first chunk, 2.5 us of stores).  Without any loads 17.3 us, without the multiplies 17.0.
+constexpr int kSplitQuads = 32;                   // position quads of a tile
+constexpr int kSplitRowTiles = 16;
+constexpr int kSplitCells = 16 * 4 * kSplitQuads;  // 16-byte cells of a chunk: (channel group of 16, position of the quad, quad)
+constexpr int kSplitSteps = 4;                    // 64-channel steps of a chunk
+constexpr int kSplitThreads = 768;
+
+// Where a quad's cells lie: the quads of a block turned round by the block's number over four and the channel group's parity, so that lanes
+// that write the same quad of neighbouring blocks (64 bytes apart) and of two groups use all banks.
+__device__ __forceinline__ int QuadSlot(int group, int block, int quad) { return 4 * block + ((quad + (block >> 2) + 2 * (group & 1)) & 3); }
+
+template <int OUT>
+__device__ __forceinline__ void ChunkSplitBody(const ChunkMfmaParams& p, uint4* xt) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // each XCD owns a contiguous range of tiles, the row groups of one tile follow each other there
+  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+  const int first_tile = (xcd * p.tiles) >> 3, last_tile = ((xcd + 1) * p.tiles) >> 3;
+  const int tile = first_tile + slot / p.row_groups, rg = slot % p.row_groups;
+  if (tile >= last_tile) return;
+
+  const uint32_t blocks_per_image = (uint32_t)p.qpi >> 2, tile_block0 = (uint32_t)tile * ((uint32_t)p.tile_quads >> 2);
+  const uint32_t total_blocks = p.total_quads >> 2;
+  float* const table = reinterpret_cast<float*>(xt + 2 * kSplitCells);
+  if (wave >= 8) {
+    // the thread's part of a chunk: eight channels (half of group kg) of block j; threads behind the tile's or the tensor's last
+    // block repeat that one
+    const int j = tid & 7, kg = (tid >> 4) & 15, half = (tid >> 3) & 1;
+    const uint32_t block = min(tile_block0 + (uint32_t)min(j, (p.tile_quads >> 2) - 1), total_blocks - 1u);
+    const uint32_t img = block / blocks_per_image;
+    const int first = min(16 * (int)(block - img * blocks_per_image), p.hw - 16);
+    const uint32_t vbase = img * (uint32_t)p.K * (uint32_t)p.hw + (uint32_t)first;
+    u4 r[2][8];
+    const __amdgpu_buffer_rsrc_t xbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(p.x), 0, (int)((uint32_t)p.batch * (uint32_t)p.K * (uint32_t)p.hw), 0x00020000);
+    auto issue = [&](u4 (&rd)[8], int chunk) {
+      // The last group of a channel count that is no multiple of 16 holds the last 16 channels.  Groups behind it meet weights of zero:
+      // they lie outside the buffer, so nothing is fetched for them, and no condition around the loads makes the wait for older ones wait for these too.
+      const int k = chunk * (64 * kSplitSteps) + 16 * kg;
+      const uint32_t voff = k < p.K ? vbase + (uint32_t)((min(k, p.K - 16) + 8 * half) * p.hw) : 0x80000000u;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) rd[i] = __builtin_amdgcn_raw_buffer_load_b128(xbuf, (int)voff, i * p.hw, 0);
+    };
+    // two stages of byte permutes: pairs of channels, then the eight bytes of each position
+    char* const cells = reinterpret_cast<char*>(xt + kg * (4 * kSplitQuads)) + 8 * half;
+    auto commit = [&](u4 (&rd)[8], int buf) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        char* const dst = cells + (buf * kSplitCells + QuadSlot(kg, j, t)) * 16;
+#pragma unroll
+        for (int pos = 0; pos < 4; pos += 2) {
+          uint32_t pair[4];
+#pragma unroll
+          for (int m = 0; m < 4; ++m) pair[m] = __builtin_amdgcn_perm(rd[2 * m + 1][t], rd[2 * m][t], pos ? 0x07030602u : 0x05010400u);
+#pragma unroll
+          for (int c = 0; c < 2; ++c) {
+            const uint32_t sel = c ? 0x07060302u : 0x05040100u;
+            *reinterpret_cast<uint2*>(dst + (pos + c) * (kSplitQuads * 16)) = make_uint2(__builtin_amdgcn_perm(pair[1], pair[0], sel), __builtin_amdgcn_perm(pair[3], pair[2], sel));
+          }
+        }
+      }
+    };
+    issue(r[0], 0);
+    __builtin_amdgcn_sched_barrier(0);
+    issue(r[1], 1);
+    __builtin_amdgcn_sched_barrier(0);
+    commit(r[0], 0);
+    issue(r[0], 2);
+    __syncthreads();
+    int chunk = 0;
+    for (; chunk + 2 < p.chunks; chunk += 2) {
+      commit(r[1], 1);
+      issue(r[1], chunk + 3);
+      __syncthreads();
+      commit(r[0], 0);
+      issue(r[0], chunk + 4);
+      __syncthreads();
+    }
+    if (chunk + 1 < p.chunks) {
+      commit(r[1], 1);
+      __syncthreads();
+    }
+    __syncthreads();
+    return;
+  }
+
+  // the wavefront's row tiles (past the last one: the last one again, not stored)
+  const int rt = rg * kSplitRowTiles + 2 * wave;
+  const int n = lane & 15, kq = lane >> 4;
+  const v4i* const wt0 = static_cast<const v4i*>(p.wtiles) + (size_t)min(rt, p.row_tiles - 1) * p.padded_ksteps * 64 + lane;
+  const v4i* const wt1 = static_cast<const v4i*>(p.wtiles) + (size_t)min(rt + 1, p.row_tiles - 1) * p.padded_ksteps * 64 + lane;
+  v4i a[kSplitSteps][2];
+  auto load_weights = [&](int chunk, int ks) {
+    a[ks][0] = wt0[(chunk * kSplitSteps + ks) * 64];
+    a[ks][1] = wt1[(chunk * kSplitSteps + ks) * 64];
+  };
+  const uint4* const operand0 = xt + kq * (4 * kSplitQuads) + QuadSlot(kq, n >> 2, n & 3);
+  const uint4* const operand1 = xt + kq * (4 * kSplitQuads) + QuadSlot(kq, 4 + (n >> 2), n & 3);
+  v4i acc[2][2][4];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int w = 0; w < 2; ++w)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[t][w][c] = v4i{0, 0, 0, 0};
+
+  // One chunk: eight (step, window) pairs of eight multiplies, operand cells read PF cells ahead.  The weights of a step are requested for
+  // the next chunk as soon as the step has used their registers.
+  constexpr int PF = 4;
+  auto run_chunk = [&](auto last_c, int chunk) {
+    constexpr bool LAST = decltype(last_c)::value;
+    const uint4* const in0 = operand0 + (chunk & 1) * kSplitCells;
+    const uint4* const in1 = operand1 + (chunk & 1) * kSplitCells;
+    uint4 b[PF + 1];
+    auto read = [&](int v) { b[v % (PF + 1)] = (v >> 2 & 1 ? in1 : in0)[(v >> 3) * (16 * kSplitQuads) + (v & 3) * kSplitQuads]; };
+#pragma unroll
+    for (int d = 0; d < PF; ++d) read(d);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int ks = u >> 1, w = u & 1;
+      if (LAST && w == 0 && 64 * (kSplitSteps * chunk + ks) >= p.K) break;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int v = 4 * u + c;
+        if (v + PF < 32) read(v + PF);
+        __builtin_amdgcn_sched_barrier(0);  // the reads stay ahead of the multiply
+        const uint4 q = b[v % (PF + 1)];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) acc[t][w][c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[ks][t], v4i{(int)q.x, (int)q.y, (int)q.z, (int)q.w}, acc[t][w][c], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (w == 1 && !LAST) load_weights(chunk + 1, ks);
+    }
+    __syncthreads();
+  };
+#pragma unroll
+  for (int ks = 0; ks < kSplitSteps; ++ks) load_weights(0, ks);
+  // scales and biases of the workgroup's rows wait in LDS (the arrays are padded to a multiple of 32 rows)
+  if (OUT != kOutAcc32) {
+    const int row = min(rg * (16 * kSplitRowTiles) + (tid & 255), 16 * p.row_tiles - 1);
+    table[tid] = tid < 256 ? p.scale[row] : p.bias[row];
+  }
+  __syncthreads();
+  int chunk = 0;
+  for (; chunk + 1 < p.chunks; ++chunk) run_chunk(std::false_type(), chunk);
+  run_chunk(std::true_type(), chunk);
+
+  // epilogue: lane (n, kq) holds rows 4 kq .. 4 kq + 3 of the row tiles at the four positions of quad n of the windows
+  const int row0 = rt * 16 + 4 * kq;
+  if (row0 >= p.M) return;
+  constexpr uint32_t kElem = OUT == kOutI8 ? 1u : 4u;
+  const bool stream = OUT != kOutI8 && (p.hw & 15) == 0;  // as in ChunkBody
+  DispatchAct(OUT == kOutAcc32 ? 0 : epilogue::LeakyAsMax(p.act), [&](auto act_c) {
+    constexpr int ACT = decltype(act_c)::value;
+    char* dst[2];
+    int own[2];  // the quad's first position that no block before it holds
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      const int bj = 4 * w + (n >> 2);
+      const uint32_t ob = tile_block0 + (uint32_t)bj, on = ob / blocks_per_image;
+      const int from = 16 * (int)(ob - on * blocks_per_image), opp = min(from, p.hw - 16) + 4 * (n & 3);
+      own[w] = bj >= (p.tile_quads >> 2) || ob >= total_blocks ? 4 : min(4, max(0, from - opp));
+      dst[w] = static_cast<char*>(p.out) + (((size_t)on * p.M + row0) * p.hw + opp) * kElem;
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      float s[4], o[4];
+      if (OUT != kOutAcc32) {
+        const float* const at = table + 32 * wave + 16 * t + 4 * kq;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[i] = at[i], o[i] = at[256 + i];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const bool row = row0 + 16 * t + i < p.M;
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+          if (row) {
+            u4 v;
+            if (OUT == kOutAcc32) {
+              v = u4{(uint32_t)acc[t][w][0][i], (uint32_t)acc[t][w][1][i], (uint32_t)acc[t][w][2][i], (uint32_t)acc[t][w][3][i]};
+            } else {
+              float f[4];
+#pragma unroll
+              for (int c = 0; c < 4; ++c) f[c] = __builtin_fmaf((float)acc[t][w][c][i], s[i], o[i]);
+              if (OUT == kOutI8) {
+                v = u4{TruncPackI8x4(ActQuantF<ACT>(f[0], p.act), ActQuantF<ACT>(f[1], p.act), ActQuantF<ACT>(f[2], p.act), ActQuantF<ACT>(f[3], p.act)), 0u, 0u, 0u};
+              } else {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) f[c] = ActivateT<ACT>(f[c], p.act);
+                v = u4{__float_as_uint(f[0]), __float_as_uint(f[1]), __float_as_uint(f[2]), __float_as_uint(f[3])};
+              }
+            }
+            if (own[w] == 0) {
+              if (OUT == kOutI8) {
+                *reinterpret_cast<uint32_t*>(dst[w]) = v.x;
+              } else if (stream) {
+                __builtin_nontemporal_store(v, reinterpret_cast<u4*>(dst[w]));
+              } else {
+                *reinterpret_cast<u4*>(dst[w]) = v;
+              }
+            } else {
+#pragma unroll
+              for (int c = 1; c < 4; ++c) {
+                if (c >= own[w]) {
+                  if (OUT == kOutI8) {
+                    reinterpret_cast<int8_t*>(dst[w])[c] = static_cast<int8_t>(v.x >> (8 * c));
+                  } else {
+                    reinterpret_cast<uint32_t*>(dst[w])[c] = v[c];
+                  }
+                }
+              }
+            }
+          }
+          dst[w] += (size_t)p.hw * kElem;
+        }
+      }
+#pragma unroll
+      for (int w = 0; w < 2; ++w) dst[w] += (size_t)(12 * p.hw) * kElem;
+    }
+  });
+}
+
+template <int OUT>
+__global__ void __launch_bounds__(kSplitThreads, 3) ChunkSplitKernel(PL_HEAD_PARAMS, const ChunkMfmaParams block) {
+  const ChunkMfmaParams p = WithHead(block, PL_HEAD_ARGS);
+  extern __shared__ uint4 xt[];
+  ChunkSplitBody<OUT>(p, xt);
+}
+
 template <int NW, int OUT>
 __global__ void __launch_bounds__(512, 2) ChunkMfmaKernel(PL_HEAD_PARAMS, const ChunkMfmaParams block) {
   const ChunkMfmaParams p = WithHead(block, PL_HEAD_ARGS);
@@ -296,8 +536,9 @@ __global__ void __launch_bounds__(512, 2) ChunkMfmaKernel(PL_HEAD_PARAMS, const 
 }
 
 template <int OUT>
-hipError_t Launch(int nw, const ChunkMfmaParams& p, dim3 grid, hipStream_t s) {
+hipError_t Launch(int nw, bool split, const ChunkMfmaParams& p, dim3 grid, hipStream_t s) {
   const dim3 block(512);
+  if (split) return LaunchWithHead(ChunkSplitKernel<OUT>, grid, dim3(kSplitThreads), (size_t)2 * kSplitCells * 16 + 2048, s, p);
   const size_t lds = 2 * kBufCells * 16;
   if (nw == 4) return LaunchWithHead(ChunkMfmaKernel<4, OUT>, grid, block, lds, s, p);
   if (nw == 2) return LaunchWithHead(ChunkMfmaKernel<2, OUT>, grid, block, lds, s, p);
@@ -347,6 +588,20 @@ ChunkMfmaPlan PlanChunkMfma(int out_kind, int cus, int tile_positions, int K, in
   return best;
 }
 
+// Position tiles of the form with twelve wavefronts.
+static int64_t SplitTiles(int hw, int batch) { return ((int64_t)batch * ((hw + 15) / 16) + kSplitQuads / 4 - 1) / (kSplitQuads / 4); }
+
+// Where that form is expected to be ahead of the tile width `plan` chose: a CU holds one of its workgroups, which takes about 4.4 us and
+// 1.1 us per chunk of 256 channels.  us, the width chosen / this: 2048 -> 2048 @14x14 x 16 22.0 / 19.0, 1024 -> 512 @17x17 x 32 18.4 /
+// 14.5, 900 -> 384 @13x13 x 60 15.5 / 13.0, 1024 -> 2048 @14x14 x 64 51.4 / 46.1; not taken: 192 -> 384 @17x17 x 64 (304 workgroups) 12 / 15,
+// 1024 -> 1024 @14x14 x 16 (half the CUs) 11.3 / 12.6, 1500 -> 700 @10x10 x 20 9.5 / 13.6.
+static bool SplitPays(int cus, const ChunkMfmaPlan& plan, int K, int M, int hw, int batch) {
+  if (hw < 16) return false;
+  const int64_t groups = ((M + 15) / 16 + kSplitRowTiles - 1) / kSplitRowTiles, workgroups = 8 * groups * ((SplitTiles(hw, batch) + 7) / 8);
+  const int64_t chunks = (K + 64 * kSplitSteps - 1) / (64 * kSplitSteps);
+  return (workgroups + cus - 1) / cus * (440 + 110 * chunks) < (plan.workgroups + cus - 1) / cus * (300 + 135 * plan.chunks);
+}
+
 hipError_t LaunchChunkMfma(int out_kind, int cus, int tile_positions, const ChunkMfmaParams& p, hipStream_t stream) {
   if (p.batch <= 0 || p.M <= 0) return hipSuccess;
   if (!ChunkMfmaFits(p.K, p.hw)) return hipErrorInvalidValue;
@@ -365,16 +620,26 @@ hipError_t LaunchChunkMfma(int out_kind, int cus, int tile_positions, const Chun
   q.tiles = plan.tiles;
   q.chunks = plan.chunks;
   const int nw = plan.nw;
-  const int64_t wgs = plan.workgroups;
+  int64_t wgs = plan.workgroups;
+  const bool split = (tile_positions == 0 || tile_positions == 256) && SplitPays(cus, plan, p.K, p.M, p.hw, p.batch);
+  if (split) {
+    q.qpi = 4 * ((p.hw + 15) / 16);
+    q.total_quads = (uint32_t)p.batch * (uint32_t)q.qpi;
+    q.tile_quads = kSplitQuads;
+    q.tiles = (int)SplitTiles(p.hw, p.batch);
+    q.row_groups = (q.row_tiles + kSplitRowTiles - 1) / kSplitRowTiles;
+    q.chunks = ((p.K + 63) / 64 + kSplitSteps - 1) / kSplitSteps;
+    wgs = 8ll * q.row_groups * ((q.tiles + 7) / 8);
+  }
   if (wgs > (1ll << 30)) return hipErrorInvalidValue;
   const dim3 grid((uint32_t)wgs);
   switch (out_kind) {
     case kOutF32:
-      return Launch<kOutF32>(nw, q, grid, stream);
+      return Launch<kOutF32>(nw, split, q, grid, stream);
     case kOutI8:
-      return Launch<kOutI8>(nw, q, grid, stream);
+      return Launch<kOutI8>(nw, split, q, grid, stream);
     case kOutAcc32:
-      return Launch<kOutAcc32>(nw, q, grid, stream);
+      return Launch<kOutAcc32>(nw, split, q, grid, stream);
     default:
       return hipErrorInvalidValue;
   }

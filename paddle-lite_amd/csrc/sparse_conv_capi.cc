@@ -954,8 +954,16 @@ bool ChunkMfmaBeatsBlock(const pl_sparse_conv_handle* h, int batch, int im_size,
     return ic % 16 != 0 && tiles * 4 <= cus;
   }
   const auto workgroups = [&] { return pl::PlanChunkMfma(OutKind(h->kind), cus, h->chunk_positions, ic, oc, im_size, batch).workgroups; };
+  // the block kernel skips blocks of 32 x 32 zeros and this one does not
+  const int64_t blocks = static_cast<int64_t>(h->row_blocks) * h->ksteps;
+  const bool dense = h->blocks_present * 4 >= blocks * 3;
+  // More than 256 channels and 96 rows on maps of 49 positions and more, where many positions are taken 256 rows at a time: of 128 calls with
+  // up to 11 tiles per CU that the rules below leave to the block kernel none is slower, 0.72 of its time at the median (1344 -> 896 @28x28 x 10
+  // 24.7 / 16.9, 422 -> 1004 @25x25 x 30 42.6 / 25.9, 480 -> 128 @18x18 x 82 9.8 / 8.0).  Up to 96 rows 0.9 - 1.25; up to 256 channels 1.0 - 1.76 from
+  // one tile per CU on (256 -> 64 @40x40 x 60 8.3 / 14.6), 0.62 - 0.97 below that.
+  if (ic > 256 && oc > 96 && im_size >= 49 && dense && (ic > 512 || tiles <= 6 * cus)) return true;
   if (ic <= 512) {
-    if (!ragged) return tiles * 2 <= cus;  // 512 -> 128 @28x28 5.6 / 7.3 at 8 images, 10.8 / 8.2 at 32; 256 -> 64 @56x56 4.4 / 4.6 at 1
+    if (!ragged) return tiles * 10 <= 9 * cus;  // 256 -> 64 @56x56 4.4 / 4.6 at 1 image, 512 -> 96 @28x28 10.8 / 8.2 at 32
     if (tiles <= cus) return true;         // 192 -> 384 @17x17 5.7 / 8.4 at 8 images
     // Up to two tiles per CU: 384 channels 0.76 - 1.02.  Others while rows, not positions, make the tiles many: 192 -> 384
     // @17x17 x 64 0.84, 192 -> 96 @35x35 x 32 1.12; with one-byte output in one round of workgroups: 192 -> 384 @13x13 x 128 (384
@@ -964,9 +972,6 @@ bool ChunkMfmaBeatsBlock(const pl_sparse_conv_handle* h, int batch, int im_size,
     if (ic > 256 && ic <= 384) return true;
     return one_byte ? oc > 16 && workgroups() <= cus : positions <= 150 * cus;
   }
-  // the block kernel skips blocks of 32 x 32 zeros and this one does not
-  const int64_t blocks = static_cast<int64_t>(h->row_blocks) * h->ksteps;
-  const bool dense = h->blocks_present * 4 >= blocks * 3;
   // Up to 1024 channels the block kernel holds all of them in LDS, beyond 640 (512 with one-byte output, which stages its
   // stores there) with room for one workgroup per CU: 768 -> 768 @12x12 7.8 / 19.8 at 16 images, 1024 -> 256 @28x28 x 64 39.1 /
   // 42.6; 1024 -> 1024 @20x20 x 64 (1600 tiles) with 5 / 30 % of the blocks present 1.34 / 1.2 of its time.

@@ -61,6 +61,24 @@ def test_large_calls(shape, kind):
     check(shape, kind, AP("relu"), False, shape[1])
 
 
+# The form of the widest tile with wavefronts of its own for the activations (256 rows x eight blocks of 16 positions, 256 channels a chunk):
+# channels around a group of 16, a step of 64 and a chunk, each number of chunks that its loops can end with, rows around a tile of 16, a
+# wavefront's 32 and a workgroup's 256, maps of one block, of blocks that overlap by 1 - 15 positions and of more than a tile, tiles that cross
+# images and are not full.
+SPLIT = [(1, 129, 1, 4, 4), (2, 191, 31, 1, 17), (3, 256, 33, 5, 5), (1, 257, 255, 1, 31), (5, 272, 256, 4, 8), (2, 320, 257, 3, 11), (9, 500, 15, 7, 7), (1, 513, 48, 14, 14),
+         (3, 768, 17, 9, 15), (2, 770, 300, 1, 18), (1, 1000, 129, 10, 10), (7, 1025, 40, 4, 4), (1, 1281, 20, 12, 13), (2, 1601, 520, 6, 6)]
+
+
+@pytest.mark.parametrize("kind", sorted(KINDS))
+@pytest.mark.parametrize("shape", SPLIT, ids=lambda s: "x".join(map(str, s)))
+def test_wavefronts_of_their_own_for_the_activations(shape, kind):
+    print("CASE chunk split", shape, kind, file=sys.stderr, flush=True)
+    case = chunk_case(shape, kind, [AP("relu"), AP("leaky_relu", Leaky_relu_alpha=0.1)][shape[1] % 2], shape[2] % 2 == 0, shape[1])
+    want = run_oracle(case, oracle_pack(case))
+    for width in (0, 256):
+        assert_same(case, run_hip(case, kernel=chunk_kernel(case, width)), want, "chunk split %s %s, width %d" % (shape, kind, width))
+
+
 # maps with every remainder modulo four, a last tile that is not full and rows that end inside a tile
 @pytest.mark.parametrize("kind", sorted(KINDS))
 @pytest.mark.parametrize("shape", [(3, 130, 37, 6, 6), (2, 200, 20, 5, 9), (3, 520, 129, 3, 6), (2, 77, 30, 3, 13)], ids=lambda s: "x".join(map(str, s)))
