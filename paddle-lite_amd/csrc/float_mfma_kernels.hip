@@ -135,6 +135,28 @@ constexpr int LdsTables(int wr, bool f32) {
   return cells > trade ? cells : trade;
 }
 
+// Bias, activation and store of the positions of a quad that `bits` names; the quad's first output in row 0 of its image lies `to` elements into out.
+template <bool F32>
+__device__ __forceinline__ void StoreWalked(const FloatMfmaParams& p, const float (&acc)[4], uint32_t bits, int row, uint32_t to) {
+  constexpr uint32_t kElem = F32 ? 4u : 2u;
+  char* const dst = static_cast<char*>(p.out) + ((size_t)to + (size_t)(uint32_t)row * (uint32_t)p.hw) * kElem;
+  DispatchAct(p.act.type, [&](auto act_c) {
+    constexpr int ACT = decltype(act_c)::value;
+    const uint32_t h0 = p.act_h_words[0], h1w = p.act_h_words[1];
+    const DevActH act_h = {ACT, (uint16_t)h0, (uint16_t)(h0 >> 16), (uint16_t)h1w, (uint16_t)(h1w >> 16)};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      if ((bits >> c & 1u) == 0) continue;
+      if constexpr (F32) {
+        reinterpret_cast<float*>(dst)[c] = ActivateT<ACT>(acc[c] + (p.bias ? static_cast<const float*>(p.bias)[row] : 0.0f), p.act);
+      } else {
+        const h1 v = (h1)(acc[c] + (p.bias ? (float)static_cast<const h1*>(p.bias)[row] : 0.0f));
+        reinterpret_cast<h1*>(dst)[c] = ActivateH<ACT>(h2{v, v}, act_h).x;
+      }
+    }
+  });
+}
+
 // The outputs that the product could not give, by the whole wavefront: lane (n, half) brings the bits of its own (4 i + c: row
 // first_row + 8 (i / 4) + 4 half + i % 4, position c of quad n).  A row with many such quads
 // is walked by two lanes per quad, others by sixteen lanes per row and quad, four of these at a time.
@@ -195,22 +217,53 @@ __device__ __forceinline__ void WalkOutputs(const FloatMfmaParams& p, uint64_t w
       }
     }
     if (item_bits == 0 || at != 0) continue;
-    char* const dst = static_cast<char*>(p.out) + ((size_t)to + (size_t)(uint32_t)item_row * (uint32_t)p.hw) * kElem;
-    DispatchAct(p.act.type, [&](auto act_c) {
-      constexpr int ACT = decltype(act_c)::value;
-      const uint32_t h0 = p.act_h_words[0], h1w = p.act_h_words[1];
-      const DevActH act_h = {ACT, (uint16_t)h0, (uint16_t)(h0 >> 16), (uint16_t)h1w, (uint16_t)(h1w >> 16)};
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        if ((item_bits >> c & 1u) == 0) continue;
-        if constexpr (F32) {
-          reinterpret_cast<float*>(dst)[c] = ActivateT<ACT>(acc[c] + (p.bias ? static_cast<const float*>(p.bias)[item_row] : 0.0f), p.act);
-        } else {
-          const h1 v = (h1)(acc[c] + (p.bias ? (float)static_cast<const h1*>(p.bias)[item_row] : 0.0f));
-          reinterpret_cast<h1*>(dst)[c] = ActivateH<ACT>(h2{v, v}, act_h).x;
-        }
+    StoreWalked<F32>(p, acc, item_bits, item_row, to);
+  }
+}
+
+// The same for wavefronts whose lanes hold 16 quads (n) in four parts (kq): the lane's row i is row first_row + 16 (i / 4) + 4 kq + i % 4.  Where more
+// than half of the lanes have such outputs in their rows i each walks its own, else sixteen lanes walk one row for one quad, four of these at a
+// time.  fp32 16 x 512 -> 512 @14x14 as above, a wavefront walking four times as many rows as there: one NaN 33, one in every
+// position 99 us (rows one after the other by four lanes per quad 139), without any 12.
+__device__ __forceinline__ void WalkOutputs16(const FloatMfmaParams& p, uint32_t walk, int first_row, uint32_t first_quad) {
+  const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), n = lane & 15;
+  const uint32_t image = (first_quad + (uint32_t)n) / (uint32_t)p.qpi;
+  const int position = 4 * (int)(first_quad + (uint32_t)n - image * (uint32_t)p.qpi);
+  const uint32_t inside = (uint32_t)min(position, p.hw - 4);
+  const uint32_t from_own = image * (uint32_t)p.K * (uint32_t)p.hw + inside, to_own = image * (uint32_t)p.M * (uint32_t)p.hw + inside;
+#pragma unroll 1
+  for (int i = 0; i < 8; ++i) {
+    const uint32_t bits = (walk >> (4 * i)) & 15u;
+    uint64_t left = __ballot(bits != 0);
+    const int row0 = first_row + 16 * (i >> 2) + (i & 3);
+    if (__popcll(left) > 32) {
+      float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+      if (bits != 0) {
+        WalkRow<true>(p, static_cast<const char*>(p.x) + (size_t)from_own * 4, row0 + 4 * (lane >> 4), 0, 1, acc);
+        StoreWalked<true>(p, acc, bits, row0 + 4 * (lane >> 4), to_own);
       }
-    });
+      continue;
+    }
+    while (left != 0) {
+      int from = lane;
+      bool taken = false;
+#pragma unroll
+      for (int item = 0; item < 4; ++item) {
+        if (left == 0) break;
+        const int of = __ffsll((unsigned long long)left) - 1;
+        left &= left - 1;
+        if (lane >> 4 == item) from = of, taken = true;
+      }
+      const uint32_t item_bits = (uint32_t)__shfl((int)bits, from), at = (uint32_t)__shfl((int)from_own, from), to = (uint32_t)__shfl((int)to_own, from);
+      const int row = row0 + 4 * (from >> 4);
+      float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+      if (taken) WalkRow<true>(p, static_cast<const char*>(p.x) + (size_t)at * 4, row, n, 16, acc);
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int m = 8; m >= 1; m >>= 1) acc[c] += __shfl_xor(acc[c], m);
+      if (taken && n == 0) StoreWalked<true>(p, acc, item_bits, row, to);
+    }
   }
 }
 
@@ -305,10 +358,14 @@ __device__ __forceinline__ void FloatMfmaBody(const FloatMfmaParams& p, uint4* x
   const int n = lane & 31, half = lane >> 5;
   const __amdgpu_buffer_rsrc_t wbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(static_cast<const char*>(p.wtiles)) + (size_t)min(rb, p.row_blocks - 1) * p.padded_ksteps * (1024 * PIECES), 0,
                                                                         (int)(FloatMfmaWeightTile(p.chunks, 0, PIECES, 0) + FloatMfmaWeightTail(PIECES)), 0x00020000);
+  const int weight_lane = (n >> 4) * (PIECES * 1024) + 256 * half + 16 * (n & 15);
   h8 a[ADEPTH][STEPS][PIECES];
   auto load_weights = [&](h8 (&dst)[PIECES], int chunk, int ks) {
 #pragma unroll
-    for (int q = 0; q < PIECES; ++q) dst[q] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(wbuf, lane * 16, (int)FloatMfmaWeightTile(chunk, kh * STEPS + ks, PIECES, q), 0));
+    for (int q = 0; q < PIECES; ++q) {
+      const int step = kh * STEPS + ks;  // of 16 channels: half of two tiles
+      dst[q] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(wbuf, weight_lane, (int)FloatMfmaWeightTile(chunk, step & ~1, PIECES, q) + 512 * (step & 1), 0));
+    }
   };
   const uint4* const operand = xt + (2 * STEPS * kh + half) * (4 * QT) + n;
   // fp32: the products of two high pieces, and those of a high and a low one, which would otherwise each round the sum
@@ -605,11 +662,360 @@ __global__ void __launch_bounds__(kThreads, F32 ? 2 : 4) FloatMfmaKernel(PL_HEAD
   FloatMfmaBody<WR, F32, RAGGED>(p, xt);
 }
 
+// fp32 with wavefronts of their own for the inputs: 256 rows x 64 positions, 128 channels a chunk, twelve wavefronts.  Eight multiply 32 rows
+// with all positions (16 x 16 x 32 matrix instructions: half of the sums' registers of FloatMfmaBody's wavefronts, which three wavefronts
+// per SIMD leave).  Four turn inputs into operand cells: a thread loads eight channels of a position quad, two chunks ahead of the one that
+// it writes, so the conversions, eleven instructions per pair of values, run beside the multiplies instead of between them.  us per call among
+// others, FloatMfmaBody / this: 64 x 1024 -> 1024 @7x7, row pairs, 70 % zeros 26.9 / 22.5; 32 x 512 -> 512 @14x14 16.1 / 14.8; 4 x 1248 -> 1024
+// @29x29 30.7 / 25.4.  With 128 rows x 128 positions, 64 channels a chunk, the first takes 25.3 (every input converted twice as
+// often).  What bounds it: nothing alone; 2.2 us a chunk, of which its matrix instructions take 1.4 at the rate they reach on such data
+// (32 x 32 x 16 ones 1.7: 18 ns against twice 7.7 for half the products) and its 80 KB 0.6.
+constexpr int kSplitThreads = 768;
+constexpr int kSplitQuads = 16;                                // position quads of a tile
+constexpr int kSplitChunk = 128;                               // channels of a chunk
+constexpr int kSplitCells = kSplitChunk / 8 * 4 * kSplitQuads;  // cells of a chunk and piece
+constexpr int kSplitRowBlocks = 8;
+
+template <bool RAGGED>
+__device__ __forceinline__ void FloatSplitBody(const FloatMfmaParams& p, uint4* xt) {
+  constexpr int QT = kSplitQuads, CHUNK = kSplitChunk, STEPS = CHUNK / 32, PIECES = 2, kCells = kSplitCells, kBuf = PIECES * kCells;
+  constexpr uint32_t kElem = 4u;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // each XCD owns a contiguous range of tiles, the row groups of one tile follow each other there
+  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+  const int first_tile = (xcd * p.tiles) >> 3, last_tile = ((xcd + 1) * p.tiles) >> 3;
+  const int tile = first_tile + slot / p.row_groups, rg = slot % p.row_groups;
+  if (tile >= last_tile) return;
+  const uint32_t tile_quad0 = (uint32_t)tile * (uint32_t)QT;
+  const int chunks = (p.K + CHUNK - 1) / CHUNK;
+
+  // the scales of fp32, as in FloatMfmaBody
+  uint32_t* const colmax = reinterpret_cast<uint32_t*>(xt + 2 * kBuf);
+  uint32_t* const flags = colmax + 4 * QT;
+  uint32_t* const marks = flags + 4;
+  uint32_t* const first_exp = marks + QT;
+  auto scale_exp = [](uint32_t bits) { return max(1, min(243, 266 - (int)(bits >> 23))); };
+  for (int i = tid; i < kF32Tables / 4; i += kSplitThreads) colmax[i] = 0;
+  __syncthreads();
+
+  if (wave >= 8) {
+    const int j = tid & (QT - 1), kg = (tid >> 4) & 15;
+    const uint32_t quad = min(tile_quad0 + (uint32_t)j, p.total_quads - 1u);
+    const uint32_t img = quad / (uint32_t)p.qpi;
+    const int first = min(4 * (int)(quad - img * (uint32_t)p.qpi), p.hw - 4);
+    const uint32_t vbase = img * (uint32_t)p.K * (uint32_t)p.hw + (uint32_t)first;
+    const __amdgpu_buffer_rsrc_t xbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.x), 0, (int)((uint32_t)p.batch * (uint32_t)p.K * (uint32_t)p.hw * kElem), 0x00020000);
+    const int pitch_in = p.hw * (int)kElem;
+    u4 r[2][8];
+    // The last group of a channel count that is no multiple of 8 holds the last eight channels.  Groups behind it lie outside the buffer:
+    // they read as zeros, and no condition around the loads makes the wait for older ones wait for these too.
+    auto issue = [&](u4 (&rd)[8], int chunk) {
+      const int k = chunk * CHUNK + 8 * kg;
+      const uint32_t voff = k < p.K ? (vbase + (uint32_t)min(k, p.K - 8) * (uint32_t)p.hw) * kElem : kFloatMfmaOutside;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) rd[i] = __builtin_amdgcn_raw_buffer_load_b128(xbuf, (int)voff, i * pitch_in, 0);
+    };
+    uint4* const cells = xt + kg * (4 * QT) + j;
+    float scale[4], peak = 0.0f;
+    uint32_t low = 0xffffffffu;  // the smallest magnitude but zero, as kSmallBits
+    auto commit = [&](u4 (&rd)[8], int buf) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        uint32_t hi[4], lo[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          // the first pieces are one mixed-precision multiply-add each
+          const float a = __uint_as_float(rd[2 * i][c]) * scale[c], b = __uint_as_float(rd[2 * i + 1][c]) * scale[c];
+          peak = fmaxf(fmaxf(peak, fabsf(a)), fabsf(b));
+          low = min(min(low, (__float_as_uint(a) << 1) - 1u), (__float_as_uint(b) << 1) - 1u);
+          const h2 both = {(h1)__builtin_fmaf(a, 1.0f / kFloatMfmaLow, 0.0f), (h1)__builtin_fmaf(b, 1.0f / kFloatMfmaLow, 0.0f)};
+          uint32_t word = __builtin_bit_cast(uint32_t, both);
+          asm("" : "+v"(word));  // the second value is taken from the word, not converted again
+          const h2 h = __builtin_bit_cast(h2, word);
+          const h2 l = __builtin_convertvector((v2f{__builtin_fmaf((float)h.x, -kFloatMfmaLow, a), __builtin_fmaf((float)h.y, -kFloatMfmaLow, b)}), h2);
+          hi[i] = word, lo[i] = __builtin_bit_cast(uint32_t, l);
+        }
+        uint4* const dst = cells + buf * kBuf + c * QT;
+        *dst = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+        dst[kCells] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+      }
+    };
+    auto collect = [&](u4 (&rd)[8]) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        float m = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) m = fmaxf(m, fabsf(__uint_as_float(rd[i][c])));
+        atomicMax(&colmax[4 * j + c], __float_as_uint(m));
+      }
+    };
+    // the cells of chunk `to` (its loads are rd), the barrier behind them, the loads of the chunk two behind it
+    auto bring = [&](u4 (&rd)[8], int buf, int to) {
+      commit(rd, buf);
+      if (peak >= kPeak || low < kSmallBits) {  // one branch for both
+        if (peak >= kPeak) flags[buf] = 1;
+        if (low < kSmallBits) marks[j] = 1;
+      }
+      peak = 0.0f;
+      __syncthreads();
+      if (__builtin_amdgcn_readfirstlane(flags[buf]) != 0) {
+        collect(rd);
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const uint32_t m = colmax[4 * j + c];
+          if (__uint_as_float(m) * scale[c] >= kPeak) scale[c] = __uint_as_float((uint32_t)(scale_exp(m) + 11) << 23);
+        }
+        commit(rd, buf);
+        if (low < kSmallBits) marks[j] = 1;
+        peak = 0.0f;
+        __syncthreads();
+      }
+      issue(rd, to + 2);
+    };
+    issue(r[0], 0);
+    __builtin_amdgcn_sched_barrier(0);
+    issue(r[1], 1);
+    __builtin_amdgcn_sched_barrier(0);
+    collect(r[0]);
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 4; ++c) scale[c] = __uint_as_float((uint32_t)(scale_exp(colmax[4 * j + c]) + 11) << 23);
+    commit(r[0], 0);
+    if (low < kSmallBits) marks[j] = 1;
+    peak = 0.0f;
+    issue(r[0], 2);
+    __syncthreads();
+    int chunk = 0;
+    for (; chunk + 2 < chunks; chunk += 2) {
+      bring(r[1], 1, chunk + 1);
+      bring(r[0], 0, chunk + 2);
+    }
+    if (chunk + 1 < chunks) bring(r[1], 1, chunk + 1);
+    __syncthreads();  // the last chunk is multiplied
+    return;
+  }
+
+  // the wavefront's row block (past the last one: the last one again, not stored)
+  const int rb = rg * kSplitRowBlocks + wave;
+  const int n = lane & 15, kq = lane >> 4;
+  const __amdgpu_buffer_rsrc_t wbuf = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(static_cast<const char*>(p.wtiles)) + (size_t)min(rb, p.row_blocks - 1) * p.padded_ksteps * (1024 * PIECES), 0,
+                                                                        (int)(FloatMfmaWeightTile(p.chunks, 0, PIECES, 0) + FloatMfmaWeightTail(PIECES)), 0x00020000);
+  constexpr int AHEAD = 2;  // steps of weights in registers
+  h8 a[AHEAD][2][PIECES];
+  auto load_weights = [&](int chunk, int ks) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int q = 0; q < PIECES; ++q) a[ks % AHEAD][t][q] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(wbuf, lane * 16, (int)FloatMfmaWeightTile(0, 2 * (chunk * STEPS + ks) + t, PIECES, q), 0));
+  };
+  const uint4* const operand = xt + kq * (4 * QT) + n;
+  // fp32: the products of two high pieces, and those of a high and a low one, which would otherwise each round the sum
+  // of the former (the matrix cores cut sums off rather than round them)
+  v4f acc[2][4], rest[2][4];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[t][c] = rest[t][c] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  uint32_t own_exps = 0;  // a byte each
+  auto own_exp = [&](int c) { return (int)(own_exps >> (8 * c) & 0xffu); };
+  const uint32_t* const own_max = colmax + 4 * n;
+
+  // The matrix cores cut sums off, so a long sum is off by more: behind half of the chunks the sums are added, rounded, to those that wait
+  // in LDS and begin anew (1024 channels 1.6e-7 in 2-norm, as FloatMfmaBody's two sums of 512 each; one sum 2.1e-7; four of 256
+  // 1.3e-7 and 0.8 us more on 64 x 1024 -> 1024 @7x7).
+  v4f* const waiting = reinterpret_cast<v4f*>(reinterpret_cast<char*>(colmax) + kF32Tables) + wave * (8 * 64) + lane;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) waiting[64 * i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  auto add_waiting = [&](auto keep_c) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const v4f sum = acc[t][c] + waiting[64 * (4 * t + c)];
+        if constexpr (decltype(keep_c)::value) {
+          waiting[64 * (4 * t + c)] = sum;
+          acc[t][c] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        } else {
+          acc[t][c] = sum;
+        }
+      }
+  };
+
+  // One chunk: STEPS x 4 cells, two tiles each, cells read PF ahead.  The weights of a step are requested as soon as the one two before it
+  // has used their registers.
+  constexpr int PF = 4;
+  auto run_chunk = [&](auto last_c, int chunk) {
+    constexpr bool LAST = decltype(last_c)::value;
+    const uint4* const in = operand + (chunk & 1) * kBuf;
+    uint4 b[PF + 1][PIECES];
+    auto read = [&](int v) {
+#pragma unroll
+      for (int q = 0; q < PIECES; ++q) b[v % (PF + 1)][q] = in[q * kCells + (v >> 2) * 4 * (4 * QT) + (v & 3) * QT];
+    };
+#pragma unroll
+    for (int d = 0; d < PF; ++d) read(d);
+#pragma unroll
+    for (int ks = 0; ks < STEPS; ++ks) {
+      if (LAST && ks > 0 && 32 * (STEPS * chunk + ks) >= p.K) break;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int v = 4 * ks + c;
+        if (v + PF < 4 * STEPS) read(v + PF);
+        __builtin_amdgcn_sched_barrier(0);  // the reads stay ahead of the multiply
+        const h8 xh = __builtin_bit_cast(h8, b[v % (PF + 1)][0]), xl = __builtin_bit_cast(h8, b[v % (PF + 1)][1]);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) acc[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[ks % AHEAD][t][0], xh, acc[t][c], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) rest[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[ks % AHEAD][t][1], xh, rest[t][c], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) rest[t][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[ks % AHEAD][t][0], xl, rest[t][c], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (!LAST || ks + AHEAD < STEPS) load_weights(chunk, ks + AHEAD);
+    }
+    __syncthreads();
+    if constexpr (!LAST) {
+      const int next = (chunk + 1) & 1;
+      if (__builtin_amdgcn_readfirstlane(flags[next]) != 0) {
+        __syncthreads();
+        if (tid == 0) flags[next] = 0;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const uint32_t om = own_max[c];
+          const int before = own_exp(c);
+          if (__uint_as_float(om) * __uint_as_float((uint32_t)before << 23) >= 0x1p15f) {
+            const int e = scale_exp(om);
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                acc[t][c][i] = __builtin_amdgcn_ldexpf(acc[t][c][i], e - before), rest[t][c][i] = __builtin_amdgcn_ldexpf(rest[t][c][i], e - before);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+              v4f sum = waiting[64 * (4 * t + c)];
+#pragma unroll
+              for (int i = 0; i < 4; ++i) sum[i] = __builtin_amdgcn_ldexpf(sum[i], e - before);
+              waiting[64 * (4 * t + c)] = sum;
+            }
+            own_exps = (own_exps & ~(0xffu << (8 * c))) | (uint32_t)e << (8 * c);
+            // unmarked, every term of a sum was 2^-48 or more when it was added: 2^64 less is far from the subnormal numbers
+            if ((int)first_exp[4 * n + c] - e > 64) marks[n] = 1;
+          }
+        }
+        __syncthreads();
+      }
+    }
+  };
+#pragma unroll
+  for (int ks = 0; ks < AHEAD; ++ks) load_weights(0, ks);
+  __syncthreads();  // the first chunk's maxima
+#pragma unroll
+  for (int c = 0; c < 4; ++c) own_exps |= (uint32_t)scale_exp(own_max[c]) << (8 * c);
+  if (tid < 4 * QT) first_exp[tid] = (uint32_t)scale_exp(colmax[tid]);
+  __syncthreads();
+  int chunk = 0;
+  const int half = chunks >> 1;
+  for (int begun = 0; chunk + 1 < chunks; begun = chunk) {
+    const int until = min(chunk + half, chunks - 1);
+    for (; chunk < until; ++chunk) run_chunk(std::false_type(), chunk);
+    if (chunk - begun == half) add_waiting(std::true_type());
+  }
+  run_chunk(std::true_type(), chunk);
+  add_waiting(std::false_type());
+
+  // Lane (n, kq) holds rows 4 kq .. 4 kq + 3 of its tiles at the four positions of quad n.
+  constexpr int ROWS = 8;  // row i of a lane is row 16 (i / 4) + i % 4 behind its first
+  auto total = [&](int c, int i) { return __builtin_fmaf(rest[i >> 2][c][i & 3], 1.0f / kFloatMfmaLow, acc[i >> 2][c][i & 3]); };
+  auto row_of = [](int i) { return 16 * (i >> 2) + (i & 3); };
+  const int row0 = rb * 32 + 4 * kq, table = min(rb, p.row_blocks - 1) * 32 + 4 * kq;
+  const uint32_t oq = tile_quad0 + (uint32_t)n, on = oq / (uint32_t)p.qpi;
+  const int opp = 4 * (int)(oq - on * (uint32_t)p.qpi), ofirst = min(opp, p.hw - 4);
+  const bool present = oq < p.total_quads;
+  const int own = RAGGED ? opp - ofirst : 0;  // the first position of the quad that is not one of the quad before
+  // An infinity or a NaN among the inputs of a position reaches every row of the product through the zero weights.  Such
+  // quads are walked below, those and the marked ones output by output.
+  float poison = 0.0f;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) poison = __builtin_fmaf(total(c, 0), 0.0f, poison);
+  bool suspect = poison != poison;
+  if (marks[n] != 0) {  // most marked quads hold no output that is too small
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const v4f reach = *reinterpret_cast<const v4f*>(p.row_exp + 32 * p.row_blocks + table + 16 * b);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) suspect = suspect || fabsf(total(c, 4 * b + i)) < reach[i];
+    }
+  }
+  suspect = suspect && present;
+  float bias[ROWS];
+  int row_exp[ROWS];
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    const v4f v = p.bias ? *reinterpret_cast<const v4f*>(static_cast<const float*>(p.bias) + table + 16 * b) : v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    const int4 e = *reinterpret_cast<const int4*>(p.row_exp + table + 16 * b);
+    bias[4 * b] = v.x, bias[4 * b + 1] = v.y, bias[4 * b + 2] = v.z, bias[4 * b + 3] = v.w;
+    row_exp[4 * b] = e.x, row_exp[4 * b + 1] = e.y, row_exp[4 * b + 2] = e.z, row_exp[4 * b + 3] = e.w;
+  }
+  // Stores past the end of the buffer are dropped, so lanes and rows without an output need no branch.
+  constexpr uint32_t kOutside = kFloatMfmaOutside;
+  const __amdgpu_buffer_rsrc_t obuf = __builtin_amdgcn_make_buffer_rsrc(p.out, 0, (int)((uint32_t)p.batch * (uint32_t)p.M * (uint32_t)p.hw * kElem), 0x00020000);
+  const uint32_t pitch = (uint32_t)p.hw * kElem;
+  const uint32_t obase = ((on * (uint32_t)p.M + (uint32_t)row0) * (uint32_t)p.hw + (uint32_t)ofirst) * kElem;
+  auto finish = [&](auto act_c) {
+    constexpr int ACT = decltype(act_c)::value;
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) {
+      const uint32_t at = row0 + row_of(i) < p.M && present ? obase + (uint32_t)row_of(i) * pitch : kOutside;
+      u4 o;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) o[c] = __float_as_uint(ActivateT<ACT>(__builtin_amdgcn_ldexpf(total(c, i), row_exp[i] + 127 - own_exp(c)) + bias[i], p.act));
+      __builtin_amdgcn_raw_buffer_store_b128(o, obuf, (int)(own == 0 ? at : kOutside), 0, 0);
+      if constexpr (RAGGED) {
+#pragma unroll
+        for (int c = 1; c < 4; ++c) __builtin_amdgcn_raw_buffer_store_b32(o[c], obuf, (int)(own != 0 && c >= own ? at + 4 * c : kOutside), 0, 0);
+      }
+    }
+  };
+  if (row0 < p.M) DispatchAct(p.act.type, finish);
+  if (__ballot(suspect) == 0) return;
+  uint32_t walk = 0;  // bit 4 i + c: the output of row i at position c is walked
+  if (suspect) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const v4f reach = *reinterpret_cast<const v4f*>(p.row_exp + 32 * p.row_blocks + table + 16 * b);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          if (row0 + 16 * b + i < p.M && c >= own && !(fabsf(total(c, 4 * b + i)) >= reach[i])) walk |= 1u << (16 * b + 4 * i + c);
+    }
+  }
+  // other lanes write these outputs again: what this wavefront has stored must have arrived
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  WalkOutputs16(p, walk, rb * 32, tile_quad0);
+}
+
+template <bool RAGGED>
+__global__ void __launch_bounds__(kSplitThreads, 3) FloatSplitKernel(PL_HEAD_PARAMS, const FloatMfmaParams block) {
+  const FloatMfmaParams p = WithHead(block, PL_HEAD_ARGS);
+  extern __shared__ uint4 xt[];
+  FloatSplitBody<RAGGED>(p, xt);
+}
+
 template <int WR, bool F32>
 hipError_t Launch(const FloatMfmaParams& p, dim3 grid, hipStream_t s) {
   const dim3 block(kThreads);
   constexpr size_t lds = LdsTables(WR, F32) + (F32 ? kF32Tables : 0);
   return p.quad_aligned ? LaunchWithHead(FloatMfmaKernel<WR, F32, false>, grid, block, lds, s, p) : LaunchWithHead(FloatMfmaKernel<WR, F32, true>, grid, block, lds, s, p);
+}
+
+hipError_t LaunchSplit(const FloatMfmaParams& p, dim3 grid, hipStream_t s) {
+  const dim3 block(kSplitThreads);
+  constexpr size_t lds = 2 * 2 * kSplitCells * 16 + kF32Tables + 8 * 8 * 64 * 16;
+  return p.quad_aligned ? LaunchWithHead(FloatSplitKernel<false>, grid, block, lds, s, p) : LaunchWithHead(FloatSplitKernel<true>, grid, block, lds, s, p);
 }
 
 }  // namespace
@@ -661,6 +1067,13 @@ FloatMfmaPlan PlanFloatMfma(bool f32, int cus, int row_blocks, int K, int M, int
   return best;
 }
 
+// The form with wavefronts of their own for the inputs, us: fitted to 150 random calls in fp32 that it makes one round of workgroups of (64 - 2048
+// channels, 33 - 2048 rows), within 7 % for two of three, and 0.8 for the sums that wait.
+static double SplitMicroseconds(int cus, int64_t workgroups, int K) {
+  const double chunks = (K + kSplitChunk - 1) / kSplitChunk, full = (double)workgroups / cus;
+  return 4.5 + 1.57 * chunks + full * (1.73 + 0.71 * chunks);
+}
+
 hipError_t LaunchFloatMfma(bool f32, int cus, int row_blocks, const FloatMfmaParams& p, hipStream_t stream) {
   if (p.batch <= 0 || p.M <= 0) return hipSuccess;
   if (!FloatMfmaFits(f32, p.K, p.M, p.hw, (int64_t)p.batch * p.hw)) return hipErrorInvalidValue;
@@ -675,6 +1088,18 @@ hipError_t LaunchFloatMfma(bool f32, int cus, int row_blocks, const FloatMfmaPar
   q.padded_ksteps = FloatMfmaPaddedSteps(p.K);
   q.tiles = (int)((q.total_quads + kQuads - 1) / kQuads);
   if (plan.workgroups > (1ll << 30)) return hipErrorInvalidValue;
+  // One round of workgroups of 256 rows x 64 positions where that is expected to take 0.88 of the time (of 11 of 150 random calls at 0.97 two were
+  // slower, 1536 -> 352 @11x11 x 37 31.5 / 33.4, the others 0.85 - 0.97); over more rounds it is 1.1 times as long
+  // (64 x 512 -> 512 @14x14 23.9 / 26.2).  Not in place of 64 rows per workgroup, whose four sums per output are closer to 64 bits (1024
+  // channels 1.3e-7), nor of up to 384 channels, where halves of the sums would not be chunks.
+  if (f32 && row_blocks == 0 && plan.wr >= 4 && p.K > 3 * kSplitChunk) {
+    const int groups = (q.row_blocks + kSplitRowBlocks - 1) / kSplitRowBlocks, tiles = (int)((q.total_quads + kSplitQuads - 1) / kSplitQuads);
+    const int64_t workgroups = 8ll * groups * ((tiles + 7) / 8);
+    if (workgroups <= cus && SplitMicroseconds(cus, workgroups, p.K) < 0.88 * plan.us) {
+      q.row_groups = groups, q.tiles = tiles;
+      return LaunchSplit(q, dim3((uint32_t)workgroups), stream);
+    }
+  }
   const dim3 grid((uint32_t)plan.workgroups);
   switch (plan.wr) {
     case 8:

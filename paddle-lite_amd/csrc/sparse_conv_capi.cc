@@ -637,7 +637,7 @@ bool FloatMfmaWanted(const pl_sparse_conv_handle* h) {
   return h->float_mfma != 0 && pl::FloatMfmaFits(!h->half, h->ic, h->oc, 4, 4) && (h->float_mfma == 2 || h->nnz * 32 >= static_cast<int64_t>(h->oc) * h->ic);
 }
 
-// Dense 32x16 binary16 tiles for the floating-point product (FloatMfmaParams::wtiles); none where a weight does not survive
+// Dense 16x32 binary16 tiles for the floating-point product (FloatMfmaParams::wtiles); none where a weight does not survive
 // in them.
 int BuildFloatMfma(const pl::DecodedLayout& L, pl_sparse_conv_handle* h) {
   const int blocks = CeilDiv(L.oc, 32), kss = pl::FloatMfmaPaddedSteps(L.ic), pieces = h->half ? 1 : 2;
@@ -668,8 +668,8 @@ int BuildFloatMfma(const pl::DecodedLayout& L, pl_sparse_conv_handle* h) {
   }
   auto put = [&](int row, uint32_t c, float weight) {
     const uint32_t t = c < whole ? c & 7u : 8u - (static_cast<uint32_t>(L.ic) - c);
-    const size_t lane = (static_cast<size_t>(row) & 31u) + 32u * ((c >> 3) & 1u);
-    uint16_t* at = &tiles[((static_cast<size_t>(row >> 5) * kss + (c >> 4)) * pieces * 64 + lane) * 8 + t];
+    const size_t lane = (static_cast<size_t>(row) & 15u) + 16u * ((c >> 3) & 3u), tile = 2u * (c >> 5) + (static_cast<size_t>(row) >> 4 & 1u);
+    uint16_t* at = &tiles[((static_cast<size_t>(row >> 5) * kss + tile) * pieces * 64 + lane) * 8 + t];
     if (h->half) {
       at[0] = FastHalfBits(weight);
       exact = exact && (at[0] & 0x7c00u) != 0x7c00u;

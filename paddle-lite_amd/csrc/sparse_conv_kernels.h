@@ -243,7 +243,7 @@ struct HalfWalkParams {
 // tile_pos: 128, 64, 32 or 16 positions with (K + 1) * tile_pos * 2 bytes of LDS.
 hipError_t LaunchHalfWalk(int nrows, int tile_pos, int threads, const HalfWalkParams& p, hipStream_t stream);
 
-// Floating-point SpMM on the matrix cores (float_mfma_kernels.hip): dense 32x16 weight tiles, the channels taken chunk by
+// Floating-point SpMM on the matrix cores (float_mfma_kernels.hip): dense 16x32 weight tiles, the channels taken chunk by
 // chunk.
 constexpr int kFloatMfmaChunk = 64;
 // fp32: the second binary16 piece of a scaled value is what the first one leaves, times kFloatMfmaLow.  Values of kFloatMfmaSmall
@@ -253,8 +253,8 @@ constexpr float kFloatMfmaLow = 2048.0f, kFloatMfmaSmall = 0x1p-13f;
 struct FloatMfmaParams {
   // the first 56 bytes: what the first loads of a kernel need (kernarg_head.h)
   const void* x;
-  // [row block of 32][16-channel step][64 lanes][8 x binary16]; lane l of a tile holds row l % 32, value t channel
-  // 16 step + 8 (l / 32) + t; in the last, partial group of eight channels value t is channel K - 8 + t (zero where
+  // [row block of 32][32-channel step][16 rows of the block][64 lanes][8 x binary16]; lane l of a tile holds row l % 16, value t channel
+  // 32 step + 8 (l / 16) + t; in the last, partial group of eight channels value t is channel K - 8 + t (zero where
   // that channel belongs to the group before)
   const void* wtiles;
   int K;
@@ -274,7 +274,7 @@ struct FloatMfmaParams {
   int nr;                // rows per list of the plain walk, 1 or 2
   void* out;
   const void* bias;      // fp32 or binary16, padded to a multiple of 32 rows; may be null
-  // fp32, padded to a multiple of 32 rows: the tiles of a row hold w 2^-row_exp in two binary16 pieces, [step][piece][64 lanes][8];
+  // fp32, padded to a multiple of 32 rows: the tiles of a row hold w 2^-row_exp in two binary16 pieces, [step][16 rows][piece][64 lanes][8];
   // behind these, as floats: 2^-13 of the sum of a row's |w| 2^-row_exp
   const int32_t* row_exp;
   // the plain walk's lists, for the outputs that the product cannot give
@@ -288,9 +288,9 @@ struct FloatMfmaParams {
 // A lane's offset that lies outside every buffer of that kernel: nothing is fetched or stored there.
 constexpr uint32_t kFloatMfmaOutside = 0x80000000u;
 
-// Where the weight tile of a piece of a step of a chunk begins in a row block.  The loop asks for a chunk behind the last one, too, where
+// Where a piece of a chunk's weight tile (2 step + 16 rows of the block) begins in a row block.  The loop asks for a chunk behind the last one, too, where
 // their number is even: that is the next block's first, and behind the last block's tiles there are FloatMfmaWeightTail bytes.
-constexpr uint32_t FloatMfmaWeightTile(int chunk, int step, int pieces, int piece) { return (uint32_t)((chunk * (kFloatMfmaChunk / 16) + step) * pieces + piece) * 1024u; }
+constexpr uint32_t FloatMfmaWeightTile(int chunk, int tile, int pieces, int piece) { return (uint32_t)((chunk * (kFloatMfmaChunk / 16) + tile) * pieces + piece) * 1024u; }
 constexpr uint32_t FloatMfmaWeightTail(int pieces) { return FloatMfmaWeightTile(1, 0, pieces, 0); }
 
 // How a call is divided (workgroups of wr x 32 rows x 128 positions) and what it is expected to take.
@@ -301,7 +301,7 @@ struct FloatMfmaPlan {
   double us;
 };
 
-int FloatMfmaPaddedSteps(int K);  // 16-channel steps of the weight tiles: whole chunks
+int FloatMfmaPaddedSteps(int K);  // weight tiles of a row block: whole chunks, two per 32 channels
 bool FloatMfmaFits(bool f32, int K, int M, int hw, int64_t positions);
 // row_blocks: blocks of 32 rows per workgroup, 8, 4 or 2; 0 = chosen by the call
 FloatMfmaPlan PlanFloatMfma(bool f32, int cus, int row_blocks, int K, int M, int hw, int batch);

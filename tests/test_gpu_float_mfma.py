@@ -86,6 +86,62 @@ def test_against_64_bits(kind, paired, shape, rows):
     check(case, act, run_hip(case, kernel=forced(case, rows, paired)))
 
 
+# Calls that the rule gives to the fp32 form with wavefronts of their own for the inputs (256 rows x 16 quads, 128 channels a chunk):
+# four to eleven chunks, even and odd, and channels that end inside a step of 32, a group of 8 and a chunk; rows around 32 and 256;
+# tiles that cross images, partial quads, one quad, exactly one tile
+SPLIT = [(1, 385, 2100, 2, 2), (3, 390, 2049, 5, 1), (2, 511, 2305, 3, 3), (1, 513, 2111, 4, 16), (1, 700, 2080, 11, 5), (9, 420, 2060, 1, 7), (1, 1030, 2100, 4, 17), (1, 1281, 2090, 5, 5), (24, 500, 513, 13, 13)]
+
+
+@pytest.mark.parametrize("shape", SPLIT, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("paired", [False, True], ids=["unstructured", "semi"])
+def test_fp32_wavefronts_of_their_own_for_the_inputs(paired, shape):
+    act = sorted(ACTS)[sum(shape) % len(ACTS)]
+    case = make_case("fp32", *shape, paired=paired, act=act)
+    check(case, act, run_hip(case, kernel=forced(case, 0, paired)))
+
+
+@pytest.mark.parametrize("how", ["grow", "late", "tails", "binades", "inf", "many nan"])
+def test_fp32_wavefronts_of_their_own_and_hard_inputs(how):
+    """New scales in the middle of a sum, inputs too small for their pieces, also in the last chunk; infinities and NaNs in few
+    and in most quads."""
+    case = make_case("fp32", 2, 450, 2100, 9, 7, act="none", sparsity=0.9)
+    case.bias = None
+    rng = np.random.RandomState(3)
+    if how == "grow":
+        case.x *= (2.0 ** (np.arange(450) // 60 * 4 - 14)).astype(np.float32)[None, :, None, None]
+    elif how == "late":
+        case.x[:, :128] = 0
+        case.x[1, :440] = 0
+        case.x[0, 449, 2] = 1e9
+    elif how == "tails":
+        case.x *= np.exp(3 * rng.standard_normal(case.x.shape)).astype(np.float32)
+    elif how == "binades":
+        case.x = np.ldexp(case.x, rng.randint(-60, 1, size=case.x.shape)).astype(np.float32)
+    elif how == "inf":
+        case.x[0, 3, 2, 1], case.x[1, 449, 8, 6] = np.inf, np.nan
+    else:
+        case.x[:, 200, :, 1:] = np.nan
+    got = run_hip(case, kernel=forced(case, 0))
+    bad = ~np.isfinite(case.x)
+    if bad.any():
+        hit = np.matmul(case.dense != 0, bad.reshape(2, 450, -1)).reshape(got.shape)
+        assert np.array_equal(~np.isfinite(got), hit) and hit.any() and not hit.all()
+        case.x[bad] = 0
+        ref, mag = sums(case)
+        assert (np.abs(got - ref)[~hit] <= ((6 + 450 / 16.0) * 2.0 ** -23 * mag)[~hit]).all()
+    else:
+        check(case, "none", got)
+
+
+def test_fp32_wavefronts_of_their_own_are_as_exact():
+    """2-norm against 64 bits beside the form with 128 rows that these calls would take otherwise: both add two sums of half of the
+    channels, whose errors differ by chance only (5 % is 50 times what the norm of 100 000 outputs' errors scatters by)."""
+    case = make_case("fp32", 16, 640, 2100, 5, 5, act="none", sparsity=0.8)
+    ref, _ = sums(case)
+    off = [np.linalg.norm((run_hip(case, kernel=forced(case, rows)) - ref).ravel()) for rows in (128, 0)]
+    assert off[1] <= 1.05 * off[0]
+
+
 @pytest.mark.parametrize("act", sorted(ACTS))
 @pytest.mark.parametrize("kind", sorted(KINDS))
 def test_activations_and_a_new_bias(kind, act):
