@@ -28,7 +28,7 @@
 // A second kernel (ImageRowsDwKernel) runs the int8 depthwise 3 x 3 layer that follows such a pointwise layer in
 // a MobileNet in the same launch: the tile of a wavefront is 16 output channels times all positions, i.e. 16 whole
 // planes of the depthwise layer.  With int8 output the epilogue writes them to the wavefront's own LDS instead of
-// global memory, and behind its last window the wavefront computes the depthwise layer on them (DwStage, no
+// global memory, and behind its last window the wavefront computes the depthwise layer on them (DwStageWide, DwStage, no
 // barrier: the planes are private to the wavefront).  14 x 14 maps, padding 1, stride 1 or 2.
 //
 // Reference semantics: out = act(fmaf(float(acc), scale, bias)) per output, int32 accumulation over all
@@ -52,6 +52,7 @@ using epilogue::ActivateT;
 using epilogue::ActQuantF;
 using epilogue::DispatchAct;
 using epilogue::TruncPackI8x4;
+using epilogue::TruncPackI8x8;
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
@@ -72,10 +73,25 @@ constexpr int kRowStride = 8;  // rows of a tile: w + 8 m
 // Output kind of the kernel that runs the following depthwise layer itself: int8 like kOutI8, written to the
 // wavefront's own planes in LDS (one plane of H x W bytes per row of its tile) instead of global memory.
 constexpr int kOutPlanes = 3;
+// The same with the 14 columns of a plane's row on 16 bytes, zeros behind them, and a row of zeros in front of and behind every plane (shared
+// by neighbours): rows of whole aligned dwords, for the matrix cores.
+constexpr int kOutWidePlanes = 4;
+constexpr int kWidePlane = 15 * 16, kWidePlaneBytes = (16 + 16 * kWidePlane + 31) / 32 * 32;  // of one plane; of a wavefront's sixteen
 template <int OUT>
-constexpr int kPlaneStride = OUT == kOutPlanes ? 1 : kRowStride;  // rows of the tile are this many rows apart where they are stored
+constexpr bool kToPlanes = OUT == kOutPlanes || OUT == kOutWidePlanes;
+template <int OUT>
+constexpr int kPlaneStride = kToPlanes<OUT> ? 1 : kRowStride;  // rows of the tile are this many rows apart where they are stored
 __device__ __forceinline__ void StoreLds(uint32_t v, char* p) {
   *reinterpret_cast<__attribute__((address_space(3))) uint32_t*>(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p))) = v;
+}
+// Where a position lies in a wide plane: 16 bytes a row of 14 (p / 14 for p < 200 as a multiplication).
+__device__ __forceinline__ int WideAt(int position) { return position + 2 * ((position * 147) >> 11); }
+// Positions 4 q .. 4 q + 3 of a wide plane, as two pairs, which no row's end parts.
+__device__ __forceinline__ void StoreWide(uint32_t v, char* plane, int q) {
+  typedef __attribute__((address_space(3))) uint16_t lds16;
+  const uint32_t at = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(plane));
+  *reinterpret_cast<lds16*>(at + WideAt(4 * q)) = (uint16_t)v;
+  *reinterpret_cast<lds16*>(at + WideAt(4 * q + 2)) = (uint16_t)(v >> 16);
 }
 
 // 16 bytes stored as streaming data (nt) at a wave-uniform base plus an unsigned 32-bit lane offset (no 64-bit
@@ -107,7 +123,7 @@ template <int OUT, int ACT>
 __device__ __forceinline__ u4 Finish4(int a0, int a1, int a2, int a3, float s, float b, const DevAct& act) {
   if (OUT == kOutAcc32) return u4{(uint32_t)a0, (uint32_t)a1, (uint32_t)a2, (uint32_t)a3};
   const float v0 = __builtin_fmaf((float)a0, s, b), v1 = __builtin_fmaf((float)a1, s, b), v2 = __builtin_fmaf((float)a2, s, b), v3 = __builtin_fmaf((float)a3, s, b);
-  if (OUT == kOutI8 || OUT == kOutPlanes) return u4{TruncPackI8x4(ActQuantF<ACT>(v0, act), ActQuantF<ACT>(v1, act), ActQuantF<ACT>(v2, act), ActQuantF<ACT>(v3, act)), 0u, 0u, 0u};
+  if (OUT == kOutI8 || kToPlanes<OUT>) return u4{TruncPackI8x4(ActQuantF<ACT>(v0, act), ActQuantF<ACT>(v1, act), ActQuantF<ACT>(v2, act), ActQuantF<ACT>(v3, act)), 0u, 0u, 0u};
   return u4{__float_as_uint(ActivateT<ACT>(v0, act)), __float_as_uint(ActivateT<ACT>(v1, act)), __float_as_uint(ActivateT<ACT>(v2, act)), __float_as_uint(ActivateT<ACT>(v3, act))};
 }
 
@@ -115,12 +131,14 @@ __device__ __forceinline__ u4 Finish4(int a0, int a1, int a2, int a3, float s, f
 // lane's line is shared with the end of the previous output row and merges in L2 (plain store).
 template <int OUT, int ACT>
 __device__ __forceinline__ void StoreRow(const v4i (&acc)[4], int i, float sc, float bi, const DevAct& act, char* __restrict__ orow, int pitch, int q, bool partial, Lane ln) {
-  constexpr int kElem = (OUT == kOutI8 || OUT == kOutPlanes) ? 1 : 4;
+  constexpr int kElem = (OUT == kOutI8 || kToPlanes<OUT>) ? 1 : 4;
   const u4 v = Finish4<OUT, ACT>(acc[0][i], acc[1][i], acc[2][i], acc[3][i], sc, bi, act);
   // at most 128 rows of at most 256 four-byte positions behind orow: the offset fits 32 bits; it is negative only
   // for the quads in front of a row, which are not stored
   const int off = ((kPlaneStride<OUT> * (4 * ln.kq + i)) * pitch + 4 * q) * kElem;
-  if (OUT == kOutPlanes) {
+  if (OUT == kOutWidePlanes) {
+    if (q >= 0) StoreWide(v.x, orow + (4 * ln.kq + i) * kWidePlane, q);
+  } else if (OUT == kOutPlanes) {
     if (q >= 0) StoreLds(v.x, orow + off);
   } else if (OUT == kOutI8) {
     if (q >= 0) StorePlain(v.x, orow + off);
@@ -136,12 +154,10 @@ __device__ __forceinline__ void StoreRow(const v4i (&acc)[4], int i, float sc, f
 // the depthwise output.
 constexpr int kPlaneInBytes = 16 + 16 * 196 + 48, kPlaneBufBytes = kPlaneInBytes + 16 * 196;
 
-// The depthwise layer on the wavefront's planes: one output row of one plane per lane and pass (dw_row_item.h),
+// The depthwise layer with stride 2 on the wavefront's planes: one output row of one plane per lane and pass (dw_row_item.h),
 // outputs collected plane-major in LDS, then stored: a plane of the tile's row m is channel row0 + 8 m.
-template <int STRIDE>
 __device__ __forceinline__ void DwStage(const DwConvParams& d, char* planes_in, char* planes_out, int n, int M, int row0, int lane) {
-  constexpr int NOUT = STRIDE == 1 ? 14 : 7;
-  constexpr int oh = NOUT, ow = NOUT;  // 14 x 14 planes, padding 1
+  constexpr int oh = 7, ow = 7, plane_bytes = oh * ow;  // of 14 x 14 planes, padding 1
   constexpr int items = 16 * oh, passes = (items + 63) / 64;
   dwrow::DwRowStage st;
   st.lds_in = planes_in - 16;
@@ -167,21 +183,74 @@ __device__ __forceinline__ void DwStage(const DwConvParams& d, char* planes_in, 
       const bool live = item < items;
       const int it = live ? item : items - 1;
       const int m = it / oh, oy = it - m * oh;
-      dwrow::DwRowItemWith<STRIDE, NOUT, kOutI8, ACT, 14>(d, st, (uint32_t)m, wrow[t], sc[t], bi[t], oy, live, planes_out + it * ow);
+      dwrow::DwRowItemWith<2, ow, kOutI8, ACT, 14>(d, st, (uint32_t)m, wrow[t], sc[t], bi[t], oy, live, planes_out + it * ow);
     }
   });
-  const int plane_bytes = oh * ow;
   char* obase = static_cast<char*>(d.out) + ((size_t)n * M + row0) * plane_bytes;
-  if ((plane_bytes & 3) == 0) {
-    const int per = plane_bytes >> 2;
-    for (int k = lane; k < 16 * per; k += 64) {
-      const int m = k / per, j = k - m * per;
-      StorePlain(*reinterpret_cast<const uint32_t*>(planes_out + 4 * k), obase + (size_t)(kRowStride * m) * plane_bytes + 4 * j);
+  for (int k = lane; k < 16 * plane_bytes; k += 64) {
+    const int m = k / plane_bytes, j = k - m * plane_bytes;
+    *reinterpret_cast<__attribute__((address_space(1))) char*>(reinterpret_cast<uintptr_t>(obase + (size_t)(kRowStride * m) * plane_bytes + j)) = planes_out[k];
+  }
+}
+
+// The same with stride 1 on wide planes and the matrix cores: v_mfma_i32_4x4x4 multiplies four dwords (of four output rows of a plane: its
+// columns) with the filter row at four places (the four output columns of a dword: its rows), the dword itself and the bytes its neighbours
+// add.  A lane takes one output row; sixteen rows per plane, two of them idle, so that four lanes share a plane, four planes per pass.  The
+// outputs take the input rows' place: a pass reads all of its planes before it writes them.
+// What bounds it: vector ALU issue of the requantisation (14 outputs of 4 to 5 instructions per row and pass).  With the products by v_dot4 on planes of 14
+// bytes a row, a byte stored at a time, each of five launches of 64 x 512 -> 512 @14x14 and this layer took 2.3 us more (13 layers with them 228.6 -> 216.8).
+__device__ __forceinline__ void DwStageWide(const DwConvParams& d, char* planes, int n, int M, int row0, int lane) {
+  const int j = lane & 3, oy = lane & 15, pl = lane >> 4;
+  // bytes j + 3 .. j + 5 of the twelve of three dwords: of the middle one; byte 3 of the first as byte 3 and byte 0 of the last as byte 0
+  const uint32_t sel0 = __builtin_amdgcn_alignbyte(0x0c0c0c02u, 0x01000c0cu, (uint32_t)(3 - j)), sel1 = j == 0 ? 0x000c0c0cu : (j == 3 ? 0x0c0c0c02u : 0x0c0c0c0cu);
+  // filter rows, scale and bias of every pass's channel first: one memory latency for all passes
+  uint32_t wrow[4][3];
+  float sc[4], bi[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const int c = row0 + kRowStride * (4 * t + pl);
+#pragma unroll
+    for (int r = 0; r < 3; ++r) wrow[t][r] = d.wpack[4 * c + r];
+    sc[t] = d.scale[c];
+    bi[t] = d.bias[c];
+  }
+  char* const own = planes + pl * kWidePlane + 16 * min(oy, 13);
+  DispatchAct(d.act.type, [&](auto act_c) {
+    constexpr int ACT = decltype(act_c)::value;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      char* const at = own + 4 * t * kWidePlane;
+      v4i sums[4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+      for (int r = 0; r < 3; ++r) {
+        const u4 x = *reinterpret_cast<const u4*>(at + 16 * (r - 1));
+        const int a0 = (int)__builtin_amdgcn_perm(0u, wrow[t][r], sel0), a1 = (int)__builtin_amdgcn_perm(0u, wrow[t][r], sel1);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          sums[q] = __builtin_amdgcn_mfma_i32_4x4x4i8(a0, (int)x[q], sums[q], 0, 0, 0);
+          const uint32_t beside = __builtin_amdgcn_perm(q < 3 ? x[q < 3 ? q + 1 : 0] : 0u, q > 0 ? x[q > 0 ? q - 1 : 0] : 0u, 0x03020104u);  // bytes 1 and 2 meet zeros
+          sums[q] = __builtin_amdgcn_mfma_i32_4x4x4i8(a1, (int)beside, sums[q], 0, 0, 0);
+        }
+      }
+      uint32_t out[4];
+#pragma unroll
+      for (int q = 0; q < 4; q += 2) {
+        float f[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) f[i] = 4 * q + i < 14 ? ActQuantF<ACT>(__builtin_fmaf((float)sums[q + i / 4][i % 4], sc[t], bi[t]), d.act) : 0.0f;
+        TruncPackI8x8(f[0], f[1], f[2], f[3], f[4], f[5], f[6], f[7], out[q], out[q + 1]);
+      }
+      if (oy < 14) *reinterpret_cast<u4*>(at) = u4{out[0], out[1], out[2], out[3]};
     }
-  } else {
-    for (int k = lane; k < 16 * plane_bytes; k += 64) {
-      const int m = k / plane_bytes, j = k - m * plane_bytes;
-      *reinterpret_cast<__attribute__((address_space(1))) char*>(reinterpret_cast<uintptr_t>(obase + (size_t)(kRowStride * m) * plane_bytes + j)) = planes_out[k];
+  });
+  // one plane per store: 49 dwords, each two pairs of columns
+  const int at0 = WideAt(4 * lane), at1 = WideAt(4 * lane + 2);
+  char* const obase = static_cast<char*>(d.out) + ((size_t)n * M + row0) * 196 + 4 * lane;
+  if (lane < 49) {
+#pragma unroll
+    for (int m = 0; m < 16; ++m) {
+      const uint32_t lo = *reinterpret_cast<const uint16_t*>(planes + m * kWidePlane + at0), hi = *reinterpret_cast<const uint16_t*>(planes + m * kWidePlane + at1);
+      StorePlain(lo | hi << 16, obase + (size_t)(kRowStride * m) * 196);
     }
   }
 }
@@ -197,7 +266,7 @@ __device__ __forceinline__ void Window(const uint4* __restrict__ xt, int kgs, in
   for (int c = 0; c < 4; ++c) acc[c] = v4i{0, 0, 0, 0};
   // operand cells in flight ahead of the multiply: two k-steps where the multiply is what the wavefront waits for
   // (int8 output), one where it hides behind the stores (8.13 against 8.17 us on the metric shape; three: 8.27)
-  constexpr int PF = (OUT == kOutI8 || OUT == kOutPlanes) ? 2 : 1;
+  constexpr int PF = (OUT == kOutI8 || kToPlanes<OUT>) ? 2 : 1;
   constexpr int kStepsPerRow = KS >= 4 ? KS / 4 : 1;
   uint4 bq[PF + 1][4];
 #pragma unroll
@@ -237,11 +306,11 @@ __device__ __forceinline__ void Window(const uint4* __restrict__ xt, int kgs, in
 // load of the kernel arguments from memory (8.36 -> 8.10 us on the metric shape).
 //
 // dw (kOutPlanes only): the depthwise layer that follows; the wavefront then keeps its 16 output planes in LDS
-// and runs that layer on them (DwStage below).
+// and runs that layer on them (DwStageWide, DwStage).
 //
 // SLAB: a work item takes one slab of hw positions of a larger map (p.pitch positions per channel, p.slabs slabs
 // per image): the channel rows of the input and the rows of the output are then p.pitch apart, not hw.
-template <int KS, int OUT, int QPI, int DW_STRIDE = 0, bool SLAB = false>
+template <int KS, int OUT, int QPI, bool SLAB = false>
 __device__ __forceinline__ void RowsBody(const ImageMfmaParams& p, uint4* lds_raw, const DwConvParams* dw) {
   // shifted windows read up to seven cells in front of a row of cells
   uint4* xt = lds_raw + 16;
@@ -273,6 +342,10 @@ __device__ __forceinline__ void RowsBody(const ImageMfmaParams& p, uint4* lds_ra
     }
   }
   __builtin_amdgcn_sched_barrier(0);
+  if constexpr (OUT == kOutWidePlanes) {  // while the image is under way
+    char* const zeros = reinterpret_cast<char*>(lds_raw) + 256 + (size_t)NKG * kgs * 16 + wave * kWidePlaneBytes;
+    for (int i = 16 * lane; i < kWidePlaneBytes; i += 1024) *reinterpret_cast<uint4*>(zeros + i) = make_uint4(0u, 0u, 0u, 0u);
+  }
   // every channel group becomes four cells per quad; the weights of KS / BPW k-steps are requested behind it
   char* lbase = reinterpret_cast<char*>(xt);
   v4i a[KS];
@@ -329,10 +402,10 @@ __device__ __forceinline__ void RowsBody(const ImageMfmaParams& p, uint4* lds_ra
   const int nqt = (qpi + sh) >> 4;       // full windows
   const int left = qpi + sh - 16 * nqt;  // quads after the last window
   const int ntail = (left + 3) >> 2;
-  constexpr int kElem = (OUT == kOutI8 || OUT == kOutPlanes) ? 1 : 4;
+  constexpr int kElem = (OUT == kOutI8 || kToPlanes<OUT>) ? 1 : 4;
   // kOutPlanes: the wavefront's planes behind the image's cells, 16 bytes of slack in front of them
-  char* planes = reinterpret_cast<char*>(lds_raw) + 256 + (size_t)NKG * kgs * 16 + wave * kPlaneBufBytes;
-  char* orow = OUT == kOutPlanes ? planes + 16 : Uniform(static_cast<char*>(p.out) + (((size_t)n * p.M + row0) * pitch + slab * hw) * kElem);
+  char* planes = reinterpret_cast<char*>(lds_raw) + 256 + (size_t)NKG * kgs * 16 + wave * (OUT == kOutWidePlanes ? kWidePlaneBytes : kPlaneBufBytes);
+  char* orow = kToPlanes<OUT> ? planes + 16 : Uniform(static_cast<char*>(p.out) + (((size_t)n * p.M + row0) * pitch + slab * hw) * kElem);
   DispatchAct(OUT == kOutAcc32 ? 0 : epilogue::LeakyAsMax(p.act), [&](auto act_c) {
     constexpr int ACT = decltype(act_c)::value;
     if (nqt > 0) {
@@ -376,18 +449,19 @@ __device__ __forceinline__ void RowsBody(const ImageMfmaParams& p, uint4* lds_ra
       if (q >= 0 && q < qpi) {
         const u4 v = Finish4<OUT, ACT>(acc[0], acc[1], acc[2], acc[3], sct, bit, p.act);
         char* ptr = orow + ((size_t)(kPlaneStride<OUT> * ln.n) * pitch + 4 * q) * kElem;
-        if (OUT == kOutPlanes) StoreLds(v.x, ptr); else if (OUT == kOutI8) StorePlain(v.x, ptr); else StorePlain(v, ptr);
+        if (OUT == kOutWidePlanes) StoreWide(v.x, orow + ln.n * kWidePlane, q); else if (OUT == kOutPlanes) StoreLds(v.x, ptr); else if (OUT == kOutI8) StorePlain(v.x, ptr); else StorePlain(v, ptr);
       }
     }
   });
-  if constexpr (OUT == kOutPlanes) DwStage<DW_STRIDE>(*dw, planes + 16, planes + kPlaneInBytes, n, p.M, row0, lane);
+  if constexpr (OUT == kOutWidePlanes) DwStageWide(*dw, planes + 16, n, p.M, row0, lane);
+  if constexpr (OUT == kOutPlanes) DwStage(*dw, planes + 16, planes + kPlaneInBytes, n, p.M, row0, lane);
 }
 
 template <int KS, int OUT, int QPI, bool SLAB = false>
 __global__ void __launch_bounds__(512) ImageRowsMfmaKernel(PL_HEAD_PARAMS, const ImageMfmaParams block) {
   const ImageMfmaParams p = WithHead(block, PL_HEAD_ARGS);
   extern __shared__ uint4 lds_raw[];
-  RowsBody<KS, OUT, QPI, 0, SLAB>(p, lds_raw, nullptr);
+  RowsBody<KS, OUT, QPI, SLAB>(p, lds_raw, nullptr);
 }
 
 // The same followed by the depthwise 3 x 3 layer (14 x 14 planes, padding 1, stride DW_STRIDE, int8 output) on
@@ -396,7 +470,7 @@ template <int KS, int DW_STRIDE>
 __global__ void __launch_bounds__(512) ImageRowsDwKernel(PL_HEAD_PARAMS, const ImageMfmaParams block, const DwConvParams dw) {
   const ImageMfmaParams p = WithHead(block, PL_HEAD_ARGS);
   extern __shared__ uint4 lds_raw[];
-  RowsBody<KS, kOutPlanes, 49, DW_STRIDE>(p, lds_raw, &dw);
+  RowsBody<KS, DW_STRIDE == 1 ? kOutWidePlanes : kOutPlanes, 49>(p, lds_raw, &dw);
 }
 
 template <int OUT>
@@ -510,7 +584,7 @@ hipError_t LaunchImageRowsDw(const ImageMfmaParams& p, const DwConvParams& d, in
   q.items = (int)items;
   q.per_xcd = (q.items + 7) / 8;
   q.align = 0;
-  const size_t lds = 256 + (size_t)(p.K / 16) * q.kgs * 16 + (size_t)8 * kPlaneBufBytes;
+  const size_t lds = 256 + (size_t)(p.K / 16) * q.kgs * 16 + (size_t)8 * (stride == 1 ? kWidePlaneBytes : kPlaneBufBytes);
   const dim3 grid(8u * (uint32_t)q.per_xcd), block(512);
   const int shape = 10 * (p.K / 64) + stride;
   switch (shape) {

@@ -1943,11 +1943,13 @@ int pl_sparse_conv_dwconv3x3_pays(const pl_sparse_conv_handle* conv, const pl_dw
   if (!pl_sparse_conv_dwconv3x3_fits(conv, dw, height, width) || batch <= 0) return 0;
   // us, two launches against one, replayed from a graph, at 1 / 4 / 16 / 32 / 64 images @14x14.  Stride 2: 512 -> 512 7.4 / 8.4,
   // 8.3 / 8.5, 9.4 / 8.5, 10.7 / 8.8, 12.0 / 8.9; 256 -> 512 7.4 / 6.8, 8.0 / 6.9, 8.5 / 6.9, 8.9 / 7.0, 10.3 / 7.4; 128 -> 128 7.2 / 6.0 ...
-  // 7.9 / 6.3.  Stride 1: 512 -> 512 7.7 / 11.0, 8.5 / 11.1, 10.1 / 11.2, 11.8 / 11.6, 14.1 / 12.1; 256 -> 512 7.7 / 9.4, 8.3 / 9.6, 9.2 / 9.7,
-  // 10.2 / 9.9, 12.3 / 10.6.  The one launch does the depthwise work of 128 planes on the CU that made them, whatever the batch;
+  // 7.9 / 6.3.  Stride 1: 512 -> 512 7.5 / 9.0, 8.4 / 9.1, 9.5 / 9.3, 12.7 / 9.8, 16.5 / 10.9; 256 -> 512 7.6 / 7.5, 8.4 / 7.5, 9.3 / 7.7,
+  // 10.9 / 8.0, 14.5 / 8.9.  The one launch does the depthwise work of 128 planes on the CU that made them, whatever the batch;
   // the depthwise kernel spreads a small batch over the chip.  At stride 2 one launch is kept at any batch: from the Python
   // classes 256 and 128 channels gain from one image on, and 512 channels (two / one, 1 / 4 / 8 images: 7.5 / 8.2, 8.3 / 8.4, 8.6 / 8.4)
-  // would gain from two launches below six images only.
+  // would gain from two launches below six images only.  At stride 1 the answer changes at half the
+  // CUs, as callers have it: from there on the one launch is ahead for every channel count (512 channels are even at about 16 images, and up to
+  // 256 channels gain from few images on, 4 images 0.7 - 0.9 us, 1 image at most 0.7).
   if (dw->stride == 2) return 1;
   const int64_t workgroups = static_cast<int64_t>(batch) * (conv->oc / 128);
   const int cus = std::max(1, conv->wg_slots_default / 2);

@@ -96,6 +96,25 @@ def test_batches(batch, stride):
     check_pair(batch, 512, 512, stride, seed=batch)
 
 
+@pytest.mark.parametrize("tap", range(9))
+def test_every_tap_alone_at_stride_1(tap):
+    """A filter with one tap shifts the planes: rows and columns of the border, the ends of the rows' dwords and neighbouring planes of LDS
+    would show in the outputs if a tap met the wrong byte."""
+    import torch
+
+    case, conv, _, _ = make_pair(2, 128, 256, 1, "none", "none", seed=40 + tap)
+    filt = np.zeros((256, 1, 3, 3), dtype=np.int8)
+    filt.reshape(256, 9)[:, tap] = np.where(np.arange(256) % 2, -127, 127)
+    scale, bias = np.full(256, 0.01, dtype=np.float32), np.linspace(-0.3, 0.3, 256).astype(np.float32)
+    dw = pla.DepthwiseConv(pla.ConvParam(filt, bias, strides=(1, 1), paddings=(1, 1, 1, 1), activation_param=ACTS["none"](), input_scale=0.01, weight_scale=scale, output_scale=0.015), out_precision="int8")
+    dw.PrepareForRun()
+    x = torch.from_numpy(case.x).cuda()
+    mid = conv.Run(x)
+    got = dwmod.run_conv_dw(conv, dw, x, torch.empty_like(mid)).cpu().numpy()
+    assert np.array_equal(got, O.dwconv3x3_int8(mid.cpu().numpy(), filt[:, 0], dw.w_scale_, dw.bias_, oracle_act(dw.merged_act), out="int8", stride=1, pad=1))
+    assert len(np.unique(got)) > 50
+
+
 def test_two_calls_in_a_row_reuse_nothing():
     """The planes in LDS are rebuilt by every launch: a second call with other inputs is as exact as the first."""
     check_pair(8, 512, 512, 1, seed=1)
