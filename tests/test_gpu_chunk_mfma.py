@@ -135,6 +135,17 @@ def test_a_kernel_that_a_tuning_field_names_keeps_its_calls():
             assert ALGO_NAMES[capi.check(L.pl_sparse_conv_algo_for(kernel._handle, batch, im_size))] == (other if field else "chunk_mfma"), (other, field)
 
 
+@pytest.mark.parametrize("batch, oc, chosen", [(32, 1024, "chunk_mfma"), (33, 1024, "image_mfma"), (64, 1024, "image_mfma"), (65, 1024, "chunk_mfma"), (33, 2048, "chunk_mfma"), (171, 384, "chunk_mfma")])
+@pytest.mark.parametrize("out_int8", [False, True], ids=["fp32", "int8"])
+def test_1024_channels_on_maps_of_49_positions(batch, oc, chosen, out_int8):
+    """More than one round of the image kernel's items, or at most half of one, on a device of 256 CUs; the same bits as that kernel's."""
+    case = workloads.make_int8("rounds", batch, 1024, oc, 7, 7, 0.9, False, AP(), out_int8=out_int8, seed=batch)
+    rule, image = make_kernel(case)[0], make_kernel(case, tuning=capi.tuning(chunk_mfma=capi.TUNE_NEVER))[0]
+    assert ALGO_NAMES[capi.check(capi.lib().pl_sparse_conv_algo_for(rule._handle, batch, 49))] == chosen
+    assert ALGO_NAMES[capi.check(capi.lib().pl_sparse_conv_algo_for(image._handle, batch, 49))] == "image_mfma"
+    assert_same(case, run_hip(case, kernel=rule), run_hip(case, kernel=image))
+
+
 def test_weight_tiles_are_held_where_some_call_can_use_them():
     """Device memory of a handle: tiles of 16 rows x 64 channels in whole chunks of 512 channels, none where a tuning field
     gives every call to another kernel."""
