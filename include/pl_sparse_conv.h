@@ -169,13 +169,18 @@ typedef struct pl_sparse_conv_tuning {
                                 PL_ALGO_BLOCK_MFMA; it takes 16 channels and maps
                                 of 4 positions and more.  By the rule, a kernel
                                 that another field names keeps its calls      */
-  int32_t chunk_positions;   /* that kernel: positions per tile, 64, 128 or 256 */
+  int32_t chunk_positions;   /* that kernel: positions per tile, 64, 128 or 256;
+                                by the rule of chunk_split, a width that is
+                                named is that of the form without             */
   int32_t float_mfma;        /* (switch) fp32 / fp16 calls on the matrix cores
                                 (PL_ALGO_CHUNK_MFMA), PL_ALGO_AUTO only; it takes
                                 8 channels and maps of 4 positions and more.  By
                                 the rule, a handle with a walk_* field keeps its
                                 calls with the walks                           */
   int32_t float_mfma_rows;   /* that kernel: rows per workgroup, 64, 128, 256  */
+  int32_t chunk_split;       /* (switch) the kernel of chunk_mfma with wavefronts
+                                of their own for the activations (256 rows x
+                                128 positions; maps of 16 positions and more)  */
 } pl_sparse_conv_tuning;
 
 /* Everything PrepareForRun() knows.  All pointers are HOST pointers and are
@@ -200,8 +205,9 @@ typedef struct pl_sparse_conv_desc {
   const float* bias;             /* oc merged biases or NULL                */
   pl_activation act;
   pl_sparse_conv_tuning tuning;  /* struct_size may also be the offset of this
-                                    field or of tuning.chunk_mfma: the rules
-                                    apply to what lies behind it              */
+                                    field, of tuning.chunk_mfma, float_mfma or
+                                    chunk_split: the rules apply to what lies
+                                    behind it                                 */
 } pl_sparse_conv_desc;
 
 typedef struct pl_sparse_conv_info {
@@ -267,6 +273,17 @@ int pl_sparse_conv_get_info(const pl_sparse_conv_handle* handle,
  * the registration (lite/kernels/arm/sparse_conv_compute.cc:369-430). */
 int pl_sparse_conv_algo_for(const pl_sparse_conv_handle* handle, int32_t batch,
                             int32_t im_size);
+
+/* How a call for which that is PL_ALGO_CHUNK_MFMA is divided; of an int8
+ * handle (else, or where it is another algorithm, PL_ERR_UNSUPPORTED). */
+typedef struct pl_sparse_conv_chunk_form {
+  int32_t rows;          /* of a workgroup's tile                           */
+  int32_t positions;
+  int32_t split;         /* 1 = the form that tuning.chunk_split names      */
+} pl_sparse_conv_chunk_form;
+int pl_sparse_conv_chunk_form_for(const pl_sparse_conv_handle* handle,
+                                  int32_t batch, int32_t im_size,
+                                  pl_sparse_conv_chunk_form* form);
 
 /* Replace scale / bias / activation without re-uploading weights (what a
  * second PrepareForRun with new quantisation parameters would do). Either

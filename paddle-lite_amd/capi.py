@@ -24,6 +24,7 @@ EXPORTS = [
     "pl_sparse_conv_run_sequence",
     "pl_sparse_conv_get_info",
     "pl_sparse_conv_algo_for",
+    "pl_sparse_conv_chunk_form_for",
     "pl_sparse_conv_set_epilogue",
     "pl_sparse_conv_destroy",
     "pl_sparse_count_semi",
@@ -75,7 +76,12 @@ class Tuning(C.Structure):
         ("chunk_positions", C.c_int32),
         ("float_mfma", C.c_int32),
         ("float_mfma_rows", C.c_int32),
+        ("chunk_split", C.c_int32),
     ]
+
+
+class ChunkForm(C.Structure):
+    _fields_ = [("rows", C.c_int32), ("positions", C.c_int32), ("split", C.c_int32)]
 
 
 def tuning(**fields):
@@ -178,6 +184,8 @@ def lib():
     L.pl_sparse_conv_get_info.restype = C.c_int
     L.pl_sparse_conv_algo_for.argtypes = [C.c_void_p, C.c_int32, C.c_int32]
     L.pl_sparse_conv_algo_for.restype = C.c_int
+    L.pl_sparse_conv_chunk_form_for.argtypes = [C.c_void_p, C.c_int32, C.c_int32, C.POINTER(ChunkForm)]
+    L.pl_sparse_conv_chunk_form_for.restype = C.c_int
     L.pl_sparse_conv_set_epilogue.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.POINTER(Activation)]
     L.pl_sparse_conv_set_epilogue.restype = C.c_int
     L.pl_sparse_conv_destroy.argtypes = [C.c_void_p]

@@ -536,12 +536,12 @@ __global__ void __launch_bounds__(512, 2) ChunkMfmaKernel(PL_HEAD_PARAMS, const 
 }
 
 template <int OUT>
-hipError_t Launch(int nw, bool split, const ChunkMfmaParams& p, dim3 grid, hipStream_t s) {
+hipError_t Launch(const ChunkMfmaPlan& plan, const ChunkMfmaParams& p, dim3 grid, hipStream_t s) {
   const dim3 block(512);
-  if (split) return LaunchWithHead(ChunkSplitKernel<OUT>, grid, dim3(kSplitThreads), (size_t)2 * kSplitCells * 16 + 2048, s, p);
+  if (plan.split) return LaunchWithHead(ChunkSplitKernel<OUT>, grid, dim3(kSplitThreads), (size_t)2 * kSplitCells * 16 + 2048, s, p);
   const size_t lds = 2 * kBufCells * 16;
-  if (nw == 4) return LaunchWithHead(ChunkMfmaKernel<4, OUT>, grid, block, lds, s, p);
-  if (nw == 2) return LaunchWithHead(ChunkMfmaKernel<2, OUT>, grid, block, lds, s, p);
+  if (plan.nw == 4) return LaunchWithHead(ChunkMfmaKernel<4, OUT>, grid, block, lds, s, p);
+  if (plan.nw == 2) return LaunchWithHead(ChunkMfmaKernel<2, OUT>, grid, block, lds, s, p);
   return LaunchWithHead(ChunkMfmaKernel<1, OUT>, grid, block, lds, s, p);
 }
 
@@ -550,7 +550,27 @@ hipError_t Launch(int nw, bool split, const ChunkMfmaParams& p, dim3 grid, hipSt
 int ChunkMfmaPaddedSteps(int K) { return (K + 511) / 512 * 8; }
 bool ChunkMfmaFits(int K, int hw) { return K >= 16 && hw >= 4; }
 
-ChunkMfmaPlan PlanChunkMfma(int out_kind, int cus, int tile_positions, int K, int M, int hw, int batch) {
+// The form with twelve wavefronts, and where it is expected to be ahead of the tile width `plan` chose: a CU holds one of its workgroups, which
+// takes about 4.4 us and 1.1 us per chunk of 256 channels.  us, the width chosen / this: 2048 -> 2048 @14x14 x 16 22.0 / 19.0, 1024 -> 512 @17x17 x
+// 32 18.4 / 14.5, 900 -> 384 @13x13 x 60 15.5 / 13.0, 1024 -> 2048 @14x14 x 64 51.4 / 46.1; not taken: 192 -> 384 @17x17 x 64 (304 workgroups)
+// 12 / 15, 1024 -> 1024 @14x14 x 16 (half the CUs) 11.3 / 12.6, 1500 -> 700 @10x10 x 20 9.5 / 13.6.
+static ChunkMfmaPlan PlanChunkSplit(int K, int M, int hw, int batch) {
+  ChunkMfmaPlan p{};
+  p.split = true;
+  p.tile_quads = kSplitQuads;
+  p.tiles = (int)(((int64_t)batch * ((hw + 15) / 16) + kSplitQuads / 4 - 1) / (kSplitQuads / 4));
+  p.row_groups = ((M + 15) / 16 + kSplitRowTiles - 1) / kSplitRowTiles;
+  p.chunks = ((K + 63) / 64 + kSplitSteps - 1) / kSplitSteps;
+  p.workgroups = 8ll * p.row_groups * ((p.tiles + 7) / 8);
+  return p;
+}
+static bool SplitPays(int cus, const ChunkMfmaPlan& plan, const ChunkMfmaPlan& split) {
+  return (split.workgroups + cus - 1) / cus * (440 + 110 * split.chunks) < (plan.workgroups + cus - 1) / cus * (300 + 135 * plan.chunks);
+}
+
+ChunkMfmaPlan PlanChunkMfma(int out_kind, int cus, int tile_positions, int split, int K, int M, int hw, int batch) {
+  const bool split_fits = split != 0 && hw >= 16;
+  if (split_fits && split == 2) return PlanChunkSplit(K, M, hw, batch);
   const int qpi = (hw + 3) / 4, ksteps = (K + 63) / 64;
   const int64_t total_quads = (int64_t)batch * qpi;
   auto plan_for = [&](int nw) {
@@ -564,7 +584,7 @@ ChunkMfmaPlan PlanChunkMfma(int out_kind, int cus, int tile_positions, int K, in
     p.workgroups = 8ll * p.row_groups * ((p.tiles + 7) / 8);
     return p;
   };
-  if (tile_positions != 0) return plan_for(tile_positions / 64);
+  if (tile_positions != 0) return plan_for(tile_positions / 64);  // a width that is asked for is that of the form above
   // The tile width: a CU holds one workgroup, a workgroup takes about 3 us and 1.35 us per chunk, so the fewest rounds
   // times that, rounds being what the XCD with the most workgroups needs.  2048 -> 2048 @14x14 x 16: 256 positions 24.7 us
   // (one round of 16 chunks), 128 36.6 (two of 8), 64 44.7 (four of 4); 1024 -> 256 @14x14 x 32: 14.6, 12.7 and 9.9 (one
@@ -585,32 +605,22 @@ ChunkMfmaPlan PlanChunkMfma(int out_kind, int cus, int tile_positions, int K, in
   // 2048 -> 1024 @7x7 x 300 101 / 112.
   const bool few_rounds_count = out_kind == kOutI8 || hw % 4 != 0;
   if (few_rounds_count ? 2 * widest.workgroups > 5ll * cus : 2 * widest.workgroups >= 3ll * cus) best = widest;
+  if (split_fits) {
+    const ChunkMfmaPlan own = PlanChunkSplit(K, M, hw, batch);
+    if (SplitPays(cus, best, own)) return own;
+  }
   return best;
 }
 
-// Position tiles of the form with twelve wavefronts.
-static int64_t SplitTiles(int hw, int batch) { return ((int64_t)batch * ((hw + 15) / 16) + kSplitQuads / 4 - 1) / (kSplitQuads / 4); }
-
-// Where that form is expected to be ahead of the tile width `plan` chose: a CU holds one of its workgroups, which takes about 4.4 us and
-// 1.1 us per chunk of 256 channels.  us, the width chosen / this: 2048 -> 2048 @14x14 x 16 22.0 / 19.0, 1024 -> 512 @17x17 x 32 18.4 /
-// 14.5, 900 -> 384 @13x13 x 60 15.5 / 13.0, 1024 -> 2048 @14x14 x 64 51.4 / 46.1; not taken: 192 -> 384 @17x17 x 64 (304 workgroups) 12 / 15,
-// 1024 -> 1024 @14x14 x 16 (half the CUs) 11.3 / 12.6, 1500 -> 700 @10x10 x 20 9.5 / 13.6.
-static bool SplitPays(int cus, const ChunkMfmaPlan& plan, int K, int M, int hw, int batch) {
-  if (hw < 16) return false;
-  const int64_t groups = ((M + 15) / 16 + kSplitRowTiles - 1) / kSplitRowTiles, workgroups = 8 * groups * ((SplitTiles(hw, batch) + 7) / 8);
-  const int64_t chunks = (K + 64 * kSplitSteps - 1) / (64 * kSplitSteps);
-  return (workgroups + cus - 1) / cus * (440 + 110 * chunks) < (plan.workgroups + cus - 1) / cus * (300 + 135 * plan.chunks);
-}
-
-hipError_t LaunchChunkMfma(int out_kind, int cus, int tile_positions, const ChunkMfmaParams& p, hipStream_t stream) {
+hipError_t LaunchChunkMfma(int out_kind, int cus, int tile_positions, int split, const ChunkMfmaParams& p, hipStream_t stream) {
   if (p.batch <= 0 || p.M <= 0) return hipSuccess;
   if (!ChunkMfmaFits(p.K, p.hw)) return hipErrorInvalidValue;
   const int64_t positions = (int64_t)p.batch * p.hw;
   // tensor offsets are kept in 32 bits
   if (positions * p.K >= (1ll << 31) || positions >= (1ll << 31) - 512) return hipErrorInvalidValue;
-  const ChunkMfmaPlan plan = PlanChunkMfma(out_kind, cus, tile_positions, p.K, p.M, p.hw, p.batch);
+  const ChunkMfmaPlan plan = PlanChunkMfma(out_kind, cus, tile_positions, split, p.K, p.M, p.hw, p.batch);
   ChunkMfmaParams q = p;
-  q.qpi = (p.hw + 3) / 4;
+  q.qpi = plan.split ? 4 * ((p.hw + 15) / 16) : (p.hw + 3) / 4;
   q.quad_aligned = p.hw % 4 == 0;
   q.total_quads = (uint32_t)p.batch * (uint32_t)q.qpi;
   q.row_tiles = (p.M + 15) / 16;
@@ -619,27 +629,15 @@ hipError_t LaunchChunkMfma(int out_kind, int cus, int tile_positions, const Chun
   q.tile_quads = plan.tile_quads;
   q.tiles = plan.tiles;
   q.chunks = plan.chunks;
-  const int nw = plan.nw;
-  int64_t wgs = plan.workgroups;
-  const bool split = (tile_positions == 0 || tile_positions == 256) && SplitPays(cus, plan, p.K, p.M, p.hw, p.batch);
-  if (split) {
-    q.qpi = 4 * ((p.hw + 15) / 16);
-    q.total_quads = (uint32_t)p.batch * (uint32_t)q.qpi;
-    q.tile_quads = kSplitQuads;
-    q.tiles = (int)SplitTiles(p.hw, p.batch);
-    q.row_groups = (q.row_tiles + kSplitRowTiles - 1) / kSplitRowTiles;
-    q.chunks = ((p.K + 63) / 64 + kSplitSteps - 1) / kSplitSteps;
-    wgs = 8ll * q.row_groups * ((q.tiles + 7) / 8);
-  }
-  if (wgs > (1ll << 30)) return hipErrorInvalidValue;
-  const dim3 grid((uint32_t)wgs);
+  if (plan.workgroups > (1ll << 30)) return hipErrorInvalidValue;
+  const dim3 grid((uint32_t)plan.workgroups);
   switch (out_kind) {
     case kOutF32:
-      return Launch<kOutF32>(nw, split, q, grid, stream);
+      return Launch<kOutF32>(plan, q, grid, stream);
     case kOutI8:
-      return Launch<kOutI8>(nw, split, q, grid, stream);
+      return Launch<kOutI8>(plan, q, grid, stream);
     case kOutAcc32:
-      return Launch<kOutAcc32>(nw, split, q, grid, stream);
+      return Launch<kOutAcc32>(plan, q, grid, stream);
     default:
       return hipErrorInvalidValue;
   }

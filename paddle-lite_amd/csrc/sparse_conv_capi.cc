@@ -210,6 +210,7 @@ struct pl_sparse_conv_handle {
   DevBuf wchunk;            // dense 16x64 tiles of the kernel that takes the channels chunk by chunk
   int chunk_mfma = 1;       // that kernel: 0 never, 1 by the rule, 2 whenever the shape allows
   int chunk_positions = 0;  // positions per tile of that kernel; 0 = chosen per problem
+  int chunk_split = 1;      // its form with wavefronts of its own for the activations: 0 never, 1 by the rule, 2 whenever the shape allows
   bool walk_asked = false, block_asked = false, image_asked = false;  // a tuning field names a form of the plain walk / the block kernel / an image kernel
   int mfma_stream = 1;      // streaming block MFMA: 0 never, 1 when the shape suits it, 2 whenever the shape allows
   int mfma_i8_wide = 1;
@@ -959,7 +960,7 @@ bool ChunkMfmaBeatsBlock(const pl_sparse_conv_handle* h, int batch, int im_size,
     // 9 images, 65 -> 160 @12x12 5.2 / 9.0; 125 -> 227 @18x18 6.2 / 5.2 at 17 (88 tiles).
     return ic % 16 != 0 && tiles * 4 <= cus;
   }
-  const auto workgroups = [&] { return pl::PlanChunkMfma(OutKind(h->kind), cus, h->chunk_positions, ic, oc, im_size, batch).workgroups; };
+  const auto workgroups = [&] { return pl::PlanChunkMfma(OutKind(h->kind), cus, h->chunk_positions, 0, ic, oc, im_size, batch).workgroups; };
   // the block kernel skips blocks of 32 x 32 zeros and this one does not
   const int64_t blocks = static_cast<int64_t>(h->row_blocks) * h->ksteps;
   const bool dense = h->blocks_present * 4 >= blocks * 3;
@@ -985,7 +986,7 @@ bool ChunkMfmaBeatsBlock(const pl_sparse_conv_handle* h, int batch, int im_size,
   // Two workgroups of the block kernel per CU: with four-byte output it is ahead once there are many tiles, with one-byte output
   // where many are met by tiles of this kernel that stay empty: 2048 -> 2048 @14x14 x 64 (2048 halves) 87.6 / 96.6, 1472 -> 812
   // @12x12 x 118 (1652, two fifths empty) 1.5; over 250 calls of 1024 halves and more without that 0.92 at the median, 1.23 at most.
-  const int64_t halves = 2ll * pl::PlanChunkMfma(OutKind(h->kind), cus, 256, ic, oc, im_size, batch).tiles * CeilDiv(oc, 128);
+  const int64_t halves = 2ll * pl::PlanChunkMfma(OutKind(h->kind), cus, 256, 0, ic, oc, im_size, batch).tiles * CeilDiv(oc, 128);
   const bool full = halves * 3 <= tiles * 4;
   if (one_byte) return dense ? full || halves <= 4 * cus : workgroups() <= 3 * cus;
   if (ic <= 640) {
@@ -1100,12 +1101,12 @@ int pl_sparse_conv_prepare(const pl_sparse_conv_desc* desc, pl_sparse_conv_handl
   *out_handle = nullptr;
   // callers compiled against a header without the tuning fields, or without the last ones, pass what they know
   constexpr size_t kNoTuning = offsetof(pl_sparse_conv_desc, tuning), kNoChunkTuning = kNoTuning + offsetof(pl_sparse_conv_tuning, chunk_mfma),
-                   kNoFloatTuning = kNoTuning + offsetof(pl_sparse_conv_tuning, float_mfma);
-  if (desc->struct_size != sizeof(pl_sparse_conv_desc) && desc->struct_size != kNoFloatTuning && desc->struct_size != kNoChunkTuning && desc->struct_size != kNoTuning)
+                   kNoFloatTuning = kNoTuning + offsetof(pl_sparse_conv_tuning, float_mfma), kNoSplitTuning = kNoTuning + offsetof(pl_sparse_conv_tuning, chunk_split);
+  if (desc->struct_size != sizeof(pl_sparse_conv_desc) && desc->struct_size != kNoSplitTuning && desc->struct_size != kNoFloatTuning && desc->struct_size != kNoChunkTuning && desc->struct_size != kNoTuning)
     return Fail(PL_ERR_BAD_ARG, "pl_sparse_conv_desc size mismatch (%u vs %zu)", desc->struct_size, sizeof(pl_sparse_conv_desc));
   pl_sparse_conv_tuning tune{};
   std::memcpy(&tune, reinterpret_cast<const char*>(desc) + kNoTuning, std::min<size_t>(desc->struct_size - kNoTuning, sizeof(tune)));
-  for (int32_t sw : {tune.mfma_stream, tune.mfma_sub_tiles, tune.walk_tiled, tune.walk_chunked, tune.image_tr_regroup, tune.walk_pairs, tune.chunk_mfma, tune.float_mfma})
+  for (int32_t sw : {tune.mfma_stream, tune.mfma_sub_tiles, tune.walk_tiled, tune.walk_chunked, tune.image_tr_regroup, tune.walk_pairs, tune.chunk_mfma, tune.float_mfma, tune.chunk_split})
     if (sw < PL_TUNE_RULE || sw > PL_TUNE_ALWAYS) return Fail(PL_ERR_BAD_ARG, "a tuning switch is not PL_TUNE_RULE, PL_TUNE_NEVER or PL_TUNE_ALWAYS");
   if (tune.chunk_positions != 0 && tune.chunk_positions != 64 && tune.chunk_positions != 128 && tune.chunk_positions != 256) return Fail(PL_ERR_BAD_ARG, "tuning.chunk_positions must be 0, 64, 128 or 256");
   if (tune.float_mfma_rows != 0 && tune.float_mfma_rows != 64 && tune.float_mfma_rows != 128 && tune.float_mfma_rows != 256) return Fail(PL_ERR_BAD_ARG, "tuning.float_mfma_rows must be 0, 64, 128 or 256");
@@ -1155,6 +1156,7 @@ int pl_sparse_conv_prepare(const pl_sparse_conv_desc* desc, pl_sparse_conv_handl
   h->walk_chunked = sw(tune.walk_chunked);
   h->chunk_mfma = sw(tune.chunk_mfma);
   h->chunk_positions = tune.chunk_positions;
+  h->chunk_split = sw(tune.chunk_split);
   // a handle that asks for a walk, or for a form of one, keeps its calls there
   const bool float_walk_asked = desc->algo != PL_ALGO_AUTO || tune.walk_tiled != PL_TUNE_RULE || tune.walk_split != 0 || tune.walk_chunked != PL_TUNE_RULE || tune.chunk_walk_groups != 0 || tune.walk_tile != 0 ||
                                 tune.walk_threads != 0 || tune.walk_slices != 0 || tune.walk_pairs != PL_TUNE_RULE;
@@ -1483,7 +1485,7 @@ int pl_sparse_conv_run(pl_sparse_conv_handle* h, const void* x_dev, void* out_de
     p.hw = im_size;
     p.batch = batch;
     p.act = h->act;
-    e = pl::LaunchChunkMfma(OutKind(h->kind), std::max(1, h->wg_slots_default / 2), h->chunk_positions, p, s);
+    e = pl::LaunchChunkMfma(OutKind(h->kind), std::max(1, h->wg_slots_default / 2), h->chunk_positions, h->chunk_split, p, s);
   } else if (call_algo == PL_ALGO_IMAGE_MFMA) {
     // larger maps of a multiple of 196 positions are taken slab by slab by the kernel with one row tile per wavefront
     const bool slabs = h->wtiles_rows.ptr != nullptr && (h->image_kernel == 0 || h->image_kernel == 3) && pl::ImageRowsSlabFits(h->oc, h->ic, im_size);
@@ -1685,6 +1687,16 @@ int pl_sparse_conv_algo_for(const pl_sparse_conv_handle* h, int32_t batch, int32
   if (!h) return Fail(PL_ERR_BAD_ARG, "null handle");
   if (batch < 0 || im_size <= 0) return Fail(PL_ERR_BAD_ARG, "batch must be >= 0 and im_size > 0");
   return AlgoForCall(h, batch, im_size, true);
+}
+
+int pl_sparse_conv_chunk_form_for(const pl_sparse_conv_handle* h, int32_t batch, int32_t im_size, pl_sparse_conv_chunk_form* form) {
+  if (!form) return Fail(PL_ERR_BAD_ARG, "null argument");
+  const int algo = pl_sparse_conv_algo_for(h, batch, im_size);
+  if (algo < 0) return algo;
+  if (algo != PL_ALGO_CHUNK_MFMA || !h->int8) return Fail(PL_ERR_UNSUPPORTED, "the call is not one of an int8 handle that takes the channels chunk by chunk");
+  const pl::ChunkMfmaPlan plan = pl::PlanChunkMfma(OutKind(h->kind), std::max(1, h->wg_slots_default / 2), h->chunk_positions, h->chunk_split, h->ic, h->oc, im_size, batch);
+  *form = plan.split ? pl_sparse_conv_chunk_form{256, 128, 1} : pl_sparse_conv_chunk_form{128, 64 * plan.nw, 0};
+  return PL_OK;
 }
 
 int pl_sparse_conv_set_epilogue(pl_sparse_conv_handle* h, const float* scale, const float* bias, const pl_activation* act) {

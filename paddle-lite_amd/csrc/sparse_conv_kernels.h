@@ -382,19 +382,21 @@ struct ChunkMfmaParams {
   DevAct act;
 };
 
-// How a call is divided: a tile width, the workgroups it makes (of 128 rows x one tile; a CU holds one at a time) and
-// the chunks of channels each of them takes.
+// How a call is divided: a tile width, the workgroups it makes (of 128 rows x one tile, or 256 in the form with wavefronts of its own for the
+// activations; a CU holds one at a time) and the chunks of channels each of them takes.
 struct ChunkMfmaPlan {
-  int nw;  // position quads per tile / 16
+  bool split;  // that form: 128 positions, 256 channels a chunk
+  int nw;      // else: position quads per tile / 16
   int tile_quads, tiles, row_groups, chunks;
   int64_t workgroups;
 };
 
 int ChunkMfmaPaddedSteps(int K);  // 64-channel steps of the weight tiles: whole chunks of the widest kind
 bool ChunkMfmaFits(int K, int hw);
-// tile_positions: positions of a tile (64, 128 or 256), 0 = chosen by the number of CUs
-ChunkMfmaPlan PlanChunkMfma(int out_kind, int cus, int tile_positions, int K, int M, int hw, int batch);
-hipError_t LaunchChunkMfma(int out_kind, int cus, int tile_positions, const ChunkMfmaParams& p, hipStream_t stream);
+// tile_positions: positions of a tile (64, 128 or 256), 0 = chosen by the number of CUs.  split: the form with wavefronts of its own for the
+// activations, on maps of 16 positions and more: 0 never, 1 where it is expected to be ahead, 2 always
+ChunkMfmaPlan PlanChunkMfma(int out_kind, int cus, int tile_positions, int split, int K, int M, int hw, int batch);
+hipError_t LaunchChunkMfma(int out_kind, int cus, int tile_positions, int split, const ChunkMfmaParams& p, hipStream_t stream);
 
 // Image MFMA SpMM (int8, image_mfma_kernels.hip): one workgroup per (image,
 // 128 output rows) with the whole image's activations in LDS.

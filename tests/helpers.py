@@ -155,7 +155,7 @@ def forced_algo(algo):
 def algo_times(case, warm=100, steps=500, repeats=3, max_sets=24, rotation_bytes=320 << 20, chunk_positions=()):
     """Device time per launch (us, events inside pl_sparse_conv_run_sequence) of an int8 case with the
     algorithm left to the handle ("auto") and with each algorithm forced, the one that takes the channels chunk
-    by chunk also with each of the tile widths in `chunk_positions`; an algorithm the shape is outside of is
+    by chunk also with each of the tile widths in `chunk_positions` ("split": the form that tuning.chunk_split names); an algorithm the shape is outside of is
     left out.  Every handle's output on the first two images is compared with the oracle before it is
     timed.  Buffer sets rotate (up to `max_sets` of them, `rotation_bytes` in all); the runs of the handles are
     interleaved `repeats` times and the smallest time of each is kept, so that a clock ramp or another
@@ -180,7 +180,8 @@ def algo_times(case, warm=100, steps=500, repeats=3, max_sets=24, rotation_bytes
     handles = {}
     wanted = [("auto", capi.ALGO_AUTO, forced_algo(capi.ALGO_AUTO))] + [(n, a, forced_algo(a)) for a, n in sorted(ALGO_NAMES.items())]
     for width in chunk_positions:
-        wanted.append(("chunk_mfma_%d" % width, capi.ALGO_CHUNK_MFMA, dict(algo=capi.ALGO_AUTO, tuning=capi.tuning(chunk_mfma=capi.TUNE_ALWAYS, chunk_positions=width))))
+        form = dict(chunk_split=capi.TUNE_ALWAYS) if width == "split" else dict(chunk_positions=width)
+        wanted.append(("chunk_mfma_%s" % width, capi.ALGO_CHUNK_MFMA, dict(algo=capi.ALGO_AUTO, tuning=capi.tuning(chunk_mfma=capi.TUNE_ALWAYS, **form))))
     for name, algo, how in wanted:
         try:
             k, _ = make_kernel(case, **how)

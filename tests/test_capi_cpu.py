@@ -37,7 +37,7 @@ def test_struct_layout_matches_header(tmp_path):
     import shutil
     import subprocess
 
-    structs = {"pl_activation": capi.Activation, "pl_sparse_conv_tuning": capi.Tuning, "pl_sparse_conv_desc": capi.Desc, "pl_sparse_conv_info": capi.Info, "pl_dwconv_desc": capi.DwConvDesc}
+    structs = {"pl_activation": capi.Activation, "pl_sparse_conv_tuning": capi.Tuning, "pl_sparse_conv_desc": capi.Desc, "pl_sparse_conv_info": capi.Info, "pl_sparse_conv_chunk_form": capi.ChunkForm, "pl_dwconv_desc": capi.DwConvDesc}
     assert C.sizeof(capi.Activation) == 24
     gcc = shutil.which("gcc")
     if gcc is None:
@@ -65,7 +65,7 @@ def test_struct_layout_matches_header(tmp_path):
 
 
 def test_descriptor_sizes_of_older_headers_are_taken():
-    """A caller compiled against a header without the tuning fields, or without the last two of them, passes the size it
+    """A caller compiled against a header without the tuning fields, or without the last ones of them, passes the size it
     knows; any other size is refused."""
     L = capi.lib()
     w = pla.detect_and_pack((np.arange(8 * 16).reshape(8, 16) % 3).astype(np.float32), 4)
@@ -75,8 +75,11 @@ def test_descriptor_sizes_of_older_headers_are_taken():
     d.oc_nonzeros, d.diffs, d.n_diffs = w.oc_nonzeros.ctypes.data, w.diffs.ctypes.data, w.diffs.size
     d.tuning.chunk_positions = 100  # refused where it is read at all
     tuning = capi.Desc.tuning.offset
-    for size, taken in ((tuning, True), (tuning + capi.Tuning.chunk_mfma.offset, True), (C.sizeof(capi.Desc), False), (tuning + 4, False), (C.sizeof(capi.Desc) - 4, False)):
+    for size, taken in ((tuning, True), (tuning + capi.Tuning.chunk_mfma.offset, True), (C.sizeof(capi.Desc), False), (tuning + 4, False), (C.sizeof(capi.Desc) - 4, False),
+                        (tuning + capi.Tuning.float_mfma.offset, True), (tuning + capi.Tuning.chunk_split.offset, True), (C.sizeof(capi.Desc), True)):
         d.struct_size = size
+        if size == tuning + capi.Tuning.float_mfma.offset:
+            d.tuning.chunk_positions = 0  # read in these
         h = C.c_void_p()
         rc = L.pl_sparse_conv_prepare(C.byref(d), C.byref(h))
         assert (rc in (capi.PL_OK, capi.PL_ERR_NO_DEVICE)) == taken and (taken or rc == capi.PL_ERR_BAD_ARG), (size, rc, capi.last_error())

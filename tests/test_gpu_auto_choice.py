@@ -64,9 +64,9 @@ def check_layer(batch, ic, oc, side, out, sparsity=0.85, blocked=False):
     if blocked:  # whole 32 x 32 blocks of zeros
         keep = np.random.RandomState(ic).random_sample((oc // 32, ic // 32)) >= sparsity
         case.dense = (workloads._int8_nonzero(np.random.RandomState(oc), (oc, ic)) * np.kron(keep, np.ones((32, 32), dtype=bool))).astype(np.int8)
-    times, picked = algo_times(case, warm=30, steps=100, chunk_positions=(64, 128, 256))
+    times, picked = algo_times(case, warm=30, steps=100, chunk_positions=(64, 128, 256, "split"))
     best_name, best = min(((k, v) for k, v in times.items() if k != "auto"), key=lambda kv: kv[1])
     if times["auto"] > 1.15 * best + 0.3:
-        times, picked = algo_times(case, warm=60, steps=200, repeats=5, chunk_positions=(64, 128, 256))
+        times, picked = algo_times(case, warm=60, steps=200, repeats=5, chunk_positions=(64, 128, 256, "split"))
         best_name, best = min(((k, v) for k, v in times.items() if k != "auto"), key=lambda kv: kv[1])
     assert times["auto"] <= 1.15 * best + 0.3, "auto (%s) %.2f us, %s %.2f us" % (picked, times["auto"], best_name, best)

@@ -1,7 +1,8 @@
 """The int8 kernel that takes the input channels chunk by chunk, against the CPU oracle through the C ABI, bit for
-bit, at each of its three tile widths: channel counts around a group of 16, a step of 64 and a chunk, one to 25 chunks
+bit, at each of its three tile widths and in the form with wavefronts of its own for the activations: channel counts around a group of 16, a step of 64 and a chunk, one to 25 chunks
 (each way the loop over the chunks can end), rows around a tile of 16 and a group of 128, maps of four positions and more
 with every remainder modulo four, tiles of whole images and tiles that cross images; tensors off the 16-byte grid."""
+import ctypes as C
 import sys
 
 import numpy as np
@@ -28,11 +29,26 @@ def chunk_case(shape, kind, act, paired, seed):
     return case
 
 
+def chunk_form(kernel, batch, im_size):
+    """(rows, positions, split) of the call's workgroups."""
+    form = capi.ChunkForm()
+    capi.check(capi.lib().pl_sparse_conv_chunk_form_for(kernel._handle, batch, im_size, C.byref(form)))
+    return form.rows, form.positions, form.split
+
+
 def chunk_kernel(case, width):
-    """A kernel that runs chunk by chunk on tiles of `width` positions (0: the rule's), which the library confirms."""
-    kernel, _ = make_kernel(case, tuning=capi.tuning(chunk_mfma=capi.TUNE_ALWAYS, chunk_positions=width))
+    """A kernel that runs chunk by chunk on tiles of `width` positions (0: the rule's, "split": the form with wavefronts of its own for the
+    activations), which the library confirms."""
+    how = dict(chunk_split=capi.TUNE_ALWAYS) if width == "split" else dict(chunk_positions=width)
+    kernel, _ = make_kernel(case, tuning=capi.tuning(chunk_mfma=capi.TUNE_ALWAYS, **how))
     assert capi.lib().pl_sparse_conv_algo_for(kernel._handle, case.batch, case.im_size) == capi.ALGO_CHUNK_MFMA
+    if width != 0:
+        assert chunk_form(kernel, case.batch, case.im_size) == ((256, 128, 1) if width == "split" else (128, width, 0))
     return kernel
+
+
+def widths(case):
+    return WIDTHS + (("split",) if case.im_size >= 16 else ())
 
 
 def check(shape, kind, act, paired, seed):
@@ -42,11 +58,11 @@ def check(shape, kind, act, paired, seed):
     few = case.x[:1] if batch * h * w > 1000 else case.x
     want = run_oracle(case, oracle_pack(case), x=few)
     last = run_oracle(case, oracle_pack(case), x=case.x[-1:]) if len(few) != batch else None
-    for width in (0,) + WIDTHS:
+    for width in (0,) + widths(case):
         got = run_hip(case, kernel=chunk_kernel(case, width))
-        assert_same(case, got[:len(few)], want, "chunk %s %s, width %d" % (shape, kind, width))
+        assert_same(case, got[:len(few)], want, "chunk %s %s, width %s" % (shape, kind, width))
         if last is not None:  # it ends the last tile
-            assert_same(case, got[-1:], last, "chunk %s %s, width %d, last image" % (shape, kind, width))
+            assert_same(case, got[-1:], last, "chunk %s %s, width %s, last image" % (shape, kind, width))
 
 
 @pytest.mark.parametrize("kind", sorted(KINDS))
@@ -61,7 +77,7 @@ def test_large_calls(shape, kind):
     check(shape, kind, AP("relu"), False, shape[1])
 
 
-# The form of the widest tile with wavefronts of its own for the activations (256 rows x eight blocks of 16 positions, 256 channels a chunk):
+# The form with wavefronts of its own for the activations (256 rows x eight blocks of 16 positions, 256 channels a chunk):
 # channels around a group of 16, a step of 64 and a chunk, each number of chunks that its loops can end with, rows around a tile of 16, a
 # wavefront's 32 and a workgroup's 256, maps of one block, of blocks that overlap by 1 - 15 positions and of more than a tile, tiles that cross
 # images and are not full.
@@ -75,8 +91,39 @@ def test_wavefronts_of_their_own_for_the_activations(shape, kind):
     print("CASE chunk split", shape, kind, file=sys.stderr, flush=True)
     case = chunk_case(shape, kind, [AP("relu"), AP("leaky_relu", Leaky_relu_alpha=0.1)][shape[1] % 2], shape[2] % 2 == 0, shape[1])
     want = run_oracle(case, oracle_pack(case))
-    for width in (0, 256):
-        assert_same(case, run_hip(case, kernel=chunk_kernel(case, width)), want, "chunk split %s %s, width %d" % (shape, kind, width))
+    for width in (0, "split"):
+        assert_same(case, run_hip(case, kernel=chunk_kernel(case, width)), want, "chunk split %s %s, width %s" % (shape, kind, width))
+
+
+# (batch, ic, oc, h, w) and the form the rule takes on 256 CUs: the widest tiles with four to eight chunks of 128 channels, on maps larger and
+# smaller than a tile
+RULE = [(121, 576, 320, 18, 18, (128, 256, 0)), (107, 420, 112, 18, 18, (128, 256, 0)), (120, 992, 672, 9, 9, (128, 256, 0)), (16, 500, 128, 35, 31, (128, 128, 0)), (16, 2048, 2048, 14, 14, (256, 128, 1)),
+        (60, 900, 384, 13, 13, (256, 128, 1)), (1, 512, 512, 14, 14, (128, 64, 0))]
+
+
+@pytest.mark.parametrize("kind", ["fp32out", "int8out"])
+@pytest.mark.parametrize("call", RULE, ids=lambda c: "x".join(map(str, c[:5])))
+def test_the_form_the_rule_takes(call, kind):
+    """By the rule, with the form that the library names, and forced, where that is a tile width: the bits of the block kernel, and of the
+    oracle on the first and the last image."""
+    shape, form = call[:5], call[5]
+    print("CASE chunk rule", shape, kind, file=sys.stderr, flush=True)
+    case = chunk_case(shape, kind, AP("relu"), False, shape[1])
+    kernel = chunk_kernel(case, 0)
+    assert chunk_form(kernel, case.batch, case.im_size) == form
+    got = run_hip(case, kernel=kernel)
+    for image in (0, shape[0] - 1):
+        assert_same(case, got[image:image + 1], run_oracle(case, oracle_pack(case), x=case.x[image:image + 1]), "chunk rule %s %s" % (shape, kind))
+    assert_same(case, got, run_hip(case, algo=capi.ALGO_BLOCK_MFMA), "chunk rule %s %s, block kernel" % (shape, kind))
+    # a width that a field names is that of the form with three widths, and the switch keeps the other one out
+    for width in WIDTHS:
+        assert chunk_form(chunk_kernel(case, width), case.batch, case.im_size) == (128, width, 0)
+    never, _ = make_kernel(case, tuning=capi.tuning(chunk_mfma=capi.TUNE_ALWAYS, chunk_split=capi.TUNE_NEVER))
+    assert chunk_form(never, case.batch, case.im_size)[2] == 0
+    assert_same(case, run_hip(case, kernel=never), got, "chunk rule %s %s, chunk_split NEVER" % (shape, kind))
+    # calls of other kernels have none
+    block, _ = make_kernel(case, algo=capi.ALGO_BLOCK_MFMA)
+    assert capi.lib().pl_sparse_conv_chunk_form_for(block._handle, case.batch, case.im_size, C.byref(capi.ChunkForm())) == capi.PL_ERR_UNSUPPORTED
 
 
 # maps with every remainder modulo four, a last tile that is not full and rows that end inside a tile
@@ -91,7 +138,7 @@ def test_tensors_off_the_grid_and_their_surroundings(shape, kind):
     want = run_oracle(case, oracle_pack(case))
     batch, ic, oc, h, w = shape
     fill, dtype = (77, torch.int8) if kind == "int8out" else (77, torch.int32) if kind == "acc32" else (77.0, torch.float32)
-    for width in WIDTHS:
+    for width in widths(case):
         kernel = chunk_kernel(case, width)
         for shift in (1, 2, 3):
             guard = 64 + shift
@@ -101,7 +148,7 @@ def test_tensors_off_the_grid_and_their_surroundings(shape, kind):
             kernel.Run(x[guard:guard + case.x.size].view(case.x.shape), out[guard:guard + want.size].view(want.shape))
             host = out.cpu().numpy()
             assert (host[:guard] == fill).all() and (host[guard + want.size:] == fill).all(), (width, shift)
-            assert_same(case, host[guard:guard + want.size].reshape(want.shape), want, "chunk off the grid %s %s %d %d" % (shape, kind, width, shift))
+            assert_same(case, host[guard:guard + want.size].reshape(want.shape), want, "chunk off the grid %s %s %s %d" % (shape, kind, width, shift))
 
 
 def test_the_choice_is_reported_and_can_be_overridden():
