@@ -181,6 +181,11 @@ typedef struct pl_sparse_conv_tuning {
   int32_t chunk_split;       /* (switch) the kernel of chunk_mfma with wavefronts
                                 of their own for the activations (256 rows x
                                 128 positions; maps of 16 positions and more)  */
+  int32_t float_mfma_split;  /* (switch) the kernel of float_mfma, fp32, with
+                                wavefronts of their own for the inputs (256 rows
+                                x 64 positions); by the rule, a number of rows
+                                that float_mfma_rows names is that of the form
+                                without                                        */
 } pl_sparse_conv_tuning;
 
 /* Everything PrepareForRun() knows.  All pointers are HOST pointers and are
@@ -274,12 +279,13 @@ int pl_sparse_conv_get_info(const pl_sparse_conv_handle* handle,
 int pl_sparse_conv_algo_for(const pl_sparse_conv_handle* handle, int32_t batch,
                             int32_t im_size);
 
-/* How a call for which that is PL_ALGO_CHUNK_MFMA is divided; of an int8
- * handle (else, or where it is another algorithm, PL_ERR_UNSUPPORTED). */
+/* How a call for which that is PL_ALGO_CHUNK_MFMA is divided (where it is
+ * another algorithm, PL_ERR_UNSUPPORTED). */
 typedef struct pl_sparse_conv_chunk_form {
   int32_t rows;          /* of a workgroup's tile                           */
   int32_t positions;
-  int32_t split;         /* 1 = the form that tuning.chunk_split names      */
+  int32_t split;         /* 1 = the form that tuning.chunk_split or
+                            float_mfma_split names                          */
 } pl_sparse_conv_chunk_form;
 int pl_sparse_conv_chunk_form_for(const pl_sparse_conv_handle* handle,
                                   int32_t batch, int32_t im_size,

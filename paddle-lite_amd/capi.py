@@ -77,6 +77,7 @@ class Tuning(C.Structure):
         ("float_mfma", C.c_int32),
         ("float_mfma_rows", C.c_int32),
         ("chunk_split", C.c_int32),
+        ("float_mfma_split", C.c_int32),
     ]
 
 

@@ -1032,7 +1032,7 @@ bool FloatMfmaFits(bool f32, int K, int M, int hw, int64_t positions) {
 // fastest on average.  Many rows per workgroup fetch the inputs the fewest times, few rows let small calls fill the chip
 // and halve the chain of a chunk: 64 x 1024 -> 1024 @7x7
 // fp32 256 rows 37.3, 128 rows 29.4, 64 rows 40.9; 64 x 512 -> 512 @14x14 25.9, 34.1, 47.7; one image 96 -> 192 @56x56 8.0, 6.9, 6.4.
-FloatMfmaPlan PlanFloatMfma(bool f32, int cus, int row_blocks, int K, int M, int hw, int batch) {
+static FloatMfmaPlan PlanRows(bool f32, int cus, int row_blocks, int K, int M, int hw, int batch) {
   const int64_t tiles = ((int64_t)batch * ((hw + 3) / 4) + kQuads - 1) / kQuads;
   const int chunks = (K + kChunk - 1) / kChunk;
   // us: a launch, a chunk of it; a full chip and a chunk of it; every workgroup beyond one per CU and a chunk of it (fp16,
@@ -1056,6 +1056,7 @@ FloatMfmaPlan PlanFloatMfma(bool f32, int cus, int row_blocks, int K, int M, int
     FloatMfmaPlan p{};
     p.wr = wr;
     p.row_groups = ((M + 31) / 32 + wr - 1) / wr;
+    p.tiles = (int)tiles;
     p.workgroups = 8ll * p.row_groups * ((tiles + 7) / 8);
     const Cost& c = f32 ? kF32[M <= 64 && wr == 2 ? 3 : i] : kF16[hw % 4 != 0][i];
     const int64_t used = f32 ? p.workgroups : p.row_groups * tiles;  // fp16: without those of the last eight tiles that return at once
@@ -1067,17 +1068,38 @@ FloatMfmaPlan PlanFloatMfma(bool f32, int cus, int row_blocks, int K, int M, int
   return best;
 }
 
-// The form with wavefronts of their own for the inputs, us: fitted to 150 random calls in fp32 that it makes one round of workgroups of (64 - 2048
+// The form with wavefronts of their own for the inputs (fp32).  us: fitted to 150 random calls that it makes one round of workgroups of (64 - 2048
 // channels, 33 - 2048 rows), within 7 % for two of three, and 0.8 for the sums that wait.
-static double SplitMicroseconds(int cus, int64_t workgroups, int K) {
-  const double chunks = (K + kSplitChunk - 1) / kSplitChunk, full = (double)workgroups / cus;
-  return 4.5 + 1.57 * chunks + full * (1.73 + 0.71 * chunks);
+static FloatMfmaPlan PlanFloatSplit(int cus, int K, int M, int hw, int batch) {
+  FloatMfmaPlan p{};
+  p.wr = kSplitRowBlocks;
+  p.split = true;
+  p.row_groups = ((M + 31) / 32 + kSplitRowBlocks - 1) / kSplitRowBlocks;
+  p.tiles = (int)(((int64_t)batch * ((hw + 3) / 4) + kSplitQuads - 1) / kSplitQuads);
+  p.workgroups = 8ll * p.row_groups * ((p.tiles + 7) / 8);
+  const double chunks = (K + kSplitChunk - 1) / kSplitChunk, full = (double)p.workgroups / cus;
+  p.us = 4.5 + 1.57 * chunks + full * (1.73 + 0.71 * chunks);
+  return p;
 }
 
-hipError_t LaunchFloatMfma(bool f32, int cus, int row_blocks, const FloatMfmaParams& p, hipStream_t stream) {
+FloatMfmaPlan PlanFloatMfma(bool f32, int cus, int row_blocks, int split, int K, int M, int hw, int batch) {
+  if (f32 && split == 2) return PlanFloatSplit(cus, K, M, hw, batch);
+  const FloatMfmaPlan plan = PlanRows(f32, cus, row_blocks, K, M, hw, batch);
+  // One round of workgroups of 256 rows x 64 positions where that is expected to take 0.88 of the time (of 11 of 150 random calls at 0.97 two were
+  // slower, 1536 -> 352 @11x11 x 37 31.5 / 33.4, the others 0.85 - 0.97); over more rounds it is 1.1 times as long
+  // (64 x 512 -> 512 @14x14 23.9 / 26.2).  Not in place of 64 rows per workgroup, whose four sums per output are closer to 64 bits (1024
+  // channels 1.3e-7), nor of up to 384 channels, where halves of the sums would not be chunks, nor of a number of rows that is asked for.
+  if (f32 && split == 1 && row_blocks == 0 && plan.wr >= 4 && K > 3 * kSplitChunk) {
+    const FloatMfmaPlan own = PlanFloatSplit(cus, K, M, hw, batch);
+    if (own.workgroups <= cus && own.us < 0.88 * plan.us) return own;
+  }
+  return plan;
+}
+
+hipError_t LaunchFloatMfma(bool f32, int cus, int row_blocks, int split, const FloatMfmaParams& p, hipStream_t stream) {
   if (p.batch <= 0 || p.M <= 0) return hipSuccess;
   if (!FloatMfmaFits(f32, p.K, p.M, p.hw, (int64_t)p.batch * p.hw)) return hipErrorInvalidValue;
-  const FloatMfmaPlan plan = PlanFloatMfma(f32, cus, row_blocks, p.K, p.M, p.hw, p.batch);
+  const FloatMfmaPlan plan = PlanFloatMfma(f32, cus, row_blocks, split, p.K, p.M, p.hw, p.batch);
   FloatMfmaParams q = p;
   q.qpi = (p.hw + 3) / 4;
   q.quad_aligned = p.hw % 4 == 0;
@@ -1086,21 +1108,10 @@ hipError_t LaunchFloatMfma(bool f32, int cus, int row_blocks, const FloatMfmaPar
   q.row_groups = plan.row_groups;
   q.chunks = (p.K + kChunk - 1) / kChunk;
   q.padded_ksteps = FloatMfmaPaddedSteps(p.K);
-  q.tiles = (int)((q.total_quads + kQuads - 1) / kQuads);
+  q.tiles = plan.tiles;
   if (plan.workgroups > (1ll << 30)) return hipErrorInvalidValue;
-  // One round of workgroups of 256 rows x 64 positions where that is expected to take 0.88 of the time (of 11 of 150 random calls at 0.97 two were
-  // slower, 1536 -> 352 @11x11 x 37 31.5 / 33.4, the others 0.85 - 0.97); over more rounds it is 1.1 times as long
-  // (64 x 512 -> 512 @14x14 23.9 / 26.2).  Not in place of 64 rows per workgroup, whose four sums per output are closer to 64 bits (1024
-  // channels 1.3e-7), nor of up to 384 channels, where halves of the sums would not be chunks.
-  if (f32 && row_blocks == 0 && plan.wr >= 4 && p.K > 3 * kSplitChunk) {
-    const int groups = (q.row_blocks + kSplitRowBlocks - 1) / kSplitRowBlocks, tiles = (int)((q.total_quads + kSplitQuads - 1) / kSplitQuads);
-    const int64_t workgroups = 8ll * groups * ((tiles + 7) / 8);
-    if (workgroups <= cus && SplitMicroseconds(cus, workgroups, p.K) < 0.88 * plan.us) {
-      q.row_groups = groups, q.tiles = tiles;
-      return LaunchSplit(q, dim3((uint32_t)workgroups), stream);
-    }
-  }
   const dim3 grid((uint32_t)plan.workgroups);
+  if (plan.split) return LaunchSplit(q, grid, stream);
   switch (plan.wr) {
     case 8:
       return f32 ? Launch<8, true>(q, grid, stream) : Launch<8, false>(q, grid, stream);

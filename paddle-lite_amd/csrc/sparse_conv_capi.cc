@@ -201,6 +201,7 @@ struct pl_sparse_conv_handle {
   size_t float_row_exp = 0;      // where these begin
   int float_mfma = 1;            // 0 never, 1 by the rule, 2 whenever the shape allows
   int float_mfma_rows = 0;       // rows per workgroup; 0 = chosen per problem
+  int float_split = 1;           // fp32 with wavefronts of their own for the inputs: 0 never, 1 by the rule, 2 always
   // block MFMA
   int row_blocks = 0, ksteps = 0, kmask_words = 1;
   int64_t blocks_present = 0;
@@ -1064,7 +1065,7 @@ bool FloatMfmaPays(const pl_sparse_conv_handle* h, int batch, int im_size, bool 
   const double P = static_cast<double>(positions);
   if (h->half && P * h->ic * h->oc <= 4e7) return false;
   const int cus = std::max(1, h->wg_slots_default / 2);
-  return (h->half ? 1.15 : (h->oc <= 64 ? 1.05 : 1.2)) * pl::PlanFloatMfma(!h->half, cus, h->float_mfma_rows / 32, h->ic, h->oc, im_size, batch).us < WalkMicroseconds(h, cus, P, im_size, aligned16);
+  return (h->half ? 1.15 : (h->oc <= 64 ? 1.05 : 1.2)) * pl::PlanFloatMfma(!h->half, cus, h->float_mfma_rows / 32, 0, h->ic, h->oc, im_size, batch).us < WalkMicroseconds(h, cus, P, im_size, aligned16);
 }
 
 // The algorithm of one call (pl_sparse_conv_algo_for reports it).
@@ -1106,7 +1107,7 @@ int pl_sparse_conv_prepare(const pl_sparse_conv_desc* desc, pl_sparse_conv_handl
     return Fail(PL_ERR_BAD_ARG, "pl_sparse_conv_desc size mismatch (%u vs %zu)", desc->struct_size, sizeof(pl_sparse_conv_desc));
   pl_sparse_conv_tuning tune{};
   std::memcpy(&tune, reinterpret_cast<const char*>(desc) + kNoTuning, std::min<size_t>(desc->struct_size - kNoTuning, sizeof(tune)));
-  for (int32_t sw : {tune.mfma_stream, tune.mfma_sub_tiles, tune.walk_tiled, tune.walk_chunked, tune.image_tr_regroup, tune.walk_pairs, tune.chunk_mfma, tune.float_mfma, tune.chunk_split})
+  for (int32_t sw : {tune.mfma_stream, tune.mfma_sub_tiles, tune.walk_tiled, tune.walk_chunked, tune.image_tr_regroup, tune.walk_pairs, tune.chunk_mfma, tune.float_mfma, tune.chunk_split, tune.float_mfma_split})
     if (sw < PL_TUNE_RULE || sw > PL_TUNE_ALWAYS) return Fail(PL_ERR_BAD_ARG, "a tuning switch is not PL_TUNE_RULE, PL_TUNE_NEVER or PL_TUNE_ALWAYS");
   if (tune.chunk_positions != 0 && tune.chunk_positions != 64 && tune.chunk_positions != 128 && tune.chunk_positions != 256) return Fail(PL_ERR_BAD_ARG, "tuning.chunk_positions must be 0, 64, 128 or 256");
   if (tune.float_mfma_rows != 0 && tune.float_mfma_rows != 64 && tune.float_mfma_rows != 128 && tune.float_mfma_rows != 256) return Fail(PL_ERR_BAD_ARG, "tuning.float_mfma_rows must be 0, 64, 128 or 256");
@@ -1162,6 +1163,7 @@ int pl_sparse_conv_prepare(const pl_sparse_conv_desc* desc, pl_sparse_conv_handl
                                 tune.walk_threads != 0 || tune.walk_slices != 0 || tune.walk_pairs != PL_TUNE_RULE;
   h->float_mfma = float_walk_asked && tune.float_mfma != PL_TUNE_ALWAYS ? 0 : sw(tune.float_mfma);
   h->float_mfma_rows = tune.float_mfma_rows;
+  h->float_split = sw(tune.float_mfma_split);
   h->walk_asked = tune.walk_tile != 0 || tune.walk_threads != 0 || tune.walk_slices != 0;
   h->block_asked = tune.mfma_stream != PL_TUNE_RULE || tune.mfma_sub_tiles != PL_TUNE_RULE || tune.mfma_tile_quads != 0 || tune.mfma_narrow_i8_stores != 0 || tune.wg_slots != 0;
   h->image_asked = tune.image_kernel != 0 || tune.image_min_items != 0 || tune.image_tr_regroup != PL_TUNE_RULE;
@@ -1403,7 +1405,7 @@ int pl_sparse_conv_run(pl_sparse_conv_handle* h, const void* x_dev, void* out_de
     p.act = h->act;
     p.act_h_words[0] = h->act_h.alpha | static_cast<uint32_t>(h->act_h.hs_offset) << 16;
     p.act_h_words[1] = h->act_h.hs_inv_scale | static_cast<uint32_t>(h->act_h.hs_threshold) << 16;
-    e = pl::LaunchFloatMfma(!h->half, std::max(1, h->wg_slots_default / 2), h->float_mfma_rows / 32, p, s);
+    e = pl::LaunchFloatMfma(!h->half, std::max(1, h->wg_slots_default / 2), h->float_mfma_rows / 32, h->float_split, p, s);
   } else if (half_tw) {
     const TileWalkDivision d = DivideTileWalk(h, *half_tw, CeilDiv(static_cast<int>(P), half_tile));
     pl::HalfTileWalkParams p{};
@@ -1693,7 +1695,12 @@ int pl_sparse_conv_chunk_form_for(const pl_sparse_conv_handle* h, int32_t batch,
   if (!form) return Fail(PL_ERR_BAD_ARG, "null argument");
   const int algo = pl_sparse_conv_algo_for(h, batch, im_size);
   if (algo < 0) return algo;
-  if (algo != PL_ALGO_CHUNK_MFMA || !h->int8) return Fail(PL_ERR_UNSUPPORTED, "the call is not one of an int8 handle that takes the channels chunk by chunk");
+  if (algo != PL_ALGO_CHUNK_MFMA) return Fail(PL_ERR_UNSUPPORTED, "the call does not take the channels chunk by chunk");
+  if (!h->int8) {
+    const pl::FloatMfmaPlan plan = pl::PlanFloatMfma(!h->half, std::max(1, h->wg_slots_default / 2), h->float_mfma_rows / 32, h->float_split, h->ic, h->oc, im_size, batch);
+    *form = pl_sparse_conv_chunk_form{32 * plan.wr, plan.split ? 64 : 128, plan.split ? 1 : 0};
+    return PL_OK;
+  }
   const pl::ChunkMfmaPlan plan = pl::PlanChunkMfma(OutKind(h->kind), std::max(1, h->wg_slots_default / 2), h->chunk_positions, h->chunk_split, h->ic, h->oc, im_size, batch);
   *form = plan.split ? pl_sparse_conv_chunk_form{256, 128, 1} : pl_sparse_conv_chunk_form{128, 64 * plan.nw, 0};
   return PL_OK;

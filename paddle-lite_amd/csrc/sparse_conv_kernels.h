@@ -293,20 +293,23 @@ constexpr uint32_t kFloatMfmaOutside = 0x80000000u;
 constexpr uint32_t FloatMfmaWeightTile(int chunk, int tile, int pieces, int piece) { return (uint32_t)((chunk * (kFloatMfmaChunk / 16) + tile) * pieces + piece) * 1024u; }
 constexpr uint32_t FloatMfmaWeightTail(int pieces) { return FloatMfmaWeightTile(1, 0, pieces, 0); }
 
-// How a call is divided (workgroups of wr x 32 rows x 128 positions) and what it is expected to take.
+// How a call is divided (workgroups of wr x 32 rows x 128 positions, or 256 rows x 64 positions in the form with wavefronts of its own for
+// the inputs) and what it is expected to take.
 struct FloatMfmaPlan {
+  bool split;  // that form
   int wr;
-  int row_groups;
+  int row_groups, tiles;
   int64_t workgroups;
   double us;
 };
 
 int FloatMfmaPaddedSteps(int K);  // weight tiles of a row block: whole chunks, two per 32 channels
 bool FloatMfmaFits(bool f32, int K, int M, int hw, int64_t positions);
-// row_blocks: blocks of 32 rows per workgroup, 8, 4 or 2; 0 = chosen by the call
-FloatMfmaPlan PlanFloatMfma(bool f32, int cus, int row_blocks, int K, int M, int hw, int batch);
+// row_blocks: blocks of 32 rows per workgroup, 8, 4 or 2; 0 = chosen by the call.  split: fp32 in the form with wavefronts of its own for the
+// inputs: 0 never, 1 where it is expected to be ahead, 2 always
+FloatMfmaPlan PlanFloatMfma(bool f32, int cus, int row_blocks, int split, int K, int M, int hw, int batch);
 // x and out on whole elements
-hipError_t LaunchFloatMfma(bool f32, int cus, int row_blocks, const FloatMfmaParams& p, hipStream_t stream);
+hipError_t LaunchFloatMfma(bool f32, int cus, int row_blocks, int split, const FloatMfmaParams& p, hipStream_t stream);
 
 // Block MFMA SpMM (int8): dense 32x32 weight blocks pre-arranged in operand
 // order, empty blocks skipped through a per-row-block bit mask.

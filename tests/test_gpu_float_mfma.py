@@ -1,5 +1,7 @@
 """fp32 / fp16 sparse_conv2d on the matrix cores (tuning.float_mfma) against the same sums in 64 bits, and the rule that
 gives calls to it."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -11,6 +13,8 @@ AP = pla.ActivationParam
 ACTS = {"none": AP(), "relu": AP("relu"), "relu6": AP("relu6", Relu_clipped_coef=6.0), "leaky": AP("leaky_relu", Leaky_relu_alpha=0.1), "hswish": AP("hard_swish")}
 KINDS = {"fp32": capi.KIND_FP32, "fp16": capi.KIND_FP16}
 ROWS = (64, 128, 256)
+FORMS = ROWS + ("split",)  # of fp32
+KIND_FORMS = [("fp16", rows) for rows in ROWS] + [("fp32", form) for form in FORMS]
 
 
 def make_case(kind, batch, ic, oc, h, w, paired=False, act="none", sparsity=0.75, seed=0):
@@ -21,9 +25,21 @@ def make_case(kind, batch, ic, oc, h, w, paired=False, act="none", sparsity=0.75
     return c
 
 
+def chunk_form(kernel, batch, im_size):
+    """(rows, positions, split) of the call's workgroups."""
+    form = capi.ChunkForm()
+    capi.check(capi.lib().pl_sparse_conv_chunk_form_for(kernel._handle, batch, im_size, C.byref(form)))
+    return form.rows, form.positions, form.split
+
+
 def forced(case, rows, paired=False):
-    kernel = make_kernel(case, force_semi=paired, tuning=capi.tuning(float_mfma=capi.TUNE_ALWAYS, float_mfma_rows=rows))[0]
+    """A kernel that runs the dense product with `rows` rows per workgroup (0: the rule's; "split": wavefronts of their own for the inputs), which
+    the library confirms."""
+    how = dict(float_mfma_split=capi.TUNE_ALWAYS) if rows == "split" else dict(float_mfma_rows=rows)
+    kernel = make_kernel(case, force_semi=paired, tuning=capi.tuning(float_mfma=capi.TUNE_ALWAYS, **how))[0]
     assert capi.lib().pl_sparse_conv_algo_for(kernel._handle, case.batch, case.im_size) == capi.ALGO_CHUNK_MFMA
+    if rows != 0:
+        assert chunk_form(kernel, case.batch, case.im_size) == ((256, 64, 1) if rows == "split" else (rows, 128, 0))
     return kernel
 
 
@@ -76,12 +92,11 @@ def check(case, act, got):
 SHAPES = [(1, 8, 1, 2, 2), (3, 9, 33, 5, 1), (2, 63, 31, 3, 3), (1, 65, 64, 9, 6), (5, 130, 65, 7, 7), (2, 203, 129, 11, 5), (1, 256, 257, 8, 16), (1, 64, 96, 3, 43), (2, 320, 40, 14, 14), (9, 100, 300, 1, 7)]
 
 
-@pytest.mark.parametrize("rows", ROWS)
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("paired", [False, True], ids=["unstructured", "semi"])
-@pytest.mark.parametrize("kind", sorted(KINDS))
+@pytest.mark.parametrize("kind, rows", KIND_FORMS)
 def test_against_64_bits(kind, paired, shape, rows):
-    act = sorted(ACTS)[(sum(shape) + rows // 64) % len(ACTS)]
+    act = sorted(ACTS)[(sum(shape) + (3 if rows == "split" else rows // 64)) % len(ACTS)]
     case = make_case(kind, *shape, paired=paired, act=act)
     check(case, act, run_hip(case, kernel=forced(case, rows, paired)))
 
@@ -97,7 +112,9 @@ SPLIT = [(1, 385, 2100, 2, 2), (3, 390, 2049, 5, 1), (2, 511, 2305, 3, 3), (1, 5
 def test_fp32_wavefronts_of_their_own_for_the_inputs(paired, shape):
     act = sorted(ACTS)[sum(shape) % len(ACTS)]
     case = make_case("fp32", *shape, paired=paired, act=act)
-    check(case, act, run_hip(case, kernel=forced(case, 0, paired)))
+    kernel = forced(case, 0, paired)
+    assert chunk_form(kernel, case.batch, case.im_size) == (256, 64, 1)
+    check(case, act, run_hip(case, kernel=kernel))
 
 
 @pytest.mark.parametrize("how", ["grow", "late", "tails", "binades", "inf", "many nan"])
@@ -121,7 +138,7 @@ def test_fp32_wavefronts_of_their_own_and_hard_inputs(how):
         case.x[0, 3, 2, 1], case.x[1, 449, 8, 6] = np.inf, np.nan
     else:
         case.x[:, 200, :, 1:] = np.nan
-    got = run_hip(case, kernel=forced(case, 0))
+    got = run_hip(case, kernel=forced(case, "split"))
     bad = ~np.isfinite(case.x)
     if bad.any():
         hit = np.matmul(case.dense != 0, bad.reshape(2, 450, -1)).reshape(got.shape)
@@ -134,11 +151,11 @@ def test_fp32_wavefronts_of_their_own_and_hard_inputs(how):
 
 
 def test_fp32_wavefronts_of_their_own_are_as_exact():
-    """2-norm against 64 bits beside the form with 128 rows that these calls would take otherwise: both add two sums of half of the
+    """2-norm against 64 bits beside the form with 128 rows that this call would take otherwise: both add two sums of half of the
     channels, whose errors differ by chance only (5 % is 50 times what the norm of 100 000 outputs' errors scatters by)."""
     case = make_case("fp32", 16, 640, 2100, 5, 5, act="none", sparsity=0.8)
     ref, _ = sums(case)
-    off = [np.linalg.norm((run_hip(case, kernel=forced(case, rows)) - ref).ravel()) for rows in (128, 0)]
+    off = [np.linalg.norm((run_hip(case, kernel=forced(case, rows)) - ref).ravel()) for rows in (128, "split")]
     assert off[1] <= 1.05 * off[0]
 
 
@@ -154,7 +171,7 @@ def test_activations_and_a_new_bias(kind, act):
     check(case, act, run_hip(case, kernel=kernel))
 
 
-@pytest.mark.parametrize("rows", ROWS)
+@pytest.mark.parametrize("rows", FORMS)
 @pytest.mark.parametrize("how", ["images", "late", "grow", "tails", "small", "large"])
 def test_fp32_magnitudes(how, rows):
     """The scales follow the inputs: images of very different size in one tile, positions that begin with a chunk of
@@ -177,7 +194,7 @@ def test_fp32_magnitudes(how, rows):
     check(case, "none", run_hip(case, kernel=forced(case, rows)))
 
 
-@pytest.mark.parametrize("rows", ROWS)
+@pytest.mark.parametrize("rows", FORMS)
 @pytest.mark.parametrize("channels", [[5], [150], [329], list(range(3, 330, 9))], ids=["first", "middle", "last", "many"])
 @pytest.mark.parametrize("size", [1e4, 1e6, 1e8, 1e12, 1e30])
 def test_fp32_large_inputs_stay_with_the_rows_that_read_them(size, channels, rows):
@@ -208,7 +225,7 @@ def test_fp16_large_inputs_stay_with_the_rows_that_read_them(channels, rows):
     check(case, "none", run_hip(case, kernel=forced(case, rows)))
 
 
-@pytest.mark.parametrize("rows", ROWS)
+@pytest.mark.parametrize("rows", FORMS)
 @pytest.mark.parametrize("binades", [24, 60, 230])
 def test_fp32_inputs_of_all_magnitudes(binades, rows):
     """Exponents spread evenly, so every position holds values that its largest one leaves few bits."""
@@ -254,13 +271,12 @@ def test_fp32_error_is_not_above_the_walks():
     case = make_case("fp32", 16, 512, 512, 14, 14, act="none", sparsity=0.85)
     ref, _ = sums(case)
     walk = make_kernel(case, tuning=capi.tuning(float_mfma=capi.TUNE_NEVER))[0]
-    off = [np.linalg.norm((run_hip(case, kernel=k) - ref).ravel()) for k in [walk] + [forced(case, rows) for rows in ROWS]]
+    off = [np.linalg.norm((run_hip(case, kernel=k) - ref).ravel()) for k in [walk] + [forced(case, rows) for rows in FORMS]]
     assert max(off[1:]) <= off[0]
 
 
-@pytest.mark.parametrize("rows", ROWS)
 @pytest.mark.parametrize("paired", [False, True], ids=["unstructured", "semi"])
-@pytest.mark.parametrize("kind", sorted(KINDS))
+@pytest.mark.parametrize("kind, rows", KIND_FORMS)
 def test_infinities_and_nans_reach_only_the_rows_that_read_them(kind, paired, rows):
     """A dense product would spread them through its zero weights.  Partial quads and every part of the channels."""
     case = make_case(kind, 3, 200, 70, 9, 5, paired=paired, act="leaky", sparsity=0.9)
@@ -279,12 +295,12 @@ def test_infinities_and_nans_reach_only_the_rows_that_read_them(kind, paired, ro
 
 
 @pytest.mark.parametrize("paired", [False, True], ids=["unstructured", "semi"])
-@pytest.mark.parametrize("kind", sorted(KINDS))
-def test_every_number_of_quads_to_walk(kind, paired):
+@pytest.mark.parametrize("kind, rows", [("fp16", 128), ("fp32", 128), ("fp32", "split")])
+def test_every_number_of_quads_to_walk(kind, rows, paired):
     """Positions with a NaN from one to all of a tile, partial quads among them: rows with few quads and with many take
     different ways.  The other positions keep the bits of a call without any."""
     case = make_case(kind, 2, 200, 70, 9, 9, paired=paired, act="relu", sparsity=0.8)
-    kernel = forced(case, 128, paired)
+    kernel = forced(case, rows, paired)
     clean = run_hip(case, kernel=kernel)
     reads = case.dense[:, 3] != 0
     if paired:
