@@ -96,9 +96,9 @@ def test_wavefronts_of_their_own_for_the_activations(shape, kind):
 
 
 # (batch, ic, oc, h, w) and the form the rule takes on 256 CUs: the widest tiles with four to eight chunks of 128 channels, on maps larger and
-# smaller than a tile
+# smaller than a tile; calls of one round that the other form would not make shorter
 RULE = [(121, 576, 320, 18, 18, (128, 256, 0)), (107, 420, 112, 18, 18, (128, 256, 0)), (120, 992, 672, 9, 9, (128, 256, 0)), (16, 500, 128, 35, 31, (128, 128, 0)), (16, 2048, 2048, 14, 14, (256, 128, 1)),
-        (60, 900, 384, 13, 13, (256, 128, 1)), (1, 512, 512, 14, 14, (128, 64, 0))]
+        (60, 900, 384, 13, 13, (256, 128, 1)), (1, 512, 512, 14, 14, (128, 64, 0)), (1, 1590, 1406, 40, 40, (128, 128, 0)), (9, 1905, 412, 33, 20, (128, 128, 0))]
 
 
 @pytest.mark.parametrize("kind", ["fp32out", "int8out"])
