@@ -182,6 +182,21 @@ def test_a_kernel_that_a_tuning_field_names_keeps_its_calls():
             assert ALGO_NAMES[capi.check(L.pl_sparse_conv_algo_for(kernel._handle, batch, im_size))] == (other if field else "chunk_mfma"), (other, field)
 
 
+# (batch, ic, oc, h, w, output, kernel)
+BLOCKS = [(666, 424, 105, 16, 16, "fp32out", "block_mfma"), (2064, 357, 105, 8, 8, "fp32out", "block_mfma"), (65, 492, 101, 32, 32, "fp32out", "block_mfma"), (28, 453, 519, 36, 36, "fp32out", "block_mfma"),
+          (28, 640, 1613, 25, 20, "fp32out", "block_mfma"), (155, 522, 865, 20, 20, "fp32out", "block_mfma"), (182, 443, 292, 14, 14, "int8out", "block_mfma"), (28, 640, 1613, 25, 20, "int8out", "chunk_mfma"),
+          (24, 512, 384, 28, 28, "fp32out", "block_mfma"), (12, 512, 384, 28, 28, "fp32out", "chunk_mfma"), (60, 512, 512, 18, 18, "fp32out", "chunk_mfma"), (40, 257, 768, 14, 16, "int8out", "chunk_mfma"), (5, 640, 900, 36, 36, "fp32out", "chunk_mfma"),
+          (30, 422, 1004, 25, 25, "fp32out", "chunk_mfma"), (10, 1344, 896, 28, 28, "fp32out", "chunk_mfma"), (20, 700, 97, 40, 40, "fp32out", "chunk_mfma")]
+
+
+@pytest.mark.parametrize("call", BLOCKS, ids=lambda c: "x".join(map(str, c[:6])))
+def test_the_rule_beside_the_block_kernel(call):
+    """More than 256 channels and 96 rows over many positions, on a device of 256 CUs."""
+    batch, ic, oc, h, w, kind, chosen = call
+    kernel, _ = make_kernel(chunk_case((1, ic, oc, h, w), kind, AP("relu"), False, 3))
+    assert ALGO_NAMES[capi.check(capi.lib().pl_sparse_conv_algo_for(kernel._handle, batch, h * w))] == chosen
+
+
 @pytest.mark.parametrize("batch, oc, chosen", [(32, 1024, "chunk_mfma"), (33, 1024, "image_mfma"), (64, 1024, "image_mfma"), (65, 1024, "chunk_mfma"), (33, 2048, "chunk_mfma"), (171, 384, "chunk_mfma")])
 @pytest.mark.parametrize("out_int8", [False, True], ids=["fp32", "int8"])
 def test_1024_channels_on_maps_of_49_positions(batch, oc, chosen, out_int8):
