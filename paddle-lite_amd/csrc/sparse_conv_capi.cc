@@ -934,12 +934,20 @@ bool ChunkMfmaBeatsImage(const pl_sparse_conv_handle* h, int batch, int im_size,
   const bool slabs = im_size > 256;
   const int64_t images = im_size == 49 ? (batch + 1) / 2 : static_cast<int64_t>(batch) * (slabs ? im_size / 196 : 1);
   const int64_t items = images * (h->oc / 128);
-  // 1024 channels @7x7: the image kernel holds one item per CU, and a second round costs as much as the first; this kernel takes two items at
-  // once (1024 -> 1024 18.7 / 13.4 at 66 images, 20.1 / 15.5 at 128, 26.9 / 23.7 at 130; with one-byte output 0.71 - 0.92).  From a half to one round the
+  // 1024 channels @7x7: the image kernel holds one item per CU, and a second round costs as much as the first.  Beyond one round this kernel's 256 rows x
+  // 128 positions where they make two thirds as many rounds or fewer: of 705 calls of 1.1 to 72 rounds one is 2 % slower, the others 0.70 - 1.01
+  // (1024 -> 1024 18.7 / 13.4 at 66 images, 20.1 / 15.5 at 128, 26.9 / 23.7 at 130); of 69 others 1.09 - 1.37 at two rounds each (1024 -> 1920 x 67 with
+  // one-byte output 17.0 / 22.7), 0.90 - 1.13 at four and three.  From a half to one round the
   // image kernel is ahead (11.5 / 13.6 at 64 images, 1024 -> 384 10.6 / 12.4 at 128), up to a half this one where whole
   // groups of 256 rows are full (1024 -> 256 9.6 / 7.9 at 128, 1024 -> 1024 9.3 / 8.0 at 32; 1024 -> 384 9.3 / 11.8 at 84).
   // With 512 channels and more than one round 0.97 - 1.06, with 256 1.04 - 1.29.
-  if (im_size == 49 && h->ic >= 1024 && (items > cus || (items * 2 <= cus && h->oc % 256 == 0))) return true;
+  if (im_size == 49 && h->ic >= 1024) {
+    if (items * 2 <= cus && h->oc % 256 == 0) return true;
+    if (items > cus) {
+      const pl::ChunkMfmaPlan plan = pl::PlanChunkMfma(OutKind(h->kind), cus, h->chunk_positions, h->chunk_split, h->ic, h->oc, im_size, batch);
+      return plan.split && (plan.workgroups + cus - 1) / cus * 3 <= (items + cus - 1) / cus * 2;
+    }
+  }
   if (h->ic < 512) return im_size >= 196 && items <= 8 && (slabs || batch <= 2);
   return items * 8 < 3 * cus;
 }

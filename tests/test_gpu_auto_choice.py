@@ -45,7 +45,7 @@ def test_auto_is_within_15_percent_on_wide_layers(layer):
 # positions, few of them through the row walk, small maps with 256 channels, channel blocks without weights
 BORDERS = [(64, 520, 96, 56, "fp32"), (32, 520, 2048, 20, "fp32"), (128, 1280, 512, 20, "fp32"), (64, 1536, 2048, 17, "fp32"), (128, 1472, 812, 12, "int8"), (2, 96, 128, 10, "int8"),
            (32, 256, 256, 10, "fp32"), (2, 768, 256, 8, "fp32"), (128, 192, 384, 13, "int8"), (16, 2048, 2048, 14, "fp32"), (64, 192, 384, 17, "fp32"), (16, 600, 600, 12, "fp32"),
-           (65, 492, 101, 32, "fp32"), (68, 360, 327, 28, "fp32"), (181, 581, 267, 24, "fp32"), (24, 512, 384, 28, "fp32")]
+           (65, 492, 101, 32, "fp32"), (68, 360, 327, 28, "fp32"), (181, 581, 267, 24, "fp32"), (24, 512, 384, 28, "fp32"), (67, 1024, 1920, 7, "int8")]
 
 
 @pytest.mark.parametrize("layer", BORDERS, ids=lambda l: "%dx%dx%d_%d_%s" % l)

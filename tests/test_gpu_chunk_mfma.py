@@ -197,10 +197,10 @@ def test_the_rule_beside_the_block_kernel(call):
     assert ALGO_NAMES[capi.check(capi.lib().pl_sparse_conv_algo_for(kernel._handle, batch, h * w))] == chosen
 
 
-@pytest.mark.parametrize("batch, oc, chosen", [(32, 1024, "chunk_mfma"), (33, 1024, "image_mfma"), (64, 1024, "image_mfma"), (65, 1024, "chunk_mfma"), (33, 2048, "chunk_mfma"), (171, 384, "chunk_mfma")])
+@pytest.mark.parametrize("batch, oc, chosen", [(32, 1024, "chunk_mfma"), (33, 1024, "image_mfma"), (64, 1024, "image_mfma"), (65, 1024, "chunk_mfma"), (33, 2048, "chunk_mfma"), (171, 384, "chunk_mfma"), (67, 1920, "image_mfma"), (85, 1408, "image_mfma"), (173, 640, "image_mfma"), (130, 1024, "chunk_mfma")])
 @pytest.mark.parametrize("out_int8", [False, True], ids=["fp32", "int8"])
 def test_1024_channels_on_maps_of_49_positions(batch, oc, chosen, out_int8):
-    """More than one round of the image kernel's items, or at most half of one, on a device of 256 CUs; the same bits as that kernel's."""
+    """More than one round of the image kernel's items and two thirds as many rounds here, or at most half of one, on a device of 256 CUs; the same bits as that kernel's."""
     case = workloads.make_int8("rounds", batch, 1024, oc, 7, 7, 0.9, False, AP(), out_int8=out_int8, seed=batch)
     rule, image = make_kernel(case)[0], make_kernel(case, tuning=capi.tuning(chunk_mfma=capi.TUNE_NEVER))[0]
     assert ALGO_NAMES[capi.check(capi.lib().pl_sparse_conv_algo_for(rule._handle, batch, 49))] == chosen
