@@ -973,16 +973,18 @@ bool ChunkMfmaBeatsBlock(const pl_sparse_conv_handle* h, int batch, int im_size,
   // the block kernel skips blocks of 32 x 32 zeros and this one does not
   const int64_t blocks = static_cast<int64_t>(h->row_blocks) * h->ksteps;
   const bool dense = h->blocks_present * 4 >= blocks * 3;
-  // More than 256 channels and 96 rows on maps of 49 positions and more.  Ragged maps, and channels that leave the block kernel room for one
-  // workgroup per CU: of 760 calls of up to 45 tiles per CU 5 take more than 1.05 times as long as there, 1.14 at most, 0.67 at the median (1344 -> 896
-  // @28x28 x 10 24.7 / 16.9, 422 -> 1004 @25x25 x 30 42.6 / 25.9).  Of the others, which that kernel runs two at a time per CU, those of one round of this
-  // kernel's 256 rows x 128 positions, of two that these fill to two fifths, or of three filled to half; the last not with four-byte
-  // output on maps of a multiple of 16 positions, which fill the block kernel's tiles.  There 3 of 210 take more than 1.05 times as long, 1.10 at most, 0.87 at the median; of the 250 beyond 100 do, to
-  // 1.45, and 1.03 at the median (424 -> 105 @16x16 x 666 30.6 / 41.1, 581 -> 267 @24x24 x 181 50.2 / 62.7, 640 -> 1613 @25x20 x 28 45.7 / 51.6).
+  // More than 256 channels and 96 rows on maps of 49 positions and more.  Ragged maps, with up to 512 channels where 256 rows are taken at a time
+  // (seven calls of three to six tiles per CU where they are not 0.98 - 1.14), and channels that leave the block kernel room for one workgroup per
+  // CU: of 760 calls of up to 45 tiles per CU 5 take more than 1.05 times as long as there, 1.14 at most, 0.67 at the median (1344 -> 896 @28x28
+  // x 10 24.7 / 16.9, 422 -> 1004 @25x25 x 30 42.6 / 25.9).  Of the others, which that kernel runs two at a time per CU, those of one round of this
+  // kernel's 256 rows x 128 positions, of two that these fill to two fifths, or of three filled to half; the last not with four-byte output
+  // on maps of a multiple of 16 positions, which fill the block kernel's tiles.  There 3 of 209 take more than 1.05 times as long, 1.10 at most, 0.87 at
+  // the median; of the 250 beyond 118 do, up to 1.5, 1.04 at the median (424 -> 105 @16x16 x 666 30.6 / 41.1, 581 -> 267 @24x24 x 181 50.2 /
+  // 62.7, 640 -> 1613 @25x20 x 28 45.7 / 51.6).
   if (ic > 256 && oc > 96 && im_size >= 49 && dense) {
-    if (ragged ? ic > 512 || tiles <= 6 * cus : ic > (one_byte ? 512 : 640)) return true;
     const pl::ChunkMfmaPlan plan = pl::PlanChunkMfma(OutKind(h->kind), cus, h->chunk_positions, h->chunk_split, ic, oc, im_size, batch);
     const int64_t rounds = (plan.workgroups + cus - 1) / cus;
+    if (ragged ? ic > 512 || (plan.split && tiles <= 6 * cus) : ic > (one_byte ? 512 : 640)) return true;
     if (!ragged && plan.split && (rounds == 1 || (rounds <= (one_byte || im_size % 16 != 0 ? 3 : 2) && rounds * cus * (256 * 128 / 10) * (rounds == 2 ? 4 : 5) <= positions * oc))) return true;
   }
   if (ic <= 512) {

@@ -186,7 +186,7 @@ def test_a_kernel_that_a_tuning_field_names_keeps_its_calls():
 BLOCKS = [(666, 424, 105, 16, 16, "fp32out", "block_mfma"), (2064, 357, 105, 8, 8, "fp32out", "block_mfma"), (65, 492, 101, 32, 32, "fp32out", "block_mfma"), (28, 453, 519, 36, 36, "fp32out", "block_mfma"),
           (28, 640, 1613, 25, 20, "fp32out", "block_mfma"), (155, 522, 865, 20, 20, "fp32out", "block_mfma"), (182, 443, 292, 14, 14, "int8out", "block_mfma"), (28, 640, 1613, 25, 20, "int8out", "chunk_mfma"),
           (24, 512, 384, 28, 28, "fp32out", "block_mfma"), (12, 512, 384, 28, 28, "fp32out", "chunk_mfma"), (60, 512, 512, 18, 18, "fp32out", "chunk_mfma"), (40, 257, 768, 14, 16, "int8out", "chunk_mfma"), (5, 640, 900, 36, 36, "fp32out", "chunk_mfma"),
-          (30, 422, 1004, 25, 25, "fp32out", "chunk_mfma"), (10, 1344, 896, 28, 28, "fp32out", "chunk_mfma"), (20, 700, 97, 40, 40, "fp32out", "chunk_mfma")]
+          (672, 288, 109, 13, 13, "fp32out", "block_mfma"), (144, 322, 103, 39, 21, "fp32out", "block_mfma"), (30, 422, 1004, 25, 25, "fp32out", "chunk_mfma"), (10, 1344, 896, 28, 28, "fp32out", "chunk_mfma"), (20, 700, 97, 40, 40, "fp32out", "chunk_mfma")]
 
 
 @pytest.mark.parametrize("call", BLOCKS, ids=lambda c: "x".join(map(str, c[:6])))
