@@ -988,7 +988,7 @@ bool ChunkMfmaBeatsBlock(const pl_sparse_conv_handle* h, int batch, int im_size,
     if (!ragged && plan.split && (rounds == 1 || (rounds <= (one_byte || im_size % 16 != 0 ? 3 : 2) && rounds * cus * (256 * 128 / 10) * (rounds == 2 ? 4 : 5) <= positions * oc))) return true;
   }
   if (ic <= 512) {
-    if (!ragged) return tiles * 10 <= 9 * cus;  // 256 -> 64 @56x56 4.4 / 4.6 at 1 image, 512 -> 96 @28x28 10.8 / 8.2 at 32
+    if (!ragged) return tiles * 10 <= 9 * cus;  // 0.61 of the time at the median of 211 calls, 1.02 at most; beyond 1.15 on 172 (256 -> 64 @40x40 x 60 14.6 / 8.3)
     if (tiles <= cus) return true;         // 192 -> 384 @17x17 5.7 / 8.4 at 8 images
     // Up to two tiles per CU: 384 channels 0.76 - 1.02.  Others while rows, not positions, make the tiles many: 192 -> 384
     // @17x17 x 64 0.84, 192 -> 96 @35x35 x 32 1.12; with one-byte output in one round of workgroups: 192 -> 384 @13x13 x 128 (384
@@ -997,28 +997,31 @@ bool ChunkMfmaBeatsBlock(const pl_sparse_conv_handle* h, int batch, int im_size,
     if (ic > 256 && ic <= 384) return true;
     return one_byte ? oc > 16 && workgroups() <= cus : positions <= 150 * cus;
   }
+  // What follows decides calls of up to 96 rows, of maps below 49 positions and of layers with empty blocks, and what the rule above leaves of
+  // maps of whole quads with up to 640 channels and four-byte output.
   // Up to 1024 channels the block kernel holds all of them in LDS, beyond 640 (512 with one-byte output, which stages its
-  // stores there) with room for one workgroup per CU: 768 -> 768 @12x12 7.8 / 19.8 at 16 images, 1024 -> 256 @28x28 x 64 39.1 /
-  // 42.6; 1024 -> 1024 @20x20 x 64 (1600 tiles) with 5 / 30 % of the blocks present 1.34 / 1.2 of its time.
+  // stores there) with room for one workgroup per CU: 739 -> 357 @5x6 x 145 7.7 / 29.7, 694 -> 32 @14x8 x 473 13.8 / 20.5, 794 -> 12 @7x7 x
+  // 1250 35.9 / 29.9, the one of 290 that is more than 1.06 times as long; few of the blocks present over many tiles would gain by now: 704 -> 1648 @29x19
+  // x 35 with 5 % of them 66.8 / 90.0.
   if (ic <= 1024 && ic > (one_byte ? 512 : 640)) return one_byte || h->blocks_present * 2 >= blocks || tiles <= 4 * cus;
   // Two workgroups of the block kernel per CU: with four-byte output it is ahead once there are many tiles, with one-byte output
-  // where many are met by tiles of this kernel that stay empty: 2048 -> 2048 @14x14 x 64 (2048 halves) 87.6 / 96.6, 1472 -> 812
-  // @12x12 x 118 (1652, two fifths empty) 1.5; over 250 calls of 1024 halves and more without that 0.92 at the median, 1.23 at most.
+  // where many are met by tiles of this kernel that stay empty: 1669 -> 25 @12x12 x 3110 (two fifths empty) 228.6 / 212.8; without that
+  // 0.29 - 1.11 on 185 calls, 0.67 at the median.
   const int64_t halves = 2ll * pl::PlanChunkMfma(OutKind(h->kind), cus, 256, 0, ic, oc, im_size, batch).tiles * CeilDiv(oc, 128);
   const bool full = halves * 3 <= tiles * 4;
   if (one_byte) return dense ? full || halves <= 4 * cus : workgroups() <= 3 * cus;
   if (ic <= 640) {
-    // 520 -> 2048 @20x20 x 32 (1600 tiles) 56.1 / 39.4, 600 -> 96 @28x28 x 64 (392) 15.7 / 13.6, 520 -> 1024 @14x14 x 32 (392) 13.2 /
-    // 16.6; half a block of rows is padding for the block kernel: 600 -> 48 @28x28 x 64 0.89
+    // 514 -> 163 @40x40 x 16 (1.6 tiles per CU) 11.4 / 11.9, 619 -> 1123 @14x14 x 235 (12.7) 96.3 / 90.6, 576 -> 1201 @36x36 x 27 with 5 % of the blocks
+    // 70.2 / 50.2, but 550 -> 1993 @4x7 x 637 60.9 / 100.6; taken 0.34 - 1.08 on 59 calls.  Half a block of rows is padding for the block kernel:
+    // 600 -> 48 @28x28 x 64 0.89
     if (ragged) return halves <= 4 * cus || (halves <= 6 * cus && oc <= 48);
     return tiles * 5 <= 7 * cus || (im_size <= 256 && full && dense && tiles <= 3 * cus) || (oc <= 48 && oc % 32 != 0 && tiles <= 4 * cus);
   }
-  // 1536 -> 2048 @13x11 x 128 200 / 139, 1280 -> 512 @20x20 x 128 85.9 / 61.2
+  // taken 0.36 - 0.94 on 68 calls; beyond, 0.57 - 0.95 on 26 since 256 rows come at a time: 1675 -> 21 @31x23 x 471 176.8 / 186.4
   if (ragged) return tiles <= 2 * cus || (halves <= 4 * cus && h->blocks_present * 4 >= blocks);
-  // Small maps whose images fill this kernel's tiles, though not the grid of 64 positions that the block kernel's end on:
-  // 2048 -> 2048 @14x14 x 16 (400 tiles) 24.7 / 31.5, with 10 % of the blocks present 24.8 / 29.0, @10x10 x 64 (800) 0.85, but
-  // @8x8 x 128 1.13.  Elsewhere 1280 -> 256 @28x28 x 32 (392 tiles, 208 workgroups) 1.14, 1325 -> 1243 @22x22 x 11 (420, 240) 0.78,
-  // 2048 -> 256 @28x28 x 64 (784) 0.88.
+  // Small maps whose images fill this kernel's tiles, though not the grid of 64 positions that the block kernel's end on: 0.30 - 0.92 on 52
+  // calls (1505 -> 1095 @4x4 x 61 7.7 / 25.5).  Layers with empty blocks else 0.77 - 1.13 on 21; few rows of many channels over many tiles 0.82 -
+  // 1.11 (1728 -> 83 @26x12 x 176 29.0 / 36.5, 1610 -> 11 @12x12 x 1818 127.1 / 114.4).
   if (tiles * 2 <= 3 * cus || (halves <= 4 * cus && im_size <= 256 && im_size % 64 != 0 && full)) return true;
   if (!dense) return false;
   if (ic > 1920 && oc <= 256 && tiles <= 4 * cus) return true;
