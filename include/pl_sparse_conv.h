@@ -102,7 +102,8 @@ enum {
  * |weight * input| (tested: (6 + ic / 16) 2^-23 of it), whatever else the
  * input holds: outputs that the product cannot give to that, and those that
  * an infinity or a NaN reached through a zero weight, are walked there
- * (a call with many of them takes up to five times as long), and a layer with
+ * (one NaN: up to 2.5 times the call's time, 3 times with tuning.float_mfma_rows;
+ * one in every position: 5 to 20 times), and a layer with
  * a weight below about 2^-28 of its row's largest stays with the walks.
  * pl_sparse_conv_algo_for() reports the choice, these dense products as
  *   PL_ALGO_CHUNK_MFMA (a report only: pl_sparse_conv_desc.algo takes the

@@ -221,19 +221,126 @@ __device__ __forceinline__ void WalkOutputs(const FloatMfmaParams& p, uint64_t w
   }
 }
 
-// The same for wavefronts whose lanes hold 16 quads (n) in four parts (kq): the lane's row i is row first_row + 16 (i / 4) + 4 kq + i % 4.  Where more
-// than half of the lanes have such outputs in their rows i each walks its own, else sixteen lanes walk one row for one quad, four of these at a
-// time.  fp32 16 x 512 -> 512 @14x14 as above, a wavefront walking four times as many rows as there: one NaN 33, one in every
-// position 99 us (rows one after the other by four lanes per quad 139), without any 12.
-__device__ __forceinline__ void WalkOutputs16(const FloatMfmaParams& p, uint32_t walk, int first_row, uint32_t first_quad) {
+// The same for wavefronts whose lanes hold 16 quads (n) in four parts (kq): the lane's row i is row first_row + 16 (i / 4) + 4 kq + i % 4.  Up to
+// kStagedQuads quads of which eight rows and more are walked have their inputs brought to LDS: from memory every nonzero of every row fetches
+// a line of its own for them, and one CU does the work of 256 rows.  Two positions of up to 2048 channels at a time, those without such an output
+// left out.  Eight rows at a time, two by sixteen lanes.
+// Of more quads every lane walks its own rows where more than half of the lanes have such outputs in their rows i, else sixteen lanes walk one row
+// for one quad, four of these at a time.
+// What bounds it: with one quad its inputs and lists on the one CU, with all of them the inputs.  Time with one NaN / one in every position, of that
+// with the form above (119 calls of 400 - 2048 channels that the rule gives to this one): 0.84 / 1.00 at
+// the median, 0.93 / 1.36 at most; with every row's inputs from memory 1.24 / 1.01, 1.63 / 1.48 at most.
+constexpr int kStagedBytes = 16 * 1024, kStagedFirst = 8 * 1024, kStagedQuads = 6;  // of a wavefront; those in the first of its two parts of LDS; quads
+constexpr int kStagedSums = 33 * 8;  // zeros and a wavefront's sums
+__device__ __forceinline__ void WalkOutputs16(const FloatMfmaParams& p, uint32_t walk, int first_row, uint32_t first_quad, const void* part0, const void* part1, const void* part2) {
   const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), n = lane & 15;
   const uint32_t image = (first_quad + (uint32_t)n) / (uint32_t)p.qpi;
   const int position = 4 * (int)(first_quad + (uint32_t)n - image * (uint32_t)p.qpi);
   const uint32_t inside = (uint32_t)min(position, p.hw - 4);
   const uint32_t from_own = image * (uint32_t)p.K * (uint32_t)p.hw + inside, to_own = image * (uint32_t)p.M * (uint32_t)p.hw + inside;
+
+  int rows_of_quad = 0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) rows_of_quad += (walk >> (4 * i) & 15u) != 0;
+  rows_of_quad += __shfl_xor(rows_of_quad, 16);
+  rows_of_quad += __shfl_xor(rows_of_quad, 32);
+  uint32_t staged = (uint32_t)__ballot(rows_of_quad >= 8) & 0xffffu;
+  if (__popc(staged) > kStagedQuads) staged = 0;
+  const uint32_t few = staged >> n & 1u ? 0u : walk;
+  // two positions at a time
+  constexpr int W = 2, CELLS = kStagedBytes / (4 * W), LOADS = 16, BATCH = 8;
+  typedef __attribute__((address_space(3))) v2f lds;
+  const uint32_t base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(part0)), apart = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(part1)) - base - kStagedFirst;
+  auto at_lds = [&](uint32_t i) { return reinterpret_cast<lds*>(base + i * (4u * W) + (i >= kStagedFirst / (4u * W) ? apart : 0u)); };
+  lds* const zeros = reinterpret_cast<lds*>(static_cast<uint32_t>(reinterpret_cast<uintptr_t>(part2)));
+  lds* const sums = zeros + 1;
+  *zeros = v2f{0.0f, 0.0f};
+#pragma unroll 1
+  for (int item = 0; staged != 0; ++item) {
+    const int q = __ffs(staged) - 1, c = W * (item & 1);
+    if ((item & 1) != 0) staged &= staged - 1;
+    if (__ballot(n == q && (walk & 0x33333333u << c) != 0) == 0) continue;
+    const char* const x = static_cast<const char*>(p.x) + ((size_t)(uint32_t)__shfl((int)from_own, q) + (uint32_t)c) * 4;
+    const uint32_t to = (uint32_t)__shfl((int)to_own, q) + (uint32_t)c;
+#pragma unroll 1
+    for (int c0 = 0; c0 < p.K; c0 += CELLS) {
+#pragma unroll 1
+      for (int i = 0; i < CELLS && c0 + i < p.K; i += 64 * LOADS) {
+        v2f v[LOADS];
+#pragma unroll
+        for (int u = 0; u < LOADS; ++u) __builtin_memcpy(&v[u], x + (size_t)min(c0 + i + 64 * u + lane, p.K - 1) * ((uint32_t)p.hw * 4u), 4 * W);
+#pragma unroll
+        for (int u = 0; u < LOADS; ++u) *at_lds(i + 64 * u + lane) = v[u];
+      }
+      const uint32_t present = (uint32_t)min(CELLS, p.K - c0);
+      // lanes read what others wrote; LDS serves a wavefront in order
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+      for (int pass = 0; pass < 4; ++pass) {
+        uint32_t bits[2], first[2], count[2], most = 0;
+        int of[2];
+        float acc[2][W];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const int r = 8 * pass + 2 * (lane >> 4) + j;  // of the wavefront's 32
+          bits[j] = (uint32_t)__shfl((int)walk, q + 16 * (r >> 2 & 3)) >> (4 * (4 * (r >> 4) + (r & 3)) + c) & ((1u << W) - 1u);
+          const int row = bits[j] != 0 ? first_row + r : 0;
+          const DevGroup g = p.groups[p.nr == 2 ? row >> 1 : row];
+          const bool any = bits[j] != 0 && g.count != 0;
+          first[j] = any ? g.first : 0u, count[j] = any ? g.count : 0u, of[j] = any ? row - g.row0 : 0;
+          most = max(most, count[j]);
+          const v2f before = c0 != 0 && n == 0 ? sums[r] : v2f{0.0f, 0.0f};
+#pragma unroll
+          for (int i = 0; i < W; ++i) acc[j][i] = before[i];
+        }
+        for (uint32_t e = (uint32_t)n; e < most; e += BATCH * 16) {
+          uint32_t k[2][BATCH], w[2][BATCH];
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u) {
+              const uint32_t entry = first[j] + min(e + 16u * u, max(count[j], 1u) - 1u);
+              k[j][u] = p.kidx[entry];
+              w[j][u] = p.wts[(size_t)entry * p.nr + of[j]];
+            }
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u) {
+              // zeros for what is not there: channels of another window, what pads the lists
+              const uint32_t at = k[j][u] - (uint32_t)c0;
+              const v2f in = *(e + 16u * u < count[j] && at < present ? at_lds(at) : zeros);
+#pragma unroll
+              for (int i = 0; i < W; ++i) acc[j][i] = __builtin_fmaf(in[i], __uint_as_float(w[j][u]), acc[j][i]);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int i = 0; i < W; ++i)
+#pragma unroll
+            for (int m = 8; m >= 1; m >>= 1) acc[j][i] += __shfl_xor(acc[j][i], m);
+        if (n == 0) {
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const int r = 8 * pass + 2 * (lane >> 4) + j;
+            if (c0 + CELLS < p.K) {
+              sums[r] = v2f{acc[j][0], acc[j][1]};
+            } else if (bits[j] != 0) {
+              const float out[4] = {acc[j][0], acc[j][1]};
+              StoreWalked<true>(p, out, bits[j], first_row + r, to);
+            }
+          }
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
 #pragma unroll 1
   for (int i = 0; i < 8; ++i) {
-    const uint32_t bits = (walk >> (4 * i)) & 15u;
+    const uint32_t bits = (few >> (4 * i)) & 15u;
     uint64_t left = __ballot(bits != 0);
     const int row0 = first_row + 16 * (i >> 2) + (i & 3);
     if (__popcll(left) > 32) {
@@ -995,7 +1102,10 @@ __device__ __forceinline__ void FloatSplitBody(const FloatMfmaParams& p, uint4* 
   }
   // other lanes write these outputs again: what this wavefront has stored must have arrived
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  WalkOutputs16(p, walk, rb * 32, tile_quad0);
+  // the cells are multiplied and the sums that waited are taken: a part of either for every wavefront
+  static_assert(2 * kBuf * 16 == 8 * kStagedFirst && kStagedBytes - kStagedFirst <= 8 * 64 * 16, "LDS of a wavefront");
+  char* const sums = reinterpret_cast<char*>(colmax) + kF32Tables + 8 * 8 * 64 * 16;
+  WalkOutputs16(p, walk, rb * 32, tile_quad0, reinterpret_cast<const char*>(xt) + wave * kStagedFirst, waiting - lane, sums + wave * kStagedSums);
 }
 
 template <bool RAGGED>
@@ -1014,7 +1124,7 @@ hipError_t Launch(const FloatMfmaParams& p, dim3 grid, hipStream_t s) {
 
 hipError_t LaunchSplit(const FloatMfmaParams& p, dim3 grid, hipStream_t s) {
   const dim3 block(kSplitThreads);
-  constexpr size_t lds = 2 * 2 * kSplitCells * 16 + kF32Tables + 8 * 8 * 64 * 16;
+  constexpr size_t lds = 2 * 2 * kSplitCells * 16 + kF32Tables + 8 * 8 * 64 * 16 + 8 * kStagedSums;
   return p.quad_aligned ? LaunchWithHead(FloatSplitKernel<false>, grid, block, lds, s, p) : LaunchWithHead(FloatSplitKernel<true>, grid, block, lds, s, p);
 }
 

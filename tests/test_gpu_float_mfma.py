@@ -356,6 +356,51 @@ def test_time_with_nans(kind):
     assert times[0] <= 4 * clean and times[1] <= 10 * clean, (clean, times)
 
 
+@pytest.mark.parametrize("shape, sparsity, paired", [((1, 1712, 1933, 36, 36), 0.8, False), ((4, 662, 1530, 22, 22), 0.7, False), ((64, 1024, 1024, 7, 7), 0.7, True)], ids=["1712", "662", "1024"])
+def test_time_with_nans_and_wavefronts_of_their_own_for_the_inputs(shape, sparsity, paired):
+    """A call that the rule gives to that form, with one NaN and with one in every position: not above what it would take with 128 rows (0.84
+    - 0.93 and 0.9 - 1.2 times; 1.2 - 1.6 and 1 - 1.5 when every row fetched its inputs from memory)."""
+    import torch
+
+    case = make_case("fp32", *shape, paired=paired, act="none", sparsity=sparsity)
+    kernel, rows = forced(case, 0, paired), forced(case, 128, paired)
+    assert chunk_form(kernel, case.batch, case.im_size) == (256, 64, 1)
+    x = torch.from_numpy(case.x).cuda()
+    one, every = x.clone(), x.clone()
+    one[0, 77, 4, 4] = float("nan")
+    every[:, 77] = float("nan")
+    out = kernel.Run(x)
+    microseconds(kernel, x, out)
+    times = [[microseconds(k, t, out) for t in (x, one, every)] for k in (kernel, rows)]
+    print(", ".join("clean %.1f us, one NaN %.1f, all %.1f" % tuple(t) for t in times))
+    assert times[0][1] <= 1.15 * times[1][1] and times[0][2] <= 1.4 * times[1][2], times
+
+
+@pytest.mark.parametrize("paired", [False, True], ids=["unstructured", "semi"])
+@pytest.mark.parametrize("ic", [450, 1024, 2048, 2049, 2500])
+def test_inputs_of_walked_quads_beside_the_lists(ic, paired):
+    """Few quads with a NaN, whose inputs are brought to LDS up to 2048 channels at a time: every output of theirs that reads none is a sum
+    over the whole row.  Channels at the ends of what is brought at a time, positions in either half of a quad, a partial quad, all rows of
+    some wavefronts and few of the last; rows without nonzeros."""
+    case = make_case("fp32", 2, ic, 300, 7, 9, paired=paired, act="none", sparsity=0.9)
+    case.bias = np.linspace(-1, 1, 300).astype(np.float32)
+    case.dense = np.sign(case.dense) * np.maximum(np.abs(case.dense), np.float32(1e-3))  # a weight far below its row's largest would keep the layer with the walks
+    case.dense[40:44] = 0
+    bad = np.zeros(case.x.shape, bool)
+    for image, c, y, x in ((0, 0, 0, 0), (0, min(ic - 1, 2047), 3, 3), (0, ic - 1, 6, 8), (1, min(ic - 1, 2048), 2, 6), (1, 7, 2, 7), (1, ic // 2, 5, 1)):
+        bad[image, c, y, x] = True
+    case.x[bad] = np.nan
+    got = run_hip(case, kernel=forced(case, "split", paired))
+    reads = case.dense != 0
+    if paired:
+        reads = np.repeat(reads.reshape(-1, 2, ic).any(axis=1), 2, axis=0)  # the walk of a pair of rows multiplies both of its weights
+    hit = np.matmul(reads, bad.reshape(2, ic, -1)).reshape(got.shape)
+    assert np.array_equal(~np.isfinite(got), hit) and hit.any()
+    case.x[bad] = 0
+    ref, mag = sums(case)
+    assert (np.abs(got - ref)[~hit] <= ((6 + ic / 16.0) * 2.0 ** -23 * mag)[~hit]).all()
+
+
 def test_time_with_channels_of_different_size():
     """New scales in every position, but no output that is too small: at most 1.3 times a call without (1.03; with every marked
     quad looked at output by output it was 1.4 and 1.5)."""
