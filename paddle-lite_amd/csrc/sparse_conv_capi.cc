@@ -1073,6 +1073,9 @@ double WalkMicroseconds(const pl_sparse_conv_handle* h, int cus, double position
 // 3070 of 4600 in half precision are taken, 18 and 13 of these are more than 10 % slower than the walk, 830 and 96 others would have
 // gained more than 10 %.  On 2567 and 1980 other calls 15 and 13 are more than 5 % slower, by up to 1.28 and 1.44 times; on
 // average the rule makes fp32 1.10 and half precision 1.49 times as fast.
+// The time is that of the form that will run.  Calls that wavefronts of their own for the inputs bring ahead of the walk, where the form without is
+// not: 184 of 3936 that make one round of its workgroups, 0.80 of the walk's time at the median, 1.06 at most, 0.72 of its error against 64
+// bits; of row pairs 1.35 times, at 1.2 13 of 62 with 90 and 95 % zeros were slower, up to 1.29 times.
 // fp32 layers of at most 64 rows: 1.05 times, by their own times of both.  On 3615 calls 1575 are taken, 48 more than 5 % slower, by up
 // to 1.26 times, and they are 1.21 times as fast on average; by the times for all rows 1646, 156, 1.47 and 1.20.
 bool FloatMfmaPays(const pl_sparse_conv_handle* h, int batch, int im_size, bool aligned16) {
@@ -1085,7 +1088,9 @@ bool FloatMfmaPays(const pl_sparse_conv_handle* h, int batch, int im_size, bool 
   const double P = static_cast<double>(positions);
   if (h->half && P * h->ic * h->oc <= 4e7) return false;
   const int cus = std::max(1, h->wg_slots_default / 2);
-  return (h->half ? 1.15 : (h->oc <= 64 ? 1.05 : 1.2)) * pl::PlanFloatMfma(!h->half, cus, h->float_mfma_rows / 32, 0, h->ic, h->oc, im_size, batch).us < WalkMicroseconds(h, cus, P, im_size, aligned16);
+  const pl::FloatMfmaPlan plan = pl::PlanFloatMfma(!h->half, cus, h->float_mfma_rows / 32, h->float_split, h->ic, h->oc, im_size, batch);
+  const double ahead = h->half ? 1.15 : (h->oc <= 64 ? 1.05 : (plan.split && h->semi ? 1.35 : 1.2));
+  return ahead * plan.us < WalkMicroseconds(h, cus, P, im_size, aligned16);
 }
 
 // The algorithm of one call (pl_sparse_conv_algo_for reports it).

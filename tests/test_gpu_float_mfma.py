@@ -464,6 +464,9 @@ def test_the_rule():
     assert algo(make_case("fp32", 1, 1184, 62, 9, 11, sparsity=0.82), 38, 99)[0] == capi.ALGO_ROW_WALK
     assert algo(make_case("fp32", 1, 800, 64, 33, 33, sparsity=0.88), 7, 1089)[0] == capi.ALGO_ROW_WALK
     assert algo(make_case("fp32", 1, 1624, 40, 8, 8, sparsity=0.76), 10, 2209)[0] == capi.ALGO_CHUNK_MFMA
+    # by the time of the form that runs: 26 us with wavefronts of its own for the inputs, 30 without, 44 as a walk
+    wide = make_case("fp32", 1, 1088, 736, 15, 15, sparsity=0.95)
+    assert algo(wide, 19, 225)[0] == capi.ALGO_CHUNK_MFMA and algo(wide, 19, 225, float_mfma_split=capi.TUNE_NEVER)[0] == capi.ALGO_ROW_WALK
     # few nonzeros per row
     assert algo(make_case("fp32", 1, 96, 192, 8, 8, sparsity=0.9), 1, 3136)[0] == capi.ALGO_ROW_WALK
     assert algo(make_case("fp16", 1, 96, 200, 8, 8, sparsity=0.86), 102, 400)[0] == capi.ALGO_ROW_WALK
