@@ -1991,19 +1991,17 @@ int pl_sparse_conv_dwconv3x3_fits(const pl_sparse_conv_handle* conv, const pl_dw
 
 int pl_sparse_conv_dwconv3x3_pays(const pl_sparse_conv_handle* conv, const pl_dwconv_handle* dw, int32_t batch, int32_t height, int32_t width) {
   if (!pl_sparse_conv_dwconv3x3_fits(conv, dw, height, width) || batch <= 0) return 0;
-  // us, two launches against one, replayed from a graph, at 1 / 4 / 16 / 32 / 64 images @14x14.  Stride 2: 512 -> 512 7.4 / 8.4,
-  // 8.3 / 8.5, 9.4 / 8.5, 10.7 / 8.8, 12.0 / 8.9; 256 -> 512 7.4 / 6.8, 8.0 / 6.9, 8.5 / 6.9, 8.9 / 7.0, 10.3 / 7.4; 128 -> 128 7.2 / 6.0 ...
-  // 7.9 / 6.3.  Stride 1: 512 -> 512 7.5 / 9.0, 8.4 / 9.1, 9.5 / 9.3, 12.7 / 9.8, 16.5 / 10.9; 256 -> 512 7.6 / 7.5, 8.4 / 7.5, 9.3 / 7.7,
-  // 10.9 / 8.0, 14.5 / 8.9.  The one launch does the depthwise work of 128 planes on the CU that made them, whatever the batch;
-  // the depthwise kernel spreads a small batch over the chip.  At stride 2 one launch is kept at any batch: from the Python
-  // classes 256 and 128 channels gain from one image on, and 512 channels (two / one, 1 / 4 / 8 images: 7.5 / 8.2, 8.3 / 8.4, 8.6 / 8.4)
-  // would gain from two launches below six images only.  At stride 1 the answer changes at half the
-  // CUs, as callers have it: from there on the one launch is ahead for every channel count (512 channels are even at about 16 images, and up to
-  // 256 channels gain from few images on, 4 images 0.7 - 0.9 us, 1 image at most 0.7).
-  if (dw->stride == 2) return 1;
+  // us, two launches against one, replayed from a graph, at 1 / 4 / 16 / 32 / 64 images @14x14.  Stride 1: 512 -> 512 7.2 / 8.7, 8.0 / 8.7, 9.0 / 9.0,
+  // 12.3 / 9.3, 13.9 / 9.8; 512 -> 256 7.2 / 8.6, 7.8 / 8.7, 8.4 / 8.8, 9.2 / 8.9, 11.8 / 9.2; 512 -> 1024 7.3 / 8.7, 8.3 / 8.8, 12.3 / 9.2, 14.0 / 9.7, 23.3 /
+  // 18.0; 256 -> 512 7.2 / 7.0, 8.0 / 7.2, 8.8 / 7.3, 10.7 / 7.5, 12.4 / 8.1; 128 -> 128 6.8 / 6.2 ... 8.1 / 6.6.  Stride 2: 512 -> 512 6.8 / 8.1,
+  // 7.5 / 8.1, 8.2 / 8.2, 11.0 / 8.3, 11.6 / 8.5; 256 -> 512 6.8 / 6.5, 7.5 / 6.5, 8.1 / 6.6, 9.2 / 6.7, 10.1 / 6.8; 128 -> 128 6.6 / 5.6 ... 7.4 / 5.9.
+  // The one launch does the depthwise work of 128 planes on the CU that made them, whatever the batch; the depthwise kernel
+  // spreads a small batch over the chip, which is ahead with 512 channels only, up to a workgroup for every fourth CU.  At stride 2 one launch is kept at any
+  // batch, as callers have it: with 512 channels up to fourteen images two would be ahead by at most 1.3 us.
+  if (dw->stride == 2 || conv->ic <= 256) return 1;
   const int64_t workgroups = static_cast<int64_t>(batch) * (conv->oc / 128);
   const int cus = std::max(1, conv->wg_slots_default / 2);
-  return workgroups * 2 >= static_cast<int64_t>(cus) ? 1 : 0;
+  return workgroups * 4 > static_cast<int64_t>(cus) ? 1 : 0;
 }
 
 int pl_sparse_conv_dwconv3x3_run(pl_sparse_conv_handle* conv, pl_dwconv_handle* dw, const void* x_dev, void* out_dev, int32_t batch, int32_t height, int32_t width, void* stream) {
