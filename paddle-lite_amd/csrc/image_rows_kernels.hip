@@ -149,10 +149,11 @@ __device__ __forceinline__ void StoreRow(const v4i (&acc)[4], int i, float sc, f
   }
 }
 
-// LDS of a wavefront behind the image's cells when the depthwise layer follows: its 16 planes of 14 x 14 int8
+// LDS of a wavefront behind the image's cells when the depthwise layer with stride 2 follows: its 16 planes of 14 x 14 int8
 // (16 bytes of slack in front, 48 behind: the rows are read as aligned dwords around them), then the planes of
-// the depthwise output.
-constexpr int kPlaneInBytes = 16 + 16 * 196 + 48, kPlaneBufBytes = kPlaneInBytes + 16 * 196;
+// the depthwise output, 7 x 7.
+constexpr int kPlaneInBytes = 16 + 16 * 196 + 48, kPlaneBufBytes = kPlaneInBytes + 16 * 49;
+constexpr int DwPlaneBytes(int stride) { return stride == 1 ? kWidePlaneBytes : kPlaneBufBytes; }
 
 // The depthwise layer with stride 2 on the wavefront's planes: one output row of one plane per lane and pass (dw_row_item.h),
 // outputs collected plane-major in LDS, then stored: a plane of the tile's row m is channel row0 + 8 m.
@@ -563,7 +564,7 @@ hipError_t LaunchImageRowsMfma(int out_kind, const ImageMfmaParams& p, hipStream
 // The pointwise layer followed by the depthwise 3 x 3 layer on its output, in one launch (14 x 14 maps).
 bool ImageRowsDwFits(int M, int K, int hw, int h, int w, int pad, int stride) {
   if (!ImageRowsMfmaFits(M, K, hw) || hw != 196 || h != 14 || w != 14 || pad != 1 || (stride != 1 && stride != 2)) return false;
-  return 256 + (size_t)(K / 16) * 208 * 16 + (size_t)8 * kPlaneBufBytes <= (size_t)kMaxLdsBytes;
+  return 256 + (size_t)(K / 16) * 208 * 16 + (size_t)8 * DwPlaneBytes(stride) <= (size_t)kMaxLdsBytes;
 }
 
 hipError_t LaunchImageRowsDw(const ImageMfmaParams& p, const DwConvParams& d, int stride, hipStream_t stream) {
@@ -584,7 +585,7 @@ hipError_t LaunchImageRowsDw(const ImageMfmaParams& p, const DwConvParams& d, in
   q.items = (int)items;
   q.per_xcd = (q.items + 7) / 8;
   q.align = 0;
-  const size_t lds = 256 + (size_t)(p.K / 16) * q.kgs * 16 + (size_t)8 * (stride == 1 ? kWidePlaneBytes : kPlaneBufBytes);
+  const size_t lds = 256 + (size_t)(p.K / 16) * q.kgs * 16 + (size_t)8 * DwPlaneBytes(stride);
   const dim3 grid(8u * (uint32_t)q.per_xcd), block(512);
   const int shape = 10 * (p.K / 64) + stride;
   switch (shape) {
