@@ -412,12 +412,12 @@ void pl_dwconv3x3_destroy(pl_dwconv_handle* handle);
 int pl_sparse_conv_dwconv3x3_fits(const pl_sparse_conv_handle* conv, const pl_dwconv_handle* dw,
                                   int32_t h, int32_t w);
 /* 1 when the pair fits and the one launch is expected to be faster than the
- * two at this batch: up to 256 input channels always; with 512 and stride 1
- * when the launch has more workgroups (batch * oc / 128) than a quarter of the
- * device's CUs - the one launch keeps the depthwise work of a workgroup's 128
- * planes on its CU, which loses to the depthwise kernel's spread at small
- * batches.  Always for stride 2, too, where two launches of 512 channels would
- * be up to 1.3 us ahead below that. */
+ * two at this batch: always for stride 2 (with 512 input channels two would be
+ * up to 1.3 us ahead below fifteen images); for stride 1 from four images on,
+ * with 512 input channels when the launch has more workgroups (batch * oc /
+ * 128) than a quarter of the device's CUs - the one launch keeps the depthwise
+ * work of a workgroup's 128 planes on its CU, which loses to the depthwise
+ * kernel's spread at small batches. */
 int pl_sparse_conv_dwconv3x3_pays(const pl_sparse_conv_handle* conv, const pl_dwconv_handle* dw,
                                   int32_t batch, int32_t h, int32_t w);
 int pl_sparse_conv_dwconv3x3_run(pl_sparse_conv_handle* conv, pl_dwconv_handle* dw,

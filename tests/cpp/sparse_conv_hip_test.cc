@@ -1354,7 +1354,7 @@ static void PairLaunches(bool run_on_device) {
       std::vector<char> two_launches(static_cast<const char*>(got->raw_data()), static_cast<const char*>(got->raw_data()) + got->memory_size());
       program.set_pair_launch(true);
       program.Run();
-      // stride 2 pays at any batch, stride 1 only when the launch fills the chip
+      // stride 2 pays at any batch, stride 1 not for two images
       const size_t expect_pairs = (stride == 2 && !second_reader) ? 1 : 0;
       EXPECT(program.pairs_joined_last_enqueue() == expect_pairs);
       EXPECT(got->memory_size() == two_launches.size() && std::memcmp(got->raw_data(), two_launches.data(), two_launches.size()) == 0);

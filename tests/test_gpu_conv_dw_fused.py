@@ -152,7 +152,7 @@ def test_pairs_that_do_not_fit_are_refused():
 
 
 def test_when_the_one_launch_pays():
-    """pl_sparse_conv_dwconv3x3_pays: stride 2 and up to 256 channels at any batch; 512 channels and stride 1 only when the launch
+    """pl_sparse_conv_dwconv3x3_pays: stride 2 at any batch; stride 1 from four images on with up to 256 channels, with 512 only when the launch
     has more workgroups (batch * oc / 128) than a quarter of the device's CUs."""
     L = capi.lib()
     _, conv, dw1, _ = make_pair(1, 512, 512, 1, "relu", "relu", 21)
@@ -165,7 +165,7 @@ def test_when_the_one_launch_pays():
     assert L.pl_sparse_conv_dwconv3x3_pays(conv._handle, dw1._handle, cus // 16, 14, 14) == 0
     assert L.pl_sparse_conv_dwconv3x3_pays(conv._handle, dw1._handle, cus // 8, 14, 14) == 1  # 512 / 128 = 4 workgroups per image: half the CUs
     assert L.pl_sparse_conv_dwconv3x3_pays(conv._handle, dw1._handle, cus // 16 + 1, 14, 14) == 1
-    for ic, oc, batch, pays in ((128, 128, 1, 1), (256, 512, 1, 1), (256, 512, 16, 1), (256, 128, 4, 1), (512, 1024, cus // 32, 0), (512, 1024, cus // 32 + 1, 1), (512, 256, cus // 8, 0), (512, 256, cus // 8 + 1, 1)):
+    for ic, oc, batch, pays in ((128, 128, 3, 0), (128, 128, 4, 1), (256, 512, 2, 0), (256, 512, 16, 1), (256, 128, 4, 1), (512, 1024, cus // 32, 0), (512, 1024, cus // 32 + 1, 1), (512, 256, cus // 8, 0), (512, 256, cus // 8 + 1, 1)):
         _, c, d, _ = make_pair(1, ic, oc, 1, "relu", "relu", 23)
         assert L.pl_sparse_conv_dwconv3x3_pays(c._handle, d._handle, batch, 14, 14) == pays, (ic, oc, batch)
     assert L.pl_sparse_conv_dwconv3x3_pays(conv._handle, dw1._handle, 2 * cus, 14, 14) == 1
