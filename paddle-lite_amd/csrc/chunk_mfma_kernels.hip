@@ -565,11 +565,12 @@ static ChunkMfmaPlan PlanChunkSplit(int K, int M, int hw, int batch) {
 // about 4.4 us and 1.1 us per chunk of 256 channels.  us, the width chosen / this: 2048 -> 2048 @14x14 x 16 22.0 / 19.0, 1024 -> 512 @17x17 x 32
 // 18.4 / 14.5, 900 -> 384 @13x13 x 60 15.5 / 13.0, 1024 -> 2048 @14x14 x 64 51.4 / 46.1; not taken: 192 -> 384 @17x17 x 64 (304
 // workgroups) 12 / 15, 1024 -> 1024 @14x14 x 16 (half the CUs) 11.3 / 12.6, 1500 -> 700 @10x10 x 20 9.5 / 13.6.
-// In place of a single round it must be expected to take less than 0.95 of the time: of 19 calls between that and level 15 were slower, 1.08 times
-// in the middle (1590 -> 1406 @40x40 11.6 / 13.1), of 282 below one.  Over more rounds 5 of 1388 calls, to 1.14 (1169 -> 125 @14x14 x 1583).
+// In place of a single round of 128 positions, which take as many chunks, it must be expected to take less than 0.9 of the time: of 17 calls between that
+// and level 16 were slower, 1.09 times in the middle (1590 -> 1406 @40x40 11.6 / 13.1), in place of 256 positions none of 38 (162 -> 1888 @11x11 x 20
+// 11.1 / 8.6).  Over more rounds 5 of 1388 calls are, to 1.14 (1169 -> 125 @14x14 x 1583).
 static bool SplitPays(int cus, const ChunkMfmaPlan& plan, const ChunkMfmaPlan& split) {
   const int64_t rounds = (plan.workgroups + cus - 1) / cus, others = rounds * (300 + 135 * plan.chunks), own = (split.workgroups + cus - 1) / cus * (440 + 110 * split.chunks);
-  return rounds == 1 ? own * 20 < others * 19 : own < others;
+  return rounds == 1 && plan.nw == 2 ? own * 10 < others * 9 : own < others;
 }
 
 ChunkMfmaPlan PlanChunkMfma(int out_kind, int cus, int tile_positions, int split, int K, int M, int hw, int batch) {

@@ -973,19 +973,32 @@ bool ChunkMfmaBeatsBlock(const pl_sparse_conv_handle* h, int batch, int im_size,
   // the block kernel skips blocks of 32 x 32 zeros and this one does not
   const int64_t blocks = static_cast<int64_t>(h->row_blocks) * h->ksteps;
   const bool dense = h->blocks_present * 4 >= blocks * 3;
-  // More than 256 channels and 96 rows on maps of 49 positions and more.  Ragged maps, with up to 512 channels where 256 rows are taken at a time
-  // (seven calls of three to six tiles per CU where they are not 0.98 - 1.14), and channels that leave the block kernel room for one workgroup per
-  // CU: of 760 calls of up to 45 tiles per CU 5 take more than 1.05 times as long as there, 1.14 at most, 0.67 at the median (1344 -> 896 @28x28
-  // x 10 24.7 / 16.9, 422 -> 1004 @25x25 x 30 42.6 / 25.9).  Of the others, which that kernel runs two at a time per CU, those of one round of this
-  // kernel's 256 rows x 128 positions, of two that these fill to two fifths, or of three filled to half; the last not with four-byte output
-  // on maps of a multiple of 16 positions, which fill the block kernel's tiles.  There 3 of 209 take more than 1.05 times as long, 1.10 at most, 0.87 at
-  // the median; of the 250 beyond 118 do, up to 1.5, 1.04 at the median (424 -> 105 @16x16 x 666 30.6 / 41.1, 581 -> 267 @24x24 x 181 50.2 /
+  // More than 256 channels and 96 rows on maps of 49 positions and more.  Channels that leave the block kernel room for one workgroup per CU, and all
+  // beyond 512 on ragged maps: of 760 calls of up to 45 tiles per CU 5 take more than 1.05 times as long as there, 1.14 at most, 0.67 at the median
+  // (1344 -> 896 @28x28 x 10 24.7 / 16.9).  Of the others, which that kernel runs two at a time per CU:
+  //  * 256 rows x 128 positions at a time: up to six tiles per CU on ragged maps (422 -> 1004 @25x25 x 30 42.6 / 25.9; 0.55 - 0.92 on 26 calls); on maps of
+  //    whole quads two rounds of workgroups, three with one-byte output and on maps of more than 256 positions that are no multiple of 16, which do not
+  //    fill the block kernel's tiles (0.89 at the median of 200 calls, 9 take more than 1.05 times as long, 1.19 at most; a third round elsewhere 1.02);
+  //  * 128 rows at a time on ragged maps: one-byte output up to six tiles per CU (0.7 - 1.29 on 220 calls, 0.9 at the median), four-byte output one
+  //    round of workgroups (0.95), or two of more than three tiles per CU (0.72 - 1.24 on 107 calls, 1.01; with fewer tiles 1.07, beyond two rounds 1.07);
+  //  * 128 rows at a time on maps of whole quads: one round, with four-byte output up to 1.2 tiles per CU and not where the map fills the block kernel's
+  //    tiles but for the last (0.9 at the median; beyond 1.02 - 1.3); with one-byte output two beyond three tiles per CU where the map is
+  //    no multiple of 16 positions (0.95).
+  // Elsewhere 118 of 250 calls take more than 1.05 times as long, up to 1.5 (424 -> 105 @16x16 x 666 30.6 / 41.1, 581 -> 267 @24x24 x 181 50.2 /
   // 62.7, 640 -> 1613 @25x20 x 28 45.7 / 51.6).
   if (ic > 256 && oc > 96 && im_size >= 49 && dense) {
+    if (ic > (ragged || one_byte ? 512 : 640)) return true;
     const pl::ChunkMfmaPlan plan = pl::PlanChunkMfma(OutKind(h->kind), cus, h->chunk_positions, h->chunk_split, ic, oc, im_size, batch);
     const int64_t rounds = (plan.workgroups + cus - 1) / cus;
-    if (ragged ? ic > 512 || (plan.split && tiles <= 6 * cus) : ic > (one_byte ? 512 : 640)) return true;
-    if (!ragged && plan.split && (rounds == 1 || (rounds <= (one_byte || im_size % 16 != 0 ? 3 : 2) && rounds * cus * (256 * 128 / 10) * (rounds == 2 ? 4 : 5) <= positions * oc))) return true;
+    const bool even = im_size % 16 == 0;
+    if (plan.split) {
+      if (ragged ? tiles <= 6 * cus : rounds <= (one_byte || (!even && im_size > 256) ? 3 : 2)) return true;
+    } else if (ragged) {
+      if (one_byte ? tiles <= 6 * cus : rounds == 1 || (rounds == 2 && tiles > 3 * cus)) return true;
+    } else {
+      if (rounds == 1 && (one_byte || (tiles * 5 <= 6 * cus && (!even || im_size <= 256 || im_size % 64 == 0)))) return true;
+      if (rounds == 2 && one_byte && !even && tiles > 3 * cus) return true;
+    }
   }
   if (ic <= 512) {
     if (!ragged) return tiles * 10 <= 9 * cus;  // 0.61 of the time at the median of 211 calls, 1.02 at most; beyond 1.15 on 172 (256 -> 64 @40x40 x 60 14.6 / 8.3)

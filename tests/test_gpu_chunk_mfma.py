@@ -96,9 +96,10 @@ def test_wavefronts_of_their_own_for_the_activations(shape, kind):
 
 
 # (batch, ic, oc, h, w) and the form the rule takes on 256 CUs: the widest tiles with four to eight chunks of 128 channels, on maps larger and
-# smaller than a tile; calls of one round that the other form would not make shorter
+# smaller than a tile; calls of one round that the other form would and would not make shorter
 RULE = [(121, 576, 320, 18, 18, (128, 256, 0)), (107, 420, 112, 18, 18, (128, 256, 0)), (120, 992, 672, 9, 9, (128, 256, 0)), (16, 500, 128, 35, 31, (128, 128, 0)), (16, 2048, 2048, 14, 14, (256, 128, 1)),
-        (60, 900, 384, 13, 13, (256, 128, 1)), (1, 512, 512, 14, 14, (128, 64, 0)), (1, 1590, 1406, 40, 40, (128, 128, 0)), (9, 1905, 412, 33, 20, (128, 128, 0))]
+        (60, 900, 384, 13, 13, (256, 128, 1)), (1, 512, 512, 14, 14, (128, 64, 0)), (1, 1590, 1406, 40, 40, (128, 128, 0)), (9, 1905, 412, 33, 20, (128, 128, 0)),
+        (20, 162, 1888, 11, 11, (256, 128, 1)), (18, 192, 142, 35, 35, (256, 128, 1))]
 
 
 @pytest.mark.parametrize("kind", ["fp32out", "int8out"])
@@ -184,9 +185,9 @@ def test_a_kernel_that_a_tuning_field_names_keeps_its_calls():
 
 # (batch, ic, oc, h, w, output, kernel)
 BLOCKS = [(666, 424, 105, 16, 16, "fp32out", "block_mfma"), (2064, 357, 105, 8, 8, "fp32out", "block_mfma"), (65, 492, 101, 32, 32, "fp32out", "block_mfma"), (28, 453, 519, 36, 36, "fp32out", "block_mfma"),
-          (28, 640, 1613, 25, 20, "fp32out", "block_mfma"), (155, 522, 865, 20, 20, "fp32out", "block_mfma"), (182, 443, 292, 14, 14, "int8out", "block_mfma"), (28, 640, 1613, 25, 20, "int8out", "chunk_mfma"),
+          (28, 640, 1613, 25, 20, "fp32out", "block_mfma"), (155, 522, 865, 20, 20, "fp32out", "block_mfma"), (182, 443, 292, 14, 14, "int8out", "chunk_mfma"), (70, 320, 263, 12, 12, "fp32out", "chunk_mfma"), (28, 640, 1613, 25, 20, "int8out", "chunk_mfma"),
           (24, 512, 384, 28, 28, "fp32out", "block_mfma"), (12, 512, 384, 28, 28, "fp32out", "chunk_mfma"), (60, 512, 512, 18, 18, "fp32out", "chunk_mfma"), (40, 257, 768, 14, 16, "int8out", "chunk_mfma"), (5, 640, 900, 36, 36, "fp32out", "chunk_mfma"),
-          (672, 288, 109, 13, 13, "fp32out", "block_mfma"), (144, 322, 103, 39, 21, "fp32out", "block_mfma"), (30, 422, 1004, 25, 25, "fp32out", "chunk_mfma"), (10, 1344, 896, 28, 28, "fp32out", "chunk_mfma"), (20, 700, 97, 40, 40, "fp32out", "chunk_mfma")]
+          (18, 352, 1152, 27, 27, "fp32out", "chunk_mfma"), (36, 320, 700, 30, 30, "fp32out", "block_mfma"), (12, 416, 876, 37, 37, "fp32out", "chunk_mfma"), (30, 422, 1004, 25, 25, "fp32out", "chunk_mfma"), (10, 1344, 896, 28, 28, "fp32out", "chunk_mfma"), (20, 700, 97, 40, 40, "fp32out", "chunk_mfma")]
 
 
 @pytest.mark.parametrize("call", BLOCKS, ids=lambda c: "x".join(map(str, c[:6])))
