@@ -773,7 +773,7 @@ __global__ void __launch_bounds__(kThreads, F32 ? 2 : 4) FloatMfmaKernel(PL_HEAD
 // with all positions (16 x 16 x 32 matrix instructions: half of the sums' registers of FloatMfmaBody's wavefronts, which three wavefronts
 // per SIMD leave).  Four turn inputs into operand cells: a thread loads eight channels of a position quad, two chunks ahead of the one that
 // it writes, so the conversions, eleven instructions per pair of values, run beside the multiplies instead of between them.  us per call among
-// others, FloatMfmaBody / this: 64 x 1024 -> 1024 @7x7, row pairs, 70 % zeros 26.9 / 22.5; 32 x 512 -> 512 @14x14 16.1 / 14.8; 4 x 1248 -> 1024
+// others, FloatMfmaBody / this: 64 x 1024 -> 1024 @7x7, row pairs, 70 % zeros 26.7 / 23.0; 32 x 512 -> 512 @14x14 16.1 / 14.8; 4 x 1248 -> 1024
 // @29x29 30.7 / 25.4.  With 128 rows x 128 positions, 64 channels a chunk, the first takes 25.3 (every input converted twice as
 // often).  What bounds it: nothing alone; 2.2 us a chunk, of which its matrix instructions take 1.4 at the rate they reach on such data
 // (32 x 32 x 16 ones 1.7: 18 ns against twice 7.7 for half the products) and its 80 KB 0.6.
